@@ -4,29 +4,22 @@
 // Only entries (b,v) with reps > 0, G != 0 and mask[b,I] != 0 carry gradient
 // (g' = G*exp(-reps)*mask[b,I]). The reference scatters them with fp32 atomics into
 // zero-filled dH/dW/dbias (src/sparton/sparton_kernel.py:473-565, :676-678). Here
-// every output row is produced by exactly one wave and summed in a fixed order:
+// every output row is summed in a fixed order by one workgroup:
 //
-//   dW / dbias  (bwd_dw_kernel)   row v gathers H[b, I[b,v], :] for b ascending.
-//   dH          (count -> scan -> scatter -> bwd_dh_kernel)
-//       1. count:   per (b, wave chunk of CHW vocab ids), active entries per s,
-//                   stored as hist[b][chunk][s]; the active entries (v, g') are also
-//                   compacted, in v order, into the chunk's slice of the workspace.
-//       2. scan:    per b, the exclusive scan of hist[b] in (s, chunk) order -> each
-//                   (b,s) segment start and each chunk's first slot inside it (one
-//                   thread per s sums its chunks; a block scan over s gives the bases).
-//       3. scatter: per (b, chunk), write its compacted entries to their slots, ranked
-//                   among equal s with one ballot per bit of s, so each segment lists
-//                   its vocab ids in ascending order (a stable counting sort).
-//       4. dh:      one wave per (b,s) row sums g' * W[v,:] over its segment,
-//                   gathering several W rows per batch before accumulating.
-//   dW / dbias for B <= 128 and S <= 65536 (bwd_dw_staged_kernel): a workgroup stages g'
-//   and I of all batch rows for 64 consecutive vocab ids in LDS (coalesced loads), then
-//   each wave gathers the H rows of one id at a time.
-//   The fused path (B <= 128, S <= 1024, V <= 65536; configs 2 and 3) is two launches:
-//   bwd_compact_kernel lists each (b, 64-id block)'s active entries sorted by 16-row
-//   range, and bwd_fused_kernel runs the dH workgroups (one per (b, 8 rows), which
-//   gather the entries of their rows from every block) and the staged dW workgroups
-//   side by side.
+//   dW / dbias  row v gathers H[b, I[b,v], :] for b ascending. For B <= 128 and S <= 65536 a
+//               workgroup stages g' and I of all batch rows for 32 consecutive ids in LDS
+//               (coalesced loads) and its waves gather the H rows of one id at a time;
+//               bwd_dw_wide_kernel and bwd_dw_kernel take larger batches.
+//   dH          bucket_run sorts each batch row's entries by position, at most 16 runs of
+//               consecutive ids per batch row; then bwd_dh_kernel's 16-lane groups sum
+//               g' * W[v,:] over a row's entries, run by run, ids ascending.
+//
+// The bucketing and the staged dW share a launch (neither needs the other), so a backward is
+// two launches. At most 64 dH rows take the few-row path instead.
+// Measured against the kernels it replaced, which sorted by 64-id blocks and gave each dH row
+// one wave, 4 rows of W in flight (backward kernels, one box): dense gradients, 16 x 256 rows
+// bf16 into fp32 341 -> 187 us, 8 x 128 rows fp32 557 -> 161 us; 5% dense, 32 x 256 rows
+// 47 -> 48 us, 8 x 512 rows 23 -> 24 us, V = 250002 337 -> 298 us, D = 4096 515 -> 438 us.
 // The only atomics are integer counts in LDS, which are order-independent.
 //
 // Gradients are written as fp32 (what the reference returns) or in the input dtype
@@ -36,6 +29,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "sparton_common.h"
 
 extern __shared__ __attribute__((aligned(16))) unsigned char sparton_bwd_smem[];
@@ -43,50 +38,53 @@ extern __shared__ __attribute__((aligned(16))) unsigned char sparton_bwd_smem[];
 namespace sparton {
 namespace bwd {
 
-constexpr int CHW = 1024;          // vocab ids per wave chunk (16 rounds of 64 lanes)
-constexpr int ROUNDS = CHW / 64;
-constexpr int MAX_S = 16384;       // positions per dH window (LDS: S mask floats + S counters per wave)
-constexpr int MAX_B = 8192;        // batch rows per dH chunk
-constexpr int MAX_NP = 16;         // D up to 16 * 256 per register pass
+constexpr int BK_WAVES = 8;         // waves of a bucketing or dW workgroup
+constexpr int BK_ROUNDS = 8;        // rounds of 64 ids whose loads a bucketing wave has in flight
+constexpr int BK_IDS = 64 * BK_ROUNDS * BK_WAVES;  // ids of a workgroup's turn
+constexpr int BK_RUNS = 16;         // bucketing workgroups (runs) per batch row, at most
+constexpr int MAX_S = 4096;         // positions per dH window (LDS: S counters per wave)
+constexpr int64_t MAX_ROWS = 1 << 20;  // dH rows per pass (bounds the run offsets)
+constexpr int MAX_NP = 16;          // D up to 16 * 256 per register pass
+
+// How a batch row's ids are cut: `runs` runs of `cap` ids (a multiple of BK_IDS).
+struct Cut {
+  int64_t runs, cap;
+};
+static Cut cut_ids(int64_t V) {
+  Cut c;
+  c.cap = BK_IDS * std::max<int64_t>(1, cdiv(V, (int64_t)BK_IDS * BK_RUNS));
+  c.runs = std::max<int64_t>(1, cdiv(V, c.cap));
+  return c;
+}
 
 struct Layout {
-  int64_t nch;
-  size_t hist, seg_start, seg_cnt, list, comp, ccount, cnt64, off64, hot, total;  // hist: [B][nch][S] int32
+  size_t off, run, total;
 };
-
 static Layout layout(int64_t B, int64_t S, int64_t V) {
+  const Cut c = cut_ids(V);
   Layout L;
-  L.nch = cdiv(V, CHW);
-  size_t off = 0;
-  auto take = [&](size_t bytes) { size_t o = off; off += (size_t)round_up((int64_t)bytes, 256); return o; };
-  L.hist = take((size_t)(B * L.nch * S) * 4);
-  L.seg_start = take((size_t)(B * S) * 4);
-  L.seg_cnt = take((size_t)(B * S) * 4);
-  // [B][V] segment lists; the fused path keeps [B][V/64][64] compacted entries here
-  L.list = take((size_t)(B * round_up(V, 64)) * 8);
-  L.comp = take((size_t)(B * L.nch * CHW) * 8);  // [B][nch][CHW] active (v, g') per chunk
-  L.ccount = take((size_t)(B * L.nch) * 4);      // [B][nch] their number
-  L.hot = take((size_t)(B * S + 1) * 4);          // [0]: hot rows; [1 ..]: their (b * S + s)
-  L.cnt64 = take((size_t)(B * cdiv(V, 64)) * 4);  // fused path: [B][V/64] entries per block
-  L.off64 = take((size_t)(B * cdiv(V, 64) * cdiv(std::min<int64_t>(S, 1024), 16)) * 4);  // and per row range
-  L.total = off;
+  size_t at = 0;
+  auto take = [&](size_t bytes) { size_t o = at; at += (size_t)round_up((int64_t)bytes, 256); return o; };
+  L.off = take((size_t)(B * (S + 1) * c.runs) * 4);  // [B][S + 1][runs] a position's first entry
+  L.run = take((size_t)(B * c.runs * c.cap) * 8);    // [B][runs][cap] (v, g'), by position, then v
+  L.total = at;
   return L;
 }
 
-// The workspace of one dH pass (at most MAX_B batch rows x MAX_S positions); the fused
-// path's layout (B <= DW_STAGE_B, S <= FUSE_MAX_S) is the same.
-static Layout pass_layout(int64_t B, int64_t S, int64_t V) {
-  return layout(std::min<int64_t>(B, MAX_B), std::min<int64_t>(S, MAX_S), V);
+// Batch rows and positions of one dH pass.
+static int64_t pass_s(int64_t S) { return std::min<int64_t>(S, MAX_S); }
+static int64_t pass_b(int64_t B, int64_t S) {
+  return std::min<int64_t>(B, std::max<int64_t>(1, MAX_ROWS / std::max<int64_t>(1, pass_s(S))));
 }
 
-// Waves per block of the count/scatter kernels: LDS holds S mask floats plus S
-// counters per wave (at most 40 KB with 4 waves, 128 KB with one wave at MAX_S).
-static int waves_for(int64_t S) { return S <= 2048 ? 4 : 1; }
-
-// Stage the S mask entries from element `off` on as floats in LDS.
-__device__ __forceinline__ void stage_mask(float* maskf, const void* mask, int mdt, int64_t off,
-                                           int S) {
-  for (int s = threadIdx.x; s < S; s += blockDim.x) maskf[s] = load_mask(mask, mdt, off + s);
+static int64_t mask_elem_bytes(int mdt) {
+  switch (mdt) {
+    case SPARTON_MASK_I64: return 8;
+    case SPARTON_MASK_I32:
+    case SPARTON_MASK_F32: return 4;
+    case SPARTON_MASK_U8: return 1;
+    default: return 2;
+  }
 }
 
 // Entry (b, v): whether it carries gradient, its coefficient g' and index s.
@@ -109,121 +107,82 @@ __device__ __forceinline__ bool entry(T g_raw, RT r_raw, int s, const float* mas
   return true;
 }
 
-// This wave's chunk of row b: round j, lane l holds entry v = base + j*64 + l, so every
-// load instruction reads consecutive elements. All 3 * ROUNDS loads are issued up front
-// and unconditionally (ids past V re-read id V-1 and are marked inactive): no value is
-// converted or tested until every load is in flight, so they overlap instead of each
-// waiting for the previous one.
+// ---- 1. bucketing --------------------------------------------------------------
+//
+// The active entries of each batch row are sorted by position, ids ascending, a run of
+// consecutive ids at a time: workgroup (b, c) takes run c (at most BK_RUNS of them, so that
+// a 16-lane group can look at all runs of its row at once), wave w of it a contiguous share.
+// It counts the share's entries per (wave, position) in LDS, a scan over (position, wave)
+// turns the counts into slots, and each entry goes to its slot, ranked among the equal
+// positions of its 64: a stable counting sort. off[b][s][c] is the run's first entry of
+// position s. One launch and no exchange between workgroups; dW's workgroups share the
+// launch (dW reads only the inputs) and hide it.
+//
+// A share is taken BK_ROUNDS rounds of 64 ids at a time: their 3 * BK_ROUNDS loads are issued
+// up front and unconditionally (ids past V re-read id V - 1 and are inactive), no value
+// converted or tested until all are in flight. A share of one turn (V <= 65536) keeps its
+// entries in registers between counting and writing; longer ones read them again.
 template <typename T, typename RT>
-struct ChunkData {
-  T g[ROUNDS];
-  RT r[ROUNDS];
-  int s[ROUNDS];
-  __device__ __forceinline__ void load(const T* grad, const RT* reps, const int32_t* idx,
-                                       int64_t row, int base, int V, int lane) {
+__device__ __forceinline__ void bucket_run(const T* __restrict__ grad, const RT* __restrict__ reps,
+                                           const int32_t* __restrict__ idx,
+                                           const void* __restrict__ mask, int mdt, int S, int V,
+                                           int64_t b, int c, int runs, int cap, int* __restrict__ off,
+                                           int2* __restrict__ run, int s0, int S_row) {
+  constexpr int NT = 64 * BK_WAVES;
+  int* wsum = (int*)sparton_bwd_smem;  // [BK_WAVES]
+  int* carry = wsum + BK_WAVES;
+  float* maskf = (float*)(carry + 1);  // [S]
+  int* all = (int*)(maskf + S);        // [BK_WAVES][S]
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int* cur = all + wave * S;
+  const int share = cap / BK_WAVES, v_beg = c * cap + wave * share;
+  const int turns = share / (64 * BK_ROUNDS);
+  float g[BK_ROUNDS];
+  int s[BK_ROUNDS];  // position in the window, -1: inactive
+  T gr[BK_ROUNDS];
+  RT rr[BK_ROUNDS];
+  auto load = [&](int t) {
 #pragma unroll
-    for (int j = 0; j < ROUNDS; ++j) {
-      const int64_t o = row + min(base + j * 64 + lane, V - 1);
-      g[j] = grad[o];
-      r[j] = reps[o];
+    for (int j = 0; j < BK_ROUNDS; ++j) {
+      const int64_t o = b * V + max(0, min(v_beg + (t * BK_ROUNDS + j) * 64 + lane, V - 1));
+      gr[j] = grad[o];
+      rr[j] = reps[o];
       s[j] = idx[o];
     }
-  }
-  // Entry j of this lane (v = base + j*64 + lane): active, with coefficient *g.
-  __device__ __forceinline__ bool get(int j, int base, int V, int lane, const float* maskf,
-                                      int S, float* gout) const {
-    if (base + j * 64 + lane >= V) {
-      *gout = 0.0f;
-      return false;
+  };
+  auto decide = [&](int t) {
+#pragma unroll
+    for (int j = 0; j < BK_ROUNDS; ++j) {
+      // Positions relative to the window (wrapping: an index outside it lands outside [0, S)
+      // and the entry is inactive).
+      const int sw = (int)((unsigned)s[j] - (unsigned)s0);
+      const bool act = v_beg + (t * BK_ROUNDS + j) * 64 + lane < V && entry(gr[j], rr[j], sw, maskf, S, &g[j]);
+      s[j] = act ? sw : -1;
     }
-    return entry(g[j], r[j], s[j], maskf, S, gout);
-  }
-};
-
-// ---- 1. count ----------------------------------------------------------------
-template <typename T, typename RT>
-__global__ __launch_bounds__(256) void bwd_count_kernel(
-    const T* __restrict__ grad, const RT* __restrict__ reps, const int32_t* __restrict__ idx,
-    const void* __restrict__ mask, int mdt, int S, int V, int nch, int* __restrict__ hist,
-    int2* __restrict__ comp, int* __restrict__ ccount, int s0, int64_t mrow0, int S_row,
-    int* __restrict__ hot) {
-  float* maskf = (float*)sparton_bwd_smem;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) hot[0] = 0;  // the scan lists them
-  const int wpb = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  int* h = (int*)(maskf + S) + wave * S;
-  const int b = blockIdx.y, c = blockIdx.x * wpb + wave;
-  stage_mask(maskf, mask, mdt, (mrow0 + b) * S_row + s0, S);
-  for (int s = lane; s < S; s += 64) h[s] = 0;
+  };
+  if (V > 0) load(0);
+  for (int i = tid; i < S; i += NT) maskf[i] = load_mask(mask, mdt, b * S_row + s0 + i);
+  for (int i = tid; i < BK_WAVES * S; i += NT) all[i] = 0;
+  if (tid == 0) *carry = 0;
   __syncthreads();
-  if (c < nch) {
-    ChunkData<T, RT> d;
-    d.load(grad, reps, idx, (int64_t)b * V, c * CHW, V, lane);
-    // Positions relative to the window (wrapping: an index outside it lands outside
-    // [0, S) and the entry is inactive).
+  for (int t = 0; t < turns && V > 0; ++t) {
+    if (t > 0) load(t);
+    decide(t);
 #pragma unroll
-    for (int j = 0; j < ROUNDS; ++j) d.s[j] = (int)((unsigned)d.s[j] - (unsigned)s0);
-    // Active entries are also compacted, in v order, into the chunk's slice of comp.
-    int2* cb = comp + ((int64_t)b * nch + c) * CHW;
-    const uint64_t lt = (1ull << lane) - 1ull;
-    int n = 0;
-#pragma unroll
-    for (int j = 0; j < ROUNDS; ++j) {
-      float g;
-      const bool act = d.get(j, c * CHW, V, lane, maskf, S, &g);
-      const uint64_t am = __ballot(act);
-      if (act) {
-        atomicAdd(&h[d.s[j]], 1);
-        cb[n + __popcll(am & lt)] = make_int2(c * CHW + j * 64 + lane, __float_as_int(g));
-      }
-      n += __popcll(am);
-    }
-    if (lane == 0) ccount[(int64_t)b * nch + c] = n;
+    for (int j = 0; j < BK_ROUNDS; ++j)
+      if (s[j] >= 0) atomicAdd(&cur[s[j]], 1);
   }
   __syncthreads();
-  if (c < nch) {
-    int* out = hist + ((int64_t)b * nch + c) * S;
-    for (int s = lane; s < S; s += 64) out[s] = h[s];
-  }
-}
-
-// ---- 2. scan -----------------------------------------------------------------
-constexpr int SCAN_THREADS = 1024;
-constexpr int SCAN_BATCH = 8;  // chunk counts loaded together
-
-// One workgroup per batch row, threads over s: thread s sums its chunks' counts
-// hist[b][c][s] (coalesced across threads), a block scan over s gives the segment
-// starts, and a second pass rewrites each count as its chunk's first slot.
-// Both scans also list the rows with more than hot_min entries (hot[0] counts them, set
-// to 0 by the count kernel; integer atomics, so only the list's order varies).
-__device__ __forceinline__ void list_hot_row(int* hot, int hot_min, int64_t row, int cnt) {
-  if (cnt > hot_min) hot[1 + atomicAdd(&hot[0], 1)] = (int)row;
-}
-
-__global__ __launch_bounds__(SCAN_THREADS) void bwd_scan_kernel(int* __restrict__ hist,
-                                                                int* __restrict__ seg_start,
-                                                                int* __restrict__ seg_cnt, int S,
-                                                                int nch, int* __restrict__ hot,
-                                                                int hot_min) {
-  __shared__ int wsum[SCAN_THREADS / 64];
-  __shared__ int carry;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t b = blockIdx.x;
-  int* hb = hist + b * nch * S;
-  if (tid == 0) carry = 0;
-  __syncthreads();
-  for (int s0 = 0; s0 < S; s0 += blockDim.x) {
-    const int s = s0 + tid;
-    const bool in = s < S;
-    int tot = 0;
-    for (int c0 = 0; c0 < nch; c0 += SCAN_BATCH) {
-      int x[SCAN_BATCH];
+  int* ob = off + b * (S + 1) * runs + c;
+  for (int p0 = 0; p0 < S; p0 += NT) {
+    const int p = p0 + tid;
+    int k[BK_WAVES], tot = 0;
 #pragma unroll
-      for (int i = 0; i < SCAN_BATCH; ++i)
-        x[i] = (in && c0 + i < nch) ? hb[(int64_t)(c0 + i) * S + s] : 0;
-#pragma unroll
-      for (int i = 0; i < SCAN_BATCH; ++i) tot += x[i];
+    for (int w = 0; w < BK_WAVES; ++w) {
+      k[w] = p < S ? all[w * S + p] : 0;
+      tot += k[w];
     }
-    int incl = tot;  // inclusive scan over s: within the wave, then across waves
+    int incl = tot;  // inclusive scan over p: within the wave, then across waves
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const int y = __shfl_up(incl, d);
@@ -231,148 +190,49 @@ __global__ __launch_bounds__(SCAN_THREADS) void bwd_scan_kernel(int* __restrict_
     }
     if (lane == 63) wsum[wave] = incl;
     __syncthreads();
-    int run = carry + incl - tot;
-    for (int w = 0; w < wave; ++w) run += wsum[w];
-    if (in) {
-      seg_start[b * S + s] = run;
-      seg_cnt[b * S + s] = tot;
-      list_hot_row(hot, hot_min, b * S + s, tot);
-    }
-    for (int c0 = 0; c0 < nch; c0 += SCAN_BATCH) {
-      int x[SCAN_BATCH];
+    int at = *carry + incl - tot;
+    for (int w = 0; w < wave; ++w) at += wsum[w];
+    if (p < S) {
+      ob[(int64_t)p * runs] = at;
+      if (p == S - 1) ob[(int64_t)S * runs] = at + tot;
+      int slot = at;
 #pragma unroll
-      for (int i = 0; i < SCAN_BATCH; ++i)
-        x[i] = (in && c0 + i < nch) ? hb[(int64_t)(c0 + i) * S + s] : 0;
-#pragma unroll
-      for (int i = 0; i < SCAN_BATCH; ++i) {
-        if (in && c0 + i < nch) hb[(int64_t)(c0 + i) * S + s] = run;
-        run += x[i];
+      for (int w = 0; w < BK_WAVES; ++w) {
+        all[w * S + p] = slot;
+        slot += k[w];
       }
     }
     __syncthreads();
-    if (tid == (int)blockDim.x - 1) carry = run;
+    if (tid == NT - 1) *carry = at + tot;
     __syncthreads();
   }
-}
-
-// S <= 512: one workgroup of SCAN_THREADS per batch row, as P = floor(SCAN_THREADS / Sr)
-// parts of Sr = round_up(S, 64) positions (the remaining threads idle); part p sums and rewrites chunks [p n / P, (p + 1) n / P)
-// of every position, so every thread works instead of S of them. Part 0 scans the
-// positions' totals; each part then starts its chunks at the position's segment start
-// plus the counts of the parts before it (integer sums: the same offsets as above).
-__global__ __launch_bounds__(SCAN_THREADS) void bwd_scan_parts_kernel(int* __restrict__ hist,
-                                                                      int* __restrict__ seg_start,
-                                                                      int* __restrict__ seg_cnt,
-                                                                      int S, int nch, int Sr,
-                                                                      int* __restrict__ hot,
-                                                                      int hot_min) {
-  __shared__ int ptot[SCAN_THREADS];
-  __shared__ int base[SCAN_THREADS];
-  __shared__ int wsum[SCAN_THREADS / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int P = SCAN_THREADS / Sr;            // Sr need not divide SCAN_THREADS:
-  const int part = tid / Sr, s = tid - part * Sr;
-  const bool in = s < S && part < P;          // threads past P * Sr take no chunks
-  const int c_beg = part < P ? (int)((int64_t)nch * part / P) : 0;
-  const int c_end = part < P ? (int)((int64_t)nch * (part + 1) / P) : 0;
-  const int64_t b = blockIdx.x;
-  int* hb = hist + b * nch * S;
-  int tot = 0;
-  for (int c0 = c_beg; c0 < c_end; c0 += SCAN_BATCH) {
-    int x[SCAN_BATCH];
-#pragma unroll
-    for (int i = 0; i < SCAN_BATCH; ++i)
-      x[i] = (in && c0 + i < c_end) ? hb[(int64_t)(c0 + i) * S + s] : 0;
-#pragma unroll
-    for (int i = 0; i < SCAN_BATCH; ++i) tot += x[i];
-  }
-  ptot[tid] = tot;
-  __syncthreads();
-  int t = 0, incl = 0;
-  if (part == 0) {  // waves 0 .. Sr/64 - 1: the positions' totals and their inclusive scan
-    for (int q = 0; q < P; ++q) t += ptot[q * Sr + s];
-    incl = t;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int y = __shfl_up(incl, d);
-      if (lane >= d) incl += y;
-    }
-    if (lane == 63) wsum[wave] = incl;
-  }
-  __syncthreads();
-  if (part == 0) {
-    int run = incl - t;
-    for (int w = 0; w < wave; ++w) run += wsum[w];
-    if (in) {
-      seg_start[b * S + s] = run;
-      seg_cnt[b * S + s] = t;
-      list_hot_row(hot, hot_min, b * S + s, t);
-    }
-    base[s] = run;
-  }
-  __syncthreads();
-  int off = base[s];
-  for (int q = 0; q < part; ++q) off += ptot[q * Sr + s];
-  for (int c0 = c_beg; c0 < c_end; c0 += SCAN_BATCH) {
-    int x[SCAN_BATCH];
-#pragma unroll
-    for (int i = 0; i < SCAN_BATCH; ++i)
-      x[i] = (in && c0 + i < c_end) ? hb[(int64_t)(c0 + i) * S + s] : 0;
-#pragma unroll
-    for (int i = 0; i < SCAN_BATCH; ++i) {
-      if (in && c0 + i < c_end) hb[(int64_t)(c0 + i) * S + s] = off;
-      off += x[i];
-    }
-  }
-}
-
-// ---- 3. scatter ----------------------------------------------------------------
-// One wave per chunk: its compacted entries (in v order) are ranked among equal s and
-// written to their segments. Lanes with equal s are found with one ballot per bit of
-// s: `same` keeps the lanes that agree with this lane on every bit. An entry's slot is
-// the cursor of its s plus the lower lanes of its group; all lanes read the cursor,
-// then each group's lowest lane advances it (one wave's LDS accesses complete in
-// program order), so each segment lists its vocab ids in ascending order.
-__global__ __launch_bounds__(256) void bwd_scatter_kernel(
-    const int32_t* __restrict__ idx, int S, int V, int nch, const int* __restrict__ hist_base,
-    const int2* __restrict__ comp, const int* __restrict__ ccount, int2* __restrict__ list,
-    int s0) {
-  int* cur = (int*)sparton_bwd_smem + (threadIdx.x >> 6) * S;
-  const int wpb = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int b = blockIdx.y, c = blockIdx.x * wpb + wave;
-  if (c >= nch) return;  // no workgroup barrier below: waves are independent
-  const int* in = hist_base + ((int64_t)b * nch + c) * S;
-  for (int s = lane; s < S; s += 64) cur[s] = in[s];
-  const int n = ccount[(int64_t)b * nch + c];
-  const int2* cb = comp + ((int64_t)b * nch + c) * CHW;
-  int2* lb = list + (int64_t)b * V;
-  const int32_t* ib = idx + (int64_t)b * V;
+  // Lanes with equal s are found with one ballot per bit of s: `same` keeps the lanes that
+  // agree with this lane on every bit. A slot is the cursor of its position plus the lower
+  // lanes of its group; all lanes read the cursor, then each group's lowest lane advances it
+  // (one wave's LDS accesses complete in program order).
   const uint64_t lt = (1ull << lane) - 1ull;
   const int sbits = S > 1 ? 32 - __builtin_clz((unsigned)(S - 1)) : 0;
-  // SCATTER_AHEAD rounds of 64 entries at a time: their entries, then their indices
-  // (one dependent round trip each, all rounds' loads in flight together).
-  constexpr int SCATTER_AHEAD = 4;
-  for (int i0 = 0; i0 < n; i0 += 64 * SCATTER_AHEAD) {
-    int2 e[SCATTER_AHEAD];
-    int s[SCATTER_AHEAD];
+  int2* out = run + (b * runs + c) * cap;
+  for (int t = 0; t < turns && V > 0; ++t) {
+    if (turns > 1) {
+      load(t);
+      decide(t);
+    }
 #pragma unroll
-    for (int r = 0; r < SCATTER_AHEAD; ++r) e[r] = cb[min(i0 + r * 64 + lane, max(n - 1, 0))];
-#pragma unroll
-    for (int r = 0; r < SCATTER_AHEAD; ++r) s[r] = ib[e[r].x] - s0;  // entries lie in the window
-#pragma unroll
-    for (int r = 0; r < SCATTER_AHEAD; ++r) {
-      const bool act = i0 + r * 64 + lane < n;
+    for (int j = 0; j < BK_ROUNDS; ++j) {
+      const bool act = s[j] >= 0;
       uint64_t same = __ballot(act);
-      if (same == 0) break;  // uniform: no entries left
-      const int sr = act ? s[r] : 0;
-      for (int k = 0; k < sbits; ++k) {
-        const bool bit = ((sr >> k) & 1) != 0;
-        const uint64_t ones = __ballot(bit);
-        same &= bit ? ones : ~ones;
+      if (same != 0) {  // uniform
+        const int sj = act ? s[j] : 0;
+        for (int k = 0; k < sbits; ++k) {
+          const bool bit = ((sj >> k) & 1) != 0;
+          const uint64_t ones = __ballot(bit);
+          same &= bit ? ones : ~ones;
+        }
+        const int at = act ? cur[sj] : 0;
+        if (act) out[at + __popcll(same & lt)] = make_int2(v_beg + (t * BK_ROUNDS + j) * 64 + lane, __float_as_int(g[j]));
+        if (act && (same & lt) == 0) cur[sj] = at + __popcll(same);
       }
-      const int base = act ? cur[sr] : 0;
-      if (act) lb[base + __popcll(same & lt)] = e[r];
-      if (act && (same & lt) == 0) cur[sr] = base + __popcll(same);
     }
   }
 }
@@ -415,80 +275,14 @@ template <> struct Raw4<f16> {
   __device__ __forceinline__ f32x4 f() const { return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]}; }
 };
 
-// The order every dH kernel (except the few-rows split kernel) sums a row in: the row's
-// entries, in v order, are taken DH_BATCH at a time (the last batch may hold fewer); a
-// batch's partial is P = fma(g_u, W[v_u], P) over its entries from P = 0, and the row is
-// ((0 + P_0) + P_1) + ... So the fused path, whose waves share one workgroup's batches,
-// and the five-kernel path agree bitwise.
+// The order every dH row is summed in (the few-row path aside): the row's entries, in v
+// order, are taken DH_BATCH at a time (the last batch may hold fewer); a batch's partial is
+// P = fma(g_u, W[v_u], P) over its entries from P = 0, and the row is ((0 + P_0) + P_1) + ...
+// So a row is the same bits whether one lane group sums it or a workgroup shares its batches.
 constexpr int DH_BATCH = 4;
-
-// P = fma(g, w, P) per element, written out so that every dH kernel rounds the same way.
-__device__ __forceinline__ void fma4(f32x4& P, float g, const f32x4& w) {
-  P[0] = __builtin_fmaf(g, w[0], P[0]);
-  P[1] = __builtin_fmaf(g, w[1], P[1]);
-  P[2] = __builtin_fmaf(g, w[2], P[2]);
-  P[3] = __builtin_fmaf(g, w[3], P[3]);
-}
 
 // Rows gathered per batch: all their loads are in flight together (about 24 per lane).
 template <int NP> struct Batch { static constexpr int U = NP <= 3 ? 8 : NP <= 6 ? 4 : NP <= 8 ? 3 : 2; };
-// bwd_dh_kernel takes at most DH_MAX_NP register passes (wider rows loop over D) and
-// whole DH_BATCH-entry batches per load group: U rows while at least U entries are left
-// in the 64-entry chunk, US rows otherwise. Its gathers are chains of round trips, so
-// for long rows more rows in flight beat occupancy; LONG is chosen for large vocabularies
-// (V > FUSE_V_FAST), where rows hold many entries. Measured (dH alone incl. its bucketing):
-// config 4 (V = 250002, 16-bit D = 768, ~49 entries per row) U = 8 vs 32: 279 vs 233 us
-// with every row here; with rows past HOT_MIN entries in bwd_dh_hot_kernel, U = 8 / 16 /
-// 32: 187 / 181 / 187 us. Config 5 (D = 4096, 8 passes) U = 4 vs 8: 233 vs 218 us; short
-// rows (config 2 on this path) lose 3 us with U = 32 (fewer waves in flight).
-constexpr int DH_MAX_NP = 8;
-template <int NP> struct DhPasses { static constexpr int value = NP < DH_MAX_NP ? NP : DH_MAX_NP; };
-template <typename T, int NP, bool LONG> struct DhBatch {
-  static constexpr bool B16 = sizeof(T) == 2;
-  static constexpr int U = NP <= 3 ? (LONG && B16 ? 16 : 8) : (LONG && B16 ? 8 : 4);
-  static constexpr int US = NP <= 3 ? 8 : 4;
-};
-static_assert(DhBatch<bf16, 1, true>::US % DH_BATCH == 0 && DhBatch<float, DH_MAX_NP, false>::U % DH_BATCH == 0,
-              "whole batches");
-
-// One load group of bwd_dh_kernel: entries j .. j + U - 1 of the chunk held one per lane
-// in ent (n of them valid), their W rows loaded together, then summed as DH_BATCH-entry
-// partials, one pass at a time (so that only one pass of a partial is held in registers).
-template <typename T, int NP, int U>
-__device__ __forceinline__ void dh_group(const T* __restrict__ W, int2 ent, int j, int n, int d0,
-                                         int D, int lane, f32x4* acc) {
-  Raw4<T> w[U][NP];
-  float g[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    // past the segment end: reload the last entry's row (a cache hit) with g' = 0,
-    // which keeps the batch free of branches so all its loads issue together
-    const int jj = min(j + u, n - 1);
-    const int v = __builtin_amdgcn_readlane(ent.x, jj);
-    g[u] = j + u < n ? __int_as_float(__builtin_amdgcn_readlane(ent.y, jj)) : 0.0f;
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int d = d0 + p * 256 + lane * 4;
-      if (d < D) w[u][p].load(W + (int64_t)v * D + d);
-      else w[u][p].zero();
-    }
-  }
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-#pragma unroll
-    for (int a = 0; a < U; a += DH_BATCH) {
-      if (j + a < n) {  // uniform: the batch exists
-        f32x4 P = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int u = a; u < a + DH_BATCH; ++u)
-          if (j + u < n) fma4(P, g[u], w[u][p].f());
-        acc[p] += P;
-      }
-    }
-  }
-}
-
-
 // The staged dW kernel gathers the rows of IDC of a wave's ids together, U rows at a
 // time. For 16-bit rows of up to 768 elements one id and 4 rows keep it within 64 VGPRs:
 // two 16-wave workgroups per CU, so config 2's 477 workgroups run in one round instead
@@ -504,182 +298,236 @@ template <typename T, int NP> struct DwPasses {
   static constexpr int value = NP < CAP ? NP : CAP;
 };
 
-// ---- 4. dH ---------------------------------------------------------------------
-// One wave per (b,s) row; lane l owns elements d0 + p*256 + 4l .. +3 for p < NP. The
-// segment's entries sit one per lane; they are taken U (or US) at a time (a uniform
-// loop, so the summation order is the segment's v order), all loads of a group are
-// issued, then its rows are accumulated.
-template <typename T, typename O, int NP, bool LONG>
-__device__ __forceinline__ void dh_rows_body(const T* __restrict__ W, const int2* __restrict__ list,
-                                             const int* __restrict__ seg_start,
-                                             const int* __restrict__ seg_cnt, O* __restrict__ dH,
-                                             int B, int S, int D, int V, int S_row, int hot_min,
-                                             int blk) {
-  constexpr int U = DhBatch<T, NP, LONG>::U, US = DhBatch<T, NP, LONG>::US;
-  static_assert(NP <= DH_MAX_NP, "register passes");
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blk * 4 + wave;
-  if (row >= (int64_t)B * S) return;
-  const int64_t b = row / S;
-  const int start = __builtin_amdgcn_readfirstlane(seg_start[row]);
-  const int cnt = __builtin_amdgcn_readfirstlane(seg_cnt[row]);
-  if (cnt > hot_min) return;  // bwd_dh_hot_kernel writes this row
-  const int2* seg = list + b * V + start;
-  for (int d0 = 0; d0 < D; d0 += NP * 256) {
-    f32x4 acc[NP];
+// ---- 2. dH ---------------------------------------------------------------------
+// A row of D elements is cut into slices of DH_LANES 16-byte chunks, and 16 lanes (one DPP
+// row) sum one slice of one row, a chunk each, over the row's entries. The lanes look up 16
+// entries together, one each, and hand them round with row broadcasts; then the 16 W chunks
+// are loaded, 256 bytes of a W row per lane group.
+// What bounds it: with dense gradients the W rows' way from the MALL into the L2s (every
+// entry's row is read once, 6 TB/s), with sparse ones the round trips of the longest row. So
+// many lane groups are in flight, each with 16 rows of W.
+constexpr int DH_LANES = 16;
+constexpr int DH_WAVES = 4;
+constexpr int DH_GROUPS = 64 / DH_LANES * DH_WAVES;  // lane groups (rows) of a workgroup
+
+template <typename T> struct Chunk {
+  static constexpr int E = 16 / (int)sizeof(T);  // elements of a 16-byte chunk
+  static constexpr int COLS = DH_LANES * E;      // columns of a slice
+};
+template <typename T>
+__device__ __forceinline__ void chunk_f32(const u32x4& c, float* f);
+template <> __device__ __forceinline__ void chunk_f32<float>(const u32x4& c, float* f) {
 #pragma unroll
-    for (int p = 0; p < NP; ++p) acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int e0 = 0; e0 < cnt; e0 += 64) {
-      const int2 ent = e0 + lane < cnt ? seg[e0 + lane] : make_int2(0, 0);
-      const int n = min(64, cnt - e0);
-      // j stays a multiple of DH_BATCH (chunks of 64 too): whole batches per group.
-      int j = 0;
-      if constexpr (U > US) {
-        for (; j + U <= n; j += U) dh_group<T, NP, U>(W, ent, j, n, d0, D, lane, acc);
-      }
-      for (; j < n; j += US) dh_group<T, NP, US>(W, ent, j, n, d0, D, lane, acc);
-    }
-    O* out = dH + (b * S_row + (row - b * S)) * D;
+  for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(c[i]);
+}
+template <> __device__ __forceinline__ void chunk_f32<bf16>(const u32x4& c, float* f) {
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int d = d0 + p * 256 + lane * 4;
-      if (d < D) store4(out + d, acc[p]);
-    }
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = __uint_as_float(c[i] << 16);
+    f[2 * i + 1] = __uint_as_float(c[i] & 0xffff0000u);
   }
 }
-template <typename T, typename O, int NP, bool LONG>
-__global__ __launch_bounds__(256) void bwd_dh_kernel(
-    const T* __restrict__ W, const int2* __restrict__ list, const int* __restrict__ seg_start,
-    const int* __restrict__ seg_cnt, O* __restrict__ dH, int B, int S, int D, int V, int S_row,
-    int hot_min) {
-  dh_rows_body<T, O, NP, LONG>(W, list, seg_start, seg_cnt, dH, B, S, D, V, S_row, hot_min,
-                               (int)blockIdx.x);
+template <> __device__ __forceinline__ void chunk_f32<f16>(const u32x4& c, float* f) {
+  const f16x8 h = __builtin_bit_cast(f16x8, c);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) f[i] = (float)h[i];
 }
 
-// Hot rows (more than hot_min entries, e.g. a position that wins most vocab ids; at
-// config 4, V = 250002, rows hold ~49 entries and up to 776): one wave per row would
-// gather them alone. Measured at config 4, backward with HOT_MIN = 64 / 128 / 256 / 512 /
-// off: 341 / 342 / 369 / 398 / 390 us; configs 1, 2, 3 (five-kernel) and 5 unchanged. Here a workgroup of HOT_WAVES waves takes one
-// (hot row, 256-column slice) at a time from the list the scan built (a grid of fixed
-// size walks the list). Each step its waves compute HOT_PER_WAVE consecutive batch
-// partials each (the DH_BATCH-entry partials of bwd_dh_kernel, over the slice) into LDS,
-// and wave 0 adds them in batch order: the same sums as bwd_dh_kernel, bitwise.
+// Lane U of the 16-lane row, to all its lanes (which must be active together).
+template <int U> __device__ __forceinline__ uint32_t row_bcast(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + U, 0xF, 0xF, true);  // row_newbcast:U
+}
+template <int I, int N, typename F> __device__ __forceinline__ void static_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+// The entries of one dH row, spread over the batch row's runs: lane l of the group holds run
+// l's. Entry i of the row (ids ascending) lies in the run q that holds the i-th of the
+// running total, at place base_q + i of the batch row's runs.
+struct RowEntries {
+  int incl, base, total;
+  __device__ __forceinline__ void load(const int* off, int runs, int cap, int l) {
+    const int o0 = l < runs ? off[l] : 0, o1 = l < runs ? off[runs + l] : 0;
+    incl = o1 - o0;
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xF, 0xF, true);  // row_shr:1
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, true);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xF, true);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xF, 0xF, true);
+    base = l * cap + o0 - (incl - (o1 - o0));
+    total = (int)row_bcast<15>((uint32_t)incl);
+  }
+  __device__ __forceinline__ int place(int i, int runs) const {
+    int q = 0;
+    static_for<0, 8>([&](auto k) { q += (int)row_bcast<decltype(k)::value>((uint32_t)incl) <= i ? 1 : 0; });
+    if (runs > 8)  // uniform
+      static_for<8, 15>([&](auto k) { q += (int)row_bcast<decltype(k)::value>((uint32_t)incl) <= i ? 1 : 0; });
+    return i + __builtin_amdgcn_ds_bpermute((((int)threadIdx.x & 48) + min(q, 15)) * 4, base);
+  }
+};
+
+// 16 entries of a row, one per lane: g' (0 past the row's end) and the place of the W row in
+// 16-byte units (the last entry's past its end).
+struct Entries {
+  uint32_t off;
+  float g;
+  __device__ __forceinline__ void load(const int2* run, const RowEntries& re, int runs, int e,
+                                       uint32_t row16, int l) {
+    const int2 x = run[re.place(min(e + l, re.total - 1), runs)];
+    off = (uint32_t)x.x * row16;
+    g = e + l < re.total ? __int_as_float(x.y) : 0.0f;
+  }
+};
+
+// The partials P of the DH_BATCHes of entries 0 .. N - 1 over one chunk of their W rows (wp:
+// the chunk in row 0), handed to put(batch, P) in order. With MASKED only the first `left`
+// count; the others add 0 * 0, which leaves the sums as they are.
+template <typename T, bool MASKED, int N, typename Put>
+__device__ __forceinline__ void dh_partials(const char* wp, const Entries& en, int left, Put put) {
+  constexpr int E = Chunk<T>::E;
+  u32x4 w[N];
+  static_for<0, N>([&](auto u) {
+    w[u] = *(const u32x4*)(wp + ((uint64_t)row_bcast<decltype(u)::value>(en.off) << 4));
+  });
+  static_for<0, N / DH_BATCH>([&](auto a) {
+    float P[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) P[i] = 0.0f;
+    static_for<0, DH_BATCH>([&](auto k) {
+      constexpr int u = decltype(a)::value * DH_BATCH + decltype(k)::value;
+      const float g = __uint_as_float(row_bcast<u>(__float_as_uint(en.g)));
+      u32x4 x = w[u];
+      if (MASKED && u >= left) x = u32x4{0u, 0u, 0u, 0u};
+      float f[E];
+      chunk_f32<T>(x, f);
+#pragma unroll
+      for (int i = 0; i < E; ++i) P[i] = __builtin_fmaf(g, f[i], P[i]);
+    });
+    put(decltype(a)::value, P);
+  });
+}
+// The same for the last `left` < DH_LANES entries, no more of them loaded than a few.
+template <typename T, typename Put>
+__device__ __forceinline__ void dh_partials_tail(const char* wp, const Entries& en, int left, Put put) {
+  if (left > 8) dh_partials<T, true, 16>(wp, en, left, put);
+  else if (left > 4) dh_partials<T, true, 8>(wp, en, left, put);
+  else dh_partials<T, true, 4>(wp, en, left, put);
+}
+
+template <typename O, int E>
+__device__ __forceinline__ void store_chunk(O* out, const float* a) {
+#pragma unroll
+  for (int i = 0; i < E; i += 4) store4(out + i, f32x4{a[i], a[i + 1], a[i + 2], a[i + 3]});
+}
+
+// Hot rows: a lane group sums a row serially, so one that holds many times the entries of
+// the others (a [CLS]-like position wins most ids), or any row of a launch with few rows,
+// would outlast the launch. A workgroup's lane groups therefore share such rows: each step
+// every group computes the batch partials of 16 consecutive entries into LDS, and the
+// slice's columns add them in batch order: the same sums. A workgroup takes DH_GROUPS rows,
+// of which those past max(HOT_MIN, HOT_REL times its mean) are shared, or, of fewer rows
+// (dh_rows_per_group), every one that is not short (HOT_FEW).
 constexpr int HOT_MIN = 128;
-constexpr int HOT_WAVES = 16;
-constexpr int HOT_PER_WAVE = 2;
-constexpr int HOT_STEP = HOT_WAVES * HOT_PER_WAVE;  // batches per step
-constexpr int HOT_GRID = 512;
+constexpr int HOT_REL = 4;
+constexpr int HOT_FEW = 32;
+constexpr int HOT_NB = DH_LANES / DH_BATCH;  // partials per lane group and step
+
+template <typename T>
+struct HotSmem {
+  float part[DH_GROUPS * HOT_NB][Chunk<T>::COLS];
+  int total[DH_GROUPS];
+};
+
 template <typename T, typename O>
-__global__ __launch_bounds__(64 * HOT_WAVES) void bwd_dh_hot_kernel(
-    const T* __restrict__ W, const int2* __restrict__ list, const int* __restrict__ seg_start,
-    const int* __restrict__ seg_cnt, const int* __restrict__ hot, O* __restrict__ dH, int S,
-    int D, int V, int S_row, int ns) {
-  __shared__ f32x4 part[HOT_STEP][64];
-  constexpr int U = HOT_PER_WAVE * DH_BATCH;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n_items = __builtin_amdgcn_readfirstlane(hot[0]) * ns;
-  for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
-    const int64_t row = __builtin_amdgcn_readfirstlane(hot[1 + item / ns]);
-    const int d = (item % ns) * 256 + lane * 4;
+__global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
+    const T* __restrict__ W, const int* __restrict__ off, const int2* __restrict__ run,
+    O* __restrict__ dH, int B, int S, int D, int runs, int cap, int S_row, int n_slices, int rpw,
+    int hot_min) {
+  constexpr int E = Chunk<T>::E;
+  static_assert(Chunk<T>::COLS <= 64 * DH_WAVES, "one thread per column");
+  __shared__ HotSmem<T> sm;
+  const int slice = (int)blockIdx.x % n_slices, blk = (int)blockIdx.x / n_slices;
+  const int tid = threadIdx.x, grp = tid / DH_LANES, l = tid % DH_LANES;
+  const uint32_t row16 = (uint32_t)(D * (int)sizeof(T) / 16);  // 16-byte units per row
+  const int d0 = slice * Chunk<T>::COLS;
+  // Lanes past the row's end work on its last chunk (the row broadcasts need them) and do not
+  // store.
+  const int d = d0 + l * E;
+  const char* wp = (const char*)(W + min(d, D - E));
+  const int64_t n_rows = (int64_t)B * S, row0 = (int64_t)blk * rpw;
+  auto entries_of = [&](int64_t row, RowEntries& re) {  // returns the batch row's runs
     const int64_t b = row / S;
-    const int start = __builtin_amdgcn_readfirstlane(seg_start[row]);
-    const int cnt = __builtin_amdgcn_readfirstlane(seg_cnt[row]);
-    const int2* seg = list + b * V + start;
-    const int nbat = (cnt + DH_BATCH - 1) / DH_BATCH;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int t0 = 0; t0 < nbat; t0 += HOT_STEP) {
-      const int e0 = (t0 + wave * HOT_PER_WAVE) * DH_BATCH;  // this wave's first entry
-      if (e0 < cnt) {  // uniform
-        const int2 ent = lane < U ? seg[min(e0 + lane, cnt - 1)] : make_int2(0, 0);
-        Raw4<T> w[U];
-        float g[U];
+    re.load(off + (b * (S + 1) + (row - b * S)) * runs, runs, cap, l);
+    return run + b * runs * cap;
+  };
+  auto out_of = [&](int64_t row) {
+    const int64_t b = row / S;
+    return dH + (b * S_row + (row - b * S)) * D;
+  };
+  const bool live = grp < rpw && row0 + grp < n_rows;
+  RowEntries re;
+  re.total = 0;
+  const int2* rb = nullptr;
+  if (live) rb = entries_of(row0 + grp, re);
+  if (l == 0) sm.total[grp] = re.total;
+  __syncthreads();
+  int lim = HOT_FEW;
+  if (rpw == DH_GROUPS) {
+    int sum = 0;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          // past the row's last entry: reload that entry's row (a cache hit), unused
-          const int v = __builtin_amdgcn_readlane(ent.x, u);
-          g[u] = __int_as_float(__builtin_amdgcn_readlane(ent.y, u));
-          if (d < D) w[u].load(W + (int64_t)v * D + d);
-          else w[u].zero();
-        }
+    for (int k = 0; k < DH_GROUPS; ++k) sum += sm.total[k];
+    lim = max(HOT_MIN, HOT_REL * (sum / DH_GROUPS));
+  }
+  if (hot_min >= 0) lim = hot_min;
+  if (live && re.total <= lim) {
+    float acc[E];
 #pragma unroll
-        for (int h = 0; h < HOT_PER_WAVE; ++h) {
-          f32x4 P = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < E; ++i) acc[i] = 0.0f;
+    if (re.total > 0) {
+      auto add = [&](int, const float* P) {
 #pragma unroll
-          for (int u = h * DH_BATCH; u < (h + 1) * DH_BATCH; ++u)
-            if (e0 + u < cnt) fma4(P, g[u], w[u].f());  // uniform condition
-          part[wave * HOT_PER_WAVE + h][lane] = P;
-        }
+        for (int i = 0; i < E; ++i) acc[i] += P[i];
+      };
+      Entries next;
+      next.load(rb, re, runs, 0, row16, l);
+      int e = 0;
+      for (; e + DH_LANES <= re.total; e += DH_LANES) {
+        const Entries en = next;
+        next.load(rb, re, runs, e + DH_LANES, row16, l);
+        dh_partials<T, false, DH_LANES>(wp, en, DH_LANES, add);
+      }
+      if (e < re.total) dh_partials_tail<T>(wp, next, re.total - e, add);
+    }
+    if (d < D) store_chunk<O, E>(out_of(row0 + grp) + d, acc);
+  }
+  for (int k = 0; k < rpw; ++k) {
+    const int n = __builtin_amdgcn_readfirstlane(sm.total[k]);
+    if (n <= lim) continue;  // workgroup-uniform
+    RowEntries rk;
+    const int2* rbk = entries_of(row0 + k, rk);
+    float acc = 0.0f;  // column `tid` of the slice
+    for (int e0 = 0; e0 < n; e0 += DH_GROUPS * DH_LANES) {
+      const int e = e0 + grp * DH_LANES;
+      if (e < n) {
+        Entries en;
+        en.load(rbk, rk, runs, e, row16, l);
+        auto put = [&](int p, const float* P) {
+#pragma unroll
+          for (int j = 0; j < E; ++j) sm.part[grp * HOT_NB + p][l * E + j] = P[j];
+        };
+        if (n - e >= DH_LANES) dh_partials<T, false, DH_LANES>(wp, en, DH_LANES, put);
+        else dh_partials_tail<T>(wp, en, n - e, put);
       }
       __syncthreads();
-      if (wave == 0) {
-        const int m = min(HOT_STEP, nbat - t0);
-        for (int j = 0; j < m; ++j) acc += part[j][lane];
-      }
+      const int m = min(DH_GROUPS * HOT_NB, (n - e0 + DH_BATCH - 1) / DH_BATCH);
+      if (tid < Chunk<T>::COLS)
+        for (int j = 0; j < m; ++j) acc += sm.part[j][tid];
       __syncthreads();  // the partials are rewritten next step
     }
-    if (wave == 0 && d < D) store4(dH + (b * S_row + (row - b * S)) * D + d, acc);
+    if (tid < Chunk<T>::COLS && d0 + tid < D) out_of(row0 + k)[d0 + tid] = from_f32<O>(acc);
   }
-}
-
-// Few rows (B*S < SPLIT_ROWS, e.g. 2 x 32 with every v active): one workgroup of
-// SPLIT_WAVES waves per (row, 256-column slice of D) instead of one wave per row, so that
-// even a handful of rows keeps thousands of waves gathering. Wave w sums entries
-// [w c, (w + 1) c) of the row's segment (c = ceil(cnt / SPLIT_WAVES)) in v order over its
-// slice, and wave 0 adds the partial slices in wave order through LDS: deterministic
-// (each element's sum does not depend on the slicing).
-constexpr int SPLIT_WAVES = 8;
-constexpr int SPLIT_ROWS = 1024;
-constexpr int SPLIT_U = 16;  // rows gathered per batch (one 256-column slice each)
-template <typename T, typename O>
-__device__ __forceinline__ void dh_split_body(float (*red)[256], const T* __restrict__ W,
-                                              const int2* __restrict__ list,
-                                              const int* __restrict__ seg_start,
-                                              const int* __restrict__ seg_cnt, O* __restrict__ dH,
-                                              int S, int D, int V, int S_row, int ns, int blk) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t row = blk / ns;  // workgroups = B * S * ns exactly
-  const int d = (int)(blk % ns) * 256 + lane * 4;
-  const int64_t b = row / S;
-  const int start = __builtin_amdgcn_readfirstlane(seg_start[row]);
-  const int cnt = __builtin_amdgcn_readfirstlane(seg_cnt[row]);
-  const int per = (cnt + SPLIT_WAVES - 1) / SPLIT_WAVES;
-  const int e_beg = min(cnt, wave * per), e_end = min(cnt, e_beg + per);
-  const int2* seg = list + b * V + start;
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int e0 = e_beg; e0 < e_end; e0 += 64) {
-    const int2 ent = e0 + lane < e_end ? seg[e0 + lane] : make_int2(0, 0);
-    const int n = min(64, e_end - e0);
-    for (int j = 0; j < n; j += SPLIT_U) {
-      Raw4<T> w[SPLIT_U];
-      float g[SPLIT_U];
-#pragma unroll
-      for (int u = 0; u < SPLIT_U; ++u) {
-        const int jj = min(j + u, n - 1);
-        const int v = __builtin_amdgcn_readlane(ent.x, jj);
-        g[u] = j + u < n ? __int_as_float(__builtin_amdgcn_readlane(ent.y, jj)) : 0.0f;
-        if (d < D) w[u].load(W + (int64_t)v * D + d);
-        else w[u].zero();
-      }
-#pragma unroll
-      for (int u = 0; u < SPLIT_U; ++u) acc += g[u] * w[u].f();
-    }
-  }
-  *(f32x4*)&red[wave][lane * 4] = acc;
-  __syncthreads();
-  if (wave == 0) {
-    f32x4 t = *(const f32x4*)&red[0][lane * 4];
-#pragma unroll
-    for (int w = 1; w < SPLIT_WAVES; ++w) t += *(const f32x4*)&red[w][lane * 4];
-    if (d < D) store4(dH + (b * S_row + (row - b * S)) * D + d, t);
-  }
-}
-template <typename T, typename O>
-__global__ __launch_bounds__(64 * SPLIT_WAVES) void bwd_dh_split_kernel(
-    const T* __restrict__ W, const int2* __restrict__ list, const int* __restrict__ seg_start,
-    const int* __restrict__ seg_cnt, O* __restrict__ dH, int B, int S, int D, int V, int S_row,
-    int ns) {
-  __shared__ __attribute__((aligned(16))) float red[SPLIT_WAVES][256];
-  dh_split_body<T, O>(red, W, list, seg_start, seg_cnt, dH, S, D, V, S_row, ns, (int)blockIdx.x);
 }
 
 // Entries (b_i, v) for N batch rows (b_i >= B or v >= V: inactive): g' (0 if inactive) and
@@ -791,23 +639,14 @@ __global__ __launch_bounds__(256) void bwd_dw_kernel(
 
 // ---- 5b. dW and dbias, staged (B <= DW_STAGE_B) ---------------------------------
 constexpr int DW_STAGE_B = 128;
-// The fused dH path (B <= DW_STAGE_B, S <= FUSE_MAX_S, V <= 2^FUSE_V_BITS, D in one
-// register pass): an entry packs v and s into one int.
-constexpr int FUSE_V_BITS = 18;
-constexpr int FUSE_MAX_S = 1024;
-constexpr int FUSE_ROWS = 16;                          // rows per range (one workgroup)
-constexpr int FUSE_V_FAST = 1 << 16;    // above this the five-kernel path is faster
-constexpr int FUSE_MAX_NVB = FUSE_V_FAST / 64;         // 64-id blocks the fused path takes
-constexpr int FUSE_MIN_RANGES = 64;     // below this too (too few workgroups)
-constexpr int FUSE_MAX_NR = FUSE_MAX_S / FUSE_ROWS;    // ranges (<= 64: one lane each)
-
 // The staged dW: a workgroup of NW waves owns NIDS consecutive vocab ids (NIDS / NW per
 // wave). It loads G, reps and I of all batch rows for them (each load instruction reads
 // NIDS consecutive elements of 64 / NIDS rows) and keeps g' (0 = inactive) and I in LDS;
 // then each wave handles its ids: lanes scan the batch rows, ballots list the active
 // ones, and their H rows are gathered up to U at a time and accumulated, each id in
 // ascending b. I is kept as 16 bits: the staged kernels take S <= DW_STAGE_S.
-constexpr int DW_WAVES = 16;
+constexpr int DW_WAVES = 16;  // of the wide kernel
+constexpr int DW_IDS = 4 * BK_WAVES;  // ids of a staged workgroup
 constexpr int DW_LD = DW_STAGE_B + 1;  // odd row stride: conflict-free column and row access
 constexpr int DW_STAGE_S = 1 << 16;
 
@@ -940,20 +779,28 @@ __device__ __forceinline__ void dw_gather(const float* gl, const uint16_t* sl,
   }
 }
 
-// dW / dbias for B <= DW_STAGE_B and S <= DW_STAGE_S (the five-kernel path's).
+// The bucketing's workgroups (n_bucket of them), then dW's, DW_IDS ids each: dW reads only the
+// inputs, so both run side by side. Either part may be empty. grad, reps, idx and mask start
+// at the pass's first batch row.
 template <typename T, typename O, int NP, typename RT>
-__global__ __launch_bounds__(64 * DW_WAVES) void bwd_dw_staged_kernel(
-    const T* __restrict__ grad, const RT* __restrict__ reps,
-    const int32_t* __restrict__ idx, const void* __restrict__ mask, int mdt,
-    const T* __restrict__ H, O* __restrict__ dW, O* __restrict__ dbias, int B, int S, int D,
-    int V) {
-  __shared__ float gl[64 * DW_LD];
-  __shared__ uint16_t sl[64 * DW_LD];
+__global__ __launch_bounds__(64 * BK_WAVES) void bwd_bucket_dw_kernel(
+    const T* __restrict__ grad, const RT* __restrict__ reps, const int32_t* __restrict__ idx,
+    const void* __restrict__ mask, int mdt, const T* __restrict__ H, O* __restrict__ dW,
+    O* __restrict__ dbias, int B, int S, int D, int V, int n_bucket, int runs, int cap, int win_s0,
+    int win_s, int* __restrict__ off, int2* __restrict__ run) {
+  const int blk = blockIdx.x;
+  if (blk < n_bucket) {  // workgroup-uniform
+    bucket_run<T, RT>(grad, reps, idx, mask, mdt, win_s, V, blk / runs, blk % runs, runs, cap, off, run,
+                      win_s0, S);
+    return;
+  }
+  float* gl = (float*)sparton_bwd_smem;
+  uint16_t* sl = (uint16_t*)(gl + DW_IDS * DW_LD);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int v0 = blockIdx.x * 64;
-  dw_stage<T, RT, 64, DW_WAVES>(gl, sl, grad, reps, idx, mask, mdt, B, S, V, v0, wave, lane);
+  const int v0 = (blk - n_bucket) * DW_IDS;
+  dw_stage<T, RT, DW_IDS, BK_WAVES>(gl, sl, grad, reps, idx, mask, mdt, B, S, V, v0, wave, lane);
   __syncthreads();
-  dw_gather<T, O, NP, RT, 64, DW_WAVES>(gl, sl, H, dW, dbias, B, S, D, V, v0, wave, lane);
+  dw_gather<T, O, NP, RT, DW_IDS, BK_WAVES>(gl, sl, H, dW, dbias, B, S, D, V, v0, wave, lane);
 }
 
 // dW / dbias for DW_STAGE_B < B <= DW_WIDE_B and S <= DW_STAGE_S: the staged kernel with
@@ -978,418 +825,25 @@ __global__ __launch_bounds__(64 * DW_WAVES) void bwd_dw_wide_kernel(
   dw_gather<T, O, NP, RT, NIDS, DW_WAVES, LD>(gl, sl, H, dW, dbias, B, S, D, V, v0, wave, lane);
 }
 
-// dH and the staged dW in one launch, for the five-kernel path when it makes one pass
-// (B <= MAX_B, S <= MAX_S), dW is staged (B <= DW_STAGE_B, S <= DW_STAGE_S) and the rows
-// are wide (the launch rule is at the host dispatch): the dH workgroups first, then dW
-// workgroups of 4 ids per wave. dW reads only the inputs, so its workgroups fill the CUs
-// that the dH rows leave idle, and its own launch (about 4.5 us of dispatch and cache
-// work at each kernel boundary) is saved. The sums are those of the separate kernels.
-template <typename T, typename O, int NP, bool LONG, int DNP, typename RT>
-__global__ __launch_bounds__(256) void bwd_dh_dw_kernel(
-    const T* __restrict__ W, const int2* __restrict__ list, const int* __restrict__ seg_start,
-    const int* __restrict__ seg_cnt, O* __restrict__ dH, int B, int S, int D, int V,
-    int hot_min, int n_dh, const T* __restrict__ grad, const RT* __restrict__ reps,
-    const int32_t* __restrict__ idx, const void* __restrict__ mask, int mdt,
-    const T* __restrict__ H, O* __restrict__ dW, O* __restrict__ dbias) {
-  constexpr int NW = 4, NIDS = 4 * NW;
-  __shared__ float gl[NIDS * DW_LD];
-  __shared__ uint16_t sl[NIDS * DW_LD];
-  if ((int)blockIdx.x < n_dh) {  // workgroup-uniform
-    dh_rows_body<T, O, NP, LONG>(W, list, seg_start, seg_cnt, dH, B, S, D, V, S, hot_min,
-                                 (int)blockIdx.x);
-    return;
-  }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int v0 = ((int)blockIdx.x - n_dh) * NIDS;
-  dw_stage<T, RT, NIDS, NW>(gl, sl, grad, reps, idx, mask, mdt, B, S, V, v0, wave, lane);
-  __syncthreads();
-  dw_gather<T, O, DNP, RT, NIDS, NW>(gl, sl, H, dW, dbias, B, S, D, V, v0, wave, lane);
-}
-
-// The same for few rows: the split dH workgroups, then dW workgroups of 4 ids per wave.
-template <typename T, typename O, int DNP, typename RT>
-__global__ __launch_bounds__(64 * SPLIT_WAVES) void bwd_dh_split_dw_kernel(
-    const T* __restrict__ W, const int2* __restrict__ list, const int* __restrict__ seg_start,
-    const int* __restrict__ seg_cnt, O* __restrict__ dH, int B, int S, int D, int V, int ns,
-    int n_dh, const T* __restrict__ grad, const RT* __restrict__ reps,
-    const int32_t* __restrict__ idx, const void* __restrict__ mask, int mdt,
-    const T* __restrict__ H, O* __restrict__ dW, O* __restrict__ dbias) {
-  constexpr int NW = SPLIT_WAVES, NIDS = 4 * NW;
-  struct DwSmem {
-    float gl[NIDS * DW_LD];
-    uint16_t sl[NIDS * DW_LD];
-  };
-  union Smem {
-    float red[SPLIT_WAVES][256];
-    DwSmem w;
-  };
-  __shared__ __attribute__((aligned(16))) Smem sm;
-  if ((int)blockIdx.x < n_dh) {  // workgroup-uniform
-    dh_split_body<T, O>(sm.red, W, list, seg_start, seg_cnt, dH, S, D, V, S, ns, (int)blockIdx.x);
-    return;
-  }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int v0 = ((int)blockIdx.x - n_dh) * NIDS;
-  dw_stage<T, RT, NIDS, NW>(sm.w.gl, sm.w.sl, grad, reps, idx, mask, mdt, B, S, V, v0, wave, lane);
-  __syncthreads();
-  dw_gather<T, O, DNP, RT, NIDS, NW>(sm.w.gl, sm.w.sl, H, dW, dbias, B, S, D, V, v0, wave, lane);
-}
-
-// The fused path's compaction, for the dH workgroups: for batch row b and 64-id block
-// blk, the active entries sorted by row range k = s / FUSE_ROWS and then by v, as
-// (v | s << FUSE_V_BITS, g') at comp[(b * nvb + blk) * 64 + rank]; their number
-// cnt[b * nvb + blk], and the first rank of each range (offs[(b * nvb + blk) * nr + k],
-// lane k). Ranks come from one pass over the active lanes (a handful per block). One
-// wave per (block, two batch rows b, b + 4).
-template <typename T, typename RT>
-__global__ __launch_bounds__(256) void bwd_compact_kernel(
-    const T* __restrict__ grad, const RT* __restrict__ reps, const int32_t* __restrict__ idx,
-    const void* __restrict__ mask, int mdt, int B, int S, int V, int2* __restrict__ comp,
-    int* __restrict__ cnt, int* __restrict__ offs) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int nvb = gridDim.x, blk = blockIdx.x, v0 = blk * 64;
-  const int nr = (S + FUSE_ROWS - 1) / FUSE_ROWS;
-  const int bs[2] = {(int)blockIdx.y * 8 + wave, (int)blockIdx.y * 8 + 4 + wave};
-  float g[2];
-  int sv[2];
-  entries_n<T, RT, 2>(grad, reps, idx, mask, mdt, bs, v0 + lane, B, S, V, g, sv);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    if (bs[i] >= B) break;  // wave-uniform
-    const bool on = g[i] != 0.0f;
-    const int k = sv[i] / FUSE_ROWS;
-    const uint64_t bal = __ballot(on);
-    uint64_t act = bal;
-    const int64_t base = (int64_t)bs[i] * nvb + blk;
-    int rank = 0, first = 0;  // this entry's rank; the first rank of range `lane`
-    while (act) {
-      const int j = __ffsll((unsigned long long)act) - 1;
-      act &= act - 1;
-      const int kj = __builtin_amdgcn_readlane(k, j);
-      rank += (kj < k || (kj == k && j < lane)) ? 1 : 0;
-      first += kj < lane ? 1 : 0;
-    }
-    if (on) comp[base * 64 + rank] = make_int2((v0 + lane) | (sv[i] << FUSE_V_BITS), __float_as_int(g[i]));
-    if (lane < nr) offs[base * nr + lane] = first;
-    if (lane == 0) cnt[base] = __popcll(bal);
-  }
-}
-
-// ---- 4b. dH from the staged dW kernel's compacted entries (the fused path) -------------
-// FUSE_HALVES workgroups per (b, range of FUSE_ROWS consecutive rows); wave w of
-// workgroup h owns row s = FUSE_ROWS * range + FUSE_WAVES * h + w. Each 64-id block of row b lists its active
-// entries sorted by row range, then v, so a range's entries are one contiguous run per
-// block: thread t copies the t-th of them into LDS (its block found by binary search over
-// the runs' prefix sums), 64 * FUSE_WAVES per round, in block (= v) order. Each wave
-// appends the entries of its row to its own list, keeping v order.
-// The workgroup's waves then share the gathering: the rows' DH_BATCH-entry batches, in
-// (row, batch) order, are taken FUSE_SLOTS at a time, one per wave; each wave gathers its
-// batch's W rows and writes the batch partial to LDS, and each row's own wave adds its
-// rows' partials in batch order. A row with many entries is gathered by all the waves of
-// its workgroup, and the sums are exactly those of bwd_dh_kernel.
-// With the compaction in the dW kernel this replaces the count, scan and scatter passes.
-constexpr int FUSE_CAP = 120;  // a wave's list; the lists are gathered before one could overflow
-constexpr int FUSE_WAVES = 8;  // rows per workgroup (one 16-wave workgroup per range measured
-                               // slower: 56.5 vs 49.4 us at config 2)
-constexpr int FUSE_HALVES = FUSE_ROWS / FUSE_WAVES;  // workgroups per row range
-static_assert(FUSE_ROWS % FUSE_WAVES == 0, "whole workgroups per row range");
-// Register passes the fused path takes (a batch of rows and the accumulators in ~64 VGPRs).
-template <typename T> struct FuseMaxNp { static constexpr int value = sizeof(T) == 2 ? 6 : 3; };
-// W rows loaded at a time by the fused dH gather (a divisor of DH_BATCH): fewer for wide
-// rows, so that the kernel stays near 64 VGPRs (8 waves per SIMD: four workgroups per CU).
-template <int NP> struct FuseBatch { static constexpr int U = NP <= 3 ? 4 : 2; };
-// Batches gathered per step (one per wave; half the waves for wide rows, whose partials
-// take twice the LDS).
-template <int NP> struct FuseSlots { static constexpr int value = NP <= 3 ? FUSE_WAVES : FUSE_WAVES / 2; };
-static_assert(DH_BATCH % FuseBatch<1>::U == 0 && DH_BATCH % FuseBatch<6>::U == 0, "whole batches");
-
-// PER: 64-id blocks per thread in the prefix (nvb <= PER * 64 * FUSE_WAVES).
-template <int PER, int NP>
-struct DhSmem {
-  static constexpr int NT = 64 * FUSE_WAVES;
-  static constexpr int SLOTS = FuseSlots<NP>::value;
-  static_assert(PER * NT <= FUSE_MAX_NVB, "prefix arrays");
-  int pre[PER * NT];    // prefix of the runs' lengths
-  int lo_of[PER * NT];  // each run's first rank in its block
-  int2 stage[NT];
-  int2 lst[FUSE_WAVES][FUSE_CAP];
-  f32x4 part[SLOTS][NP * 64];  // one step's batch partials, [slot][p * 64 + lane]
-  int wsum[FUSE_WAVES];
-  int nlist[FUSE_WAVES];       // entries in each row's list
-  int nbat[FUSE_WAVES];        // batches of each row to gather now
-  int full[2][FUSE_WAVES];     // a row's list could overflow (two buffers: no WAR barrier)
-};
-static_assert(sizeof(DhSmem<1, 3>) <= 40 * 1024, "four dH workgroups per CU at config 2's widths");
-
-// One batch's partial (entries e0 .. e0 + m - 1 of `list`), pass by pass: pass p goes to
-// dst[p * 64 + lane] (ADD = false) or is added to acc[p] (ADD = true).
-template <typename T, int NP, bool ADD>
-__device__ __forceinline__ void dh_batch(const T* __restrict__ W, const int2* list, int e0, int m,
-                                         int D, int lane, f32x4* dst, f32x4* acc) {
-  constexpr int U = FuseBatch<NP>::U;
-  constexpr int VMASK = (1 << FUSE_V_BITS) - 1;
-  f32x4 Pr[NP];  // ADD with two load groups: the partial between them
-#pragma unroll
-  for (int u0 = 0; u0 < DH_BATCH; u0 += U) {
-    Raw4<T> w[U][NP];
-    float g[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // past the batch's last entry: reload that entry's row (a cache hit), unused
-      const int2 ent = list[e0 + min(u0 + u, m - 1)];
-      const int v = __builtin_amdgcn_readfirstlane(ent.x) & VMASK;  // uniform
-      g[u] = __int_as_float(__builtin_amdgcn_readfirstlane(ent.y));
-#pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        const int d = p * 256 + lane * 4;
-        if (d < D) w[u][p].load(W + (int64_t)v * D + d);
-        else w[u][p].zero();
-      }
-    }
-    // One pass at a time, so that only one pass of the partial is held in registers when
-    // the batch is one load group.
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      f32x4 P = u0 == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : (ADD ? Pr[p] : dst[p * 64 + lane]);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (u0 + u < m) fma4(P, g[u], w[u][p].f());  // uniform condition
-      if (!ADD) dst[p * 64 + lane] = P;
-      else if (u0 + U >= DH_BATCH) acc[p] += P;
-      else Pr[p] = P;
-    }
-  }
-}
-
-// The workgroup's gather of every listed batch of its rows (only the complete ones unless
-// `last`); row `wave`'s partials are added to acc in batch order, and the gathered entries
-// leave the lists (a row keeps its incomplete last batch). When one row holds more than
-// `share` times the batches per wave, the waves share them: SLOTS per step, each wave's
-// partial through LDS to the row's wave. Otherwise each wave gathers its own row.
-template <typename T, int NP, int PER>
-__device__ __forceinline__ void dh_gather(DhSmem<PER, NP>& sm, const T* __restrict__ W, int D,
-                                          int wave, int lane, int& n, bool last, int share,
-                                          f32x4* acc) {
-  constexpr int SLOTS = DhSmem<PER, NP>::SLOTS;
-  const int mine = last ? (n + DH_BATCH - 1) / DH_BATCH : n / DH_BATCH;
-  if (lane == 0) {
-    sm.nlist[wave] = n;
-    sm.nbat[wave] = mine;
-  }
-  __syncthreads();
-  int st[FUSE_WAVES + 1];  // first batch of each row in the workgroup's order (uniform)
-  st[0] = 0;
-  int most = 0;
-#pragma unroll
-  for (int w = 0; w < FUSE_WAVES; ++w) {
-    const int c = __builtin_amdgcn_readfirstlane(sm.nbat[w]);
-    st[w + 1] = st[w] + c;
-    most = max(most, c);
-  }
-  const int nb = st[FUSE_WAVES];
-  if (most > share * ((nb + SLOTS - 1) / SLOTS)) {
-    for (int t0 = 0; t0 < nb; t0 += SLOTS) {
-      const int q = t0 + wave;  // this wave's batch
-      if (wave < SLOTS && q < nb) {
-        int r = 0;
-#pragma unroll
-        for (int w = 1; w < FUSE_WAVES; ++w) r += q >= st[w] ? 1 : 0;
-        const int e0 = (q - st[r]) * DH_BATCH;
-        const int m = min(DH_BATCH, __builtin_amdgcn_readfirstlane(sm.nlist[r]) - e0);
-        dh_batch<T, NP, false>(W, sm.lst[r], e0, m, D, lane, sm.part[wave], acc);
-      }
-      __syncthreads();
-      // This wave's row: its batches among this step's, in order.
-      const int b0 = max(st[wave], t0), b1 = min(st[wave + 1], t0 + SLOTS);
-      for (int q2 = b0; q2 < b1; ++q2)
-#pragma unroll
-        for (int p = 0; p < NP; ++p) acc[p] += sm.part[q2 - t0][p * 64 + lane];
-      __syncthreads();  // the partials are rewritten next step
-    }
-  } else {
-    for (int k = 0; k < mine; ++k)
-      dh_batch<T, NP, true>(W, sm.lst[wave], k * DH_BATCH, min(DH_BATCH, n - k * DH_BATCH), D,
-                            lane, nullptr, acc);
-  }
-  // The row keeps only its incomplete batch (at most DH_BATCH - 1 entries).
-  const int taken = mine * DH_BATCH;
-  const int keep = max(0, n - taken);
-  int2 e = make_int2(0, 0);
-  if (lane < keep) e = sm.lst[wave][taken + lane];
-  if (lane < keep) sm.lst[wave][lane] = e;
-  n = keep;
-}
-
-// The workgroup for batch row b and xb = FUSE_HALVES * range + half.
-template <typename T, typename O, int NP, int PER>
-__device__ __forceinline__ void dh_fused_body(DhSmem<PER, NP>& sm, const T* __restrict__ W,
-                                              const int2* __restrict__ comp,
-                                              const int* __restrict__ cnt,
-                                              const int* __restrict__ offs, O* __restrict__ dH,
-                                              int S, int D, int nvb, int64_t b, int xb,
-                                              int share) {
-  constexpr int NT = DhSmem<PER, NP>::NT;
-  int* pre = sm.pre;
-  int* lo_of = sm.lo_of;
-  int2* stage = sm.stage;
-  int* wsum = sm.wsum;
-  auto& lst = sm.lst;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int k = xb / FUSE_HALVES, nr = (S + FUSE_ROWS - 1) / FUSE_ROWS;
-  // >= S: no row (the wave still keeps the barriers and helps gather)
-  const int s = k * FUSE_ROWS + (xb % FUSE_HALVES) * FUSE_WAVES + wave;
-  // Run of block `blk`: ranks [offs[k], offs[k+1]) (the last range ends at the count).
-  int c[PER], sum = 0;
-  {
-    int lo[PER], hi[PER];
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      const int blk = min(PER * tid + q, nvb - 1);
-      const int64_t o = (b * nvb + blk) * nr + k;
-      lo[q] = offs[o];
-      hi[q] = k + 1 < nr ? offs[o + 1] : cnt[b * nvb + blk];
-    }
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      const int blk = PER * tid + q;
-      c[q] = blk < nvb ? hi[q] - lo[q] : 0;
-      if (blk < nvb) lo_of[blk] = lo[q];
-      sum += c[q];
-    }
-  }
-  int x = sum;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int y = __shfl_up(x, d);
-    if (lane >= d) x += y;
-  }
-  if (lane == 63) wsum[wave] = x;
-  __syncthreads();
-  int before = 0, total = 0;
-#pragma unroll
-  for (int w = 0; w < FUSE_WAVES; ++w) {
-    before += w < wave ? wsum[w] : 0;
-    total += wsum[w];
-  }
-  int run = before + x - sum;
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    pre[PER * tid + q] = run;
-    run += c[q];
-  }
-  __syncthreads();
-  f32x4 acc[NP];
-#pragma unroll
-  for (int p = 0; p < NP; ++p) acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int n = 0;  // entries in this wave's list (uniform)
-  int par = 0;
-  for (int t0 = 0; t0 < total; t0 += NT) {
-    const int t = t0 + tid;
-    if (t < total) {
-      int lo = 0, hi = nvb;  // pre[lo] <= t < pre[hi]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (pre[mid] <= t) lo = mid;
-        else hi = mid;
-      }
-      stage[tid] = comp[(b * nvb + lo) * 64 + lo_of[lo] + (t - pre[lo])];
-    }
-    __syncthreads();
-    const int here = min(NT, total - t0);
-    for (int i = 0; i * 64 < here; ++i) {
-      const int j = i * 64 + lane;
-      const int2 e = j < here ? stage[j] : make_int2(-1, 0);
-      const bool mine = j < here && (e.x >> FUSE_V_BITS) == s;
-      const uint64_t bal = __ballot(mine);
-      if (mine) lst[wave][n + __popcll(bal & ((1ull << lane) - 1ull))] = e;
-      n += __popcll(bal);
-      // If any row's list could overflow on the next 64 entries, gather the complete
-      // batches listed (workgroup-uniform decision).
-      if (i * 64 + 64 < here || t0 + NT < total) {
-        if (lane == 0) sm.full[par][wave] = n > FUSE_CAP - 64 ? 1 : 0;
-        __syncthreads();
-        int any = 0;
-#pragma unroll
-        for (int w = 0; w < FUSE_WAVES; ++w) any |= sm.full[par][w];
-        par ^= 1;
-        if (any) dh_gather<T, NP, PER>(sm, W, D, wave, lane, n, false, share, acc);
-      }
-    }
-    __syncthreads();  // stage is refilled next round
-  }
-  dh_gather<T, NP, PER>(sm, W, D, wave, lane, n, true, share, acc);
-  if (s < S) {
-    O* out = dH + (b * S + s) * D;
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int d = p * 256 + lane * 4;
-      if (d < D) store4(out + d, acc[p]);
-    }
-  }
-}
-
-// The fused path after the compaction: the dH workgroups (the first n_dh_x * B; the
-// long rows start first) and the staged dW workgroups (FUSE_DW_IDS ids each) in one
-// launch. The two read only the compaction and the inputs, so the dW work fills the
-// CUs while the dH workgroups with long rows finish.
-constexpr int FUSE_DW_IDS = 4 * FUSE_WAVES;
-template <typename T, typename O, int NP, typename RT, int PER>
-__global__ __launch_bounds__(64 * FUSE_WAVES) void bwd_fused_kernel(
-    const T* __restrict__ grad, const RT* __restrict__ reps, const int32_t* __restrict__ idx,
-    const void* __restrict__ mask, int mdt, const T* __restrict__ H, const T* __restrict__ W,
-    const int2* __restrict__ comp, const int* __restrict__ cnt, const int* __restrict__ offs,
-    O* __restrict__ dH, O* __restrict__ dW, O* __restrict__ dbias, int B, int S, int D, int V,
-    int nvb, int n_dh_x, int share) {
-  struct DwSmem {
-    float gl[FUSE_DW_IDS * DW_LD];
-    uint16_t sl[FUSE_DW_IDS * DW_LD];
-  };
-  union Smem {
-    DhSmem<PER, NP> h;
-    DwSmem w;
-  };
-  __shared__ Smem sm;
-  const int n_dh = n_dh_x * B;
-  if ((int)blockIdx.x < n_dh) {  // workgroup-uniform
-    dh_fused_body<T, O, NP, PER>(sm.h, W, comp, cnt, offs, dH, S, D, nvb, blockIdx.x / n_dh_x,
-                                 blockIdx.x % n_dh_x, share);
-  } else {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int v0 = ((int)blockIdx.x - n_dh) * FUSE_DW_IDS;
-    dw_stage<T, RT, FUSE_DW_IDS, FUSE_WAVES>(sm.w.gl, sm.w.sl, grad, reps, idx, mask, mdt, B, S,
-                                             V, v0, wave, lane);
-    __syncthreads();
-    dw_gather<T, O, NP, RT, FUSE_DW_IDS, FUSE_WAVES>(sm.w.gl, sm.w.sl, H, dW, dbias, B, S, D, V,
-                                                     v0, wave, lane);
-  }
-}
-
 // Register passes for a row of D elements (4 per lane, 256 per pass), capped at MAX_NP
 // (longer rows loop over D in chunks of MAX_NP * 256).
 static int passes_for(int64_t D) {
   return (int)std::min<int64_t>(MAX_NP, std::max<int64_t>(1, cdiv(D, 256)));
 }
 
-// Fused dH: a workgroup's waves share the gathering when one row holds more than this
-// many times the batches per wave (SPARTON_BWD_SHARE overrides it; tests use 0, always).
-static int dh_share() {
-  const char* e = getenv("SPARTON_BWD_SHARE");
-  return e != nullptr ? atoi(e) : 2;
+// Rows a dH workgroup takes: all its lane groups' worth once there are enough rows to fill the
+// chip, fewer (whose entries the groups share) below. Measured at 1024 fp32 rows of 424
+// entries: 16 / 4 / 1 rows 123 / 134 / 111 us, but at 4096 rows of 7: 11 / - / 48 us, so only
+// launches under 1024 rows give way.
+static int dh_rows_per_group(int64_t rows) {
+  return rows >= 1024 ? DH_GROUPS : rows >= 512 ? 4 : rows >= 256 ? 2 : 1;
 }
-// Rows with more entries than this go to bwd_dh_hot_kernel (SPARTON_BWD_HOT_MIN overrides
-// it; tests compare both).
+// SPARTON_BWD_HOT_MIN sets the number of entries past which a row is shared (tests compare
+// shared and unshared rows).
 static int dh_hot_min() {
   const char* e = getenv("SPARTON_BWD_HOT_MIN");
-  return e != nullptr ? atoi(e) : HOT_MIN;
+  return e != nullptr ? atoi(e) : -1;
 }
-// The five-kernel dH takes its long-row load groups for large vocabularies
-// (SPARTON_BWD_DH_LONG=1 forces them; tests compare the two).
-static bool dh_long_rows(int64_t V) {
-  const char* e = getenv("SPARTON_BWD_DH_LONG");
-  return V > FUSE_V_FAST || (e != nullptr && strcmp(e, "1") == 0);
-}
-// Register passes from which the many-rows dH launch also takes dW's workgroups.
-constexpr int DH_MERGE_NP = 6;
 // ---- few dH rows (B * S <= FEW_ROWS) ------------------------------------------------------
 //
 // With few dH rows every W row serves several of them (config 1: each of the 30522 ids is
@@ -1703,16 +1157,12 @@ __global__ __launch_bounds__(64 * FEW_SUM_WAVES) void bwd_few_sum_kernel(
   }
 }
 
-// The five-kernel path runs dW in the dH launch where it can (SPARTON_BWD_DW_MERGE=0 keeps
-// it a separate launch; tests compare the two).
+// dW's workgroups run in the bucketing's launch
+// (SPARTON_BWD_DW_MERGE=0 keeps them apart; tests compare the two).
+constexpr int64_t DW_MERGE_S = 1024;
 static bool dw_merge_on() {
   const char* e = getenv("SPARTON_BWD_DW_MERGE");
   return e == nullptr || strcmp(e, "0") != 0;
-}
-// SPARTON_BWD_PATH=five forces the five-kernel path (tests compare the two paths).
-static bool fused_path_enabled() {
-  const char* e = getenv("SPARTON_BWD_PATH");
-  return e == nullptr || strcmp(e, "five") != 0;
 }
 
 // The wide staged dW with 16 ids per workgroup (B <= DW_WIDE_B), for 16-bit types: fp32
@@ -1737,11 +1187,6 @@ template <typename T, typename O, int NP, typename RT>
 static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void* mask,
                         int mdt, const T* H, const T* W, O* dH, O* dW, O* dbias, void* ws,
                         int64_t B, int64_t S, int64_t D, int64_t V, hipStream_t st) {
-  constexpr int FNP = NP <= FuseMaxNp<T>::value ? NP : FuseMaxNp<T>::value;
-  // The fused path stages, per (b, 16-row range), a prefix over every 64-id block, and
-  // gives each dH row one wave: it needs many ranges and few blocks. Measured on MI355X:
-  // B = 32, S = 256, V = 30522: fused 61 us vs 65 us; B = 2, S = 32 (dense grads):
-  // 1133 us vs 331 us; V = 250002: 753 us vs 460 us.
   const FewPlan few = few_plan(B, S, D, V);
   if (few.fits && few_enabled() && dH != nullptr) {
     float* part = (float*)ws;
@@ -1754,144 +1199,50 @@ static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void*
                        (const float*)part, dH, n, few.ranges);
     return;
   }
-  const bool fused = fused_path_enabled() && dH != nullptr && dW != nullptr && B * S > 0 &&
-                     D > 0 && V > 0 &&
-                     B <= DW_STAGE_B && S <= FUSE_MAX_S && V <= FUSE_V_FAST &&
-                     B * cdiv(S, FUSE_ROWS) >= FUSE_MIN_RANGES &&
-                     D <= (int64_t)FNP * 256;
-  if (fused) {
-    const Layout L = layout(B, S, V);
-    int2* comp = (int2*)((char*)ws + L.list);
-    int* cnt = (int*)((char*)ws + L.cnt64);
-    int* offs = (int*)((char*)ws + L.off64);
-    const int nvb = (int)cdiv(V, 64);
-    hipLaunchKernelGGL((bwd_compact_kernel<T, RT>), dim3((unsigned)nvb, (unsigned)cdiv(B, 8)), dim3(256),
-                       0, st, g, r, idx, mask, mdt, (int)B, (int)S, (int)V, comp, cnt, offs);
-    const int n_dh_x = (int)(FUSE_HALVES * cdiv(S, FUSE_ROWS));
-    const dim3 grid((unsigned)(n_dh_x * B + cdiv(V, FUSE_DW_IDS)));
-#define FUSED(PER)                                                                                  \
-  hipLaunchKernelGGL((bwd_fused_kernel<T, O, FNP, RT, PER>), grid, dim3(64 * FUSE_WAVES), 0, st, g,  \
-                     r, idx, mask, mdt, H, W, (const int2*)comp, (const int*)cnt, (const int*)offs, \
-                     dH, dW, dbias, (int)B, (int)S, (int)D, (int)V, nvb, n_dh_x, dh_share())
-    if (nvb <= 64 * FUSE_WAVES) FUSED(1);
-    else FUSED(FUSE_MAX_NVB / (64 * FUSE_WAVES));
-#undef FUSED
-    return;
-  }
-  bool merged_dw = false;
+  constexpr int DNP = DwPasses<T, NP>::value;
+  const bool need_dw = (dW != nullptr || dbias != nullptr) && V > 0;
+  const bool staged = B <= DW_STAGE_B && S <= DW_STAGE_S;
+  const size_t dw_lds = (size_t)DW_IDS * DW_LD * 6;
+  const int n_dw = need_dw && staged ? (int)cdiv(V, DW_IDS) : 0;
+  bool dw_done = false;
   if (dH != nullptr && B * S > 0 && D > 0) {
-    // Batch rows in chunks of at most MAX_B and positions in windows of at most MAX_S:
-    // each pass runs count -> scan -> scatter -> dH over rows [b0, b0 + nb) and
-    // positions [s0, s0 + sw), with entries whose index lies outside the window
-    // inactive, so every dH row is written by exactly one pass. The workspace holds
-    // one pass; the passes reuse it in stream order.
-    const int64_t Bc = std::min<int64_t>(B, MAX_B), Sc = std::min<int64_t>(S, MAX_S);
+    // Batch rows in chunks and positions in windows (pass_b, pass_s): each pass buckets the
+    // entries of rows [b0, b0 + nb) and positions [s0, s0 + sw) (entries whose index lies
+    // outside the window are inactive) and sums its dH rows, so every dH row is written by
+    // exactly one pass. The workspace holds one pass; the passes reuse it in stream order.
+    const int64_t Bc = pass_b(B, S), Sc = pass_s(S);
     const Layout L = layout(Bc, Sc, V);
-    int* hist = (int*)((char*)ws + L.hist);
-    int* seg_start = (int*)((char*)ws + L.seg_start);
-    int* seg_cnt = (int*)((char*)ws + L.seg_cnt);
-    int2* list = (int2*)((char*)ws + L.list);
-    int2* comp = (int2*)((char*)ws + L.comp);
-    int* ccount = (int*)((char*)ws + L.ccount);
-    int* hot = (int*)((char*)ws + L.hot);
-    const int hot_min = dh_hot_min();
-    // One pass and a staged dW: dW's workgroups join the dH launch when that launch
-    // does not take dW's occupancy away. Measured (backward, one box): few rows (config
-    // 1, split dH) 78.9 -> 73.6 us; wide rows (config 5, D = 4096: 182 VGPRs for dH
-    // against 107 for dW) 520 -> 504 us; but config 4 (D = 768, long rows: dH at 125
-    // VGPRs, dW at 58) 328 -> 346 us, so rows under DH_MERGE_NP passes keep two launches.
-    const bool few_rows = B * S < SPLIT_ROWS;
-    merged_dw = (dW != nullptr || dbias != nullptr) && V > 0 && B <= Bc && S <= Sc &&
-                B <= DW_STAGE_B && S <= DW_STAGE_S && L.nch > 0 && dw_merge_on() &&
-                (few_rows || DhPasses<NP>::value >= DH_MERGE_NP);
+    const Cut c = cut_ids(V);
+    int* off = (int*)((char*)ws + L.off);
+    int2* run = (int2*)((char*)ws + L.run);
+    const int64_t n_slices = cdiv(D, Chunk<T>::COLS);
     for (int64_t b0 = 0; b0 < B; b0 += Bc) {
       const int64_t nb = std::min(Bc, B - b0);
-      const T* gb = g + b0 * V;
-      const RT* rb = r + b0 * V;
-      const int32_t* ib = idx + b0 * V;
       for (int64_t s0 = 0; s0 < S; s0 += Sc) {
         const int64_t sw = std::min(Sc, S - s0);
-        O* dhb = dH + (b0 * S + s0) * D;
-        const int wpb = waves_for(sw);
-        const dim3 cgrid((unsigned)cdiv(L.nch, wpb), (unsigned)nb);
-        const size_t cl = (size_t)sw * 4 * (1 + wpb);
-        if (L.nch > 0)
-          hipLaunchKernelGGL((bwd_count_kernel<T, RT>), cgrid, dim3(64 * wpb), cl, st, gb, rb, ib,
-                             mask, mdt, (int)sw, (int)V, (int)L.nch, hist, comp, ccount, (int)s0,
-                             b0, (int)S, hot);
-        if (sw <= SCAN_THREADS / 2)
-          hipLaunchKernelGGL(bwd_scan_parts_kernel, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st,
-                             hist, seg_start, seg_cnt, (int)sw, (int)L.nch, (int)round_up(sw, 64),
-                             hot, hot_min);
-        else
-          hipLaunchKernelGGL(bwd_scan_kernel, dim3((unsigned)nb),
-                             dim3((unsigned)std::min<int64_t>(SCAN_THREADS, round_up(sw, 64))), 0, st,
-                             hist, seg_start, seg_cnt, (int)sw, (int)L.nch, hot, hot_min);
-        if (L.nch > 0)
-          hipLaunchKernelGGL(bwd_scatter_kernel, cgrid, dim3(64 * wpb), (size_t)sw * 4 * wpb, st, ib,
-                             (int)sw, (int)V, (int)L.nch, (const int*)hist, (const int2*)comp,
-                             (const int*)ccount, list, (int)s0);
-        if (nb * sw < SPLIT_ROWS) {
-          const int64_t ns = cdiv(D, 256);
-          if (merged_dw)
-            hipLaunchKernelGGL((bwd_dh_split_dw_kernel<T, O, DwPasses<T, NP>::value, RT>),
-                               dim3((unsigned)(nb * sw * ns + cdiv(V, 4 * SPLIT_WAVES))),
-                               dim3(64 * SPLIT_WAVES), 0, st, W, (const int2*)list,
-                               (const int*)seg_start, (const int*)seg_cnt, dhb, (int)B, (int)S,
-                               (int)D, (int)V, (int)ns, (int)(nb * sw * ns), g, r, idx, mask, mdt,
-                               H, dW, dbias);
-          else
-            hipLaunchKernelGGL((bwd_dh_split_kernel<T, O>), dim3((unsigned)(nb * sw * ns)),
-                               dim3(64 * SPLIT_WAVES), 0, st, W, (const int2*)list,
-                               (const int*)seg_start, (const int*)seg_cnt, dhb, (int)nb, (int)sw,
-                               (int)D, (int)V, (int)S, (int)ns);
-        } else if (merged_dw) {
-          if constexpr (DhPasses<NP>::value >= DH_MERGE_NP) {
-            const int n_dh = (int)cdiv(nb * sw, 4);
-            const dim3 grid((unsigned)(n_dh + cdiv(V, 16)));
-            if (dh_long_rows(V))
-              hipLaunchKernelGGL((bwd_dh_dw_kernel<T, O, DhPasses<NP>::value, true, DwPasses<T, NP>::value, RT>),
-                                 grid, dim3(256), 0, st, W, (const int2*)list, (const int*)seg_start,
-                                 (const int*)seg_cnt, dhb, (int)B, (int)S, (int)D, (int)V, hot_min,
-                                 n_dh, g, r, idx, mask, mdt, H, dW, dbias);
-            else
-              hipLaunchKernelGGL((bwd_dh_dw_kernel<T, O, DhPasses<NP>::value, false, DwPasses<T, NP>::value, RT>),
-                                 grid, dim3(256), 0, st, W, (const int2*)list, (const int*)seg_start,
-                                 (const int*)seg_cnt, dhb, (int)B, (int)S, (int)D, (int)V, hot_min,
-                                 n_dh, g, r, idx, mask, mdt, H, dW, dbias);
-          }
-          if (L.nch > 0)
-            hipLaunchKernelGGL((bwd_dh_hot_kernel<T, O>), dim3(HOT_GRID), dim3(64 * HOT_WAVES), 0, st, W,
-                               (const int2*)list, (const int*)seg_start, (const int*)seg_cnt,
-                               (const int*)hot, dhb, (int)sw, (int)D, (int)V, (int)S,
-                               (int)cdiv(D, 256));
-        } else {
-          if (dh_long_rows(V))
-            hipLaunchKernelGGL((bwd_dh_kernel<T, O, DhPasses<NP>::value, true>), dim3((unsigned)cdiv(nb * sw, 4)),
-                               dim3(256), 0, st, W, (const int2*)list, (const int*)seg_start,
-                               (const int*)seg_cnt, dhb, (int)nb, (int)sw, (int)D, (int)V, (int)S,
-                               hot_min);
-          else
-            hipLaunchKernelGGL((bwd_dh_kernel<T, O, DhPasses<NP>::value, false>), dim3((unsigned)cdiv(nb * sw, 4)),
-                               dim3(256), 0, st, W, (const int2*)list, (const int*)seg_start,
-                               (const int*)seg_cnt, dhb, (int)nb, (int)sw, (int)D, (int)V, (int)S,
-                               hot_min);
-          // The rows bwd_dh_kernel left (listed by the scan; the count kernel zeroed the list).
-          if (L.nch > 0)
-            hipLaunchKernelGGL((bwd_dh_hot_kernel<T, O>), dim3(HOT_GRID), dim3(64 * HOT_WAVES), 0, st, W,
-                               (const int2*)list, (const int*)seg_start, (const int*)seg_cnt,
-                               (const int*)hot, dhb, (int)sw, (int)D, (int)V, (int)S,
-                               (int)cdiv(D, 256));
-        }
+        const int nbk = (int)(nb * c.runs);
+        // dW's workgroups join where the bucketing's counters take little more LDS than dW's.
+        const bool with_dw = n_dw > 0 && S <= DW_MERGE_S && nb == B && dw_merge_on();
+        const size_t lds = (size_t)(BK_WAVES + 1 + (BK_WAVES + 1) * sw) * 4;
+        hipLaunchKernelGGL((bwd_bucket_dw_kernel<T, O, DNP, RT>), dim3((unsigned)(nbk + (with_dw ? n_dw : 0))),
+                           dim3(64 * BK_WAVES), with_dw ? std::max(lds, dw_lds) : lds, st, g + b0 * V,
+                           r + b0 * V, idx + b0 * V, (const char*)mask + b0 * S * mask_elem_bytes(mdt), mdt,
+                           H, dW, dbias, (int)B, (int)S, (int)D, (int)V, nbk, (int)c.runs, (int)c.cap,
+                           (int)s0, (int)sw, off, run);
+        dw_done |= with_dw;
+        const int rpw = dh_rows_per_group(nb * sw);
+        hipLaunchKernelGGL((bwd_dh_kernel<T, O>), dim3((unsigned)(cdiv(nb * sw, rpw) * n_slices)),
+                           dim3(64 * DH_WAVES), 0, st, W, (const int*)off, (const int2*)run,
+                           dH + (b0 * S + s0) * D, (int)nb, (int)sw, (int)D, (int)c.runs, (int)c.cap,
+                           (int)S, (int)n_slices, rpw, dh_hot_min());
       }
     }
   }
-  if ((dW != nullptr || dbias != nullptr) && V > 0 && !merged_dw) {
-    constexpr int DNP = DwPasses<T, NP>::value;
-    if (B <= DW_STAGE_B && S <= DW_STAGE_S)
-      hipLaunchKernelGGL((bwd_dw_staged_kernel<T, O, DNP, RT>),
-                         dim3((unsigned)cdiv(V, 64)), dim3(64 * DW_WAVES), 0,
-                         st, g, r, idx, mask, mdt, H, dW, dbias, (int)B, (int)S, (int)D, (int)V);
+  if (need_dw && !dw_done) {
+    if (staged)
+      hipLaunchKernelGGL((bwd_bucket_dw_kernel<T, O, DNP, RT>), dim3((unsigned)n_dw), dim3(64 * BK_WAVES),
+                         dw_lds, st, g, r, idx, mask, mdt, H, dW, dbias, (int)B, (int)S, (int)D, (int)V,
+                         0, 1, 0, 0, 0, nullptr, nullptr);
     else if (B <= DW_WIDE_IDS_ROWS / 64 && S <= DW_STAGE_S)
       hipLaunchKernelGGL((bwd_dw_wide_kernel<T, O, DNP, RT, 64>), dim3((unsigned)cdiv(V, 64)),
                          dim3(64 * DW_WAVES), 0, st, g, r, idx, mask, mdt, H, dW, dbias, (int)B,
@@ -1943,7 +1294,7 @@ extern "C" __attribute__((visibility("default"))) size_t sparton_bwd_workspace_b
     int64_t B, int64_t S, int64_t D, int64_t V) {
   if (B <= 0 || S <= 0 || D <= 0 || V < 0) return 0;
   const bwd::FewPlan few = bwd::few_plan(B, S, D, V);
-  return std::max(bwd::pass_layout(B, S, V).total, few.fits ? few.part_bytes : (size_t)0);
+  return std::max(bwd::layout(bwd::pass_b(B, S), bwd::pass_s(S), V).total, few.fits ? few.part_bytes : (size_t)0);
 }
 
 extern "C" __attribute__((visibility("default"))) int sparton_bwd(

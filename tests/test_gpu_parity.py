@@ -332,6 +332,36 @@ def test_backward_hot_rows_five_kernel(case, device, monkeypatch):
     check_bwd_isolated(H, W, b, m, G, reps32, idx, *hot)
 
 
+@pytest.mark.parametrize("case", [
+    ("bf16", 70, 4, 136, 3000, True, "int64"),      # 280 rows: 2 a workgroup; a slice of one chunk
+    ("fp16", 5, 120, 72, 9000, False, "holes"),     # 600 rows: 4 a workgroup; 3 runs of ids
+    ("fp32", 9, 131, 68, 40000, True, "int64"),     # 1179 rows: 16 a workgroup, the last ragged; 10 runs
+    ("bf16", 2, 5000, 16, 300, True, "int64"),      # two windows of positions
+    ("fp16", 1, 90, 40, 70000, True, "int64"),      # two turns per bucketing wave; 1 row a workgroup
+    ("bf16", 3, 30, 2056, 130, True, "holes"),      # 17 slices, the last of one chunk
+], ids=lambda c: "-".join(map(str, c)))
+def test_backward_row_sharing(case, device, monkeypatch):
+    """dH at the edges of its bucketing and its workgroups: rows shared by a workgroup's lane
+    groups, or never (SPARTON_BWD_HOT_MIN past every row), or always (0), are the same bits,
+    and the oracle's."""
+    say(f"dH row sharing, case {case}")
+    H, W, b, m, G = make_case(*case)
+    Hd, Wd, md, Gd = H.to(device), W.to(device), m.to(device), G.to(device)
+    bd = None if b is None else b.to(device)
+    _, idx, reps32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
+    runs = []
+    for hot_min in (None, "0", str(2 ** 30)):
+        if hot_min is not None:
+            monkeypatch.setenv("SPARTON_BWD_HOT_MIN", hot_min)
+        runs.append([None if t is None else t.clone()
+                     for t in torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)])
+    torch.cuda.synchronize()
+    for out in runs[1:]:
+        for a, c in zip(runs[0], out):
+            assert (a is None and c is None) or torch.equal(a, c)
+    check_bwd_isolated(H, W, b, m, G, reps32, idx, *runs[0])
+
+
 def test_graph_capture_replays(device):
     """Forward and backward captured into one HIP graph (all of their kernels and workspace
     allocations) replay to the eager results, bitwise, with eager work and synchronizations
