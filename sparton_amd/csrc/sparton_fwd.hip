@@ -17,6 +17,9 @@
 // for 256 live rows instead of one batch row's (often partly padded) 256 positions,
 // and a batch row wastes less than 16 rows of padding.
 //
+// fp32 batches past the small-batch kernel run on fp16 MFMAs (fwd_split_rows_kernel): H and W
+// as exact pairs of fp16, three products per value.
+//
 // Main kernel. A "unit" is one M-tile x one vocab tile of BN columns. The grid is
 // persistent (one workgroup per CU) and each workgroup walks its units in rounds; for
 // each it computes the 256 x BN logit tile with bf16/fp16 (or fp32) MFMA, K = D
@@ -435,6 +438,8 @@ struct __align__(16) UnitMeta {
   int grp_s[NGRP];           // first position of each group (16 j)
   int mask_binary;           // every maskf value is 0 or 1
   float bias[BN];            // bias of the tile's columns (0 past V or without bias)
+  int rexp[BM];              // fp32 operands as fp16 pairs: the scales' exponents, negated, of
+  int cexp[BN];              // the tile's rows and columns
 };
 
 struct Smem {
@@ -582,11 +587,15 @@ __device__ __forceinline__ void unit_tile(int u, int n_mt, int n_vt, int* m, int
 }
 
 // Launch-wide, wave-uniform parameters.
-template <typename T>
+// T: the operands' type; O: the type of bias and reps. PAIR: the operands are fp32 values
+// split into pairs of fp16 (split_rows_kernel below), H's rows in tile-row order.
+template <typename T, typename O, bool PAIR>
 struct Args {
   const char* H;      // H[0, 0, :]
   const char* W;
-  const T* bias;
+  const O* bias;
+  const int* rexp;       // PAIR: [n_mt * BM]
+  const int* cexp;       // PAIR: [V]
   const float* rowmask;  // [n_mt * BM] mask of each tile row
   const int* list;
   int n_grp;          // active groups
@@ -596,6 +605,18 @@ struct Args {
   int nk_full;        // slabs lying entirely inside the row
   int nk;             // slabs per unit
   int V;
+  int part_bytes;     // PAIR: bytes of a row's hi (or lo) part
+  // Byte offsets of K slab k in a row of A and of W. A PAIR product runs over K three times:
+  // lo x hi, hi x lo, hi x hi.
+  __device__ __forceinline__ void slab_at(int k, uint32_t* ka, uint32_t* kb) const {
+    *ka = *kb = (uint32_t)k * SLAB;
+    if constexpr (PAIR) {
+      const uint32_t part = (uint32_t)part_bytes;
+      const uint32_t at = *ka;  // bytes into the three runs
+      *ka = at < part ? at + part : at < 2 * part ? at - part : at - 2 * part;
+      *kb = at < part ? at : at < 2 * part ? at : at - 2 * part;
+    }
+  }
 };
 
 // One unit as the copy waves see it.
@@ -646,6 +667,17 @@ __device__ __forceinline__ void row_offsets(const UnitMeta& um, int n_valid, int
   }
 }
 
+// The same for rows in tile order (PAIR): tile row 256 m + r lies at that row.
+__device__ __forceinline__ void pair_row_offsets(int m, int n_valid, int row_bytes, int c, int lane,
+                                                 uint32_t* a_off) {
+#pragma unroll
+  for (int i = 0; i < A_LOADS; ++i) {
+    const int row = (i * COPY_WAVES + c) * ROWS_PER_LOAD + (lane >> 3);
+    const int r = min(row / GROUP, n_valid - 1) * GROUP + row % GROUP;
+    a_off[i] = (uint32_t)(m * BM + r) * (uint32_t)row_bytes + lane_chunk(row, lane);
+  }
+}
+
 // Raw loads for the in-loop prefetch: the bits are loaded without any conversion or
 // select, and converted two K steps later, after the steps' drains.
 template <typename T> __device__ __forceinline__ uint32_t load_bits(const T* p, int64_t i);
@@ -675,16 +707,17 @@ template <> __device__ __forceinline__ float bits_to_f32<float>(uint32_t x) { re
 // before use (a zero W times a finite H adds exactly 0). W rows past V re-read row V-1
 // (never stored). Rows of groups past the last active one (n_valid) re-read a row of the
 // last active group (their keys are never used), so every copy is issued unconditionally.
-template <typename T, bool TAIL>
-__device__ __forceinline__ void issue_slab_k(Smem& sm, const Args<T>& a, const CopyUnit& cu, int k,
+template <bool TAIL, typename A>
+__device__ __forceinline__ void issue_slab_k(Smem& sm, const A& a, const CopyUnit& cu, int k,
                                              int buf, int c, int lane) {
-  const uint32_t kb = (uint32_t)k * SLAB;
+  uint32_t ka, kb;
+  a.slab_at(k, &ka, &kb);
 #pragma unroll
   for (int i = 0; i < A_LOADS; ++i) {
     const int grp = i * COPY_WAVES + c;
     const uint32_t c16 = lane_chunk(grp * ROWS_PER_LOAD + (lane >> 3), lane);
     // a_off includes c16: adding 0 - c16 (mod 2^32) lands on the row's first chunk.
-    const uint32_t step = (!TAIL || kb + c16 < (uint32_t)a.row_bytes) ? kb : 0u - c16;
+    const uint32_t step = (!TAIL || ka + c16 < (uint32_t)a.row_bytes) ? ka : 0u - c16;
     __builtin_amdgcn_global_load_lds((const void*)(a.H + (cu.a_off[i] + step)),
                                      (lds_void*)&sm.a[buf][grp * 64], 16, 0, 0);
   }
@@ -700,11 +733,11 @@ __device__ __forceinline__ void issue_slab_k(Smem& sm, const Args<T>& a, const C
     __builtin_amdgcn_global_load_lds((const void*)(bb + off), (lds_void*)&sm.b[buf][grp * 64], 16, 0, 0);
   }
 }
-template <typename T>
-__device__ __forceinline__ void issue_slab(Smem& sm, const Args<T>& a, const CopyUnit& cu, int k,
+template <typename A>
+__device__ __forceinline__ void issue_slab(Smem& sm, const A& a, const CopyUnit& cu, int k,
                                            int buf, int c, int lane) {
-  if (k >= a.nk_full) issue_slab_k<T, true>(sm, a, cu, k, buf, c, lane);
-  else issue_slab_k<T, false>(sm, a, cu, k, buf, c, lane);
+  if (k >= a.nk_full) issue_slab_k<true>(sm, a, cu, k, buf, c, lane);
+  else issue_slab_k<false>(sm, a, cu, k, buf, c, lane);
 }
 
 // Zero the W chunks of slab k (in stage buf) that lie past D; each copy wave clears the
@@ -842,8 +875,8 @@ struct Outputs {
 
 // Start a unit without prefetch: fetch its metadata into um, write the previous unit's
 // results (prev.u >= 0, metadata in um_prev), and land its first two slabs. Two barriers.
-template <typename T>
-__device__ __forceinline__ void copy_start(Smem& sm, const Args<T>& a, const Outputs<T>& o,
+template <typename T, typename O, bool PAIR>
+__device__ __forceinline__ void copy_start(Smem& sm, const Args<T, O, PAIR>& a, const Outputs<O>& o,
                                            UnitMeta& um, CopyUnit& cu, int buf,
                                            const Unit& prev, const UnitMeta& um_prev, int ct,
                                            int c, int lane) {
@@ -851,19 +884,24 @@ __device__ __forceinline__ void copy_start(Smem& sm, const Args<T>& a, const Out
   const float mv = a.rowmask[(int64_t)cu.m * BM + ct];
   const int col = cu.v0 + ct;
   const float bv = (a.bias != nullptr && col < a.V) ? to_f32(a.bias[col]) : 0.0f;
+  if constexpr (PAIR) {
+    um.rexp[ct] = a.rexp[(int64_t)cu.m * BM + ct];
+    um.cexp[ct] = a.cexp[min(col, a.V - 1)];
+  }
   put_groups(um, code, a.ngrp, ct);
   um.maskf[ct] = mv;
   um.bias[ct] = bv;
   if (ct == 0) um.mask_binary = 1;
   lds_barrier();  // S1
-  row_offsets(um, cu.n_valid, a.S, a.row_bytes, c, lane, cu.a_off);
+  if constexpr (PAIR) pair_row_offsets(cu.m, cu.n_valid, a.row_bytes, c, lane, cu.a_off);
+  else row_offsets(um, cu.n_valid, a.S, a.row_bytes, c, lane, cu.a_off);
   if (a.nk > 0) {
     issue_slab(sm, a, cu, 0, buf, c, lane);
     issue_slab(sm, a, cu, 1, buf ^ 1, c, lane);
   }
   put_mask_words(um, mv, ct, lane);
   if (prev.u >= 0)
-    write_unit<T>(sm, um_prev, prev.m, prev.v0, a.V, prev.n_valid, ct, o.reps, o.argmax,
+    write_unit<O>(sm, um_prev, prev.m, prev.v0, a.V, prev.n_valid, ct, o.reps, o.argmax,
                   o.reps_f32, o.part);
   wait_all();
   if (a.nk > 0) {
@@ -873,8 +911,8 @@ __device__ __forceinline__ void copy_start(Smem& sm, const Args<T>& a, const Out
   lds_barrier();  // S2
 }
 
-template <typename T>
-__device__ void copy_path(Smem& sm, const Args<T>& a, const Outputs<T>& o, int w, int G,
+template <typename T, typename O, bool PAIR>
+__device__ void copy_path(Smem& sm, const Args<T, O, PAIR>& a, const Outputs<O>& o, int w, int G,
                           int n_units, int n_mt, int n_vt, int ct, int c, int lane) {
   const int nk = a.nk;
   Unit cur = unit_of(w, 0, G, n_units, n_mt, n_vt, a.n_grp);
@@ -895,13 +933,18 @@ __device__ void copy_path(Smem& sm, const Args<T>& a, const Outputs<T>& o, int w
     float mv;
     int code;
     uint32_t bias;
+    int rexp, cexp;
   };
   auto load_meta = [&](const Unit& x) {
-    MetaRegs mr{0.0f, 0, 0u};
+    MetaRegs mr{0.0f, 0, 0u, 0, 0};
     if (x.u >= 0 && nk >= PREFETCH_MIN_NK) {
       mr.mv = a.rowmask[(int64_t)x.m * BM + ct];
       mr.code = a.list[min(max(group_entry(x.m, min(ct, NGRP + 1)), 0), a.n_grp - 1)];
       if (a.bias != nullptr) mr.bias = load_bits(a.bias + min(x.v0 + ct, a.V - 1), 0);
+      if constexpr (PAIR) {
+        mr.rexp = a.rexp[(int64_t)x.m * BM + ct];
+        mr.cexp = a.cexp[min(x.v0 + ct, a.V - 1)];
+      }
     }
     return mr;
   };
@@ -932,13 +975,18 @@ __device__ void copy_path(Smem& sm, const Args<T>& a, const Outputs<T>& o, int w
           um_next.maskf[ct] = meta.mv;
           put_mask_words(um_next, meta.mv, ct, lane);
           const int col = nx.v0 + ct;
-          um_next.bias[ct] = (a.bias != nullptr && col < a.V) ? bits_to_f32<T>(meta.bias) : 0.0f;
+          um_next.bias[ct] = (a.bias != nullptr && col < a.V) ? bits_to_f32<O>(meta.bias) : 0.0f;
+          if constexpr (PAIR) {
+            um_next.rexp[ct] = meta.rexp;
+            um_next.cexp[ct] = meta.cexp;
+          }
         } else if (k == 3) {
-          row_offsets(um_next, nx.n_valid, a.S, a.row_bytes, c, lane, nx.a_off);
+          if constexpr (PAIR) pair_row_offsets(nx.m, nx.n_valid, a.row_bytes, c, lane, nx.a_off);
+          else row_offsets(um_next, nx.n_valid, a.S, a.row_bytes, c, lane, nx.a_off);
         }
       }
       if (k == 1 && prev.u >= 0) {
-        write_unit<T>(sm, um_next, prev.m, prev.v0, a.V, prev.n_valid, ct, o.reps, o.argmax,
+        write_unit<O>(sm, um_next, prev.m, prev.v0, a.V, prev.n_valid, ct, o.reps, o.argmax,
                       o.reps_f32, o.part);
         prev.u = -1;
       }
@@ -957,7 +1005,7 @@ __device__ void copy_path(Smem& sm, const Args<T>& a, const Outputs<T>& o, int w
     if (pre) meta = load_meta(next2);
     lds_barrier();  // E: the compute waves' keys are written
     if (next.u < 0) {
-      write_unit<T>(sm, sm.um[par], cur.m, cur.v0, a.V, cur.n_valid, ct, o.reps, o.argmax,
+      write_unit<O>(sm, sm.um[par], cur.m, cur.v0, a.V, cur.n_valid, ct, o.reps, o.argmax,
                     o.reps_f32, o.part);
       return;
     }
@@ -978,7 +1026,7 @@ __device__ void copy_path(Smem& sm, const Args<T>& a, const Outputs<T>& o, int w
 
 // Mainloop + block epilogue of one unit for a compute wave with JM blocks (JM = 0: the
 // wave only keeps the barrier schedule). Stage buf holds the unit's slab 0.
-template <typename T, int JM>
+template <typename T, bool PAIR, int JM>
 __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int nk, int buf,
                                              int lane, int wm, int wn) {
   constexpr int JA = JM > 0 ? JM : 1;
@@ -989,7 +1037,8 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
   f32x16 acc[JA][NB_PER_WAVE];
 #pragma unroll
   for (int nb = 0; nb < NB_PER_WAVE; ++nb) {
-    const float bv = um.bias[wn * 64 + nb * 32 + l32];
+    float bv = PAIR ? 0.0f : um.bias[wn * 64 + nb * 32 + l32];  // (PAIR adds it unscaled, below)
+    if constexpr (PAIR) asm("" : "+v"(bv));  // a register like the bias: a constant costs spills
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[JA - 1][nb][i] = bv;
     if (nk == 0) {  // no MFMAs: x = bias
@@ -1097,6 +1146,19 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
   const float* mrow = &um.maskf[wm * 32 + 4 * h];
   const int* wrow = &um.maskw[wm * 32 + 4 * h];
   int* kw = &sm.key[2 * wm][wn * 64 + l32];
+  if constexpr (PAIR) __builtin_amdgcn_sched_barrier(0);  // (keeps the reads below out of the K loop's registers)
+  // PAIR: x = acc 2^(row exponent + column exponent) + bias.
+  const int* rrow = &um.rexp[wm * 32 + 4 * h];
+  int ce[NB_PER_WAVE];
+  float cb[NB_PER_WAVE];
+#pragma unroll
+  for (int nb = 0; nb < NB_PER_WAVE; ++nb) {
+    ce[nb] = PAIR ? um.cexp[wn * 64 + nb * 32 + l32] : 0;
+    cb[nb] = PAIR ? um.bias[wn * 64 + nb * 32 + l32] : 0.0f;
+  }
+  auto logit = [&](float x, int re, int nb) {
+    return PAIR ? __builtin_amdgcn_ldexpf(x, re + ce[nb]) + cb[nb] : x;
+  };
 #pragma unroll
   for (int j = 0; j < JM; ++j) {
     int kmax[2][NB_PER_WAVE];
@@ -1108,23 +1170,27 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const i32x4 w4 = *(const i32x4*)(wrow + j * WAVES_M * 32 + 8 * q);
+        const i32x4 r4 = PAIR ? *(const i32x4*)(rrow + j * WAVES_M * 32 + 8 * q) : i32x4{0, 0, 0, 0};
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
           for (int nb = 0; nb < NB_PER_WAVE; ++nb)
-            kmax[q >> 1][nb] = max(kmax[q >> 1][nb],
-                                   (__float_as_int(acc[j][nb][q * 4 + e]) & w4[e]) | (31 - 8 * q - e));
+            kmax[q >> 1][nb] =
+                max(kmax[q >> 1][nb],
+                    (__float_as_int(logit(acc[j][nb][q * 4 + e], r4[e], nb)) & w4[e]) | (31 - 8 * q - e));
       }
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const f32x4 m4 = *(const f32x4*)(mrow + j * WAVES_M * 32 + 8 * q);
+        const i32x4 r4 = PAIR ? *(const i32x4*)(rrow + j * WAVES_M * 32 + 8 * q) : i32x4{0, 0, 0, 0};
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
           for (int nb = 0; nb < NB_PER_WAVE; ++nb)
-            kmax[q >> 1][nb] = max(kmax[q >> 1][nb],
-                                   (__float_as_int(acc[j][nb][q * 4 + e] * m4[e]) & ~31) | (31 - 8 * q - e));
+            kmax[q >> 1][nb] =
+                max(kmax[q >> 1][nb],
+                    (__float_as_int(logit(acc[j][nb][q * 4 + e], r4[e], nb) * m4[e]) & ~31) | (31 - 8 * q - e));
       }
     }
 #pragma unroll
@@ -1143,8 +1209,8 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
   lds_barrier();  // E
 }
 
-template <typename T>
-__device__ void compute_path(Smem& sm, const Args<T>& a, int w, int G, int n_units, int n_mt,
+template <typename T, typename O, bool PAIR>
+__device__ void compute_path(Smem& sm, const Args<T, O, PAIR>& a, int w, int G, int n_units, int n_mt,
                              int n_vt, int wave, int lane) {
   const int nk = a.nk;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -1158,11 +1224,11 @@ __device__ void compute_path(Smem& sm, const Args<T>& a, int w, int G, int n_uni
     const int n_blocks = (cur.n_valid + 1) / 2;  // 32-row blocks with an active group
     const int jm = n_blocks <= wm ? 0 : min(4, (n_blocks - wm + 1) / WAVES_M);
     switch (jm) {
-      case 0: compute_unit<T, 0>(sm, um, nk, buf, lane, wm, wn); break;
-      case 1: compute_unit<T, 1>(sm, um, nk, buf, lane, wm, wn); break;
-      case 2: compute_unit<T, 2>(sm, um, nk, buf, lane, wm, wn); break;
-      case 3: compute_unit<T, 3>(sm, um, nk, buf, lane, wm, wn); break;
-      default: compute_unit<T, 4>(sm, um, nk, buf, lane, wm, wn); break;
+      case 0: compute_unit<T, PAIR, 0>(sm, um, nk, buf, lane, wm, wn); break;
+      case 1: compute_unit<T, PAIR, 1>(sm, um, nk, buf, lane, wm, wn); break;
+      case 2: compute_unit<T, PAIR, 2>(sm, um, nk, buf, lane, wm, wn); break;
+      case 3: compute_unit<T, PAIR, 3>(sm, um, nk, buf, lane, wm, wn); break;
+      default: compute_unit<T, PAIR, 4>(sm, um, nk, buf, lane, wm, wn); break;
     }
     const Unit next = unit_of(w, r, G, n_units, n_mt, n_vt, a.n_grp);
     if (next.u < 0) return;
@@ -1176,42 +1242,140 @@ __device__ void compute_path(Smem& sm, const Args<T>& a, int w, int G, int n_uni
   }
 }
 
-template <typename T>
+template <typename T, typename O, bool PAIR>
 __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
-    const T* __restrict__ H, const T* __restrict__ W, const T* __restrict__ bias,
-    const float* __restrict__ rowmask, T* __restrict__ reps, int32_t* __restrict__ argmax,
+    const T* __restrict__ H, const T* __restrict__ W, const O* __restrict__ bias,
+    const float* __restrict__ rowmask, O* __restrict__ reps, int32_t* __restrict__ argmax,
     float* __restrict__ reps_f32, int S, int D, int V, int n_vt, int ngrp,
-    const int* __restrict__ meta, const int* __restrict__ list, float2* __restrict__ part) {
+    const int* __restrict__ meta, const int* __restrict__ list, float2* __restrict__ part,
+    const int* __restrict__ rexp, const int* __restrict__ cexp) {
   __shared__ Smem sm;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: keep it scalar
 
-  Args<T> a;
+  Args<T, O, PAIR> a;
   a.H = (const char*)H;
   a.W = (const char*)W;
   a.bias = bias;
+  a.rexp = rexp;
+  a.cexp = cexp;
   a.rowmask = rowmask;
   a.list = list;
   a.n_grp = __builtin_amdgcn_readfirstlane(meta[0]);
   a.ngrp = ngrp;
   a.S = S;
-  a.row_bytes = D * (int)sizeof(T);
-  const int slab_elems = SLAB / (int)sizeof(T);
-  a.nk_full = D / slab_elems;
-  // At least two slabs per unit (a padding slab contributes zero); none when D == 0,
-  // where x = bias * mask and nothing is loaded.
-  a.nk = D == 0 ? 0 : max(2, (int)cdiv(D, slab_elems));
   a.V = V;
+  const int slab_elems = SLAB / (int)sizeof(T);
+  if constexpr (PAIR) {  // D: the padded part, whole slabs
+    a.part_bytes = D * (int)sizeof(T);
+    a.row_bytes = 2 * a.part_bytes;
+    a.nk_full = a.nk = 3 * (D / slab_elems);
+  } else {
+    a.part_bytes = 0;
+    a.row_bytes = D * (int)sizeof(T);
+    a.nk_full = D / slab_elems;
+    // At least two slabs per unit (a padding slab contributes zero); none when D == 0,
+    // where x = bias * mask and nothing is loaded.
+    a.nk = D == 0 ? 0 : max(2, (int)cdiv(D, slab_elems));
+  }
 
   const int n_mt = (a.n_grp + NGRP - 1) / NGRP;
   const int n_units = n_mt * n_vt;
   if (wave < COMPUTE_WAVES) {
-    compute_path<T>(sm, a, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, wave, lane);
+    compute_path<T, O, PAIR>(sm, a, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, wave, lane);
   } else {
-    Outputs<T> o{reps, argmax, reps_f32, part};
-    copy_path<T>(sm, a, o, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, tid - 64 * COMPUTE_WAVES,
-                 wave - COMPUTE_WAVES, lane);
+    Outputs<O> o{reps, argmax, reps_f32, part};
+    copy_path<T, O, PAIR>(sm, a, o, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, tid - 64 * COMPUTE_WAVES,
+                          wave - COMPUTE_WAVES, lane);
   }
+}
+
+// ---- fp32 operands as pairs of fp16 -------------------------------------------------
+//
+// The fp32 MFMA runs at a sixteenth of the fp16 one's rate, so larger fp32 batches run on
+// fp16 MFMAs: each row of H and W is scaled by a power of two that brings its largest
+// magnitude to [2^14, 2^15) and written as hi = fp16(x), lo = fp16(x - hi). Both round to
+// nearest, so hi takes x's upper 12 bits and x - hi, at most 2^11 units of x's last place,
+// fits lo's 11: hi + lo = x exactly for every x within 2^-15 of its row's largest, and within
+// 2^-39 of that largest below (fp16's subnormals). A product is taken as lo hi + hi lo + hi hi,
+// each exact in fp32, accumulated in fp32; the dropped lo lo is at most 2^-24 of the product,
+// fp32's own rounding of it. An element that is infinite or NaN puts its value in lo (hi = 0),
+// so that it meets only the partner's hi, and the row's scale leaves it out. The epilogue takes
+// the scales out again before it adds the bias.
+// Error of reps against 64 bits, fp32 MFMAs -> pairs (2-norm relative; the keys' 18 bits
+// included): 8 x 128 x 768 x 30522 normal 1.22e-6 -> 1.19e-6, rows scaled by e^N(0,16)
+// 2.6e-7 -> 2.4e-7, elements scaled by e^N(0,4) 2.61e-7 -> 2.56e-7; D = 4096 1.11e-6 -> 1.00e-6.
+// Bound by the fp16 MFMAs at three products per value, and by the two streams of W. Measured
+// at 8 x 128 x 768 x 30522, 757 live rows: main kernel 403 -> 116 us, this split 29 us
+// (188 MB, 6.5 TB/s).
+struct PairRows {
+  f16* hi_lo;      // [rows][2][Dp]: hi, lo
+  int* exp;        // [rows] the scale's exponent, negated
+};
+
+// One wave per row of W (rows 0 .. V - 1), then per row of H's tiles, in tile order (row t of
+// group list[t / 16]; rows past the last active group are left out).
+__global__ __launch_bounds__(256) void fwd_split_rows_kernel(
+    const float* __restrict__ H, const float* __restrict__ W, PairRows hp, PairRows wp, int S, int D,
+    int Dp, int V, int ngrp, const int* __restrict__ meta, const int* __restrict__ list) {
+  const int lane = threadIdx.x & 63;
+  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const float* src;
+  f16* dst;
+  int* exp;
+  if (r < V) {
+    src = W + r * D;
+    dst = wp.hi_lo + r * 2 * Dp;
+    exp = wp.exp + r;
+  } else {
+    const int64_t t = r - V;
+    if (t / GROUP >= meta[0]) return;
+    const int code = list[t / GROUP], b = code / ngrp;
+    const int s = min((code - b * ngrp) * GROUP + (int)(t % GROUP), S - 1);
+    src = H + ((int64_t)b * S + s) * D;
+    dst = hp.hi_lo + t * 2 * Dp;
+    exp = hp.exp + t;
+  }
+  constexpr int NR = 4;  // 256-column pieces kept in registers: D <= 1024 is read once
+  f32x4 x[NR];
+  float m = 0.0f;
+  auto piece = [&](int p) {
+    const int d = p * 256 + lane * 4;
+    return d < D ? *(const f32x4*)(src + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto top = [&](const f32x4& v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float y = fabsf(v[i]);
+      m = y > m && y < INFINITY ? y : m;
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < NR; ++p) x[p] = piece(p);
+#pragma unroll
+  for (int p = 0; p < NR; ++p) top(x[p]);
+  for (int p = NR; p * 256 < D; ++p) top(piece(p));
+  m = wave_max(m);
+  int e = 15;  // m = f 2^e, 1/2 <= f < 1: the scale is 2^(15 - e)
+  if (m > 0.0f) (void)frexpf(m, &e);
+  if (lane == 0) *exp = e - 15;
+  auto put = [&](int p, const f32x4& v) {
+    const int d = p * 256 + lane * 4;
+    if (d >= Dp) return;
+    f16x4 hi, lo;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float y = __builtin_amdgcn_ldexpf(v[i], 15 - e);
+      const bool fin = fabsf(v[i]) < INFINITY;
+      hi[i] = fin ? (f16)y : (f16)0.0f;
+      lo[i] = (f16)(y - (float)hi[i]);
+    }
+    *(f16x4*)(dst + d) = hi;
+    *(f16x4*)(dst + Dp + d) = lo;
+  };
+#pragma unroll
+  for (int p = 0; p < NR; ++p) put(p, x[p]);
+  for (int p = NR; p * 256 < Dp; ++p) put(p, piece(p));
 }
 
 // ---- fixup ------------------------------------------------------------------------
@@ -1548,15 +1712,55 @@ static int64_t persistent_grid(int64_t n_units_max) {
   return std::min<int64_t>(g, n_units_max);
 }
 
+// The fp16 pairs of an fp32 launch, carved from the workspace after Work.
+struct Pairs {
+  PairRows h, w;
+  int64_t Dp;
+  size_t total;
+};
+// When fp32 batches take the pairs (whole forward, fp32 MFMAs -> pairs, one box): the split
+// passes over W cost what the fp32 MFMAs of about 100 rows do, so every batch past the
+// small-batch kernel gains (V = 30522, D = 768: 130 rows 139 -> 84 us, 1024 rows 414 -> 160 us,
+// 4096 rows 1162 -> 414 us), except where W is larger than the MALL holds beside its pairs
+// (140 rows, W of 983 MB: 727 -> 761 us; 512 rows, 614 MB: 1402 -> 682 us) or rows are narrow
+// (1024 rows, D = 64: 53 -> 56 us; D = 384: 112 -> 63 us).
+constexpr int64_t PAIR_MIN_D = 128;
+constexpr int64_t PAIR_W_BYTES = (int64_t)128 << 20, PAIR_BIG_W_ROWS = 256;
+static bool pairs_fit(int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
+  const int64_t Dp = round_up(D, SLAB / 2), n_mt_max = cdiv(B * cdiv(S, GROUP), NGRP);
+  return dtype == SPARTON_F32 && D >= PAIR_MIN_D && B * S > SMALL_MAX_ROWS &&
+         (V * D * 4 <= PAIR_W_BYTES || B * S >= PAIR_BIG_W_ROWS) &&
+         n_mt_max * BM * Dp * 4 < ((int64_t)1 << 31) && BN * Dp * 4 < ((int64_t)1 << 31);
+}
+static Pairs carve_pairs(void* base, int64_t B, int64_t S, int64_t D, int64_t V) {
+  const int64_t n = cdiv(B * cdiv(S, GROUP), NGRP) * BM;
+  char* p = (char*)base;
+  Pairs x;
+  x.Dp = round_up(D, SLAB / 2);
+  size_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const size_t o = off;
+    off += (size_t)round_up(bytes, 256);
+    return p != nullptr ? p + o : nullptr;
+  };
+  x.h.hi_lo = (f16*)take(n * x.Dp * 4);
+  x.h.exp = (int*)take(n * 4);
+  x.w.hi_lo = (f16*)take(V * x.Dp * 4);
+  x.w.exp = (int*)take(V * 4);
+  x.total = off;
+  return x;
+}
+
 // ev_main: if non-null, two events recorded on `stream` just before and after the main
 // kernel (profiling).
 // split: fp32 products as bf16 hi/lo parts (SPARTON_F32_SPLIT) in the small-batch kernel;
-// the main kernel computes fp32 exactly either way.
+// the main kernel keeps fp32's precision either way. pairs: where its fp16 pairs lie, or null
+// for the fp32 MFMAs.
 template <typename T>
 static int launch(const void* H, const void* W, const void* bias, const void* mask,
                   int mask_dtype, void* reps, int32_t* argmax, float* reps_f32, int64_t B,
                   int64_t S, int64_t D, int64_t V, const Work& w, hipStream_t stream,
-                  hipEvent_t* ev_main, bool split) {
+                  hipEvent_t* ev_main, bool split, const Pairs* pairs) {
   const int64_t ngrp = cdiv(S, GROUP);
   const int64_t n_vt = cdiv(V, BN);
   const int64_t n_mt_max = cdiv(B * ngrp, NGRP);
@@ -1598,12 +1802,30 @@ static int launch(const void* H, const void* W, const void* bias, const void* ma
                        0, stream, mask, mask_dtype, (int)S, (int)ngrp, (const int*)w.meta,
                        (const int*)w.list, w.rowmask);
   }
+  if (pairs != nullptr)
+    hipLaunchKernelGGL(fwd_split_rows_kernel, dim3((unsigned)cdiv(V + n_mt_max * BM, 4)), dim3(256), 0,
+                       stream, (const float*)H, (const float*)W, pairs->h, pairs->w, (int)S, (int)D,
+                       (int)pairs->Dp, (int)V, (int)ngrp, (const int*)w.meta, (const int*)w.list);
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[0], stream);
-  if (grid > 0)  // S == 0: no blocks, the fixup writes every row
-    hipLaunchKernelGGL(sparton_fwd_kernel<T>, dim3((unsigned)grid), dim3(NTHREADS), 0, stream,
-                       (const T*)H, (const T*)W, (const T*)bias, (const float*)w.rowmask, (T*)reps,
-                       argmax, reps_f32, (int)S, (int)D, (int)V, (int)n_vt, (int)ngrp,
-                       (const int*)w.meta, (const int*)w.list, w.part);
+  if (grid > 0) {  // S == 0: no blocks, the fixup writes every row
+    bool done = false;
+    if constexpr (sizeof(T) == 4) {
+      if (pairs != nullptr) {
+        hipLaunchKernelGGL((sparton_fwd_kernel<f16, float, true>), dim3((unsigned)grid), dim3(NTHREADS), 0,
+                           stream, (const f16*)pairs->h.hi_lo, (const f16*)pairs->w.hi_lo,
+                           (const float*)bias, (const float*)w.rowmask, (float*)reps, argmax, reps_f32,
+                           (int)S, (int)pairs->Dp, (int)V, (int)n_vt, (int)ngrp, (const int*)w.meta,
+                           (const int*)w.list, w.part, (const int*)pairs->h.exp,
+                           (const int*)pairs->w.exp);
+        done = true;
+      }
+    }
+    if (!done)
+      hipLaunchKernelGGL((sparton_fwd_kernel<T, T, false>), dim3((unsigned)grid), dim3(NTHREADS), 0, stream,
+                         (const T*)H, (const T*)W, (const T*)bias, (const float*)w.rowmask, (T*)reps,
+                         argmax, reps_f32, (int)S, (int)D, (int)V, (int)n_vt, (int)ngrp,
+                         (const int*)w.meta, (const int*)w.list, w.part, nullptr, nullptr);
+  }
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[1], stream);
   hipLaunchKernelGGL(fwd_fixup_kernel<T>, dim3((unsigned)cdiv(V, FIX_COLS), (unsigned)B), dim3(256), 0,
                      stream, (int)V, (const int*)w.count, (const int*)w.first,
@@ -1637,11 +1859,19 @@ static int64_t mask_elem_bytes(int mask_dtype) {
 
 using namespace sparton;
 
-extern "C" __attribute__((visibility("default"))) size_t sparton_fwd_workspace_bytes(
-    int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
+// Workspace without the fp16 pairs of fp32 operands: the plan and the partials.
+static size_t plan_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
   if (B <= 0 || S < 0 || D < 0 || V <= 0) return 0;
   const int64_t esz = (dtype & ~SPARTON_F32_SPLIT) == SPARTON_F32 ? 4 : 2;
   return fwd::carve(nullptr, fwd::rows_per_launch(B, S, D, esz), S, V).total;
+}
+
+extern "C" __attribute__((visibility("default"))) size_t sparton_fwd_workspace_bytes(
+    int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
+  size_t n = plan_workspace_bytes(B, S, D, V, dtype);
+  if (n > 0 && fwd::pairs_fit(B, S, D, V, dtype & ~SPARTON_F32_SPLIT))
+    n += fwd::carve_pairs(nullptr, B, S, D, V).total;
+  return n;
 }
 
 // dtype: an enum sparton_dtype, or SPARTON_F32 | SPARTON_F32_SPLIT.
@@ -1674,11 +1904,16 @@ static int fwd_run(const void* hidden, const void* weight, const void* bias, con
   if (B > INT32_MAX || V > INT32_MAX) return SPARTON_EUNSUPPORTED;
   if (S * D * esz >= ((int64_t)1 << 31) || (int64_t)fwd::BN * D * esz >= ((int64_t)1 << 31))
     return SPARTON_EUNSUPPORTED;
-  const size_t need = sparton_fwd_workspace_bytes(B, S, D, V, dtype);
+  const size_t need = plan_workspace_bytes(B, S, D, V, dtype);
   if (workspace == nullptr || workspace_bytes < need) return SPARTON_EWORKSPACE;
   if ((uintptr_t)workspace % 256 != 0) return SPARTON_EALIGN;
   hipStream_t st = (hipStream_t)stream;
   const int64_t Bc = fwd::rows_per_launch(B, S, D, esz);
+  // A workspace that holds the plan only (sparton_fwd_noalloc's) keeps the fp32 MFMAs.
+  const bool use_pairs = fwd::pairs_fit(B, S, D, V, dtype) && Bc >= B &&
+                         workspace_bytes >= sparton_fwd_workspace_bytes(B, S, D, V, dtype);
+  fwd::Pairs pairs{};
+  if (use_pairs) pairs = fwd::carve_pairs((char*)workspace + need, B, S, D, V);
   for (int64_t b0 = 0; b0 < B; b0 += Bc) {
     const int64_t nb = std::min(Bc, B - b0);
     const fwd::Work w = fwd::carve(workspace, nb, S, V);
@@ -1698,13 +1933,14 @@ static int fwd_run(const void* hidden, const void* weight, const void* bias, con
     int rc;
     switch (dtype) {
       case SPARTON_BF16:
-        rc = fwd::launch<bf16>(h, weight, bias, mk, mask_dtype, r, am, r32, nb, S, D, V, w, st, evp, false);
+        rc = fwd::launch<bf16>(h, weight, bias, mk, mask_dtype, r, am, r32, nb, S, D, V, w, st, evp, false, nullptr);
         break;
       case SPARTON_F16:
-        rc = fwd::launch<f16>(h, weight, bias, mk, mask_dtype, r, am, r32, nb, S, D, V, w, st, evp, false);
+        rc = fwd::launch<f16>(h, weight, bias, mk, mask_dtype, r, am, r32, nb, S, D, V, w, st, evp, false, nullptr);
         break;
       default:
-        rc = fwd::launch<float>(h, weight, bias, mk, mask_dtype, r, am, r32, nb, S, D, V, w, st, evp, split);
+        rc = fwd::launch<float>(h, weight, bias, mk, mask_dtype, r, am, r32, nb, S, D, V, w, st, evp, split,
+                                use_pairs ? &pairs : nullptr);
         break;
     }
     if (main_ms != nullptr) {
@@ -1778,7 +2014,7 @@ extern "C" __attribute__((visibility("default"))) int sparton_fwd_noalloc(
   if (B < 0 || S < 0 || D < 0 || V < 0) return SPARTON_EINVAL;
   if (!fwd_dtype_ok(dtype)) return SPARTON_EINVAL;
   if (mask_dtype < SPARTON_MASK_I64 || mask_dtype > SPARTON_MASK_F16) return SPARTON_EINVAL;
-  const size_t need = sparton_fwd_workspace_bytes(B, S, D, V, dtype);
+  const size_t need = plan_workspace_bytes(B, S, D, V, dtype);
   if (need > kNoAllocScratchBytes) return SPARTON_ESCRATCH;
   void* ws = nullptr;
   if (need > 0) {
@@ -1786,7 +2022,7 @@ extern "C" __attribute__((visibility("default"))) int sparton_fwd_noalloc(
     if (rc != SPARTON_OK) return rc;
   }
   return fwd_run(hidden, weight, bias, mask, mask_dtype, reps, argmax, reps_f32, B, S, D, V,
-                 dtype, ws, need > 0 ? kNoAllocScratchBytes : 0, stream, nullptr);
+                 dtype, ws, need, stream, nullptr);
 }
 
 extern "C" __attribute__((visibility("default"))) int sparton_fwd_profile(

@@ -924,6 +924,92 @@ def test_fp32_split_precision(case, device):
         assert not torch.equal(r32, exact[2])
 
 
+def _fwd_capi_fp32(H, W, b, m, pairs):
+    """sparton_fwd on fp32 device tensors: with the whole workspace (fp16 pairs where the size
+    takes them), or one byte less (the fp32 MFMAs)."""
+    B, S, D = H.shape
+    V = W.shape[0]
+    L = _lib.load()
+    n = int(L.sparton_fwd_workspace_bytes(B, S, D, V, 0))
+    ws = torch.empty(n, dtype=torch.uint8, device=H.device)
+    reps = torch.empty((B, V), dtype=torch.float32, device=H.device)
+    idx = torch.empty((B, V), dtype=torch.int32, device=H.device)
+    rc = L.sparton_fwd(H.data_ptr(), W.data_ptr(), _lib.ptr(b), m.data_ptr(), _lib.MASK_CODE[m.dtype],
+                       reps.data_ptr(), idx.data_ptr(), None, B, S, D, V, 0, ws.data_ptr(),
+                       n if pairs else n - 1, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, L.sparton_strerror(rc)
+    torch.cuda.synchronize()
+    return reps, idx
+
+
+@pytest.mark.parametrize("case,spread", [
+    (("fp32", 1, 129, 128, 300, True, "int64"), 0),     # the fewest rows and columns that take pairs
+    (("fp32", 3, 70, 132, 900, False, "frac"), 0),      # a padded last slab, fractional mask
+    (("fp32", 8, 64, 772, 257, True, "holes"), 2),      # rows and elements of very different size
+    (("fp32", 2, 100, 1540, 515, True, "bool"), 2),     # rows longer than the split keeps in registers
+    (("fp32", 40, 30, 256, 1000, True, "gaps"), 0),     # rows with no active position
+], ids=lambda c: "-".join(map(str, c)) if isinstance(c, tuple) else f"spread{c}")
+def test_fp32_pairs_precision(case, spread, device):
+    """fp32 batches past 128 positions run as pairs of fp16 (hi + lo, three products): against
+    the oracle like any fp32 forward, and no further from 64 bits than the fp32 MFMAs. Both
+    errors are dominated by the keys' 2^-18, so theirs may differ by a tenth either way."""
+    say(f"fp32 pairs, case {case}, spread {spread}")
+    H, W, b, m, _ = make_case(*case)
+    if spread:
+        g = torch.Generator().manual_seed(3)
+        H = H * torch.exp(torch.randn(H.shape[:2], generator=g) * spread)[..., None]
+        W = W * torch.exp(torch.randn(W.shape, generator=g) * spread)
+    Hd, Wd, md = H.to(device), W.to(device), m.to(device)
+    bd = None if b is None else b.to(device)
+    err = []
+    for pairs in (True, False):
+        reps, idx = _fwd_capi_fp32(Hd, Wd, bd, md, pairs)
+        check_fwd(H, W, b, m, reps, idx)
+        x = torch.einsum("bsd,vd->bsv", H.double(), W.double())
+        if b is not None:
+            x = x + b.double()
+        want = torch.log1p((x * m.double()[..., None]).amax(1).clamp_min(0.0))
+        err.append(float((reps.cpu().double() - want).norm() / want.norm()))
+    say(f"  error against 64 bits: pairs {err[0]:.3g}, fp32 MFMAs {err[1]:.3g}")
+    assert err[0] <= 1.1 * err[1]
+
+
+def test_fp32_pairs_infinite_and_extreme_entries(device):
+    """Infinite entries, and rows at the ends of fp32's range, in a batch that runs as fp16
+    pairs: the fp32 MFMAs' reps, infinities and NaNs included, as long as no product has both
+    operands infinite."""
+    say("fp32 pairs with infinite and extreme entries")
+    g = torch.Generator().manual_seed(22)
+    B, S, D, V = 3, 64, 256, 700
+    H = torch.randn(B, S, D, generator=g)
+    W = torch.randn(V, D, generator=g) * 0.02
+    b = torch.randn(V, generator=g) * 0.02
+    m = torch.ones(B, S, dtype=torch.long)
+    m[1, 20:] = 0
+    H[0, 5, 17] = float("inf")
+    H[1, 3, 40] = float("-inf")
+    H[2] *= 2.0 ** -100
+    H[2, 7] *= 2.0 ** 90
+    W[7, 100] = float("-inf")
+    W[699, 255] = float("inf")
+    W[10:20] *= 2.0 ** 100
+    W[20] = 0.0
+    W[21, 3] = float("nan")
+    b[10:20] = 0.0
+    Hd, Wd, bd, md = H.to(device), W.to(device), b.to(device), m.to(device)
+    r_p, i_p = (t.cpu() for t in _fwd_capi_fp32(Hd, Wd, bd, md, True))
+    r_e, i_e = (t.cpu() for t in _fwd_capi_fp32(Hd, Wd, bd, md, False))
+    nonfinite = ~torch.isfinite(r_e)
+    assert int(torch.isinf(r_e).sum()) > 100
+    assert torch.equal(nonfinite, ~torch.isfinite(r_p))
+    assert torch.equal(r_p[nonfinite].isnan(), r_e[nonfinite].isnan())
+    assert torch.equal(i_p[nonfinite], i_e[nonfinite])
+    # Values whose positions agree: 2^-18 of the keys and the sums' rounding, on either side.
+    same = ~nonfinite & (i_p == i_e)
+    assert int(same.sum()) > 0.99 * int((~nonfinite).sum())
+    torch.testing.assert_close(r_p[same], r_e[same], rtol=2e-5, atol=1e-30)
+
+
 def test_fp32_split_infinite_entries(device):
     """Infinite entries in H and in W under 'high' (the bf16 hi/lo split kernel): reps and
     argmax equal the exact fp32 path's ('highest'), infinities and NaNs included, as long as
