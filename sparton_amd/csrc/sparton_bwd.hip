@@ -427,8 +427,8 @@ __device__ __forceinline__ void store_chunk(O* out, const float* a) {
 // would outlast the launch. A workgroup's lane groups therefore share such rows: each step
 // every group computes the batch partials of 16 consecutive entries into LDS, and the
 // slice's columns add them in batch order: the same sums. A workgroup takes DH_GROUPS rows,
-// of which those past max(HOT_MIN, HOT_REL times its mean) are shared, or, of fewer rows
-// (dh_rows_per_group), every one that is not short (HOT_FEW).
+// of which those past max(HOT_MIN, HOT_REL times its mean) are shared, or one row, which is unless it is short
+// (HOT_FEW).
 constexpr int HOT_MIN = 128;
 constexpr int HOT_REL = 4;
 constexpr int HOT_FEW = 32;
@@ -436,7 +436,7 @@ constexpr int HOT_NB = DH_LANES / DH_BATCH;  // partials per lane group and step
 
 template <typename T>
 struct HotSmem {
-  float part[DH_GROUPS * HOT_NB][Chunk<T>::COLS];
+  __attribute__((aligned(16))) float part[DH_GROUPS * HOT_NB][Chunk<T>::COLS];
   int total[DH_GROUPS];
 };
 
@@ -508,14 +508,17 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
     RowEntries rk;
     const int2* rbk = entries_of(row0 + k, rk);
     float acc = 0.0f;  // column `tid` of the slice
+    Entries next;
+    next.load(rbk, rk, runs, grp * DH_LANES, row16, l);
     for (int e0 = 0; e0 < n; e0 += DH_GROUPS * DH_LANES) {
       const int e = e0 + grp * DH_LANES;
+      const Entries en = next;
+      next.load(rbk, rk, runs, e + DH_GROUPS * DH_LANES, row16, l);
       if (e < n) {
-        Entries en;
-        en.load(rbk, rk, runs, e, row16, l);
         auto put = [&](int p, const float* P) {
 #pragma unroll
-          for (int j = 0; j < E; ++j) sm.part[grp * HOT_NB + p][l * E + j] = P[j];
+          for (int j = 0; j < E; j += 4)
+            *(f32x4*)&sm.part[grp * HOT_NB + p][l * E + j] = f32x4{P[j], P[j + 1], P[j + 2], P[j + 3]};
         };
         if (n - e >= DH_LANES) dh_partials<T, false, DH_LANES>(wp, en, DH_LANES, put);
         else dh_partials_tail<T>(wp, en, n - e, put);
@@ -832,12 +835,12 @@ static int passes_for(int64_t D) {
 }
 
 // Rows a dH workgroup takes: all its lane groups' worth once there are enough rows to fill the
-// chip, fewer (whose entries the groups share) below. Measured at 1024 fp32 rows of 424
-// entries: 16 / 4 / 1 rows 123 / 134 / 111 us, but at 4096 rows of 7: 11 / - / 48 us, so only
-// launches under 1024 rows give way.
-static int dh_rows_per_group(int64_t rows) {
-  return rows >= 1024 ? DH_GROUPS : rows >= 512 ? 4 : rows >= 256 ? 2 : 1;
-}
+// chip, one (shared by the groups) below. Measured as whole passes with bf16 rows of 768,
+// V = 30522, at 16 rows / 1 row a workgroup: dense gradients, 16 x 64 positions 295 / 214 us,
+// 16 x 128 256 / 233 us, 16 x 200 282 / 263 us; 5% dense, 16 x 64 93 / 89 us, 16 x 128 99 /
+// 116 us (8 x 512, dH alone: 11 / 48 us).
+constexpr int64_t DH_MANY_ROWS = 2048;
+static int dh_rows_per_group(int64_t rows) { return rows >= DH_MANY_ROWS ? DH_GROUPS : 1; }
 // SPARTON_BWD_HOT_MIN sets the number of entries past which a row is shared (tests compare
 // shared and unshared rows).
 static int dh_hot_min() {

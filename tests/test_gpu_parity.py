@@ -333,9 +333,9 @@ def test_backward_hot_rows_five_kernel(case, device, monkeypatch):
 
 
 @pytest.mark.parametrize("case", [
-    ("bf16", 70, 4, 136, 3000, True, "int64"),      # 280 rows: 2 a workgroup; a slice of one chunk
-    ("fp16", 5, 120, 72, 9000, False, "holes"),     # 600 rows: 4 a workgroup; 3 runs of ids
-    ("fp32", 9, 131, 68, 40000, True, "int64"),     # 1179 rows: 16 a workgroup, the last ragged; 10 runs
+    ("bf16", 70, 4, 136, 3000, True, "int64"),      # 280 rows: a row a workgroup; a slice of one chunk
+    ("fp16", 5, 120, 72, 9000, False, "holes"),     # 600 rows; 3 runs of ids
+    ("fp32", 17, 131, 68, 40000, True, "int64"),    # 2227 rows: 16 a workgroup, the last ragged; 10 runs
     ("bf16", 2, 5000, 16, 300, True, "int64"),      # two windows of positions
     ("fp16", 1, 90, 40, 70000, True, "int64"),      # two turns per bucketing wave; 1 row a workgroup
     ("bf16", 3, 30, 2056, 130, True, "holes"),      # 17 slices, the last of one chunk
