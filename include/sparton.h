@@ -203,6 +203,20 @@ int sparton_transform_bwd(const void* dy, const void* z, const float* dense_bias
                           int dtype, void* stream);
 
 /*
+ * The same two with the vectors (dense_bias, ln_weight, ln_bias) and their gradients in
+ * `vec_dtype`: SPARTON_F32, or `dtype`, for a model held in 16 bits (16- or 8-byte aligned).
+ * The gradients' fp32 sums are rounded once.
+ */
+int sparton_transform_fwd_typed(const void* z, const void* dense_bias, const void* ln_weight,
+                                const void* ln_bias, int vec_dtype, float eps, void* y, float* mean,
+                                float* rstd, int64_t M, int64_t D, int dtype, void* stream);
+int sparton_transform_bwd_typed(const void* dy, const void* z, const void* dense_bias,
+                                const void* ln_weight, int vec_dtype, const float* mean,
+                                const float* rstd, void* dz, void* d_ln_weight, void* d_ln_bias,
+                                void* d_dense_bias, void* workspace, size_t workspace_bytes, int64_t M,
+                                int64_t D, int dtype, void* stream);
+
+/*
  * Weight gradient of the transform's dense layer, dW = dz^T x, as a batched GEMM over C row
  * chunks (the caller runs the GEMM): sparton_transform_dz_chunks writes dzt [C, D, M/C] with
  * dzt[c][i][l] = dz[c (M/C) + l][i] (bf16/fp16; M % C == 0, (M/C) % 64 == 0, D % 64 == 0,

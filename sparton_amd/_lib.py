@@ -50,6 +50,8 @@ EXPORTED_SYMBOLS = (
     "sparton_bwd_workspace_bytes",
     "sparton_transform_fwd",
     "sparton_transform_bwd",
+    "sparton_transform_fwd_typed",
+    "sparton_transform_bwd_typed",
     "sparton_transform_workspace_bytes",
     "sparton_transform_dz_chunks",
     "sparton_transform_chunk_sum",

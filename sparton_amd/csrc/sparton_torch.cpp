@@ -15,6 +15,7 @@
 //       -> reps; weight_c/bias_c are the compute-dtype copies of the fp32 masters weight/bias
 //       (D zero-padded by pad); the backward writes fp32 gradients straight to the masters
 //   sparton_eager::mlm_transform(x, weight, dense_bias, ln_weight, ln_bias, eps) -> y
+//   sparton_eager::mlm_transform_typed(the same, with the vectors in x's dtype)
 //       LayerNorm(gelu(x W^T + b)) (training/model.py:14-40)
 //   sparton_eager::splade_loss(q, d?, temperature, w_ce, w_l1, w_flops) -> out[6]
 //       (total, CE, L1 q, L1 d, FLOPS q, FLOPS d)  (training/train.py:73-94, :164-197)
@@ -433,10 +434,11 @@ struct TransformFn : public torch::autograd::Function<TransformFn> {
     Tensor y = at::empty_like(z);
     Tensor mean = at::empty({M}, x.options().dtype(at::kFloat));
     Tensor rstd = at::empty({M}, x.options().dtype(at::kFloat));
-    Tensor vb = dense_bias.contiguous(), vg = ln_weight.contiguous(), vt = ln_bias.contiguous();
-    check(sparton_transform_fwd(z.data_ptr(), vb.data_ptr<float>(), vg.data_ptr<float>(),
-                                vt.data_ptr<float>(), (float)eps, y.data_ptr(), mean.data_ptr<float>(),
-                                rstd.data_ptr<float>(), M, D, dtype_code(x.scalar_type()), stream_of(x)),
+    Tensor vb = dense(dense_bias), vg = dense(ln_weight), vt = dense(ln_bias);
+    check(sparton_transform_fwd_typed(z.data_ptr(), vb.data_ptr(), vg.data_ptr(), vt.data_ptr(),
+                                      dtype_code(vb.scalar_type()), (float)eps, y.data_ptr(),
+                                      mean.data_ptr<float>(), rstd.data_ptr<float>(), M, D,
+                                      dtype_code(x.scalar_type()), stream_of(x)),
           "sparton_transform_fwd");
     ctx->save_for_backward({x, weight, z, vb, vg, mean, rstd});
     return y.view(x.sizes());
@@ -451,14 +453,15 @@ struct TransformFn : public torch::autograd::Function<TransformFn> {
     const int64_t M = x2.size(0);
     Tensor dy2 = grads[0].reshape({-1, D}).to(x.scalar_type()).contiguous();
     Tensor dz = at::empty_like(z);
-    Tensor dg = at::empty({D}, x.options().dtype(at::kFloat));
+    Tensor dg = at::empty({D}, vb.options());
     Tensor dbt = at::empty_like(dg), dbd = at::empty_like(dg);
     const size_t ws_bytes = sparton_transform_workspace_bytes(M, D);
     Tensor ws = workspace(ws_bytes, x);
-    check(sparton_transform_bwd(dy2.data_ptr(), z.data_ptr(), vb.data_ptr<float>(), vg.data_ptr<float>(),
-                                mean.data_ptr<float>(), rstd.data_ptr<float>(), dz.data_ptr(),
-                                dg.data_ptr<float>(), dbt.data_ptr<float>(), dbd.data_ptr<float>(),
-                                ws.data_ptr(), ws_bytes, M, D, dtype_code(x.scalar_type()), stream_of(x)),
+    check(sparton_transform_bwd_typed(dy2.data_ptr(), z.data_ptr(), vb.data_ptr(), vg.data_ptr(),
+                                      dtype_code(vb.scalar_type()), mean.data_ptr<float>(),
+                                      rstd.data_ptr<float>(), dz.data_ptr(), dg.data_ptr(), dbt.data_ptr(),
+                                      dbd.data_ptr(), ws.data_ptr(), ws_bytes, M, D,
+                                      dtype_code(x.scalar_type()), stream_of(x)),
           "sparton_transform_bwd");
     Tensor dx = lt_gemm_ok(dz) ? lt_dgrad(dz, dense(weight)) : at::mm(dz, weight);
     Tensor dw = transform_weight_grad(dz, lt_gemm_ok(dz) ? dense(x2) : x2, M, D);
@@ -466,13 +469,25 @@ struct TransformFn : public torch::autograd::Function<TransformFn> {
   }
 };
 
+// The vectors' dtype: float32 (mlm_transform), or x's own (mlm_transform_typed).
+void check_vectors(const Tensor& b, const Tensor& g, const Tensor& t, at::ScalarType dt, const char* op) {
+  TORCH_CHECK(b.scalar_type() == dt && g.scalar_type() == dt && t.scalar_type() == dt, "sparton: ", op,
+              " takes its bias and LayerNorm vectors in ", dt);
+}
+
 Tensor transform_autograd(const Tensor& x, const Tensor& weight, const Tensor& dense_bias,
                           const Tensor& ln_weight, const Tensor& ln_bias, double eps) {
+  check_vectors(dense_bias, ln_weight, ln_bias, at::kFloat, "mlm_transform");
+  return TransformFn::apply(x, weight, dense_bias, ln_weight, ln_bias, eps);
+}
+Tensor transform_typed_autograd(const Tensor& x, const Tensor& weight, const Tensor& dense_bias,
+                                const Tensor& ln_weight, const Tensor& ln_bias, double eps) {
+  check_vectors(dense_bias, ln_weight, ln_bias, x.scalar_type(), "mlm_transform_typed");
   return TransformFn::apply(x, weight, dense_bias, ln_weight, ln_bias, eps);
 }
 
-Tensor transform_cuda(const Tensor& x, const Tensor& weight, const Tensor& dense_bias,
-                      const Tensor& ln_weight, const Tensor& ln_bias, double eps) {
+Tensor transform_run(const Tensor& x, const Tensor& weight, const Tensor& dense_bias,
+                     const Tensor& ln_weight, const Tensor& ln_bias, double eps) {
   c10::OptionalDeviceGuard guard(x.device());
   const int64_t D = x.size(-1);
   Tensor x2 = x.reshape({-1, D});
@@ -480,12 +495,23 @@ Tensor transform_cuda(const Tensor& x, const Tensor& weight, const Tensor& dense
   const int64_t M = z.size(0);
   Tensor y = at::empty_like(z);
   Tensor mean = at::empty({M}, x.options().dtype(at::kFloat)), rstd = at::empty_like(mean);
-  Tensor vb = dense_bias.contiguous(), vg = ln_weight.contiguous(), vt = ln_bias.contiguous();
-  check(sparton_transform_fwd(z.data_ptr(), vb.data_ptr<float>(), vg.data_ptr<float>(),
-                              vt.data_ptr<float>(), (float)eps, y.data_ptr(), mean.data_ptr<float>(),
-                              rstd.data_ptr<float>(), M, D, dtype_code(x.scalar_type()), stream_of(x)),
+  Tensor vb = dense(dense_bias), vg = dense(ln_weight), vt = dense(ln_bias);
+  check(sparton_transform_fwd_typed(z.data_ptr(), vb.data_ptr(), vg.data_ptr(), vt.data_ptr(),
+                                    dtype_code(vb.scalar_type()), (float)eps, y.data_ptr(),
+                                    mean.data_ptr<float>(), rstd.data_ptr<float>(), M, D,
+                                    dtype_code(x.scalar_type()), stream_of(x)),
         "sparton_transform_fwd");
   return y.view(x.sizes());
+}
+Tensor transform_cuda(const Tensor& x, const Tensor& weight, const Tensor& dense_bias,
+                      const Tensor& ln_weight, const Tensor& ln_bias, double eps) {
+  check_vectors(dense_bias, ln_weight, ln_bias, at::kFloat, "mlm_transform");
+  return transform_run(x, weight, dense_bias, ln_weight, ln_bias, eps);
+}
+Tensor transform_typed_cuda(const Tensor& x, const Tensor& weight, const Tensor& dense_bias,
+                            const Tensor& ln_weight, const Tensor& ln_bias, double eps) {
+  check_vectors(dense_bias, ln_weight, ln_bias, x.scalar_type(), "mlm_transform_typed");
+  return transform_run(x, weight, dense_bias, ln_weight, ln_bias, eps);
 }
 
 // ---- the SPLADE loss ----------------------------------------------------------------------
@@ -586,6 +612,8 @@ TORCH_LIBRARY(sparton_eager, m) {
         "Tensor weight_c, Tensor? bias_c, int pad) -> Tensor");
   m.def("mlm_transform(Tensor x, Tensor weight, Tensor dense_bias, Tensor ln_weight, "
         "Tensor ln_bias, float eps) -> Tensor");
+  m.def("mlm_transform_typed(Tensor x, Tensor weight, Tensor dense_bias, Tensor ln_weight, "
+        "Tensor ln_bias, float eps) -> Tensor");
   m.def("splade_loss(Tensor q, Tensor? d, float temperature, float w_ce, float w_l1, "
         "float w_flops) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
 }
@@ -595,6 +623,7 @@ TORCH_LIBRARY_IMPL(sparton_eager, CUDA, m) {
   m.impl("head_encode", &head_encode_cuda);
   m.impl("head_train_autocast", &head_train_autocast_cuda);
   m.impl("mlm_transform", &transform_cuda);
+  m.impl("mlm_transform_typed", &transform_typed_cuda);
   m.impl("splade_loss", &loss_cuda);
 }
 
@@ -602,6 +631,7 @@ TORCH_LIBRARY_IMPL(sparton_eager, AutogradCUDA, m) {
   m.impl("head_train", &head_train_autograd);
   m.impl("head_train_autocast", &head_train_autocast_autograd);
   m.impl("mlm_transform", &transform_autograd);
+  m.impl("mlm_transform_typed", &transform_typed_autograd);
   m.impl("splade_loss", &loss_autograd);
 }
 
@@ -617,6 +647,8 @@ TORCH_LIBRARY_IMPL(sparton_eager, CPU, m) {
             const c10::optional<Tensor>&, int64_t) -> Tensor { cpu_refused("sparton_eager::head_train_autocast"); });
   m.impl("mlm_transform", [](const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
                              double) -> Tensor { cpu_refused("sparton_eager::mlm_transform"); });
+  m.impl("mlm_transform_typed", [](const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+                                   double) -> Tensor { cpu_refused("sparton_eager::mlm_transform_typed"); });
   m.impl("splade_loss", [](const Tensor&, const c10::optional<Tensor>&, double, double, double,
                            double) -> Loss6 { cpu_refused("sparton_eager::splade_loss"); });
 }

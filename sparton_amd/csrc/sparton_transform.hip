@@ -103,17 +103,19 @@ __device__ __forceinline__ void store4t(T* p, int d, int D, f32x4 v) {
     __builtin_nontemporal_store(o, (vec4_t<T>*)(p + d));
   }
 }
-template <bool FULL>
-__device__ __forceinline__ f32x4 load4p(const float* p, int d, int D) {
-  return *(const f32x4*)(p + (FULL ? d : min(d, D - 4)));
+// Four elements of a bias or LayerNorm vector, of type VT: float, or the rows' own type (a
+// model held in 16 bits), which spares its caller casts there and back around every call.
+template <typename VT, bool FULL>
+__device__ __forceinline__ f32x4 load4p(const VT* p, int d, int D) {
+  return to_f32<VT>(load4<VT, FULL>(p, d, D));
 }
 
 // ---- forward epilogue: one wave per row ------------------------------------------------
 // u = gelu(Z + b_d), mean and 1/std of u over the row, Y = (u - mean) / std * gamma + beta.
-template <typename T, int NP, bool FULL>
+template <typename T, typename VT, int NP, bool FULL>
 __global__ __launch_bounds__(64 * FWD_WAVES) void xf_fwd_kernel(
-    const T* __restrict__ Z, const float* __restrict__ bd, const float* __restrict__ gamma,
-    const float* __restrict__ beta, float eps, T* __restrict__ Y, float* __restrict__ mean_out,
+    const T* __restrict__ Z, const VT* __restrict__ bd, const VT* __restrict__ gamma,
+    const VT* __restrict__ beta, float eps, T* __restrict__ Y, float* __restrict__ mean_out,
     float* __restrict__ rstd_out, int M, int D) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * FWD_WAVES + (threadIdx.x >> 6);
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void xf_fwd_kernel(
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int d = p * 256 + lane * 4;
-    const f32x4 zz = to_f32<T>(zr[p]), bb = load4p<FULL>(bd, d, D);
+    const f32x4 zz = to_f32<T>(zr[p]), bb = load4p<VT, FULL>(bd, d, D);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       u[p][e] = in_row<FULL>(d, D) ? gelu(zz[e] + bb[e]) : 0.0f;
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void xf_fwd_kernel(
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int d = p * 256 + lane * 4;
-    const f32x4 g = load4p<FULL>(gamma, d, D), bt = load4p<FULL>(beta, d, D);
+    const f32x4 g = load4p<VT, FULL>(gamma, d, D), bt = load4p<VT, FULL>(beta, d, D);
     f32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = (u[p][e] - mu) * rs * g[e] + bt[e];
@@ -180,10 +182,10 @@ template <int NP> struct BwdCfg {
   static constexpr int threads = 64 * waves;
 };
 
-template <typename T, int NP, bool FULL>
+template <typename T, typename VT, int NP, bool FULL>
 __global__ __launch_bounds__(BwdCfg<NP>::threads) void xf_bwd_kernel(
-    const T* __restrict__ dY, const T* __restrict__ Z, const float* __restrict__ bd,
-    const float* __restrict__ gamma, const float* __restrict__ mean_in,
+    const T* __restrict__ dY, const T* __restrict__ Z, const VT* __restrict__ bd,
+    const VT* __restrict__ gamma, const float* __restrict__ mean_in,
     const float* __restrict__ rstd_in, T* __restrict__ dZ, float* __restrict__ part, int M, int D,
     int rows_per_wave) {
   constexpr bool KEEP = BwdCfg<NP>::keep;
@@ -200,8 +202,8 @@ __global__ __launch_bounds__(BwdCfg<NP>::threads) void xf_bwd_kernel(
   if constexpr (KEEP) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      vb[p] = load4p<FULL>(bd, p * 256 + lane * 4, D);
-      vg[p] = load4p<FULL>(gamma, p * 256 + lane * 4, D);
+      vb[p] = load4p<VT, FULL>(bd, p * 256 + lane * 4, D);
+      vg[p] = load4p<VT, FULL>(gamma, p * 256 + lane * 4, D);
     }
   }
   vec4_t<T> ny[NP], nz[NP];  // the next row's dY and Z
@@ -234,8 +236,8 @@ __global__ __launch_bounds__(BwdCfg<NP>::threads) void xf_bwd_kernel(
     for (int p = 0; p < NP; ++p) {
       const int d = p * 256 + lane * 4;
       const f32x4 dy = to_f32<T>(cy[p]), zz = to_f32<T>(cz[p]);
-      const f32x4 bb = KEEP ? vb[p] : load4p<FULL>(bd, d, D);
-      const f32x4 ga = KEEP ? vg[p] : load4p<FULL>(gamma, d, D);
+      const f32x4 bb = KEEP ? vb[p] : load4p<VT, FULL>(bd, d, D);
+      const f32x4 ga = KEEP ? vg[p] : load4p<VT, FULL>(gamma, d, D);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float zb = zz[e] + bb[e];
@@ -263,7 +265,7 @@ __global__ __launch_bounds__(BwdCfg<NP>::threads) void xf_bwd_kernel(
         for (int e = 0; e < 4; ++e) o[e] = rs * (gg[p][e] - c1 - xh[p][e] * c2) * gp[p][e];
       } else {
         const f32x4 dy = to_f32<T>(cy[p]), zz = to_f32<T>(cz[p]);
-        const f32x4 bb = load4p<FULL>(bd, d, D), ga = load4p<FULL>(gamma, d, D);
+        const f32x4 bb = load4p<VT, FULL>(bd, d, D), ga = load4p<VT, FULL>(gamma, d, D);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float zb = zz[e] + bb[e];
@@ -308,11 +310,12 @@ __global__ __launch_bounds__(BwdCfg<NP>::threads) void xf_bwd_kernel(
 // Workgroup c owns columns [64 c, 64 c + 64) of part's 3D columns, one per lane; wave w sums
 // blocks [w S, (w + 1) S) (S = ceil(nblk / COL_WAVES)) in block order, eight loads in flight,
 // and lane i of wave 0 adds the 16 wave sums in wave order. Fixed order: reproducible.
+template <typename VT>
 __global__ __launch_bounds__(64 * COL_WAVES) void xf_colsum_kernel(const float* __restrict__ part,
                                                                    int nblk, int D,
-                                                                   float* __restrict__ dgamma,
-                                                                   float* __restrict__ dbeta,
-                                                                   float* __restrict__ dbd) {
+                                                                   VT* __restrict__ dgamma,
+                                                                   VT* __restrict__ dbeta,
+                                                                   VT* __restrict__ dbd) {
   __shared__ float wsum[COL_WAVES][64];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int col = blockIdx.x * 64 + lane;
@@ -336,8 +339,8 @@ __global__ __launch_bounds__(64 * COL_WAVES) void xf_colsum_kernel(const float* 
 #pragma unroll
     for (int w = 0; w < COL_WAVES; ++w) t += wsum[w][lane];
     const int which = col / D, d = col - which * D;
-    float* dst = which == 0 ? dgamma : which == 1 ? dbeta : dbd;
-    if (dst != nullptr) dst[d] = t;
+    VT* dst = which == 0 ? dgamma : which == 1 ? dbeta : dbd;
+    if (dst != nullptr) dst[d] = from_f32<VT>(t);
   }
 }
 
@@ -404,18 +407,18 @@ static int64_t bwd_blocks(int64_t M, int64_t D) {
   return cdiv(M, (int64_t)bwd_waves(D) * rows_per_wave(M, D));
 }
 
-template <typename T>
-static int fwd(const void* z, const float* bd, const float* gamma, const float* beta, float eps,
+template <typename T, typename VT>
+static int fwd(const void* z, const VT* bd, const VT* gamma, const VT* beta, float eps,
                void* y, float* mean, float* rstd, int64_t M, int64_t D, hipStream_t st) {
   const dim3 grid((unsigned)cdiv(M, FWD_WAVES)), block(64 * FWD_WAVES);
   const bool full = D % 256 == 0;
 #define XF_FWD(NP)                                                                            \
   do {                                                                                        \
     if (full && D == NP * 256)                                                                \
-      hipLaunchKernelGGL((xf_fwd_kernel<T, NP, true>), grid, block, 0, st, (const T*)z, bd,   \
+      hipLaunchKernelGGL((xf_fwd_kernel<T, VT, NP, true>), grid, block, 0, st, (const T*)z, bd,   \
                          gamma, beta, eps, (T*)y, mean, rstd, (int)M, (int)D);                \
     else                                                                                      \
-      hipLaunchKernelGGL((xf_fwd_kernel<T, NP, false>), grid, block, 0, st, (const T*)z, bd,  \
+      hipLaunchKernelGGL((xf_fwd_kernel<T, VT, NP, false>), grid, block, 0, st, (const T*)z, bd,  \
                          gamma, beta, eps, (T*)y, mean, rstd, (int)M, (int)D);                \
   } while (0)
   switch (passes(D)) {
@@ -432,10 +435,10 @@ static int fwd(const void* z, const float* bd, const float* gamma, const float* 
   return e == hipSuccess ? SPARTON_OK : (int)e;
 }
 
-template <typename T>
-static int bwd(const void* dy, const void* z, const float* bd, const float* gamma,
-               const float* mean, const float* rstd, void* dz, float* part, float* dgamma,
-               float* dbeta, float* dbd, int64_t M, int64_t D, hipStream_t st) {
+template <typename T, typename VT>
+static int bwd(const void* dy, const void* z, const VT* bd, const VT* gamma,
+               const float* mean, const float* rstd, void* dz, float* part, VT* dgamma,
+               VT* dbeta, VT* dbd, int64_t M, int64_t D, hipStream_t st) {
   const int rpw = rows_per_wave(M, D);
   const int nblk = (int)bwd_blocks(M, D);
   const dim3 grid((unsigned)nblk), block(64 * bwd_waves(D));
@@ -444,10 +447,10 @@ static int bwd(const void* dy, const void* z, const float* bd, const float* gamm
 #define XF_BWD(NP)                                                                               \
   do {                                                                                           \
     if (full && D == NP * 256)                                                                   \
-      hipLaunchKernelGGL((xf_bwd_kernel<T, NP, true>), grid, block, lds, st, (const T*)dy,       \
+      hipLaunchKernelGGL((xf_bwd_kernel<T, VT, NP, true>), grid, block, lds, st, (const T*)dy,       \
                          (const T*)z, bd, gamma, mean, rstd, (T*)dz, part, (int)M, (int)D, rpw); \
     else                                                                                         \
-      hipLaunchKernelGGL((xf_bwd_kernel<T, NP, false>), grid, block, lds, st, (const T*)dy,      \
+      hipLaunchKernelGGL((xf_bwd_kernel<T, VT, NP, false>), grid, block, lds, st, (const T*)dy,      \
                          (const T*)z, bd, gamma, mean, rstd, (T*)dz, part, (int)M, (int)D, rpw); \
   } while (0)
   switch (passes(D)) {
@@ -460,7 +463,7 @@ static int bwd(const void* dy, const void* z, const float* bd, const float* gamm
     default: XF_BWD(12); break;
   }
 #undef XF_BWD
-  hipLaunchKernelGGL(xf_colsum_kernel, dim3((unsigned)cdiv(3 * D, 64)), dim3(64 * COL_WAVES), 0, st,
+  hipLaunchKernelGGL(xf_colsum_kernel<VT>, dim3((unsigned)cdiv(3 * D, 64)), dim3(64 * COL_WAVES), 0, st,
                      (const float*)part, nblk, (int)D, dgamma, dbeta, dbd);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? SPARTON_OK : (int)e;
@@ -485,23 +488,67 @@ extern "C" __attribute__((visibility("default"))) size_t sparton_transform_works
   return (size_t)(xf::bwd_blocks(M, D) * 3 * D) * sizeof(float);
 }
 
-extern "C" __attribute__((visibility("default"))) int sparton_transform_fwd(
-    const void* z, const float* dense_bias, const float* ln_weight, const float* ln_bias,
+// The vectors are float, or of the rows' dtype.
+static bool xf_vec_ok(int vec_dtype, int dtype) { return vec_dtype == SPARTON_F32 || vec_dtype == dtype; }
+static uintptr_t xf_vec_align(int vec_dtype) { return vec_dtype == SPARTON_F32 ? 16 : 8; }
+
+extern "C" __attribute__((visibility("default"))) int sparton_transform_fwd_typed(
+    const void* z, const void* dense_bias, const void* ln_weight, const void* ln_bias, int vec_dtype,
     float eps, void* y, float* mean, float* rstd, int64_t M, int64_t D, int dtype, void* stream) {
   const int rc = xf_check(M, D, dtype);
   if (rc != SPARTON_OK) return rc;
+  if (!xf_vec_ok(vec_dtype, dtype)) return SPARTON_EINVAL;
   if (M == 0 || D == 0) return SPARTON_OK;
   if (z == nullptr || y == nullptr || mean == nullptr || rstd == nullptr || dense_bias == nullptr ||
       ln_weight == nullptr || ln_bias == nullptr || !(eps >= 0.0f))
     return SPARTON_EINVAL;
-  if (((uintptr_t)dense_bias | (uintptr_t)ln_weight | (uintptr_t)ln_bias) % 16 != 0)
+  if (((uintptr_t)dense_bias | (uintptr_t)ln_weight | (uintptr_t)ln_bias) % xf_vec_align(vec_dtype) != 0)
     return SPARTON_EALIGN;
   hipStream_t st = (hipStream_t)stream;
+#define XF(T, VT) \
+  xf::fwd<T, VT>(z, (const VT*)dense_bias, (const VT*)ln_weight, (const VT*)ln_bias, eps, y, mean, rstd, M, D, st)
   switch (dtype) {
-    case SPARTON_BF16: return xf::fwd<bf16>(z, dense_bias, ln_weight, ln_bias, eps, y, mean, rstd, M, D, st);
-    case SPARTON_F16: return xf::fwd<f16>(z, dense_bias, ln_weight, ln_bias, eps, y, mean, rstd, M, D, st);
-    default: return xf::fwd<float>(z, dense_bias, ln_weight, ln_bias, eps, y, mean, rstd, M, D, st);
+    case SPARTON_BF16: return vec_dtype == SPARTON_F32 ? XF(bf16, float) : XF(bf16, bf16);
+    case SPARTON_F16: return vec_dtype == SPARTON_F32 ? XF(f16, float) : XF(f16, f16);
+    default: return XF(float, float);
   }
+#undef XF
+}
+
+extern "C" __attribute__((visibility("default"))) int sparton_transform_bwd_typed(
+    const void* dy, const void* z, const void* dense_bias, const void* ln_weight, int vec_dtype,
+    const float* mean, const float* rstd, void* dz, void* d_ln_weight, void* d_ln_bias,
+    void* d_dense_bias, void* workspace, size_t workspace_bytes, int64_t M, int64_t D, int dtype,
+    void* stream) {
+  const int rc = xf_check(M, D, dtype);
+  if (rc != SPARTON_OK) return rc;
+  if (!xf_vec_ok(vec_dtype, dtype)) return SPARTON_EINVAL;
+  if (M == 0 || D == 0) return SPARTON_OK;
+  if (dy == nullptr || z == nullptr || dz == nullptr || mean == nullptr || rstd == nullptr ||
+      dense_bias == nullptr || ln_weight == nullptr)
+    return SPARTON_EINVAL;
+  if (((uintptr_t)dense_bias | (uintptr_t)ln_weight) % xf_vec_align(vec_dtype) != 0) return SPARTON_EALIGN;
+  if (workspace == nullptr || workspace_bytes < sparton_transform_workspace_bytes(M, D))
+    return SPARTON_EWORKSPACE;
+  if ((uintptr_t)workspace % 16 != 0) return SPARTON_EALIGN;
+  hipStream_t st = (hipStream_t)stream;
+  float* part = (float*)workspace;
+#define XF(T, VT)                                                                                   \
+  xf::bwd<T, VT>(dy, z, (const VT*)dense_bias, (const VT*)ln_weight, mean, rstd, dz, part,          \
+                 (VT*)d_ln_weight, (VT*)d_ln_bias, (VT*)d_dense_bias, M, D, st)
+  switch (dtype) {
+    case SPARTON_BF16: return vec_dtype == SPARTON_F32 ? XF(bf16, float) : XF(bf16, bf16);
+    case SPARTON_F16: return vec_dtype == SPARTON_F32 ? XF(f16, float) : XF(f16, f16);
+    default: return XF(float, float);
+  }
+#undef XF
+}
+
+extern "C" __attribute__((visibility("default"))) int sparton_transform_fwd(
+    const void* z, const float* dense_bias, const float* ln_weight, const float* ln_bias,
+    float eps, void* y, float* mean, float* rstd, int64_t M, int64_t D, int dtype, void* stream) {
+  return sparton_transform_fwd_typed(z, dense_bias, ln_weight, ln_bias, SPARTON_F32, eps, y, mean, rstd, M, D,
+                                     dtype, stream);
 }
 
 extern "C" __attribute__((visibility("default"))) int sparton_transform_bwd(
@@ -509,29 +556,8 @@ extern "C" __attribute__((visibility("default"))) int sparton_transform_bwd(
     const float* mean, const float* rstd, void* dz, float* d_ln_weight, float* d_ln_bias,
     float* d_dense_bias, void* workspace, size_t workspace_bytes, int64_t M, int64_t D, int dtype,
     void* stream) {
-  const int rc = xf_check(M, D, dtype);
-  if (rc != SPARTON_OK) return rc;
-  if (M == 0 || D == 0) return SPARTON_OK;
-  if (dy == nullptr || z == nullptr || dz == nullptr || mean == nullptr || rstd == nullptr ||
-      dense_bias == nullptr || ln_weight == nullptr)
-    return SPARTON_EINVAL;
-  if (((uintptr_t)dense_bias | (uintptr_t)ln_weight) % 16 != 0) return SPARTON_EALIGN;
-  if (workspace == nullptr || workspace_bytes < sparton_transform_workspace_bytes(M, D))
-    return SPARTON_EWORKSPACE;
-  if ((uintptr_t)workspace % 16 != 0) return SPARTON_EALIGN;
-  hipStream_t st = (hipStream_t)stream;
-  float* part = (float*)workspace;
-  switch (dtype) {
-    case SPARTON_BF16:
-      return xf::bwd<bf16>(dy, z, dense_bias, ln_weight, mean, rstd, dz, part, d_ln_weight,
-                           d_ln_bias, d_dense_bias, M, D, st);
-    case SPARTON_F16:
-      return xf::bwd<f16>(dy, z, dense_bias, ln_weight, mean, rstd, dz, part, d_ln_weight,
-                          d_ln_bias, d_dense_bias, M, D, st);
-    default:
-      return xf::bwd<float>(dy, z, dense_bias, ln_weight, mean, rstd, dz, part, d_ln_weight,
-                            d_ln_bias, d_dense_bias, M, D, st);
-  }
+  return sparton_transform_bwd_typed(dy, z, dense_bias, ln_weight, SPARTON_F32, mean, rstd, dz, d_ln_weight,
+                                     d_ln_bias, d_dense_bias, workspace, workspace_bytes, M, D, dtype, stream);
 }
 
 extern "C" __attribute__((visibility("default"))) int sparton_transform_dz_chunks(

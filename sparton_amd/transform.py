@@ -29,7 +29,7 @@ from . import _eager, _lib
 _FLOAT_DTYPES = tuple(_lib.DTYPE_CODE)
 
 
-def _check(x: Tensor, weight: Tensor, vecs, op: str) -> int:
+def _check(x: Tensor, weight: Tensor, vecs, op: str, vec_dtype: torch.dtype = torch.float32) -> int:
     if not x.is_cuda:
         raise RuntimeError(f"{op} only supports ROCm/HIP device tensors (got device {x.device})")
     D = x.shape[-1]
@@ -38,8 +38,8 @@ def _check(x: Tensor, weight: Tensor, vecs, op: str) -> int:
     if x.dtype not in _FLOAT_DTYPES or weight.dtype != x.dtype:
         raise TypeError(f"{op}: x and weight must share a float dtype, got {x.dtype}/{weight.dtype}")
     for v in vecs:
-        if tuple(v.shape) != (D,) or v.dtype != torch.float32:
-            raise ValueError(f"{op}: bias and LayerNorm vectors must be float32 [{D}], got "
+        if tuple(v.shape) != (D,) or v.dtype != vec_dtype:
+            raise ValueError(f"{op}: bias and LayerNorm vectors must be {vec_dtype} [{D}], got "
                              f"{v.dtype} {tuple(v.shape)}")
     for t in (weight,) + tuple(vecs):
         if t.device != x.device:
@@ -227,8 +227,15 @@ class SpartonMLMTransform(nn.Module):
             x, weight = x.to(dt), weight.to(dt)
         elif weight.dtype != x.dtype:
             weight = weight.to(x.dtype)
-        args = (x, weight, self.dense.bias.float(), self.layer_norm.weight.float(),
-                self.layer_norm.bias.float(), float(self.layer_norm.eps))
+        vecs = (self.dense.bias, self.layer_norm.weight, self.layer_norm.bias)
+        eps = float(self.layer_norm.eps)
+        if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and all(v.dtype == x.dtype for v in vecs)
+                and not torch.compiler.is_compiling()):
+            # a model held in 16 bits: the kernels read the vectors, and write their gradients,
+            # as they are (six casts and their autograd nodes fewer per step)
+            _check(x, weight, vecs, "SpartonMLMTransform", x.dtype)
+            return _eager.load().mlm_transform_typed(x, weight, *vecs, eps)
+        args = (x, weight, *(v.float() for v in vecs), eps)
         if torch.compiler.is_compiling() or not x.is_cuda:  # the registered op: fake + autograd
             return torch.ops.sparton.mlm_transform_fwd(*args)[0]
         # eager: the C++ op (autograd in C++), the same implementation as the custom ops

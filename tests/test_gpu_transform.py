@@ -202,3 +202,47 @@ def test_transform_auxiliary_outputs_not_differentiable(device):
     x.requires_grad_()
     y, z, mean, rstd = torch.ops.sparton.mlm_transform_fwd(x, w, b, g, bt, 1e-5)
     assert y.requires_grad and not (z.requires_grad or mean.requires_grad or rstd.requires_grad)
+
+
+@pytest.mark.parametrize("dt,M,D", [("bf16", 33, 8), ("fp16", 130, 1000), ("bf16", 2048, 768), ("fp16", 70, 1500)])
+def test_module_in_16_bits_equals_float_vectors(dt, M, D, device):
+    """A module held in 16 bits runs on its vectors as they are (mlm_transform_typed): what the
+    op gives on their float32 copies, each vector's gradient rounded once from its float32
+    sum. bf16 the same bits; fp16 within one rounding (2^-11 of a value, 2^-24 below fp16's
+    normal range), as the last multiply-add may round straight to fp16, and what the GEMMs
+    make of that."""
+    dtype = {"bf16": torch.bfloat16, "fp16": torch.float16}[dt]
+    g = torch.Generator().manual_seed(M + D)
+    rand = lambda *n: torch.randn(*n, generator=g)
+    dense, norm = torch.nn.Linear(D, D), torch.nn.LayerNorm(D)
+    with torch.no_grad():
+        dense.weight.copy_(rand(D, D) * D ** -0.5)
+        dense.bias.copy_(rand(D) * 0.1)
+        norm.weight.copy_(1 + rand(D) * 0.1)
+        norm.bias.copy_(rand(D) * 0.1)
+    module = sparton_amd.SpartonMLMTransform(dense, norm).to(device, dtype)
+    x = rand(M, D).to(device, dtype).requires_grad_()
+    dy = rand(M, D).to(device, dtype)
+    y = module(x)
+    y.backward(dy)
+    x2, w2 = x.detach().clone().requires_grad_(), dense.weight.detach().clone().requires_grad_()
+    vecs = [v.detach().float().requires_grad_() for v in (dense.bias, norm.weight, norm.bias)]
+    from sparton_amd import _eager
+    y2 = _eager.load().mlm_transform(x2, w2, *vecs, float(norm.eps))
+    y2.backward(dy)
+    def same(a, b):
+        if dt == "bf16":
+            assert torch.equal(a, b)
+        else:  # relative to the tensor's scale: the GEMMs' sums mix rounded values
+            a, b = a.detach().double(), b.detach().double()
+            assert float((a - b).abs().max()) <= 2.0 ** -10 * float(b.abs().max())
+    same(y, y2)
+    same(x.grad, x2.grad)
+    same(dense.weight.grad, w2.grad)
+    for p, v in zip((dense.bias, norm.weight, norm.bias), vecs):
+        assert p.grad.dtype == dtype
+        same(p.grad, v.grad.to(dtype))
+    with torch.no_grad():
+        assert torch.equal(module(x), y)
+    with pytest.raises(RuntimeError):
+        _eager.load().mlm_transform(x2, w2, dense.bias, norm.weight, norm.bias, 1e-5)
