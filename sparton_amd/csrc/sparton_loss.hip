@@ -388,10 +388,12 @@ static void bwd_all(const void* q, const void* d, const float* P, const Grads6& 
 // The kernels above stage every row of a 64-column slice and keep per-slice partials of all
 // Bq x Bd scores; their per-thread work grows with the rows, and past 64 rows a side the
 // kernels below are faster (V 30522, fwd+bwd device time: 96 rows 134 us against 81 us, 128
-// rows 190 against 90; 64 rows 62 against 70). Larger batches take GEMM-shaped kernels on the
-// fp32 matrix cores (v_mfma_f32_32x32x2f32: the products of any reps dtype are exact in fp32,
-// and the sums accumulate in fp32, as above; 16-bit reps have the variants further down):
-//   forward   loss_stats_kernel   per 64-column slice: each row's sum of |x| over the slice,
+// rows 190 against 90; 64 rows 62 against 70). Larger batches take GEMM-shaped kernels; the
+// score and gradient kernels further down run on the 16-bit matrix cores, those here on the fp32
+// ones (v_mfma_f32_32x32x2f32: the products of any reps dtype are exact in fp32, and the sums
+// accumulate in fp32, as above), which tests compare them with and which the tiles of fp32 and
+// fp16 reps with an entry that is not finite take:
+//   forward   loss_stats_kernel   per 128-column slice: each row's sum of |x| over the slice,
 //                                 and sum_v (sum_b x)^2 of Q and of R;
 //             loss_score_kernel   S = Q R^T in 128 x 128 tiles, the vocabulary split into
 //                                 chunks (one partial S per chunk);
@@ -412,6 +414,7 @@ constexpr int LDA = 161;  // floats per k row of a [KS][128] tile
 constexpr int NC = 64;    // backward: vocabulary columns per workgroup
 constexpr int LDB = 97;   // floats per k row of a [KS][64] tile
 constexpr int ST_ROWS = 32;  // stats: rows whose loads are in flight together per wave
+constexpr int ST_COLS = 128;  // and columns per workgroup
 
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 z;
@@ -426,11 +429,13 @@ template <typename T>
 __device__ __forceinline__ void load_kc(const T* __restrict__ X, int64_t ld, int m0, int M, int k0,
                                         int kend, T (&v)[16]) {
   const int t = threadIdx.x, k = k0 + (t & 31), rb = t >> 5;
+  // every load from a clamped place, zeroed afterwards: a load under its own condition would be
+  // waited for before the next
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
-    const int m = m0 + rb + 8 * u;
-    v[u] = (m < M && k < kend) ? X[(int64_t)m * ld + k] : T(0.0f);
-  }
+  for (int u = 0; u < 16; ++u) v[u] = X[(int64_t)min(m0 + rb + 8 * u, M - 1) * ld + min(k, kend - 1)];
+#pragma unroll
+  for (int u = 0; u < 16; ++u)
+    if (!(m0 + rb + 8 * u < M && k < kend)) v[u] = T(0.0f);
 }
 template <typename T>
 __device__ __forceinline__ void store_kc(float* s, const T (&v)[16]) {
@@ -447,10 +452,11 @@ __device__ __forceinline__ void load_nc(const T* __restrict__ X, int64_t ld, int
   constexpr int KSTEP = NT / NN;
   const int t = threadIdx.x, n = n0 + t % NN, kb = t / NN;
 #pragma unroll
-  for (int u = 0; u < KS / KSTEP; ++u) {
-    const int k = k0 + kb + KSTEP * u;
-    v[u] = (k < kend && n < nend) ? X[(int64_t)k * ld + n] : T(0.0f);
-  }
+  for (int u = 0; u < KS / KSTEP; ++u)
+    v[u] = X[(int64_t)min(k0 + kb + KSTEP * u, kend - 1) * ld + min(n, nend - 1)];
+#pragma unroll
+  for (int u = 0; u < KS / KSTEP; ++u)
+    if (!(k0 + kb + KSTEP * u < kend && n < nend)) v[u] = T(0.0f);
 }
 template <typename T, int NN, int LD>
 __device__ __forceinline__ void store_nc(float* s, const T (&v)[KS * NN / NT]) {
@@ -485,6 +491,28 @@ __device__ __forceinline__ void mma_stage(const float* sA, int am0, const float*
 // lane % 32).
 __device__ __forceinline__ int acc_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
 
+// acc += Q R^T over columns [kc0, kc1) for the 128 x 128 tile at (i0, j0), in [KS][LDA] tiles.
+template <typename T>
+__device__ __forceinline__ void score_tile(float* sA, float* sB, const T* __restrict__ Q,
+                                           const T* __restrict__ R, int Bq, int Bd, int V, int i0, int j0,
+                                           int kc0, int kc1, f32x16 (&acc)[2][2]) {
+  const int wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
+  T ra[16], rb[16];
+  load_kc(Q, V, i0, Bq, kc0, kc1, ra);
+  load_kc(R, V, j0, Bd, kc0, kc1, rb);
+  for (int k0 = kc0; k0 < kc1; k0 += KS) {
+    __syncthreads();  // the previous stage is read
+    store_kc(sA, ra);
+    store_kc(sB, rb);
+    __syncthreads();
+    if (k0 + KS < kc1) {  // the next stage's loads run under this stage's MFMAs
+      load_kc(Q, V, i0, Bq, k0 + KS, kc1, ra);
+      load_kc(R, V, j0, Bd, k0 + KS, kc1, rb);
+    }
+    mma_stage<2, 2, LDA, LDA>(sA, wm * 64, sB, wn * 64, acc);
+  }
+}
+
 // Partial S = Q R^T over the vocabulary chunk blockIdx.y (columns [chunk y, chunk (y+1))) for
 // the 128 x 128 tile blockIdx.x, at part + y Bq Bd. Four waves of 64 x 64 (2 x 2 blocks).
 template <typename T>
@@ -502,20 +530,7 @@ __global__ __launch_bounds__(NT) void loss_score_kernel(const T* __restrict__ Q,
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
-  T ra[16], rb[16];
-  load_kc(Q, V, i0, Bq, kc0, kc1, ra);
-  load_kc(R, V, j0, Bd, kc0, kc1, rb);
-  for (int k0 = kc0; k0 < kc1; k0 += KS) {
-    __syncthreads();  // the previous stage is read
-    store_kc(sA, ra);
-    store_kc(sB, rb);
-    __syncthreads();
-    if (k0 + KS < kc1) {  // the next stage's loads run under this stage's MFMAs
-      load_kc(Q, V, i0, Bq, k0 + KS, kc1, ra);
-      load_kc(R, V, j0, Bd, k0 + KS, kc1, rb);
-    }
-    mma_stage<2, 2, LDA, LDA>(sA, wm * 64, sB, wn * 64, acc);
-  }
+  score_tile(sA, sB, Q, R, Bq, Bd, V, i0, j0, kc0, kc1, acc);
   float* out = part + (size_t)blockIdx.y * Bq * Bd;
   const int l32 = lane & 31, h = lane >> 5;
 #pragma unroll
@@ -531,50 +546,72 @@ __global__ __launch_bounds__(NT) void loss_score_kernel(const T* __restrict__ Q,
     }
 }
 
-// Per 64-column slice (blockIdx.x), at part + slice K: entries [0, Bq) and [Bq, Bq + Bd) the
-// rows' sums of |x| over the slice, Bq + Bd and Bq + Bd + 1 the slice's sum_v (sum_b x)^2 of Q
-// and of R. Wave w takes rows w, w + 4, ...; column sums are added over the waves in order.
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+template <typename T> using Two = T __attribute__((ext_vector_type(2)));
+
+// N rows r0, r0 + step, .. (r0 uniform) of X at columns c, c + 1 (c even), two to a load where rows
+// and columns allow it (pair: V even, X aligned to two elements). Rows past K read zero; columns
+// past V whatever is there (nothing of theirs is stored).
+template <typename T, int N>
+__device__ __forceinline__ void load_x(const T* __restrict__ X, bool pair, int K, int r0, int step, int c,
+                                       int V, Two<T> (&v)[N]) {
+  if (pair) {  // uniform
+    const uint32_t cc = (uint32_t)min(c, V - 2);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const T* row = X + (int64_t)min(r0 + step * i, K - 1) * V;
+      v[i] = *(const Two<T>*)(row + cc);
+    }
+  } else {
+    const uint32_t ca = (uint32_t)min(c, V - 1), cb = (uint32_t)min(c + 1, V - 1);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const T* row = X + (int64_t)min(r0 + step * i, K - 1) * V;
+      v[i] = Two<T>{row[ca], row[cb]};
+    }
+  }
+  if (r0 + step * (N - 1) >= K)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (r0 + step * i >= K) v[i] = Two<T>{T(0.0f), T(0.0f)};
+}
+// Side blockIdx.y (Q, R) of the 128-column slice blockIdx.x, at part + slice K: entries [0, Bq) and
+// [Bq, Bq + Bd) the rows' sums of |x| over the slice, Bq + Bd and Bq + Bd + 1 the slice's
+// sum_v (sum_b x)^2 of Q and of R. Wave w takes rows w, w + 4, ..., two columns a lane; column sums
+// are added over the waves in order. Bound by the loads' latency: a workgroup for each side, and
+// ST_ROWS rows' loads in flight (256 x 512 x 30522 fp16: 28 -> 20 us).
 template <typename T>
 __global__ __launch_bounds__(NT) void loss_stats_kernel(const T* __restrict__ Q, const T* __restrict__ R,
-                                                        int Bq, int Bd, int V, float* __restrict__ part,
-                                                        int K) {
-  __shared__ float cpart[4][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c = blockIdx.x * 64 + lane;
-  const bool cv = c < V;
+                                                        bool pair, int Bq, int Bd, int V,
+                                                        float* __restrict__ part, int K) {
+  __shared__ f32x2 cpart[4][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = blockIdx.x * ST_COLS + 2 * lane, side = blockIdx.y;
+  const T* X = side ? R : Q;
+  const int rows = side ? Bd : Bq, o = side ? Bq : 0;
   float* out = part + (size_t)blockIdx.x * K;
-  for (int side = 0; side < 2; ++side) {
-    const T* X = side ? R : Q;
-    const int rows = side ? Bd : Bq, o = side ? Bq : 0;
-    float cs = 0.0f;
-    for (int b0 = wave; b0 < rows; b0 += 4 * ST_ROWS) {  // uniform per wave
-      // every load issued, from clamped indices, before any is used
-      T v[ST_ROWS];
+  f32x2 cs = {0.0f, 0.0f};
+  for (int b0 = wave; b0 < rows; b0 += 4 * ST_ROWS) {
+    Two<T> v[ST_ROWS];
+    load_x<T>(X, pair, rows, b0, 4, c, V, v);
 #pragma unroll
-      for (int u = 0; u < ST_ROWS; ++u)
-        v[u] = X[(int64_t)min(b0 + 4 * u, rows - 1) * V + min(c, V - 1)];
-#pragma unroll
-      for (int u = 0; u < ST_ROWS; ++u)
-        if (!(b0 + 4 * u < rows && cv)) v[u] = T(0.0f);
-#pragma unroll
-      for (int u = 0; u < ST_ROWS; ++u) {
-        const int b = b0 + 4 * u;
-        if (b < rows) {
-          const float x = to_f32(v[u]);
-          cs += x;
-          const float a = wave_sum(fabsf(x));
-          if (lane == 0) out[o + b] = a;
-        }
+    for (int u = 0; u < ST_ROWS; ++u) {
+      const int b = b0 + 4 * u;
+      if (b < rows) {  // uniform
+        const float x0 = c < V ? to_f32((T)v[u][0]) : 0.0f, x1 = c + 1 < V ? to_f32((T)v[u][1]) : 0.0f;
+        cs[0] += x0;
+        cs[1] += x1;
+        const float a = wave_sum(fabsf(x0) + fabsf(x1));
+        if (lane == 0) out[o + b] = a;
       }
     }
-    cpart[wave][lane] = cs;
-    __syncthreads();
-    if (wave == 0) {
-      const float tot = ((cpart[0][lane] + cpart[1][lane]) + cpart[2][lane]) + cpart[3][lane];
-      const float sq = wave_sum(tot * tot);
-      if (lane == 0) out[Bq + Bd + side] = sq;
-    }
-    __syncthreads();
+  }
+  cpart[wave][lane] = cs;
+  __syncthreads();
+  if (wave == 0) {
+    const f32x2 tot = ((cpart[0][lane] + cpart[1][lane]) + cpart[2][lane]) + cpart[3][lane];
+    const float sq = wave_sum(tot[0] * tot[0] + tot[1] * tot[1]);
+    if (lane == 0) out[Bq + Bd + side] = sq;
   }
 }
 
@@ -625,275 +662,6 @@ __global__ __launch_bounds__(64) void loss_final_large_kernel(const float* __res
     out[4] = flq;
     out[5] = fld;
   }
-}
-
-// ---- 16-bit reps on 16-bit MFMAs ----
-//
-// A product of two bf16 (or two fp16) values is exact in fp32, so for 16-bit reps the score
-// GEMM runs on v_mfma_f32_32x32x16_{bf16,f16}: 8 times the k per instruction of the fp32
-// MFMA, in the same 32 x 32 output layout. The stage's operands are kept in LDS as [row][k]
-// 16-bit values, rows LDH apart: 80 bytes, so the 16 rows of one ds_read_b128 phase fall in
-// distinct banks. A lane's MFMA operand (8 consecutive k of one row) is one 16-byte read.
-// The global loads are those of the fp32 path (element by element: a row of V elements is
-// not 16-byte aligned in general).
-// The gradients' products P R and P^T Q take P (fp32) as two bf16 parts, p = hi + lo + r
-// with |r| <= 2^-18 |p| (both round to nearest even, p - hi is exact), against R or Q exact
-// in bf16: two MFMAs per step, lo first. fp16 reps keep the fp32 MFMA there (P's range does
-// not fit fp16).
-constexpr int LDH = 40;
-
-template <typename T> struct Mfma16;
-template <> struct Mfma16<bf16> {
-  static __device__ __forceinline__ f32x16 run(const u32x4& a, const u32x4& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mfma16<f16> {
-  static __device__ __forceinline__ f32x16 run(const u32x4& a, const u32x4& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
-
-template <typename T> __device__ __forceinline__ uint16_t bits16(T x) {
-  return __builtin_bit_cast(uint16_t, x);
-}
-
-// load_kc's registers (thread t: k = t % 32 of rows t / 32 + 8 u) into a [rows][KS] tile.
-template <typename T>
-__device__ __forceinline__ void store_kc16(uint16_t* s, const T (&v)[16]) {
-  const int t = threadIdx.x, kk = t & 31, rb = t >> 5;
-#pragma unroll
-  for (int u = 0; u < 16; ++u) s[(rb + 8 * u) * LDH + kk] = bits16(v[u]);
-}
-
-// The operand of lane (l32, h) for k step s of a stage: row `row`, k = 16 s + 8 h .. + 7.
-__device__ __forceinline__ u32x4 frag16(const uint16_t* s, int row, int ks) {
-  const int h = (threadIdx.x & 63) >> 5;
-  return *(const u32x4*)(s + row * LDH + 16 * ks + 8 * h);
-}
-
-// acc[bi][bj] += A[am0 + 32 bi .., :] B[bn0 + 32 bj .., :]^T over one stage.
-template <typename T, int BI, int BJ>
-__device__ __forceinline__ void mma16_stage(const uint16_t* sA, int am0, const uint16_t* sB, int bn0,
-                                            f32x16 (&acc)[BI][BJ]) {
-  const int l32 = threadIdx.x & 31;
-#pragma unroll
-  for (int ks = 0; ks < KS / 16; ++ks) {
-    u32x4 a[BI], b[BJ];
-#pragma unroll
-    for (int i = 0; i < BI; ++i) a[i] = frag16(sA, am0 + 32 * i + l32, ks);
-#pragma unroll
-    for (int j = 0; j < BJ; ++j) b[j] = frag16(sB, bn0 + 32 * j + l32, ks);
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) acc[i][j] = Mfma16<T>::run(a[i], b[j], acc[i][j]);
-  }
-}
-
-// loss_score_kernel for 16-bit reps.
-template <typename T>
-__global__ __launch_bounds__(NT) void loss_score16_kernel(const T* __restrict__ Q,
-                                                          const T* __restrict__ R, int Bq, int Bd,
-                                                          int V, int chunk, float* __restrict__ part) {
-  __shared__ __attribute__((aligned(16))) uint16_t sA[TM * LDH];
-  __shared__ __attribute__((aligned(16))) uint16_t sB[TM * LDH];
-  const int tj = (Bd + TM - 1) / TM;
-  const int i0 = (blockIdx.x / tj) * TM, j0 = (blockIdx.x % tj) * TM;
-  const int kc0 = blockIdx.y * chunk, kc1 = min(V, kc0 + chunk);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wm = wave >> 1, wn = wave & 1;
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
-  T ra[16], rb[16];
-  load_kc(Q, V, i0, Bq, kc0, kc1, ra);
-  load_kc(R, V, j0, Bd, kc0, kc1, rb);
-  for (int k0 = kc0; k0 < kc1; k0 += KS) {
-    __syncthreads();  // the previous stage is read
-    store_kc16(sA, ra);
-    store_kc16(sB, rb);
-    __syncthreads();
-    if (k0 + KS < kc1) {  // the next stage's loads run under this stage's MFMAs
-      load_kc(Q, V, i0, Bq, k0 + KS, kc1, ra);
-      load_kc(R, V, j0, Bd, k0 + KS, kc1, rb);
-    }
-    mma16_stage<T, 2, 2>(sA, wm * 64, sB, wn * 64, acc);
-  }
-  float* out = part + (size_t)blockIdx.y * Bq * Bd;
-  const int l32 = lane & 31, h = lane >> 5;
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj) {
-      const int j = j0 + wn * 64 + 32 * bj + l32;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = i0 + wm * 64 + 32 * bi + acc_row(r, h);
-        if (i < Bq && j < Bd) out[(size_t)i * Bd + j] = acc[bi][bj][r];
-      }
-    }
-}
-
-// p as bf16 hi and lo bits.
-__device__ __forceinline__ void split_bf16(float p, uint16_t& hi, uint16_t& lo) {
-  const bf16 h = (bf16)p;
-  hi = bits16(h);
-  lo = bits16((bf16)(p - (float)h));
-}
-
-// ---- bf16 gradients as one tiled GEMM grid ----
-//
-// Both gradients are GEMMs over the other side's rows plus per-element terms:
-//   dQ = c_ce P R + ...  (K = Bd),   dR = c_ce P^T Q + ...  (K = Bq).
-// A workgroup owns GC columns and row tile t of both (dQ rows and dR rows 128 t ..
-// 128 t + 127; either may be empty), four waves of 64 x 64 per tile. The dQ GEMM streams
-// all of R's rows for its columns, so it also sums R's columns (the FLOPS term of dR), and
-// the dR GEMM sums Q's (that of dQ); a workgroup with only one of the tiles streams the
-// other side for its sums alone. No workspace: everything stays in the workgroup.
-constexpr int GC = 128;
-
-// One GEMM tile: acc += A B^T over k in [0, K), A = P rows m0.. (A_KC) or P columns m0..,
-// B = X[k][c0 ..] (bf16). cs accumulates thread t's share of X's column sums (column
-// t % GC, k rows of parity t / GC). With MM false only the sums are taken.
-template <bool A_KC, bool MM>
-__device__ __forceinline__ void gemm16(uint16_t* sAh, uint16_t* sAl, uint16_t* sB,
-                                       const float* __restrict__ P, int Bq, int Bd,
-                                       const bf16* __restrict__ X, int K, int m0, int c0, int V,
-                                       f32x16 (&acc)[2][2], float& cs) {
-  const int t = threadIdx.x, wave = t >> 6, l32 = t & 31, wm = wave >> 1, wn = wave & 1;
-  if (K <= 0) return;
-  float pa[16];
-  bf16 rbv[KS * GC / NT];
-  auto load = [&](int k0) {
-    if (MM) {
-      if (A_KC) load_kc(P, Bd, m0, Bq, k0, K, pa);         // A[m][k] = P[m0 + m][k]
-      else load_nc<float, TM>(P, Bd, k0, K, m0, Bd, pa);   // A[m][k] = P[k][m0 + m]
-    }
-    load_nc<bf16, GC>(X, V, k0, K, c0, V, rbv);            // B[n][k] = X[k][c0 + n]
-  };
-  load(0);
-  for (int k0 = 0; k0 < K; k0 += KS) {
-#pragma unroll
-    for (int u = 0; u < KS * GC / NT; ++u) cs += to_f32(rbv[u]);
-    if (MM) {
-      __syncthreads();  // the previous stage is read
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        // load_kc: k = t % 32 of rows t / 32 + 8 u; load_nc<TM>: m = t % 128 of k rows t / 128 + 2 u
-        const int m = A_KC ? (t >> 5) + 8 * u : t % TM;
-        const int k = A_KC ? (t & 31) : t / TM + 2 * u;
-        uint16_t hi, lo;
-        split_bf16(pa[u], hi, lo);
-        sAh[m * LDH + k] = hi;
-        sAl[m * LDH + k] = lo;
-      }
-#pragma unroll
-      for (int u = 0; u < KS * GC / NT; ++u)  // load_nc<GC>: n = t % GC of k rows t / GC + 2 u
-        sB[(t % GC) * LDH + t / GC + (NT / GC) * u] = bits16(rbv[u]);
-      __syncthreads();
-    }
-    if (k0 + KS < K) load(k0 + KS);  // the next stage's loads run under this stage's MFMAs
-    if (MM) {
-#pragma unroll
-      for (int ks = 0; ks < KS / 16; ++ks) {
-        u32x4 ah[2], al[2], b[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          ah[i] = frag16(sAh, wm * 64 + 32 * i + l32, ks);
-          al[i] = frag16(sAl, wm * 64 + 32 * i + l32, ks);
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = frag16(sB, wn * 64 + 32 * j + l32, ks);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            acc[i][j] = Mfma16<bf16>::run(al[i], b[j], acc[i][j]);
-            acc[i][j] = Mfma16<bf16>::run(ah[i], b[j], acc[i][j]);
-          }
-      }
-    }
-  }
-}
-
-// G[i][c] = c_ce acc + c_s sign(X[i][c]) + c_f colsum[c] for the tile's rows below `rows`.
-__device__ __forceinline__ void grad16_epilogue(const f32x16 (&acc)[2][2], const bf16* __restrict__ X,
-                                                int rows, int m0, int c0, int V, float c_ce,
-                                                float c_s, float c_f, const float* colsum,
-                                                bf16* __restrict__ G) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
-  const int wm = wave >> 1, wn = wave & 1;
-#pragma unroll
-  for (int bj = 0; bj < 2; ++bj) {
-    const int cl = wn * 64 + 32 * bj + l32, c = c0 + cl;
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi) {
-      bf16 xv[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = m0 + wm * 64 + 32 * bi + acc_row(r, h);
-        xv[r] = (i < rows && c < V) ? X[(int64_t)i * V + c] : bf16(0.0f);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = m0 + wm * 64 + 32 * bi + acc_row(r, h);
-        if (i < rows && c < V) {
-          const float x = to_f32(xv[r]);
-          const float sg = x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f);
-          G[(int64_t)i * V + c] = from_f32<bf16>(c_ce * acc[bi][bj][r] + c_s * sg + c_f * colsum[cl]);
-        }
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(NT) void loss_grad16_kernel(const bf16* __restrict__ Q,
-                                                         const bf16* __restrict__ R,
-                                                         const float* __restrict__ P, const Grads6 g,
-                                                         int Bq, int Bd, int V, float w_ce,
-                                                         float w_l1, float w_fl,
-                                                         bf16* __restrict__ GQ,
-                                                         bf16* __restrict__ GR) {
-  __shared__ __attribute__((aligned(16))) uint16_t sAh[TM * LDH];
-  __shared__ __attribute__((aligned(16))) uint16_t sAl[TM * LDH];
-  __shared__ __attribute__((aligned(16))) uint16_t sB[GC * LDH];
-  __shared__ float csp[2][2][GC];   // [side][k parity][column]
-  __shared__ float colsum[2][GC];
-  const int t = threadIdx.x;
-  const int c0 = blockIdx.x * GC, m0 = blockIdx.y * TM;
-  const bool has_q = m0 < Bq, has_r = m0 < Bd;
-  f32x16 accq[2][2], accr[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      accq[i][j] = zero16();
-      accr[i][j] = zero16();
-    }
-  float csq = 0.0f, csr = 0.0f;
-  // dQ streams R (K = Bd): R's column sums for dR
-  if (has_q) gemm16<true, true>(sAh, sAl, sB, P, Bq, Bd, R, Bd, m0, c0, V, accq, csr);
-  else if (has_r) gemm16<true, false>(sAh, sAl, sB, P, Bq, Bd, R, Bd, m0, c0, V, accq, csr);
-  // dR streams Q (K = Bq): Q's column sums for dQ
-  if (has_r) gemm16<false, true>(sAh, sAl, sB, P, Bq, Bd, Q, Bq, m0, c0, V, accr, csq);
-  else if (has_q) gemm16<false, false>(sAh, sAl, sB, P, Bq, Bd, Q, Bq, m0, c0, V, accr, csq);
-  csp[0][t / GC][t % GC] = csq;
-  csp[1][t / GC][t % GC] = csr;
-  __syncthreads();
-  if (t < 2 * GC) colsum[t / GC][t % GC] = csp[t / GC][0][t % GC] + csp[t / GC][1][t % GC];
-  __syncthreads();
-  const float g0 = grad_of(g, 0);
-  const float c_ce = g0 * w_ce + grad_of(g, 1);
-  const float c_sq = (g0 * w_l1 + grad_of(g, 2)) / (float)Bq;
-  const float c_sd = Bd > 0 ? (g0 * w_l1 + grad_of(g, 3)) / (float)Bd : 0.0f;
-  const float c_fq = 2.0f * (g0 * w_fl + grad_of(g, 4)) / (float)V;
-  const float c_fd = 2.0f * (g0 * w_fl + grad_of(g, 5)) / (float)V;
-  if (has_q) grad16_epilogue(accq, Q, Bq, m0, c0, V, c_ce, c_sq, c_fq, colsum[0], GQ);
-  if (has_r) grad16_epilogue(accr, R, Bd, m0, c0, V, c_ce, c_sd, c_fd, colsum[1], GR);
 }
 
 // 128 rows of one gradient over the workgroup's 64 columns: acc = sum_k A[m][k] B[k][n] with A
@@ -950,6 +718,511 @@ __device__ __forceinline__ void grad_tile(float* sA, float* sB, const float* __r
         G[(int64_t)i * V + c] = from_f32<T>(c_ce * acc[0][bj][r] + c_s * sg + c_f * colsum[cl]);
       }
     }
+  }
+}
+
+// ---- score and gradients on 16-bit MFMAs ----
+//
+// A product of two bf16 (or two fp16) values is exact in fp32, so for 16-bit reps the score
+// GEMM runs on v_mfma_f32_32x32x16_{bf16,f16}: 8 times the k per instruction of the fp32
+// MFMA, in the same 32 x 32 output layout. The stage's operands are kept in LDS as [row][k]
+// 16-bit values, rows LDH apart: 80 bytes, so the 16 rows of one ds_read_b128 phase fall in
+// distinct banks. A lane's MFMA operand (8 consecutive k of one row) is one 16-byte read.
+// Other operands are taken as sums of bf16 parts, x = x0 + x1 + ... (each part rounds what
+// the ones before it left to nearest even; the remainders are exact): three parts hold an
+// fp32 value's 24 bits, two an fp16 value's 11, and bf16 has fp32's exponents, so no scales
+// are needed. A product takes the pairs of parts down to 2^-24 of it:
+//   scores     fp32 reps 3 x 3 parts, 6 MFMAs per step (against 8 fp32 ones of twice the time)
+//   gradients  P (fp32) against bf16 reps 2 x 1 parts (p within 2^-18), 2 MFMAs; fp16 reps
+//              3 x 2 parts, 5; fp32 reps 3 x 3, 6
+// The products of the lower parts have accumulators of their own, added at the end: the main
+// sums then round once per 16 k (the fp32 MFMA's: 8 times), and over batches of 65 to 500 rows
+// and V 257 to 30522 the gradients' rms error against fp64 is that of the fp32 MFMAs or below
+// (0.65 to 1.0 of it, also where it is all sums; with one set of accumulators it was twice that).
+// Every load of a row goes two elements at a time: a row of V elements starts on any 2- or
+// 4-byte boundary, and 16-byte loads off theirs took 1.6 times as long (256 x 512 x 30522 fp16
+// score 42.6 us against 27.2).
+// Forward and backward of 256 x 512 x 30522, before (fp32 MFMAs, bf16 reps on bf16 ones) -> now:
+// fp16 398 -> 184 us, bf16 326 -> 154, fp32 436 -> 236; 512 x 1024 bf16 972 -> 400, fp32
+// 1448 -> 710; 65 x 130 and 128 x 128, where the launches weigh most, 93-112 -> 90-109.
+constexpr int LDH = 40;
+
+template <typename T> struct Mfma16;
+template <> struct Mfma16<bf16> {
+  static __device__ __forceinline__ f32x16 run(const u32x4& a, const u32x4& b, const f32x16& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+template <> struct Mfma16<f16> {
+  static __device__ __forceinline__ f32x16 run(const u32x4& a, const u32x4& b, const f32x16& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+};
+
+template <typename T> __device__ __forceinline__ uint16_t bits16(T x) {
+  return __builtin_bit_cast(uint16_t, x);
+}
+
+// Parts of the reps in the score GEMM, of P and of the reps in the gradients.
+template <typename T> struct Parts {
+  static constexpr int S = sizeof(T) == 4 ? 3 : 1;
+  static constexpr int P = std::is_same<T, bf16>::value ? 2 : 3;
+  static constexpr int X = sizeof(T) == 4 ? 3 : std::is_same<T, f16>::value ? 2 : 1;
+  typedef typename std::conditional<sizeof(T) == 4, bf16, T>::type ST;  // the score MFMA's type
+};
+
+// Two values as N parts, a pair of bf16 each.
+template <int N>
+__device__ __forceinline__ void parts2(f32x2 r, uint32_t (&p)[N]) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    p[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+    r = r - f32x2{__uint_as_float(p[i] << 16), __uint_as_float(p[i] & 0xffff0000u)};
+  }
+}
+// Eight consecutive k of one row as N parts, 16 bytes each.
+template <int N>
+__device__ __forceinline__ void parts8(const float (&x)[8], u32x4 (&p)[N]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t w[N];
+    parts2<N>(f32x2{x[2 * q], x[2 * q + 1]}, w);
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i][q] = w[i];
+  }
+}
+
+// A stage of a K-contiguous operand X[m][k] (row stride V): thread t holds k = k0 + 2 (t % 16), + 1
+// of rows m0 + t / 16 + 16 u, two to a load where rows lie on 4-byte boundaries (`pair`); from
+// clamped places otherwise and at the end of K, zero past it. Rows past M repeat the last one
+// (nothing of theirs is stored).
+template <typename T>
+__device__ __forceinline__ void load_rows(const T* __restrict__ X, bool pair, int V, int m0, int M, int k0,
+                                          int kend, Two<T> (&v)[8]) {
+  const int t = threadIdx.x, k = k0 + 2 * (t & 15);
+  typedef Two<T> __attribute__((aligned(4))) two;
+  if (pair && k0 + KS <= kend) {  // uniform
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      v[u] = *(const two*)(X + (int64_t)min(m0 + (t >> 4) + 16 * u, M - 1) * V + k);
+  } else {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const T* row = X + (int64_t)min(m0 + (t >> 4) + 16 * u, M - 1) * V;
+      const T a = row[min(k, kend - 1)], b = row[min(k + 1, kend - 1)];
+      v[u] = Two<T>{k < kend ? a : T(0.0f), k + 1 < kend ? b : T(0.0f)};
+    }
+  }
+}
+// Into [rows][KS] tiles, one per part, TM * LDH apart.
+template <int N, typename T>
+__device__ __forceinline__ void store_rows(uint16_t* s, const Two<T> (&v)[8]) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    uint16_t* to = s + ((t >> 4) + 16 * u) * LDH + 2 * (t & 15);
+    if constexpr (N == 1) {
+      *(uint32_t*)to = __builtin_bit_cast(uint32_t, v[u]);
+    } else {
+      uint32_t p[N];
+      parts2<N>(v[u], p);
+#pragma unroll
+      for (int i = 0; i < N; ++i) *(uint32_t*)(to + i * TM * LDH) = p[i];
+    }
+  }
+}
+
+// The operand of lane (l32, h) for k step s of a stage: row `row`, k = 16 s + 8 h .. + 7.
+__device__ __forceinline__ u32x4 frag16(const uint16_t* s, int row, int ks) {
+  const int h = (threadIdx.x & 63) >> 5;
+  return *(const u32x4*)(s + row * LDH + 16 * ks + 8 * h);
+}
+
+// acc[bi][bj] += A[am0 + 32 bi .., :] B[bn0 + 32 bj .., :]^T over one stage, A in NA parts and B
+// in NB (tiles of 128 rows): the pairs (i, j) with i + j < max(NA, NB), smallest first.
+template <typename T, int NA, int NB, bool SPLIT>
+__device__ __forceinline__ void mma16_stage(const uint16_t* sA, int am0, const uint16_t* sB, int bn0,
+                                            f32x16 (&acc)[2][2], f32x16 (&low)[2][2]) {
+  constexpr int W = NA > NB ? NA : NB;
+  const int l32 = threadIdx.x & 31;
+#pragma unroll
+  for (int ks = 0; ks < KS / 16; ++ks) {
+    u32x4 a[NA][2], b[NB][2];
+#pragma unroll
+    for (int p = 0; p < NA; ++p)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) a[p][i] = frag16(sA + p * TM * LDH, am0 + 32 * i + l32, ks);
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) b[p][j] = frag16(sB + p * TM * LDH, bn0 + 32 * j + l32, ks);
+#pragma unroll
+    for (int d = W - 1; d >= 0; --d)
+#pragma unroll
+      for (int p = 0; p < NA; ++p) {
+        const int q = d - p;
+        if (q < 0 || q >= NB) continue;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            f32x16& to = d > 0 && SPLIT ? low[i][j] : acc[i][j];
+            to = Mfma16<T>::run(a[p][i], b[q][j], to);
+          }
+      }
+  }
+}
+
+__device__ __forceinline__ void zero4(f32x16 (&acc)[2][2]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
+}
+__device__ __forceinline__ void add4(f32x16 (&acc)[2][2], const f32x16 (&low)[2][2]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] += low[i][j];
+}
+
+// Whether any sum of the workgroup's is not finite (every thread calls it). A part of an infinite
+// value, or of one that rounds to infinity in bf16, is infinite and its remainder no number: such a
+// tile is done again on the fp32 MFMAs, whose products are those of the values themselves.
+__device__ __forceinline__ bool any_nonfinite(const f32x16 (&acc)[2][2]) {
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) < INFINITY);
+  return __syncthreads_or(bad);
+}
+
+// loss_score_kernel on the 16-bit MFMAs.
+template <typename T>
+__global__ __launch_bounds__(NT, 2) void loss_score16_kernel(const T* __restrict__ Q,
+                                                          const T* __restrict__ R, bool pair, int Bq,
+                                                          int Bd, int V, int chunk,
+                                                          float* __restrict__ part) {
+  constexpr int NS = Parts<T>::S;
+  __shared__ __attribute__((aligned(16))) uint16_t sA[NS * TM * LDH];
+  __shared__ __attribute__((aligned(16))) uint16_t sB[NS * TM * LDH];
+  static_assert(NS == 1 || sizeof(sA) >= KS * LDA * sizeof(float), "score_tile's tiles");
+  // Workgroups go round the 8 XCDs in launch order: a chunk's tiles share one, so its columns of Q
+  // and R come into one L2 once.
+  const int tj = (Bd + TM - 1) / TM, tiles = tj * ((Bq + TM - 1) / TM), slot = blockIdx.x >> 3;
+  const int tile = slot % tiles, c = 8 * (slot / tiles) + (blockIdx.x & 7);
+  const int i0 = (tile / tj) * TM, j0 = (tile % tj) * TM;
+  const int64_t kc = (int64_t)c * chunk;
+  if (kc >= V) return;  // uniform
+  const int kc0 = (int)kc, kc1 = min(V, kc0 + chunk);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wm = wave >> 1, wn = wave & 1;
+  f32x16 acc[2][2], low[2][2];
+  zero4(acc);
+  zero4(low);
+  // Two stages of loads are in flight where registers allow: a stage's MFMAs are shorter than the
+  // loads' way.
+  constexpr int ST = NS > 1 ? 1 : 2;
+  Two<T> ra[ST][8], rb[ST][8];
+  auto load = [&](int k0, int b) {
+    if (k0 >= kc1) return;  // uniform
+    load_rows(Q, pair, V, i0, Bq, k0, kc1, ra[b]);
+    load_rows(R, pair, V, j0, Bd, k0, kc1, rb[b]);
+  };
+  auto stage = [&](int k0, int b) {
+    if (k0 >= kc1) return;
+    __syncthreads();  // the previous stage is read
+    store_rows<NS>(sA, ra[b]);
+    store_rows<NS>(sB, rb[b]);
+    __syncthreads();
+    load(k0 + ST * KS, b);
+    mma16_stage<typename Parts<T>::ST, NS, NS, (NS > 1)>(sA, wm * 64, sB, wn * 64, acc, low);
+  };
+  load(kc0, 0);
+  if (ST > 1) load(kc0 + KS, ST - 1);
+  for (int k0 = kc0; k0 < kc1; k0 += ST * KS) {
+    stage(k0, 0);
+    if (ST > 1) stage(k0 + KS, ST - 1);
+  }
+  if (NS > 1) add4(acc, low);
+  if (NS > 1 && any_nonfinite(acc)) {
+    zero4(acc);
+    score_tile((float*)sA, (float*)sB, Q, R, Bq, Bd, V, i0, j0, kc0, kc1, acc);
+  }
+  float* out = part + (size_t)c * Bq * Bd;
+  const int l32 = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj) {
+      const int j = j0 + wn * 64 + 32 * bj + l32;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = i0 + wm * 64 + 32 * bi + acc_row(r, h);
+        if (i < Bq && j < Bd) out[(size_t)i * Bd + j] = acc[bi][bj][r];
+      }
+    }
+}
+
+// ---- gradients as one tiled GEMM grid ----
+//
+// Both gradients are GEMMs over the other side's rows plus per-element terms:
+//   dQ = c_ce P R + ...  (K = Bd),   dR = c_ce P^T Q + ...  (K = Bq).
+// A workgroup owns GC columns of one 128-row tile of dQ or of dR, four waves of 64 x 64. It sums
+// its own side's columns (the FLOPS term) while the first stages of the GEMM load. No workspace:
+// everything stays in the workgroup.
+// Two workgroups fit a CU, so what bounds it is the latency that a stage does not hide, in turn
+// with the parts' vector arithmetic and the MFMAs (28% of the time for fp16): two stages are in
+// flight, from uniform addresses at constant distances, and the sums' and the epilogue's loads
+// are issued all at once. 256 x 512 x 30522 fp16, each with what comes before: parts in place of
+// fp32 MFMAs 273 -> 174 us, two stages 155, uniform addresses and one side a workgroup 128,
+// loads at once 105; fp32 132, bf16 78.
+constexpr int GC = 128;
+
+static_assert(GC == TM, "one tile shape for both operands");
+static_assert(KS == 32 && NT == 256, "the loaders' thread mappings");
+
+// A stage of A = P rows m0.. (A_KC: thread t holds k = 8 (t % 4) .. + 7 of rows t / 4 + 64 u) or
+// of P's columns m0.. (row t % 128, k = 8 (t / 128 + 2 u) .. + 7). k past P reads zero; rows past P
+// repeat its last one (nothing of theirs is stored). A whole stage is loaded at constant distances
+// from a uniform address, so it costs no vector arithmetic.
+template <bool A_KC>
+__device__ __forceinline__ void load_p(const float* __restrict__ P, int Bq, int Bd, int m0, int k0,
+                                       float (&v)[2][8]) {
+  const int t = threadIdx.x, K = A_KC ? Bd : Bq;
+  typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+  const bool whole = k0 + KS <= K;  // uniform
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    if (A_KC) {
+      const uint32_t m = (uint32_t)min(m0 + (t >> 2) + 64 * u, Bq - 1), k = 8 * (t & 3);
+      if (whole) {
+        const uint32_t off = m * (uint32_t)Bd + k;  // Bq Bd fits an int
+        const f32x4 a = *(const f32x4_any*)(P + k0 + off), b = *(const f32x4_any*)(P + k0 + 4 + off);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[u][i] = a[i];
+          v[u][4 + i] = b[i];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int kk = k0 + (int)k + i;
+          const float x = P[m * (uint32_t)Bd + (uint32_t)min(kk, K - 1)];
+          v[u][i] = kk < K ? x : 0.0f;
+        }
+      }
+    } else {
+      const int k = k0 + 8 * (__builtin_amdgcn_readfirstlane(t >> 7) + 2 * u);
+      const uint32_t m = (uint32_t)min(m0 + (t & 127), Bd - 1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float* row = P + (int64_t)min(k + i, K - 1) * Bd;
+        v[u][i] = row[m];
+      }
+      if (!whole)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (k + i >= K) v[u][i] = 0.0f;
+    }
+  }
+}
+template <bool A_KC, int N>
+__device__ __forceinline__ void store_p(uint16_t* s, const float (&v)[2][8]) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int m = A_KC ? (t >> 2) + 64 * u : t & 127, kg = A_KC ? t & 3 : (t >> 7) + 2 * u;
+    u32x4 p[N];
+    parts8<N>(v[u], p);
+#pragma unroll
+    for (int i = 0; i < N; ++i) *(u32x4*)(s + i * TM * LDH + m * LDH + 8 * kg) = p[i];
+  }
+}
+
+// Sums of X's columns c0 .. c0 + GC - 1 into sum: thread t adds columns 2 (t % 64), + 1 over rows
+// t / 64 + 4 i, the four waves' shares are added in wave order. Every thread of the workgroup.
+template <typename T>
+__device__ __forceinline__ void column_sums(const T* __restrict__ X, bool pair, int K, int c0, int V,
+                                            float (&share)[4][GC], float (&sum)[GC]) {
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), c = 2 * (t & 63);
+  float a = 0.0f, b = 0.0f;
+  constexpr int N = 128 / sizeof(T);  // loads in flight
+  for (int k0 = 0; k0 < K; k0 += 4 * N) {
+    Two<T> v[N];
+    load_x<T>(X, pair, K, k0 + wave, 4, c0 + c, V, v);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      a += to_f32((T)v[i][0]);
+      b += to_f32((T)v[i][1]);
+    }
+  }
+  share[wave][c] = a;
+  share[wave][c + 1] = b;
+  __syncthreads();
+  if (t < GC) sum[t] = ((share[0][t] + share[1][t]) + share[2][t]) + share[3][t];
+  __syncthreads();
+}
+
+// A stage of X: thread t holds columns c0 + 2 (t % 64), + 1 of rows k0 + 8 (t / 64) .. + 7.
+template <typename T, int N>
+__device__ __forceinline__ void store_x(uint16_t* s, const Two<T> (&v)[8]) {
+  const int t = threadIdx.x, kg = t >> 6, n = 2 * (t & 63);
+#pragma unroll
+  for (int col = 0; col < 2; ++col) {
+    uint16_t* to = s + (n + col) * LDH + 8 * kg;
+    if constexpr (N == 1) {
+      u32x4 w;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        w[q] = (uint32_t)bits16<T>(v[2 * q][col]) | ((uint32_t)bits16<T>(v[2 * q + 1][col]) << 16);
+      *(u32x4*)to = w;
+    } else {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = to_f32((T)v[i][col]);
+      u32x4 p[N];
+      parts8<N>(x, p);
+#pragma unroll
+      for (int i = 0; i < N; ++i) *(u32x4*)(to + i * GC * LDH) = p[i];
+    }
+  }
+}
+
+// One GEMM tile: acc += A B^T over k in [0, K), A = P rows m0.. (A_KC) or P columns m0..,
+// B = X[k][c0 ..]. `meanwhile` (barriers in it are reached by every thread) runs under the first
+// loads.
+template <typename T, bool A_KC, typename F>
+__device__ __forceinline__ void gemm16(uint16_t* sA, uint16_t* sB, const float* __restrict__ P, int Bq,
+                                       int Bd, const T* __restrict__ X, bool pair, int K, int m0, int c0,
+                                       int V, f32x16 (&acc)[2][2], const F& meanwhile) {
+  f32x16 low[2][2];
+  zero4(low);
+  constexpr int NP = Parts<T>::P, NX = Parts<T>::X;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 1, wn = wave & 1;
+  // Two stages of loads are in flight: a stage's MFMAs are shorter than the loads' way.
+  float pa0[2][8], pa1[2][8];
+  Two<T> xv0[8], xv1[8];
+  auto load = [&](int k0, float (&p)[2][8], Two<T> (&x)[8]) __attribute__((always_inline)) {
+    if (k0 >= K) return;  // uniform
+    load_p<A_KC>(P, Bq, Bd, m0, k0, p);
+    load_x<T>(X, pair, K, k0 + 8 * wave, 1, c0 + 2 * (t & 63), V, x);
+  };
+  auto stage = [&](int k0, float (&p)[2][8], Two<T> (&x)[8]) __attribute__((always_inline)) {
+    if (k0 >= K) return;
+    __syncthreads();  // the previous stage is read
+    store_p<A_KC, NP>(sA, p);
+    store_x<T, NX>(sB, x);
+    __syncthreads();
+    load(k0 + 2 * KS, p, x);
+    mma16_stage<bf16, NP, NX, (NX > 1)>(sA, wm * 64, sB, wn * 64, acc, low);
+  };
+  load(0, pa0, xv0);
+  load(KS, pa1, xv1);
+  meanwhile();
+  for (int k0 = 0; k0 < K; k0 += 2 * KS) {
+    stage(k0, pa0, xv0);
+    stage(k0 + KS, pa1, xv1);
+  }
+  if (NX > 1) add4(acc, low);
+}
+
+// G[i][c] = c_ce acc + c_s sign(X[i][c]) + c_f colsum[c] for the tile's rows below `rows`.
+template <typename T>
+__device__ __forceinline__ void grad16_epilogue(const f32x16 (&acc)[2][2], const T* __restrict__ X,
+                                                int rows, int m0, int c0, int V, float c_ce,
+                                                float c_s, float c_f, const float* colsum,
+                                                T* __restrict__ G) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
+  const int wm = wave >> 1, wn = wave & 1;
+  T xv[2][2][16];  // every load issued, from clamped places, before any is used
+#pragma unroll
+  for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = m0 + wm * 64 + 32 * bi + acc_row(r, h), c = c0 + wn * 64 + 32 * bj + l32;
+        xv[bi][bj][r] = X[(int64_t)min(i, rows - 1) * V + min(c, V - 1)];
+      }
+#pragma unroll
+  for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj) {
+      const int cl = wn * 64 + 32 * bj + l32, c = c0 + cl;
+      const float add = c_f * colsum[cl];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = m0 + wm * 64 + 32 * bi + acc_row(r, h);
+        if (i < rows && c < V) {
+          const float x = to_f32(xv[bi][bj][r]);
+          const float sg = x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f);
+          G[(int64_t)i * V + c] = from_f32<T>(c_ce * acc[bi][bj][r] + c_s * sg + add);
+        }
+      }
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(NT, 2) void loss_grad16_kernel(const T* __restrict__ Q,
+                                                            const T* __restrict__ R,
+                                                            const float* __restrict__ P, const Grads6 g,
+                                                            bool pair, int Bq, int Bd, int V, float w_ce,
+                                                            float w_l1, float w_fl,
+                                                            T* __restrict__ GQ,
+                                                            T* __restrict__ GR) {
+  __shared__ __attribute__((aligned(16))) uint16_t sA[Parts<T>::P * TM * LDH];
+  __shared__ __attribute__((aligned(16))) uint16_t sB[Parts<T>::X * GC * LDH];
+  __shared__ float share[4][GC];
+  __shared__ float colsum[GC];
+  // One bf16 part (bf16 reps) is the value itself.
+  constexpr bool REDO = Parts<T>::X > 1;
+  static_assert(!REDO || (sizeof(sA) >= KS * LDA * sizeof(float) && sizeof(sB) >= KS * LDB * sizeof(float)),
+                "grad_tile's tiles");
+  // Workgroups go round the 8 XCDs in launch order: the tiles of one side and column tile share an
+  // XCD, so what they stream comes into one L2 once. The side with the longer GEMMs goes first.
+  const int nq = (Bq + TM - 1) / TM, nd = (Bd + TM - 1) / TM, cols8 = (V + 8 * GC - 1) / (8 * GC);
+  const bool q_first = Bd >= Bq;
+  const int n0 = q_first ? nq : nd, n1 = q_first ? nd : nq;
+  int slot = blockIdx.x >> 3;
+  const bool second = slot >= cols8 * n0;  // uniform, as all below
+  if (second) slot -= cols8 * n0;
+  const int n = second ? n1 : n0;
+  const int c0 = (8 * (slot / n) + (int)(blockIdx.x & 7)) * GC, m0 = (slot % n) * TM;
+  if (c0 >= V) return;
+  const float g0 = grad_of(g, 0);
+  const float c_ce = g0 * w_ce + grad_of(g, 1);
+  f32x16 acc[2][2];
+  zero4(acc);
+  if (second != q_first) {
+    gemm16<T, true>(sA, sB, P, Bq, Bd, R, pair, Bd, m0, c0, V, acc,
+                    [&] { column_sums<T>(Q, pair, Bq, c0, V, share, colsum); });
+    const float c_s = (g0 * w_l1 + grad_of(g, 2)) / (float)Bq;
+    const float c_f = 2.0f * (g0 * w_fl + grad_of(g, 4)) / (float)V;
+    if (REDO && any_nonfinite(acc)) {
+      for (int c = 0; c < GC && c0 + c < V; c += NC)
+        grad_tile<T, true>((float*)sA, (float*)sB, P, Bq, Bd, R, Bd, Q, Bq, m0, c0 + c, V, c_ce, c_s, c_f,
+                           colsum + c, GQ);
+      return;
+    }
+    grad16_epilogue(acc, Q, Bq, m0, c0, V, c_ce, c_s, c_f, colsum, GQ);
+  } else {
+    gemm16<T, false>(sA, sB, P, Bq, Bd, Q, pair, Bq, m0, c0, V, acc,
+                     [&] { column_sums<T>(R, pair, Bd, c0, V, share, colsum); });
+    const float c_s = (g0 * w_l1 + grad_of(g, 3)) / (float)Bd;
+    const float c_f = 2.0f * (g0 * w_fl + grad_of(g, 5)) / (float)V;
+    if (REDO && any_nonfinite(acc)) {
+      for (int c = 0; c < GC && c0 + c < V; c += NC)
+        grad_tile<T, false>((float*)sA, (float*)sB, P, Bq, Bd, Q, Bq, R, Bd, m0, c0 + c, V, c_ce, c_s, c_f,
+                            colsum + c, GR);
+      return;
+    }
+    grad16_epilogue(acc, R, Bd, m0, c0, V, c_ce, c_s, c_f, colsum, GR);
   }
 }
 
@@ -1025,10 +1298,16 @@ static int64_t workspace_floats(int64_t Bq, int64_t Bd, int64_t V) {
   return s + (slices(V) + 1) * stats_entries(Bq, Bd) + Bq;
 }
 
-// SPARTON_LOSS_MFMA16=0 keeps 16-bit reps on the fp32 MFMA (tests compare the two).
+// SPARTON_LOSS_MFMA16=0 takes the fp32 MFMAs throughout (tests compare the two).
 static bool mfma16_on() {
   const char* e = getenv("SPARTON_LOSS_MFMA16");
   return e == nullptr || strcmp(e, "0") != 0;
+}
+
+// Two columns to a load: rows of an even number of elements, from a place aligned to two.
+template <typename T>
+static bool pairs(const void* q, const void* d, int V) {
+  return V % 2 == 0 && ((uintptr_t)q | (uintptr_t)d) % (2 * sizeof(T)) == 0;
 }
 
 template <typename T>
@@ -1039,29 +1318,25 @@ static void fwd(const void* q, const void* d, int Bq, int Bd, int V, float inv_t
   if (Bd > 0) {
     const ScorePlan p = score_plan(Bq, Bd, V);
     S = spart + (size_t)p.nchunk * Bq * Bd;
-    const dim3 grid((unsigned)p.tiles, (unsigned)p.nchunk);
-    if constexpr (sizeof(T) == 2) {
-      if (mfma16_on()) {
-        hipLaunchKernelGGL((loss_score16_kernel<T>), grid, dim3(NT), 0, st, (const T*)q, (const T*)d,
-                           Bq, Bd, V, p.chunk, spart);
-      } else {
-        hipLaunchKernelGGL((loss_score_kernel<T>), grid, dim3(NT), 0, st, (const T*)q, (const T*)d,
-                           Bq, Bd, V, p.chunk, spart);
-      }
+    if (mfma16_on()) {
+      const dim3 grid((unsigned)(p.tiles * round_up(p.nchunk, 8)));
+      const bool pair = V * sizeof(T) % 4 == 0 && ((uintptr_t)q | (uintptr_t)d) % 4 == 0;
+      hipLaunchKernelGGL((loss_score16_kernel<T>), grid, dim3(NT), 0, st, (const T*)q, (const T*)d,
+                         pair, Bq, Bd, V, p.chunk, spart);
     } else {
-      hipLaunchKernelGGL((loss_score_kernel<T>), grid, dim3(NT), 0, st, (const T*)q, (const T*)d,
-                         Bq, Bd, V, p.chunk, spart);
+      hipLaunchKernelGGL((loss_score_kernel<T>), dim3((unsigned)p.tiles, (unsigned)p.nchunk), dim3(NT),
+                         0, st, (const T*)q, (const T*)d, Bq, Bd, V, p.chunk, spart);
     }
     const int K = Bq * Bd;
     hipLaunchKernelGGL(loss_slice_sum_kernel, dim3((unsigned)cdiv(K, 64)), dim3(64 * SUM_WAVES), 0, st,
                        (const float*)spart, p.nchunk, K, S);
   }
   float* tpart = Bd > 0 ? S + (size_t)Bq * Bd : ws;
-  const int KS2 = (int)stats_entries(Bq, Bd), ns = (int)slices(V);
+  const int KS2 = (int)stats_entries(Bq, Bd), ns = (int)cdiv(V, ST_COLS);
   float* stats = tpart + (size_t)ns * KS2;
   float* row_loss = stats + KS2;
-  hipLaunchKernelGGL((loss_stats_kernel<T>), dim3((unsigned)ns), dim3(NT), 0, st, (const T*)q,
-                     (const T*)d, Bq, Bd, V, tpart, KS2);
+  hipLaunchKernelGGL((loss_stats_kernel<T>), dim3((unsigned)ns, 2), dim3(NT), 0, st, (const T*)q,
+                     (const T*)d, pairs<T>(q, d, V), Bq, Bd, V, tpart, KS2);
   hipLaunchKernelGGL(loss_slice_sum_kernel, dim3((unsigned)cdiv(KS2, 64)), dim3(64 * SUM_WAVES), 0, st,
                      (const float*)tpart, ns, KS2, stats);
   if (Bd > 0)
@@ -1074,13 +1349,11 @@ static void fwd(const void* q, const void* d, int Bq, int Bd, int V, float inv_t
 template <typename T>
 static void bwd(const void* q, const void* d, const float* P, const Grads6& g, int Bq, int Bd, int V,
                 float w_ce, float w_l1, float w_fl, void* gq, void* gd, hipStream_t st) {
-  if constexpr (std::is_same<T, bf16>::value) {
-    if (mfma16_on()) {
-      const dim3 grid((unsigned)cdiv(V, GC), (unsigned)cdiv(std::max(Bq, Bd), TM));
-      hipLaunchKernelGGL(loss_grad16_kernel, grid, dim3(NT), 0, st, (const bf16*)q, (const bf16*)d, P,
-                         g, Bq, Bd, V, w_ce, w_l1, w_fl, (bf16*)gq, (bf16*)gd);
-      return;
-    }
+  if (mfma16_on()) {
+    const dim3 grid((unsigned)(round_up(cdiv(V, GC), 8) * (cdiv(Bq, TM) + cdiv(Bd, TM))));
+    hipLaunchKernelGGL(loss_grad16_kernel<T>, grid, dim3(NT), 0, st, (const T*)q, (const T*)d, P, g,
+                       pairs<T>(q, d, V), Bq, Bd, V, w_ce, w_l1, w_fl, (T*)gq, (T*)gd);
+    return;
   }
   hipLaunchKernelGGL((loss_bwd_large_kernel<T>), dim3((unsigned)cdiv(V, NC)), dim3(NT), 0, st,
                      (const T*)q, (const T*)d, P, g, Bq, Bd, V, w_ce, w_l1, w_fl, (T*)gq, (T*)gd);

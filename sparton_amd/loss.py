@@ -18,11 +18,11 @@ runs in the reps dtype), deterministically. Device tensors only, like the head.
     sparton::splade_loss_bwd(grad_out[6], q, d?, probs, w_ce, w_l1, w_flops) -> (dq, dd)
 
 Batches of up to 64 rows on each side take the slice-staged kernels above. Larger batches
-take GEMM-shaped HIP kernels on the matrix cores (16-bit reps on the bf16/fp16 MFMA, whose
-products are exact in fp32; fp32 reps on the fp32 MFMA): a split-vocabulary score GEMM with a
-fixed-order sum of its partials, per-slice row and column statistics, a row softmax, and a
-backward that recomputes each vocabulary slice's column sums and forms both gradients tile by
-tile (sparton_loss.hip). Limits: 1 <= Bq <= Bd when documents are given (the labels
+take GEMM-shaped HIP kernels on the matrix cores (the bf16/fp16 MFMA: products of 16-bit
+reps are exact in fp32, fp32 values are sums of bf16 parts that hold all their bits): a
+split-vocabulary score GEMM with a fixed-order sum of its partials, per-slice row and column
+statistics, a row softmax, and a backward that recomputes each vocabulary slice's column sums
+and forms both gradients tile by tile (sparton_loss.hip). Limits: 1 <= Bq <= Bd when documents are given (the labels
 arange(Bq) index d's rows); the C ABI reports sizes past its int offsets as unsupported.
 """
 from __future__ import annotations

@@ -150,6 +150,70 @@ def test_loss_large_batch_16bit_mfma_matches_fp32_mfma(dt, Bq, Bd, V, device, mo
         assert (a - b).abs().max().item() <= tol * scale, (a - b).abs().max().item() / scale
 
 
+@pytest.mark.parametrize("dt,Bq,Bd,V,off", [
+    ("fp32", 65, 129, 257, 0), ("fp32", 129, 300, 770, 0), ("fp32", 66, 66, 1000, 1), ("fp32", 1, 65, 1, 0),
+    ("fp16", 65, 257, 385, 0), ("fp16", 128, 160, 1026, 1), ("bf16", 97, 128, 259, 1), ("bf16", 65, 65, 258, 0)])
+def test_loss_parts_against_fp64(dt, Bq, Bd, V, off, device, monkeypatch):
+    """Past 64 rows, reps (and P) as sums of 16-bit parts: tiles with ragged rows and columns, K tails,
+    one row tile on one side and more on the other, rows that allow no paired loads (V odd, or a
+    base one element off). The error against fp64 is no larger than that of the same products on
+    the fp32 MFMAs, up to the roundings of the sums themselves (2^-22 of the gradient's scale) and
+    one rounding to the reps' dtype."""
+    say(f"loss parts {dt} Bq={Bq} Bd={Bd} V={V} off={off}")
+
+    def make(B, seed):
+        x = torch.empty(B * V + off, dtype=reps_like(1, 1, dt, 0).dtype, device=device)[off:].view(B, V)
+        return x.copy_(reps_like(B, V, dt, seed=seed))
+
+    q, d = make(Bq, 41), make(Bd, 42)
+    q64, d64 = (x.cpu().double().requires_grad_() for x in (q, d))
+    ref = F.cross_entropy(q64 @ d64.T / 0.6, torch.arange(Bq))
+    ref.backward()
+    err = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("SPARTON_LOSS_MFMA16", mode)
+        qs, ds = q.detach().requires_grad_(), d.detach().requires_grad_()
+        res = sl.splade_loss(qs, ds, 0.6, 0.0, 0.0)
+        res.contrastive.backward()
+        err[mode] = [abs(res.contrastive.item() - ref.item()) / max(1.0, abs(ref.item()))]
+        for x, y in ((qs, q64), (ds, d64)):
+            scale = y.grad.abs().max().item() + 1e-30
+            err[mode].append((x.grad.cpu().double() - y.grad).abs().max().item() / scale)
+        qs.grad = ds.grad = None
+    eps = {"fp32": 2.0 ** -22, "fp16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
+    for a, b, e in zip(err["1"], err["0"], (2.0 ** -20, eps, eps)):
+        assert a <= b + e, (err, eps)
+
+
+@pytest.mark.parametrize("dt,big", [("fp32", float("inf")), ("fp32", 3.4e38), ("fp16", float("inf"))])
+def test_loss_parts_with_infinite_entries(dt, big, device, monkeypatch):
+    """An entry with no finite parts (infinite, or one that bf16 rounds to infinity): every score,
+    probability and gradient is the one of the fp32 MFMAs."""
+    say(f"loss parts, entry {big} {dt}")
+    q = reps_like(70, 513, dt, seed=51).to(device)
+    d = reps_like(200, 513, dt, seed=52).to(device)
+    d = d + 0.25  # no 0 * inf
+    q = q + 0.25
+    d[150, 300] = -big  # its scores are -inf or next to it: probability 0
+    out = []
+    for mode in ("1", "0"):
+        monkeypatch.setenv("SPARTON_LOSS_MFMA16", mode)
+        qs, ds = q.clone().requires_grad_(), d.clone().requires_grad_()
+        res = sl.splade_loss(qs, ds, 1.0, 0.0, 0.0)
+        res.contrastive.backward()
+        out.append((res.contrastive.detach(), qs.grad, ds.grad))
+    q64, d64 = (x.cpu().double().requires_grad_() for x in (q, d))
+    F.cross_entropy(q64 @ d64.T, torch.arange(70)).backward()
+    assert out[0][0].isfinite()
+    eps = {"fp32": 2.0 ** -22, "fp16": 2.0 ** -11}[dt]  # as above
+    for a, b, y in zip(out[0][1:], out[1][1:], (q64.grad, d64.grad)):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+        a, b = a.cpu().double(), b.cpu().double()
+        keep = y.isfinite() & b.isfinite()
+        ea, eb = ((x[keep] - y[keep]).abs().max().item() for x in (a, b))
+        assert ea <= eb + eps * y[keep].abs().max().item()
+
+
 def test_loss_large_batch_deterministic_and_paths_agree(device):
     """The large-batch kernels are bitwise reproducible, and the custom op (what torch.compile
     traces) and the eager C++ op run the same kernels."""
