@@ -434,6 +434,14 @@ constexpr int HOT_REL = 4;
 constexpr int HOT_FEW = 32;
 constexpr int HOT_NB = DH_LANES / DH_BATCH;  // partials per lane group and step
 
+// A row's partials are summed in blocks of FOLD entries, those in blocks of FOLD2 and these in
+// order: a row may hold every id, and one chain over thousands of them has the larger error. fp32
+// dH against fp64, rms, one chain -> these blocks (the kernels before, per-wave parts):
+// 3 x 60 x 1024 x 180001 5.6e-7 -> 0.63e-7 (1.8e-7), 40 x 20 x 1024 x 40001 6.0e-7 -> 0.76e-7
+// (2.3e-7), 2 x 50 x 772 x 200000 with 5% of the gradients 1.3e-7 -> 0.85e-7 (0.94e-7); the time
+// is the same.
+constexpr int FOLD = 64, FOLD2 = 1024;
+
 template <typename T>
 struct HotSmem {
   __attribute__((aligned(16))) float part[DH_GROUPS * HOT_NB][Chunk<T>::COLS];
@@ -447,6 +455,9 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
     int hot_min) {
   constexpr int E = Chunk<T>::E;
   static_assert(Chunk<T>::COLS <= 64 * DH_WAVES, "one thread per column");
+  static_assert(FOLD % DH_LANES == 0 && DH_GROUPS * DH_LANES % FOLD == 0 &&
+                    FOLD2 % (DH_GROUPS * DH_LANES) == 0,
+                "blocks of whole steps");
   __shared__ HotSmem<T> sm;
   const int slice = (int)blockIdx.x % n_slices, blk = (int)blockIdx.x / n_slices;
   const int tid = threadIdx.x, grp = tid / DH_LANES, l = tid % DH_LANES;
@@ -482,9 +493,9 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
   }
   if (hot_min >= 0) lim = hot_min;
   if (live && re.total <= lim) {
-    float acc[E];
+    float acc[E], sum[E], all[E];
 #pragma unroll
-    for (int i = 0; i < E; ++i) acc[i] = 0.0f;
+    for (int i = 0; i < E; ++i) acc[i] = sum[i] = all[i] = 0.0f;
     if (re.total > 0) {
       auto add = [&](int, const float* P) {
 #pragma unroll
@@ -497,17 +508,31 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
         const Entries en = next;
         next.load(rb, re, runs, e + DH_LANES, row16, l);
         dh_partials<T, false, DH_LANES>(wp, en, DH_LANES, add);
+        if ((e + DH_LANES) % FOLD == 0)
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            sum[i] += acc[i];
+            acc[i] = 0.0f;
+          }
+        if ((e + DH_LANES) % FOLD2 == 0)
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            all[i] += sum[i];
+            sum[i] = 0.0f;
+          }
       }
       if (e < re.total) dh_partials_tail<T>(wp, next, re.total - e, add);
+#pragma unroll
+      for (int i = 0; i < E; ++i) all[i] += sum[i] + acc[i];
     }
-    if (d < D) store_chunk<O, E>(out_of(row0 + grp) + d, acc);
+    if (d < D) store_chunk<O, E>(out_of(row0 + grp) + d, all);
   }
   for (int k = 0; k < rpw; ++k) {
     const int n = __builtin_amdgcn_readfirstlane(sm.total[k]);
     if (n <= lim) continue;  // workgroup-uniform
     RowEntries rk;
     const int2* rbk = entries_of(row0 + k, rk);
-    float acc = 0.0f;  // column `tid` of the slice
+    float sum = 0.0f, all = 0.0f;  // column `tid` of the slice
     Entries next;
     next.load(rbk, rk, runs, grp * DH_LANES, row16, l);
     for (int e0 = 0; e0 < n; e0 += DH_GROUPS * DH_LANES) {
@@ -526,10 +551,18 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
       __syncthreads();
       const int m = min(DH_GROUPS * HOT_NB, (n - e0 + DH_BATCH - 1) / DH_BATCH);
       if (tid < Chunk<T>::COLS)
-        for (int j = 0; j < m; ++j) acc += sm.part[j][tid];
+        for (int j0 = 0; j0 < m; j0 += FOLD / DH_BATCH) {
+          float acc = 0.0f;
+          for (int j = j0; j < min(m, j0 + FOLD / DH_BATCH); ++j) acc += sm.part[j][tid];
+          sum += acc;
+        }
+      if ((e0 + DH_GROUPS * DH_LANES) % FOLD2 == 0 || e0 + DH_GROUPS * DH_LANES >= n) {
+        all += sum;
+        sum = 0.0f;
+      }
       __syncthreads();  // the partials are rewritten next step
     }
-    if (tid < Chunk<T>::COLS && d0 + tid < D) out_of(row0 + k)[d0 + tid] = from_f32<O>(acc);
+    if (tid < Chunk<T>::COLS && d0 + tid < D) out_of(row0 + k)[d0 + tid] = from_f32<O>(all);
   }
 }
 

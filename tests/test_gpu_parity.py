@@ -362,6 +362,31 @@ def test_backward_row_sharing(case, device, monkeypatch):
     check_bwd_isolated(H, W, b, m, G, reps32, idx, *runs[0])
 
 
+@pytest.mark.parametrize("B,S,D,V", [(1, 65, 68, 200001), (140, 16, 8, 30522), (2, 40, 72, 81920)])
+def test_backward_long_rows_error(B, S, D, V, device, monkeypatch):
+    """dH rows of 1000 to 3000 entries of one sign, shared by a workgroup or not: each sum is within
+    the bound of its order of adding, (4 in a partial, 16 partials, 16 blocks, one more per 1024
+    entries) roundings of 2^-24 of the sum of magnitudes, with 4 for g'. One chain of partials
+    would be bound by a quarter of the entries."""
+    say(f"long dH rows B={B} S={S} D={D} V={V}")
+    g = torch.Generator().manual_seed(3)
+    H, W = torch.randn(B, S, D, generator=g), torch.rand(V, D, generator=g) + 0.5
+    G, reps = torch.rand(B, V, generator=g) + 0.1, torch.rand(B, V, generator=g) + 0.1
+    idx = torch.randint(0, S, (B, V), generator=g, dtype=torch.int32)
+    mask = torch.ones(B, S, dtype=torch.int64)
+    args = [x.to(device) for x in (G, reps, idx, H, W)]
+    coeff = G.double() * torch.exp(-reps.double())
+    ref = torch.zeros(B, S, D, dtype=torch.float64)
+    for b in range(B):
+        ref[b].index_add_(0, idx[b].long(), coeff[b, :, None] * W.double())
+    n = max(torch.bincount(idx[b].long(), minlength=S).max().item() for b in range(B))
+    bound = (4 + 16 + 16 + n // 1024 + 2 + 4) * 2.0 ** -24
+    for hot_min in ("0", str(2 ** 30)):
+        monkeypatch.setenv("SPARTON_BWD_HOT_MIN", hot_min)
+        dH = torch.ops.sparton.fused_sparton_bwd(*args, None, mask.to(device))[0].cpu().double()
+        assert ((dH - ref).abs() <= bound * ref).all()  # every term is positive
+
+
 def test_graph_capture_replays(device):
     """Forward and backward captured into one HIP graph (all of their kernels and workspace
     allocations) replay to the eager results, bitwise, with eager work and synchronizations
