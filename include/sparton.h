@@ -139,7 +139,7 @@ int sparton_fwd_profile(const void* hidden, const void* weight, const void* bias
 
 /*
  * Bytes of device scratch sparton_bwd needs for these sizes (256-byte aligned
- * sections: per-chunk histograms, segment offsets and the bucketed entry list).
+ * sections: where each position's entries begin in each run of ids, and the entries).
  * No counterpart in the reference: its backward needs no scratch because it
  * accumulates with atomics into zero-filled outputs (sparton_kernel.py:676-678).
  */
