@@ -369,27 +369,42 @@ struct RowEntries {
 };
 
 // 16 entries of a row, one per lane: g' (0 past the row's end) and the place of the W row in
-// 16-byte units (the last entry's past its end).
-struct Entries {
-  uint32_t off;
+// 16-byte units (the last entry's past its end). WIDE: a W of 64 GiB or more, whose places need
+// more than 32 bits; the second half's broadcasts cost 1.5% (16 x 256 dense bf16 rows), so
+// smaller ones do without.
+template <bool WIDE> struct Entries {
+  uint32_t lo, hi;
   float g;
   __device__ __forceinline__ void load(const int2* run, const RowEntries& re, int runs, int e,
-                                       uint32_t row16, int l) {
+                                       uint64_t row16, int l) {
     const int2 x = run[re.place(min(e + l, re.total - 1), runs)];
-    off = (uint32_t)x.x * row16;
+    if constexpr (WIDE) {
+      const uint64_t at = (uint64_t)(uint32_t)x.x * row16;
+      lo = (uint32_t)at;
+      hi = (uint32_t)(at >> 32);
+    } else {
+      lo = (uint32_t)x.x * (uint32_t)row16;
+    }
     g = e + l < re.total ? __int_as_float(x.y) : 0.0f;
   }
+  // Byte offset of entry U's W row.
+  template <int U> __device__ __forceinline__ uint64_t at() const {
+    uint64_t u = row_bcast<U>(lo);
+    if constexpr (WIDE) u |= (uint64_t)row_bcast<U>(hi) << 32;
+    return u << 4;
+  }
 };
+constexpr uint64_t DH_WIDE_16 = 1ull << 32;  // 16-byte units of W from which on it is WIDE
 
 // The partials P of the DH_BATCHes of entries 0 .. N - 1 over one chunk of their W rows (wp:
 // the chunk in row 0), handed to put(batch, P) in order. With MASKED only the first `left`
 // count; the others add 0 * 0, which leaves the sums as they are.
-template <typename T, bool MASKED, int N, typename Put>
-__device__ __forceinline__ void dh_partials(const char* wp, const Entries& en, int left, Put put) {
+template <typename T, bool MASKED, int N, bool WIDE, typename Put>
+__device__ __forceinline__ void dh_partials(const char* wp, const Entries<WIDE>& en, int left, Put put) {
   constexpr int E = Chunk<T>::E;
   u32x4 w[N];
   static_for<0, N>([&](auto u) {
-    w[u] = *(const u32x4*)(wp + ((uint64_t)row_bcast<decltype(u)::value>(en.off) << 4));
+    w[u] = *(const u32x4*)(wp + en.template at<decltype(u)::value>());
   });
   static_for<0, N / DH_BATCH>([&](auto a) {
     float P[E];
@@ -409,8 +424,8 @@ __device__ __forceinline__ void dh_partials(const char* wp, const Entries& en, i
   });
 }
 // The same for the last `left` < DH_LANES entries, no more of them loaded than a few.
-template <typename T, typename Put>
-__device__ __forceinline__ void dh_partials_tail(const char* wp, const Entries& en, int left, Put put) {
+template <typename T, bool WIDE, typename Put>
+__device__ __forceinline__ void dh_partials_tail(const char* wp, const Entries<WIDE>& en, int left, Put put) {
   if (left > 8) dh_partials<T, true, 16>(wp, en, left, put);
   else if (left > 4) dh_partials<T, true, 8>(wp, en, left, put);
   else dh_partials<T, true, 4>(wp, en, left, put);
@@ -448,7 +463,7 @@ struct HotSmem {
   int total[DH_GROUPS];
 };
 
-template <typename T, typename O>
+template <typename T, typename O, bool WIDE>
 __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
     const T* __restrict__ W, const int* __restrict__ off, const int2* __restrict__ run,
     O* __restrict__ dH, int B, int S, int D, int runs, int cap, int S_row, int n_slices, int rpw,
@@ -461,7 +476,7 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
   __shared__ HotSmem<T> sm;
   const int slice = (int)blockIdx.x % n_slices, blk = (int)blockIdx.x / n_slices;
   const int tid = threadIdx.x, grp = tid / DH_LANES, l = tid % DH_LANES;
-  const uint32_t row16 = (uint32_t)(D * (int)sizeof(T) / 16);  // 16-byte units per row
+  const uint64_t row16 = (uint64_t)D * sizeof(T) / 16;  // 16-byte units per row
   const int d0 = slice * Chunk<T>::COLS;
   // Lanes past the row's end work on its last chunk (the row broadcasts need them) and do not
   // store.
@@ -501,11 +516,11 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
 #pragma unroll
         for (int i = 0; i < E; ++i) acc[i] += P[i];
       };
-      Entries next;
+      Entries<WIDE> next;
       next.load(rb, re, runs, 0, row16, l);
       int e = 0;
       for (; e + DH_LANES <= re.total; e += DH_LANES) {
-        const Entries en = next;
+        const Entries<WIDE> en = next;
         next.load(rb, re, runs, e + DH_LANES, row16, l);
         dh_partials<T, false, DH_LANES>(wp, en, DH_LANES, add);
         if ((e + DH_LANES) % FOLD == 0)
@@ -533,11 +548,11 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
     RowEntries rk;
     const int2* rbk = entries_of(row0 + k, rk);
     float sum = 0.0f, all = 0.0f;  // column `tid` of the slice
-    Entries next;
+    Entries<WIDE> next;
     next.load(rbk, rk, runs, grp * DH_LANES, row16, l);
     for (int e0 = 0; e0 < n; e0 += DH_GROUPS * DH_LANES) {
       const int e = e0 + grp * DH_LANES;
-      const Entries en = next;
+      const Entries<WIDE> en = next;
       next.load(rbk, rk, runs, e + DH_GROUPS * DH_LANES, row16, l);
       if (e < n) {
         auto put = [&](int p, const float* P) {
@@ -1267,7 +1282,9 @@ static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void*
                            (int)s0, (int)sw, off, run);
         dw_done |= with_dw;
         const int rpw = dh_rows_per_group(nb * sw);
-        hipLaunchKernelGGL((bwd_dh_kernel<T, O>), dim3((unsigned)(cdiv(nb * sw, rpw) * n_slices)),
+        const bool wide = (uint64_t)V * ((uint64_t)D * sizeof(T) / 16) > DH_WIDE_16;
+        hipLaunchKernelGGL((wide ? bwd_dh_kernel<T, O, true> : bwd_dh_kernel<T, O, false>),
+                           dim3((unsigned)(cdiv(nb * sw, rpw) * n_slices)),
                            dim3(64 * DH_WAVES), 0, st, W, (const int*)off, (const int2*)run,
                            dH + (b0 * S + s0) * D, (int)nb, (int)sw, (int)D, (int)c.runs, (int)c.cap,
                            (int)S, (int)n_slices, rpw, dh_hot_min());

@@ -833,6 +833,40 @@ def test_backward_dw_in_dh_launch(case, long_rows, device, monkeypatch):
     check_bwd_isolated(H, W, b, m, G, reps32, idx, *merged)
 
 
+@pytest.mark.parametrize("V,D,ids", [
+    # 8192 bf16 columns are 16 KiB a row: 2^22 rows are 64 GiB, and ids past them land past it
+    (2 ** 22 + 64, 8192, [5, 70, 2 ** 22 + 5, 2 ** 22 + 63]),
+])
+def test_backward_weight_past_64_gib(V, D, ids, device):
+    """dH of ids whose W row starts 64 GiB or more into W: each row is g' W[v] of its own id. (Each
+    dH row takes one entry here, so the sum is one product: 4 roundings, of exp and of g'.)"""
+    say(f"backward, W of {V * D * 2 / 2 ** 30:.2f} GiB")
+    if torch.cuda.mem_get_info()[0] < V * D * 2 + 2 ** 32:
+        pytest.skip("W does not fit this card's free memory")
+    S = 65  # past the few-row path
+    W = torch.empty(V, D, dtype=torch.bfloat16, device=device)  # only the rows below are read
+    g = torch.Generator().manual_seed(1)
+    rows = torch.randn(len(ids), D, generator=g).bfloat16()
+    for v, row in zip(ids, rows):
+        W[v] = row.to(device)
+    W[V - 1] = rows[-1].to(device)
+    G = torch.zeros(1, V, dtype=torch.bfloat16, device=device)
+    reps = torch.zeros(1, V, device=device)
+    idx = torch.zeros(1, V, dtype=torch.int32, device=device)
+    for k, v in enumerate(ids):
+        G[0, v], reps[0, v], idx[0, v] = 1.0 + k, 0.25 * (k + 1), 16 * k
+    H = torch.zeros(1, S, D, dtype=torch.bfloat16, device=device)
+    m = torch.ones(1, S, dtype=torch.int64, device=device)
+    dH = torch.empty(1, S, D, device=device)
+    _bwd_capi(G, reps, idx, H, W, m, dH, None, None)
+    torch.cuda.synchronize()
+    want = torch.zeros(S, D, dtype=F64)
+    for k, v in enumerate(ids):
+        want[16 * k] = (1.0 + k) * np.exp(-0.25 * (k + 1)) * rows[k].double()
+    err = (dH[0].cpu().double() - want).abs()
+    assert bool((err <= 4 * 2.0 ** -24 * want.abs()).all())
+
+
 @pytest.mark.parametrize("case", [
     ("bf16", 2, 20000, 64, 320, True, "holes"),     # S > 16384: two dH windows
     ("fp32", 1, 40000, 32, 200, False, "int64"),    # three windows, the last partial
