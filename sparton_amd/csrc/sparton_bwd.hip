@@ -71,10 +71,21 @@ static Layout layout(int64_t B, int64_t S, int64_t V) {
   return L;
 }
 
-// Batch rows and positions of one dH pass.
-static int64_t pass_s(int64_t S) { return std::min<int64_t>(S, MAX_S); }
-static int64_t pass_b(int64_t B, int64_t S) {
-  return std::min<int64_t>(B, std::max<int64_t>(1, MAX_ROWS / std::max<int64_t>(1, pass_s(S))));
+// A launch holds fewer than 2^32 threads (past that, workgroups were left out without an error):
+// the workgroups of a dH launch, and of one with dW's.
+constexpr int64_t MAX_THREADS = ((int64_t)1 << 32) - 1;
+constexpr int64_t DH_MAX_WG = MAX_THREADS / 256, BK_MAX_WG = MAX_THREADS / (64 * BK_WAVES);
+
+// Batch rows and positions of one dH pass: 16 rows a workgroup, for each 256-byte slice of theirs.
+struct Pass {
+  int64_t b, s;
+};
+static Pass pass_of(int64_t B, int64_t S, int64_t D) {
+  const int64_t rows = std::max<int64_t>(16, std::min<int64_t>(MAX_ROWS, 16 * (DH_MAX_WG / cdiv(D * 4, 256))));
+  Pass p;
+  p.s = std::min<int64_t>({S, MAX_S, rows});
+  p.b = std::min<int64_t>(B, std::max<int64_t>(1, rows / std::max<int64_t>(1, p.s)));
+  return p;
 }
 
 static int64_t mask_elem_bytes(int mdt) {
@@ -888,7 +899,11 @@ static int passes_for(int64_t D) {
 // 16 x 128 256 / 233 us, 16 x 200 282 / 263 us; 5% dense, 16 x 64 93 / 89 us, 16 x 128 99 /
 // 116 us (8 x 512, dH alone: 11 / 48 us).
 constexpr int64_t DH_MANY_ROWS = 2048;
-static int dh_rows_per_group(int64_t rows) { return rows >= DH_MANY_ROWS ? DH_GROUPS : 1; }
+// Rows too long for a workgroup each within a launch (65 of 2^24 fp32 columns) share them too.
+static_assert(DH_MAX_WG == MAX_THREADS / (64 * DH_WAVES), "workgroups of a dH launch");
+static int dh_rows_per_group(int64_t rows, int64_t n_slices) {
+  return rows >= DH_MANY_ROWS || rows * n_slices > DH_MAX_WG ? DH_GROUPS : 1;
+}
 // SPARTON_BWD_HOT_MIN sets the number of entries past which a row is shared (tests compare
 // shared and unshared rows).
 static int dh_hot_min() {
@@ -1257,11 +1272,12 @@ static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void*
   const int n_dw = need_dw && staged ? (int)cdiv(V, DW_IDS) : 0;
   bool dw_done = false;
   if (dH != nullptr && B * S > 0 && D > 0) {
-    // Batch rows in chunks and positions in windows (pass_b, pass_s): each pass buckets the
+    // Batch rows in chunks and positions in windows (pass_of): each pass buckets the
     // entries of rows [b0, b0 + nb) and positions [s0, s0 + sw) (entries whose index lies
     // outside the window are inactive) and sums its dH rows, so every dH row is written by
     // exactly one pass. The workspace holds one pass; the passes reuse it in stream order.
-    const int64_t Bc = pass_b(B, S), Sc = pass_s(S);
+    const Pass pass = pass_of(B, S, D);
+    const int64_t Bc = pass.b, Sc = pass.s;
     const Layout L = layout(Bc, Sc, V);
     const Cut c = cut_ids(V);
     int* off = (int*)((char*)ws + L.off);
@@ -1273,7 +1289,8 @@ static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void*
         const int64_t sw = std::min(Sc, S - s0);
         const int nbk = (int)(nb * c.runs);
         // dW's workgroups join where the bucketing's counters take little more LDS than dW's.
-        const bool with_dw = n_dw > 0 && S <= DW_MERGE_S && nb == B && dw_merge_on();
+        const bool with_dw = n_dw > 0 && S <= DW_MERGE_S && nb == B && nbk + (int64_t)n_dw <= BK_MAX_WG &&
+                             dw_merge_on();
         const size_t lds = (size_t)(BK_WAVES + 1 + (BK_WAVES + 1) * sw) * 4;
         hipLaunchKernelGGL((bwd_bucket_dw_kernel<T, O, DNP, RT>), dim3((unsigned)(nbk + (with_dw ? n_dw : 0))),
                            dim3(64 * BK_WAVES), with_dw ? std::max(lds, dw_lds) : lds, st, g + b0 * V,
@@ -1281,7 +1298,7 @@ static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void*
                            H, dW, dbias, (int)B, (int)S, (int)D, (int)V, nbk, (int)c.runs, (int)c.cap,
                            (int)s0, (int)sw, off, run);
         dw_done |= with_dw;
-        const int rpw = dh_rows_per_group(nb * sw);
+        const int rpw = dh_rows_per_group(nb * sw, n_slices);
         const bool wide = (uint64_t)V * ((uint64_t)D * sizeof(T) / 16) > DH_WIDE_16;
         hipLaunchKernelGGL((wide ? bwd_dh_kernel<T, O, true> : bwd_dh_kernel<T, O, false>),
                            dim3((unsigned)(cdiv(nb * sw, rpw) * n_slices)),
@@ -1347,7 +1364,8 @@ extern "C" __attribute__((visibility("default"))) size_t sparton_bwd_workspace_b
     int64_t B, int64_t S, int64_t D, int64_t V) {
   if (B <= 0 || S <= 0 || D <= 0 || V < 0) return 0;
   const bwd::FewPlan few = bwd::few_plan(B, S, D, V);
-  return std::max(bwd::layout(bwd::pass_b(B, S), bwd::pass_s(S), V).total, few.fits ? few.part_bytes : (size_t)0);
+  const bwd::Pass p = bwd::pass_of(B, S, D);
+  return std::max(bwd::layout(p.b, p.s, V).total, few.fits ? few.part_bytes : (size_t)0);
 }
 
 extern "C" __attribute__((visibility("default"))) int sparton_bwd(

@@ -867,6 +867,29 @@ def test_backward_weight_past_64_gib(V, D, ids, device):
     assert bool((err <= 4 * 2.0 ** -24 * want.abs()).all())
 
 
+def test_backward_rows_past_the_launch_limit(device):
+    """65 dH rows of 2^24 fp32 columns: a workgroup for every row and 256-byte slice would be more
+    than the 2^32 threads that a launch may have."""
+    B, S, D, V = 1, 65, 2 ** 24, 4
+    say(f"backward, B={B} S={S} D={D} V={V}")
+    gen = torch.Generator(device=device).manual_seed(2)
+    W = torch.randn(V, D, generator=gen, device=device)
+    H = torch.zeros(B, S, D, device=device)
+    G, reps = torch.ones(B, V, device=device), torch.full((B, V), 0.5, device=device)
+    idx = torch.tensor([[0, 64, 64, 30]], dtype=torch.int32, device=device)
+    m = torch.ones(B, S, dtype=torch.int64, device=device)
+    dH = torch.full((B, S, D), float("nan"), device=device)
+    _bwd_capi(G, reps, idx, H, W, m, dH, None, None)
+    torch.cuda.synchronize()
+    c = float(np.exp(-0.5))
+    for s in range(S):
+        want = {0: c * W[0], 64: c * (W[1] + W[2]), 30: c * W[3]}.get(s)
+        if want is None:
+            assert not bool(dH[0, s].any())
+        else:
+            torch.testing.assert_close(dH[0, s], want, rtol=2e-6, atol=1e-6)
+
+
 @pytest.mark.parametrize("case", [
     ("bf16", 2, 20000, 64, 320, True, "holes"),     # S > 16384: two dH windows
     ("fp32", 1, 40000, 32, 200, False, "int64"),    # three windows, the last partial
