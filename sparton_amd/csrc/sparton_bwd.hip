@@ -44,6 +44,7 @@ constexpr int BK_IDS = 64 * BK_ROUNDS * BK_WAVES;  // ids of a workgroup's turn
 constexpr int BK_RUNS = 16;         // bucketing workgroups (runs) per batch row, at most
 constexpr int MAX_S = 4096;         // positions per dH window (LDS: S counters per wave)
 constexpr int64_t MAX_ROWS = 1 << 20;  // dH rows per pass (bounds the run offsets)
+constexpr int64_t MAX_B = 8192;     // and batch rows (bounds the runs, 8 V bytes each)
 constexpr int MAX_NP = 16;          // D up to 16 * 256 per register pass
 
 // How a batch row's ids are cut: `runs` runs of `cap` ids (a multiple of BK_IDS).
@@ -61,12 +62,11 @@ struct Layout {
   size_t off, run, total;
 };
 static Layout layout(int64_t B, int64_t S, int64_t V) {
-  const Cut c = cut_ids(V);
   Layout L;
   size_t at = 0;
   auto take = [&](size_t bytes) { size_t o = at; at += (size_t)round_up((int64_t)bytes, 256); return o; };
-  L.off = take((size_t)(B * (S + 1) * c.runs) * 4);  // [B][S + 1][runs] a position's first entry
-  L.run = take((size_t)(B * c.runs * c.cap) * 8);    // [B][runs][cap] (v, g'), by position, then v
+  L.off = take((size_t)(B * (S + 1) * cut_ids(V).runs) * 4);  // [B][S + 1][runs] a position's first entry
+  L.run = take((size_t)(B * V) * 8);  // [B][V] (v, g'): run c from id c cap on, by position, then v
   L.total = at;
   return L;
 }
@@ -84,7 +84,7 @@ static Pass pass_of(int64_t B, int64_t S, int64_t D) {
   const int64_t rows = std::max<int64_t>(16, std::min<int64_t>(MAX_ROWS, 16 * (DH_MAX_WG / cdiv(D * 4, 256))));
   Pass p;
   p.s = std::min<int64_t>({S, MAX_S, rows});
-  p.b = std::min<int64_t>(B, std::max<int64_t>(1, rows / std::max<int64_t>(1, p.s)));
+  p.b = std::min<int64_t>({B, MAX_B, std::max<int64_t>(1, rows / std::max<int64_t>(1, p.s))});
   return p;
 }
 
@@ -223,7 +223,7 @@ __device__ __forceinline__ void bucket_run(const T* __restrict__ grad, const RT*
   // (one wave's LDS accesses complete in program order).
   const uint64_t lt = (1ull << lane) - 1ull;
   const int sbits = S > 1 ? 32 - __builtin_clz((unsigned)(S - 1)) : 0;
-  int2* out = run + (b * runs + c) * cap;
+  int2* out = run + b * V + c * cap;
   for (int t = 0; t < turns && V > 0; ++t) {
     if (turns > 1) {
       load(t);
@@ -477,7 +477,7 @@ struct HotSmem {
 template <typename T, typename O, bool WIDE>
 __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
     const T* __restrict__ W, const int* __restrict__ off, const int2* __restrict__ run,
-    O* __restrict__ dH, int B, int S, int D, int runs, int cap, int S_row, int n_slices, int rpw,
+    O* __restrict__ dH, int B, int S, int D, int V, int runs, int cap, int S_row, int n_slices, int rpw,
     int hot_min) {
   constexpr int E = Chunk<T>::E;
   static_assert(Chunk<T>::COLS <= 64 * DH_WAVES, "one thread per column");
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
   auto entries_of = [&](int64_t row, RowEntries& re) {  // returns the batch row's runs
     const int64_t b = row / S;
     re.load(off + (b * (S + 1) + (row - b * S)) * runs, runs, cap, l);
-    return run + b * runs * cap;
+    return run + b * V;
   };
   auto out_of = [&](int64_t row) {
     const int64_t b = row / S;
@@ -1303,7 +1303,7 @@ static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void*
         hipLaunchKernelGGL((wide ? bwd_dh_kernel<T, O, true> : bwd_dh_kernel<T, O, false>),
                            dim3((unsigned)(cdiv(nb * sw, rpw) * n_slices)),
                            dim3(64 * DH_WAVES), 0, st, W, (const int*)off, (const int2*)run,
-                           dH + (b0 * S + s0) * D, (int)nb, (int)sw, (int)D, (int)c.runs, (int)c.cap,
+                           dH + (b0 * S + s0) * D, (int)nb, (int)sw, (int)D, (int)V, (int)c.runs, (int)c.cap,
                            (int)S, (int)n_slices, rpw, dh_hot_min());
       }
     }

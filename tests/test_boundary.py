@@ -118,6 +118,21 @@ def test_bwd_argument_validation(kw, code):
     assert bwd(**kw) == code
 
 
+@pytest.mark.parametrize("B,S,V", [(65536, 8, 30522), (65536, 16, 1000), (10 ** 6, 1, 128), (100000, 8, 1000),
+                                   (9000, 3, 64), (40, 8192, 300), (3, 500000, 70000)])
+def test_bwd_workspace_is_bounded_in_batch_rows(B, S, V):
+    """A dH pass takes at most 8192 batch rows, windows of 4096 positions and 2^20 dH rows: its
+    workspace holds 8 bytes for each of their ids, and a position's first entry for each of its
+    (at most 16) runs of ids. More rows go in more passes through the same workspace."""
+    size = _lib.load().sparton_bwd_workspace_bytes
+    sw = min(S, 4096)
+    nb = min(B, 8192, 2 ** 20 // sw)
+    runs = -(-V // (4096 * -(-V // 65536)))
+    ws = size(B, S, 64, V)
+    assert 0 <= ws - (8 * nb * V + 4 * nb * (sw + 1) * runs) < 512
+    assert (B > nb) == (ws == size(2 * B, S, 64, V))  # several passes (batch chunks), or one
+
+
 def test_fwd_profile_requires_time_output():
     a = dict(hidden=P, weight=P, bias=None, mask=P, mask_dtype=0, reps=P, argmax=P, reps_f32=None,
              B=2, S=4, D=64, V=10, dtype=1, ws=P, ws_bytes=1 << 30, stream=None, main_ms=None)
