@@ -91,7 +91,7 @@ constexpr int PLAN_THREADS = 1024;
 // Device scratch of one launch, carved from the caller's workspace (256-byte aligned
 // sections). ngrp = groups per batch row, n_mt_max = M-tiles if every group is active.
 struct Work {
-  int* meta;          // [0] active groups
+  int* meta;          // [0] active groups; [1] fp32 operands that the fp16 pairs do not hold
   int* count;         // [B] active groups per batch row
   int* first;         // [B] index of its first active group in `list`
   uint8_t* flag;      // [B][ngrp] 1 = group has a nonzero mask entry
@@ -203,7 +203,10 @@ __device__ __forceinline__ void plan_list(int B, int ngrp, const uint8_t* __rest
     if (tid == PLAN_THREADS - 1) carry = start + c;
     __syncthreads();
   }
-  if (tid == 0) meta[0] = carry;
+  if (tid == 0) {
+    meta[0] = carry;
+    meta[1] = 0;
+  }
   // One wave per batch row: lane j takes group j (64 at a time); its slot is the row
   // start plus the active groups before it (a ballot prefix), so the list stays in
   // (b, j) order.
@@ -313,7 +316,10 @@ __global__ __launch_bounds__(PLAN_THREADS) void fwd_plan_small_kernel(
     if (tid == PLAN_THREADS - 1) carry = start + c;
     __syncthreads();
   }
-  if (tid == 0) meta[0] = carry;
+  if (tid == 0) {
+    meta[0] = carry;
+    meta[1] = 0;
+  }
   for (int b = wave; b < B; b += NW) {
     int k = cnt[b];
     for (int j0 = 0; j0 < ngrp; j0 += 64) {
@@ -406,6 +412,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void fwd_plan_tiny_kernel(
   if (tid == 0) {
     slot_of[n_g] = total;
     meta[0] = total;
+    meta[1] = 0;
   }
   __syncthreads();
   for (int b = tid; b < B; b += PLAN_THREADS) {
@@ -1248,8 +1255,14 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
     const float* __restrict__ rowmask, O* __restrict__ reps, int32_t* __restrict__ argmax,
     float* __restrict__ reps_f32, int S, int D, int V, int n_vt, int ngrp,
     const int* __restrict__ meta, const int* __restrict__ list, float2* __restrict__ part,
-    const int* __restrict__ rexp, const int* __restrict__ cexp) {
+    const int* __restrict__ rexp, const int* __restrict__ cexp, int only_unheld) {
   __shared__ Smem sm;
+  // fp32 operands: the launch on pairs or, after it, the one on the values, as the split found.
+  if constexpr (PAIR) {
+    if (meta[1] != 0) return;
+  } else if constexpr (sizeof(T) == 4) {
+    if (only_unheld && meta[1] == 0) return;
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: keep it scalar
 
@@ -1299,9 +1312,10 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
 // fits lo's 11: hi + lo = x exactly for every x within 2^-15 of its row's largest, and within
 // 2^-39 of that largest below (fp16's subnormals). A product is taken as lo hi + hi lo + hi hi,
 // each exact in fp32, accumulated in fp32; the dropped lo lo is at most 2^-24 of the product,
-// fp32's own rounding of it. An element that is infinite or NaN puts its value in lo (hi = 0),
-// so that it meets only the partner's hi, and the row's scale leaves it out. The epilogue takes
-// the scales out again before it adds the bias.
+// fp32's own rounding of it. The epilogue takes the scales out again before it adds the bias.
+// An element that is infinite or NaN has no such parts (an infinity would meet zeros among its
+// partners' that are none): the split then raises meta[1], the launch on pairs ends at once and
+// one on the fp32 MFMAs, which ends at once otherwise, follows.
 // Error of reps against 64 bits, fp32 MFMAs -> pairs (2-norm relative; the keys' 18 bits
 // included): 8 x 128 x 768 x 30522 normal 1.22e-6 -> 1.19e-6, rows scaled by e^N(0,16)
 // 2.6e-7 -> 2.4e-7, elements scaled by e^N(0,4) 2.61e-7 -> 2.56e-7; D = 4096 1.11e-6 -> 1.00e-6.
@@ -1317,7 +1331,7 @@ struct PairRows {
 // group list[t / 16]; rows past the last active group are left out).
 __global__ __launch_bounds__(256) void fwd_split_rows_kernel(
     const float* __restrict__ H, const float* __restrict__ W, PairRows hp, PairRows wp, int S, int D,
-    int Dp, int V, int ngrp, const int* __restrict__ meta, const int* __restrict__ list) {
+    int Dp, int V, int ngrp, int* meta, const int* __restrict__ list) {
   const int lane = threadIdx.x & 63;
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const float* src;
@@ -1339,6 +1353,7 @@ __global__ __launch_bounds__(256) void fwd_split_rows_kernel(
   constexpr int NR = 4;  // 256-column pieces kept in registers: D <= 1024 is read once
   f32x4 x[NR];
   float m = 0.0f;
+  bool held = true;
   auto piece = [&](int p) {
     const int d = p * 256 + lane * 4;
     return d < D ? *(const f32x4*)(src + d) : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1347,7 +1362,8 @@ __global__ __launch_bounds__(256) void fwd_split_rows_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float y = fabsf(v[i]);
-      m = y > m && y < INFINITY ? y : m;
+      held &= y < INFINITY;
+      m = fmaxf(m, y);
     }
   };
 #pragma unroll
@@ -1355,6 +1371,10 @@ __global__ __launch_bounds__(256) void fwd_split_rows_kernel(
 #pragma unroll
   for (int p = 0; p < NR; ++p) top(x[p]);
   for (int p = NR; p * 256 < D; ++p) top(piece(p));
+  if (__ballot(!held) != 0) {  // uniform
+    if (lane == 0) meta[1] = 1;
+    return;
+  }
   m = wave_max(m);
   int e = 15;  // m = f 2^e, 1/2 <= f < 1: the scale is 2^(15 - e)
   if (m > 0.0f) (void)frexpf(m, &e);
@@ -1366,8 +1386,7 @@ __global__ __launch_bounds__(256) void fwd_split_rows_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float y = __builtin_amdgcn_ldexpf(v[i], 15 - e);
-      const bool fin = fabsf(v[i]) < INFINITY;
-      hi[i] = fin ? (f16)y : (f16)0.0f;
+      hi[i] = (f16)y;
       lo[i] = (f16)(y - (float)hi[i]);
     }
     *(f16x4*)(dst + d) = hi;
@@ -1805,26 +1824,23 @@ static int launch(const void* H, const void* W, const void* bias, const void* ma
   if (pairs != nullptr)
     hipLaunchKernelGGL(fwd_split_rows_kernel, dim3((unsigned)cdiv(V + n_mt_max * BM, 4)), dim3(256), 0,
                        stream, (const float*)H, (const float*)W, pairs->h, pairs->w, (int)S, (int)D,
-                       (int)pairs->Dp, (int)V, (int)ngrp, (const int*)w.meta, (const int*)w.list);
+                       (int)pairs->Dp, (int)V, (int)ngrp, w.meta, (const int*)w.list);
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[0], stream);
   if (grid > 0) {  // S == 0: no blocks, the fixup writes every row
-    bool done = false;
     if constexpr (sizeof(T) == 4) {
-      if (pairs != nullptr) {
+      if (pairs != nullptr)
         hipLaunchKernelGGL((sparton_fwd_kernel<f16, float, true>), dim3((unsigned)grid), dim3(NTHREADS), 0,
                            stream, (const f16*)pairs->h.hi_lo, (const f16*)pairs->w.hi_lo,
                            (const float*)bias, (const float*)w.rowmask, (float*)reps, argmax, reps_f32,
                            (int)S, (int)pairs->Dp, (int)V, (int)n_vt, (int)ngrp, (const int*)w.meta,
                            (const int*)w.list, w.part, (const int*)pairs->h.exp,
-                           (const int*)pairs->w.exp);
-        done = true;
-      }
+                           (const int*)pairs->w.exp, 0);
     }
-    if (!done)
-      hipLaunchKernelGGL((sparton_fwd_kernel<T, T, false>), dim3((unsigned)grid), dim3(NTHREADS), 0, stream,
-                         (const T*)H, (const T*)W, (const T*)bias, (const float*)w.rowmask, (T*)reps,
-                         argmax, reps_f32, (int)S, (int)D, (int)V, (int)n_vt, (int)ngrp,
-                         (const int*)w.meta, (const int*)w.list, w.part, nullptr, nullptr);
+    hipLaunchKernelGGL((sparton_fwd_kernel<T, T, false>), dim3((unsigned)grid), dim3(NTHREADS), 0, stream,
+                       (const T*)H, (const T*)W, (const T*)bias, (const float*)w.rowmask, (T*)reps,
+                       argmax, reps_f32, (int)S, (int)D, (int)V, (int)n_vt, (int)ngrp,
+                       (const int*)w.meta, (const int*)w.list, w.part, nullptr, nullptr,
+                       pairs != nullptr ? 1 : 0);
   }
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[1], stream);
   hipLaunchKernelGGL(fwd_fixup_kernel<T>, dim3((unsigned)cdiv(V, FIX_COLS), (unsigned)B), dim3(256), 0,

@@ -1092,6 +1092,36 @@ def test_fp32_pairs_infinite_and_extreme_entries(device):
     torch.testing.assert_close(r_p[same], r_e[same], rtol=2e-5, atol=1e-30)
 
 
+@pytest.mark.parametrize("where", ["tiny", "both", "nan", "weight", "padding"])
+def test_fp32_large_batch_nonfinite_entries(where, device):
+    """An infinite or NaN entry in an fp32 batch past the small-batch kernel: reps and argmax are the
+    fp32 MFMAs', bit for bit, whatever it meets: a finite partner far below its row's largest
+    (an infinity times it is infinite), another infinity, or a position the mask leaves out."""
+    say(f"fp32 large batch, entries that are not finite: {where}")
+    g = torch.Generator().manual_seed(23)
+    B, S, D, V = 3, 64, 256, 700
+    H, W = torch.randn(B, S, D, generator=g), torch.randn(V, D, generator=g) * 0.02
+    m = torch.ones(B, S, dtype=torch.long)
+    m[1, 20:] = 0
+    inf = float("inf")
+    if where == "tiny":
+        H[0, 5, 17], W[:, 17] = inf, 1e-20
+    elif where == "both":
+        H[0, 5, 17] = W[100, 17] = inf
+    elif where == "nan":
+        H[2, 63, 255] = float("nan")
+    elif where == "weight":
+        W[699, 255], H[..., 255] = inf, 1e-20
+    else:
+        H[1, 25, 3], W[:, 3] = inf, 1e-20
+    Hd, Wd, md = H.to(device), W.to(device), m.to(device)
+    r_p, i_p = _fwd_capi_fp32(Hd, Wd, None, md, True)
+    r_e, i_e = _fwd_capi_fp32(Hd, Wd, None, md, False)
+    if where in ("tiny", "weight", "both"):
+        assert bool(r_e.isinf().any())
+    assert torch.equal(r_p.view(torch.int32), r_e.view(torch.int32)) and torch.equal(i_p, i_e)
+
+
 def test_fp32_split_infinite_entries(device):
     """Infinite entries in H and in W under 'high' (the bf16 hi/lo split kernel): reps and
     argmax equal the exact fp32 path's ('highest'), infinities and NaNs included, as long as
