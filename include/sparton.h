@@ -51,7 +51,7 @@ enum sparton_dtype {
  * each product as hi*hi + hi*lo + lo*hi on bf16 MFMAs with fp32 accumulation, within
  * 3 * 2^-16 relative of the exact product. It applies to the small-batch kernel
  * (B*S <= 128); larger batches are computed to fp32's precision either way (fp32 MFMAs, or
- * each operand as an exact pair of fp16, see sparton_fwd_workspace_bytes).
+ * each operand as three bf16 parts that hold all its bits, see sparton_fwd_workspace_bytes).
  */
 #define SPARTON_F32_SPLIT 0x100
 
@@ -78,9 +78,10 @@ enum sparton_status {
 /*
  * Bytes of device scratch sparton_fwd needs for these sizes (256-byte aligned
  * sections: the per-row block plan, the partial results of batch rows whose
- * positions span several row tiles, and for fp32 batches past 128 positions H and W
- * as pairs of fp16, on whose MFMAs such a batch runs; given less than these bytes but
- * enough for the rest, it runs on the fp32 MFMAs instead). No counterpart in the reference: its forward
+ * positions span several row tiles, and for larger fp32 batches (B*S >= 192) H and W
+ * as three bf16 parts, on whose MFMAs such a batch runs; given less than these bytes but
+ * enough for the rest, it runs on the fp32 MFMAs instead, as do operands with a nonzero
+ * magnitude outside [2^-50, 2^48), infinities and NaN among them). No counterpart in the reference: its forward
  * materializes a [B,S,C] logits tile per vocab tile instead (sparton_kernel.py:245-247).
  */
 size_t sparton_fwd_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t V, int dtype);
@@ -109,10 +110,10 @@ int sparton_fwd(const void* hidden, const void* weight, const void* bias,
  * sparton_fwd without a workspace argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No
  * counterpart in the reference. The same kernels and results as sparton_fwd (fp32 batches
- * always on the fp32 MFMAs, without pairs of fp16); the workspace
+ * always on the fp32 MFMAs, without bf16 parts); the workspace
  * is a static device array of sparton_fwd_noalloc_max_workspace() bytes (32 MiB), one per
  * GPU, held until the process ends. Sizes that need more (sparton_fwd_workspace_bytes(), the
- * pairs aside) return SPARTON_ESCRATCH and launch nothing (at V = 30522 that allows about 68 row tiles of
+ * parts aside) return SPARTON_ESCRATCH and launch nothing (at V = 30522 that allows about 68 row tiles of
  * 256 packed positions, e.g. B = 64, S = 256). Calls that overlap on one GPU share that
  * array and race: the caller serialises them. Allocates, frees and synchronises nothing.
  */

@@ -17,8 +17,8 @@
 // for 256 live rows instead of one batch row's (often partly padded) 256 positions,
 // and a batch row wastes less than 16 rows of padding.
 //
-// fp32 batches past the small-batch kernel run on fp16 MFMAs (fwd_split_rows_kernel): H and W
-// as exact pairs of fp16, three products per value.
+// fp32 batches past the small-batch kernel run on bf16 MFMAs (fwd_split_rows_kernel): H and W
+// as sums of three bf16 parts, which hold all their bits, six products per value.
 //
 // Main kernel. A "unit" is one M-tile x one vocab tile of BN columns. The grid is
 // persistent (one workgroup per CU) and each workgroup walks its units in rounds; for
@@ -91,7 +91,7 @@ constexpr int PLAN_THREADS = 1024;
 // Device scratch of one launch, carved from the caller's workspace (256-byte aligned
 // sections). ngrp = groups per batch row, n_mt_max = M-tiles if every group is active.
 struct Work {
-  int* meta;          // [0] active groups; [1] fp32 operands that the fp16 pairs do not hold
+  int* meta;          // [0] active groups; [1] fp32 operands that the bf16 parts do not hold
   int* count;         // [B] active groups per batch row
   int* first;         // [B] index of its first active group in `list`
   uint8_t* flag;      // [B][ngrp] 1 = group has a nonzero mask entry
@@ -445,8 +445,6 @@ struct __align__(16) UnitMeta {
   int grp_s[NGRP];           // first position of each group (16 j)
   int mask_binary;           // every maskf value is 0 or 1
   float bias[BN];            // bias of the tile's columns (0 past V or without bias)
-  int rexp[BM];              // fp32 operands as fp16 pairs: the scales' exponents, negated, of
-  int cexp[BN];              // the tile's rows and columns
 };
 
 struct Smem {
@@ -593,16 +591,17 @@ __device__ __forceinline__ void unit_tile(int u, int n_mt, int n_vt, int* m, int
   *vt = group * GROUP_V + rem - mm * gv;
 }
 
+// fp32 operands as parts (fwd_split_rows_kernel): parts of a value, products of a pair of values.
+constexpr int N_PARTS = 3, PART_RUNS = 6;
+
 // Launch-wide, wave-uniform parameters.
-// T: the operands' type; O: the type of bias and reps. PAIR: the operands are fp32 values
-// split into pairs of fp16 (split_rows_kernel below), H's rows in tile-row order.
-template <typename T, typename O, bool PAIR>
+// T: the operands' type; O: the type of bias and reps. PARTS: the operands are fp32 values as
+// three bf16 parts (fwd_split_rows_kernel below), H's rows in tile-row order.
+template <typename T, typename O, bool PARTS>
 struct Args {
   const char* H;      // H[0, 0, :]
   const char* W;
   const O* bias;
-  const int* rexp;       // PAIR: [n_mt * BM]
-  const int* cexp;       // PAIR: [V]
   const float* rowmask;  // [n_mt * BM] mask of each tile row
   const int* list;
   int n_grp;          // active groups
@@ -612,16 +611,22 @@ struct Args {
   int nk_full;        // slabs lying entirely inside the row
   int nk;             // slabs per unit
   int V;
-  int part_bytes;     // PAIR: bytes of a row's hi (or lo) part
-  // Byte offsets of K slab k in a row of A and of W. A PAIR product runs over K three times:
-  // lo x hi, hi x lo, hi x hi.
+  int part_bytes;     // PARTS: bytes of one part of a row
+  // Byte offsets of K slab k in a row of A and of W. A product of PARTS runs over K six times,
+  // smallest first: A's parts 2 0 1 1 0 0 with W's 0 2 1 0 1 0.
   __device__ __forceinline__ void slab_at(int k, uint32_t* ka, uint32_t* kb) const {
     *ka = *kb = (uint32_t)k * SLAB;
-    if constexpr (PAIR) {
+    if constexpr (PARTS) {
       const uint32_t part = (uint32_t)part_bytes;
-      const uint32_t at = *ka;  // bytes into the three runs
-      *ka = at < part ? at + part : at < 2 * part ? at - part : at - 2 * part;
-      *kb = at < part ? at : at < 2 * part ? at : at - 2 * part;
+      uint32_t run = 0, at = *ka;
+#pragma unroll
+      for (int i = 0; i < PART_RUNS - 1; ++i)
+        if (at >= part) {
+          at -= part;
+          ++run;
+        }
+      *ka = at + (0x052u >> (2 * run) & 3u) * part;
+      *kb = at + (0x118u >> (2 * run) & 3u) * part;
     }
   }
 };
@@ -674,8 +679,8 @@ __device__ __forceinline__ void row_offsets(const UnitMeta& um, int n_valid, int
   }
 }
 
-// The same for rows in tile order (PAIR): tile row 256 m + r lies at that row.
-__device__ __forceinline__ void pair_row_offsets(int m, int n_valid, int row_bytes, int c, int lane,
+// The same for rows in tile order (PARTS): tile row 256 m + r lies at that row.
+__device__ __forceinline__ void tile_row_offsets(int m, int n_valid, int row_bytes, int c, int lane,
                                                  uint32_t* a_off) {
 #pragma unroll
   for (int i = 0; i < A_LOADS; ++i) {
@@ -882,8 +887,8 @@ struct Outputs {
 
 // Start a unit without prefetch: fetch its metadata into um, write the previous unit's
 // results (prev.u >= 0, metadata in um_prev), and land its first two slabs. Two barriers.
-template <typename T, typename O, bool PAIR>
-__device__ __forceinline__ void copy_start(Smem& sm, const Args<T, O, PAIR>& a, const Outputs<O>& o,
+template <typename T, typename O, bool PARTS>
+__device__ __forceinline__ void copy_start(Smem& sm, const Args<T, O, PARTS>& a, const Outputs<O>& o,
                                            UnitMeta& um, CopyUnit& cu, int buf,
                                            const Unit& prev, const UnitMeta& um_prev, int ct,
                                            int c, int lane) {
@@ -891,16 +896,12 @@ __device__ __forceinline__ void copy_start(Smem& sm, const Args<T, O, PAIR>& a, 
   const float mv = a.rowmask[(int64_t)cu.m * BM + ct];
   const int col = cu.v0 + ct;
   const float bv = (a.bias != nullptr && col < a.V) ? to_f32(a.bias[col]) : 0.0f;
-  if constexpr (PAIR) {
-    um.rexp[ct] = a.rexp[(int64_t)cu.m * BM + ct];
-    um.cexp[ct] = a.cexp[min(col, a.V - 1)];
-  }
   put_groups(um, code, a.ngrp, ct);
   um.maskf[ct] = mv;
   um.bias[ct] = bv;
   if (ct == 0) um.mask_binary = 1;
   lds_barrier();  // S1
-  if constexpr (PAIR) pair_row_offsets(cu.m, cu.n_valid, a.row_bytes, c, lane, cu.a_off);
+  if constexpr (PARTS) tile_row_offsets(cu.m, cu.n_valid, a.row_bytes, c, lane, cu.a_off);
   else row_offsets(um, cu.n_valid, a.S, a.row_bytes, c, lane, cu.a_off);
   if (a.nk > 0) {
     issue_slab(sm, a, cu, 0, buf, c, lane);
@@ -918,8 +919,8 @@ __device__ __forceinline__ void copy_start(Smem& sm, const Args<T, O, PAIR>& a, 
   lds_barrier();  // S2
 }
 
-template <typename T, typename O, bool PAIR>
-__device__ void copy_path(Smem& sm, const Args<T, O, PAIR>& a, const Outputs<O>& o, int w, int G,
+template <typename T, typename O, bool PARTS>
+__device__ void copy_path(Smem& sm, const Args<T, O, PARTS>& a, const Outputs<O>& o, int w, int G,
                           int n_units, int n_mt, int n_vt, int ct, int c, int lane) {
   const int nk = a.nk;
   Unit cur = unit_of(w, 0, G, n_units, n_mt, n_vt, a.n_grp);
@@ -940,18 +941,13 @@ __device__ void copy_path(Smem& sm, const Args<T, O, PAIR>& a, const Outputs<O>&
     float mv;
     int code;
     uint32_t bias;
-    int rexp, cexp;
   };
   auto load_meta = [&](const Unit& x) {
-    MetaRegs mr{0.0f, 0, 0u, 0, 0};
+    MetaRegs mr{0.0f, 0, 0u};
     if (x.u >= 0 && nk >= PREFETCH_MIN_NK) {
       mr.mv = a.rowmask[(int64_t)x.m * BM + ct];
       mr.code = a.list[min(max(group_entry(x.m, min(ct, NGRP + 1)), 0), a.n_grp - 1)];
       if (a.bias != nullptr) mr.bias = load_bits(a.bias + min(x.v0 + ct, a.V - 1), 0);
-      if constexpr (PAIR) {
-        mr.rexp = a.rexp[(int64_t)x.m * BM + ct];
-        mr.cexp = a.cexp[min(x.v0 + ct, a.V - 1)];
-      }
     }
     return mr;
   };
@@ -983,12 +979,8 @@ __device__ void copy_path(Smem& sm, const Args<T, O, PAIR>& a, const Outputs<O>&
           put_mask_words(um_next, meta.mv, ct, lane);
           const int col = nx.v0 + ct;
           um_next.bias[ct] = (a.bias != nullptr && col < a.V) ? bits_to_f32<O>(meta.bias) : 0.0f;
-          if constexpr (PAIR) {
-            um_next.rexp[ct] = meta.rexp;
-            um_next.cexp[ct] = meta.cexp;
-          }
         } else if (k == 3) {
-          if constexpr (PAIR) pair_row_offsets(nx.m, nx.n_valid, a.row_bytes, c, lane, nx.a_off);
+          if constexpr (PARTS) tile_row_offsets(nx.m, nx.n_valid, a.row_bytes, c, lane, nx.a_off);
           else row_offsets(um_next, nx.n_valid, a.S, a.row_bytes, c, lane, nx.a_off);
         }
       }
@@ -1033,7 +1025,7 @@ __device__ void copy_path(Smem& sm, const Args<T, O, PAIR>& a, const Outputs<O>&
 
 // Mainloop + block epilogue of one unit for a compute wave with JM blocks (JM = 0: the
 // wave only keeps the barrier schedule). Stage buf holds the unit's slab 0.
-template <typename T, bool PAIR, int JM>
+template <typename T, int JM>
 __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int nk, int buf,
                                              int lane, int wm, int wn) {
   constexpr int JA = JM > 0 ? JM : 1;
@@ -1044,8 +1036,7 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
   f32x16 acc[JA][NB_PER_WAVE];
 #pragma unroll
   for (int nb = 0; nb < NB_PER_WAVE; ++nb) {
-    float bv = PAIR ? 0.0f : um.bias[wn * 64 + nb * 32 + l32];  // (PAIR adds it unscaled, below)
-    if constexpr (PAIR) asm("" : "+v"(bv));  // a register like the bias: a constant costs spills
+    const float bv = um.bias[wn * 64 + nb * 32 + l32];
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[JA - 1][nb][i] = bv;
     if (nk == 0) {  // no MFMAs: x = bias
@@ -1153,19 +1144,6 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
   const float* mrow = &um.maskf[wm * 32 + 4 * h];
   const int* wrow = &um.maskw[wm * 32 + 4 * h];
   int* kw = &sm.key[2 * wm][wn * 64 + l32];
-  if constexpr (PAIR) __builtin_amdgcn_sched_barrier(0);  // (keeps the reads below out of the K loop's registers)
-  // PAIR: x = acc 2^(row exponent + column exponent) + bias.
-  const int* rrow = &um.rexp[wm * 32 + 4 * h];
-  int ce[NB_PER_WAVE];
-  float cb[NB_PER_WAVE];
-#pragma unroll
-  for (int nb = 0; nb < NB_PER_WAVE; ++nb) {
-    ce[nb] = PAIR ? um.cexp[wn * 64 + nb * 32 + l32] : 0;
-    cb[nb] = PAIR ? um.bias[wn * 64 + nb * 32 + l32] : 0.0f;
-  }
-  auto logit = [&](float x, int re, int nb) {
-    return PAIR ? __builtin_amdgcn_ldexpf(x, re + ce[nb]) + cb[nb] : x;
-  };
 #pragma unroll
   for (int j = 0; j < JM; ++j) {
     int kmax[2][NB_PER_WAVE];
@@ -1177,27 +1155,23 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const i32x4 w4 = *(const i32x4*)(wrow + j * WAVES_M * 32 + 8 * q);
-        const i32x4 r4 = PAIR ? *(const i32x4*)(rrow + j * WAVES_M * 32 + 8 * q) : i32x4{0, 0, 0, 0};
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
           for (int nb = 0; nb < NB_PER_WAVE; ++nb)
-            kmax[q >> 1][nb] =
-                max(kmax[q >> 1][nb],
-                    (__float_as_int(logit(acc[j][nb][q * 4 + e], r4[e], nb)) & w4[e]) | (31 - 8 * q - e));
+            kmax[q >> 1][nb] = max(kmax[q >> 1][nb],
+                                   (__float_as_int(acc[j][nb][q * 4 + e]) & w4[e]) | (31 - 8 * q - e));
       }
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const f32x4 m4 = *(const f32x4*)(mrow + j * WAVES_M * 32 + 8 * q);
-        const i32x4 r4 = PAIR ? *(const i32x4*)(rrow + j * WAVES_M * 32 + 8 * q) : i32x4{0, 0, 0, 0};
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
           for (int nb = 0; nb < NB_PER_WAVE; ++nb)
-            kmax[q >> 1][nb] =
-                max(kmax[q >> 1][nb],
-                    (__float_as_int(logit(acc[j][nb][q * 4 + e], r4[e], nb) * m4[e]) & ~31) | (31 - 8 * q - e));
+            kmax[q >> 1][nb] = max(kmax[q >> 1][nb],
+                                   (__float_as_int(acc[j][nb][q * 4 + e] * m4[e]) & ~31) | (31 - 8 * q - e));
       }
     }
 #pragma unroll
@@ -1216,8 +1190,8 @@ __device__ __forceinline__ void compute_unit(Smem& sm, const UnitMeta& um, int n
   lds_barrier();  // E
 }
 
-template <typename T, typename O, bool PAIR>
-__device__ void compute_path(Smem& sm, const Args<T, O, PAIR>& a, int w, int G, int n_units, int n_mt,
+template <typename T, typename O, bool PARTS>
+__device__ void compute_path(Smem& sm, const Args<T, O, PARTS>& a, int w, int G, int n_units, int n_mt,
                              int n_vt, int wave, int lane) {
   const int nk = a.nk;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -1231,11 +1205,11 @@ __device__ void compute_path(Smem& sm, const Args<T, O, PAIR>& a, int w, int G, 
     const int n_blocks = (cur.n_valid + 1) / 2;  // 32-row blocks with an active group
     const int jm = n_blocks <= wm ? 0 : min(4, (n_blocks - wm + 1) / WAVES_M);
     switch (jm) {
-      case 0: compute_unit<T, PAIR, 0>(sm, um, nk, buf, lane, wm, wn); break;
-      case 1: compute_unit<T, PAIR, 1>(sm, um, nk, buf, lane, wm, wn); break;
-      case 2: compute_unit<T, PAIR, 2>(sm, um, nk, buf, lane, wm, wn); break;
-      case 3: compute_unit<T, PAIR, 3>(sm, um, nk, buf, lane, wm, wn); break;
-      default: compute_unit<T, PAIR, 4>(sm, um, nk, buf, lane, wm, wn); break;
+      case 0: compute_unit<T, 0>(sm, um, nk, buf, lane, wm, wn); break;
+      case 1: compute_unit<T, 1>(sm, um, nk, buf, lane, wm, wn); break;
+      case 2: compute_unit<T, 2>(sm, um, nk, buf, lane, wm, wn); break;
+      case 3: compute_unit<T, 3>(sm, um, nk, buf, lane, wm, wn); break;
+      default: compute_unit<T, 4>(sm, um, nk, buf, lane, wm, wn); break;
     }
     const Unit next = unit_of(w, r, G, n_units, n_mt, n_vt, a.n_grp);
     if (next.u < 0) return;
@@ -1249,16 +1223,16 @@ __device__ void compute_path(Smem& sm, const Args<T, O, PAIR>& a, int w, int G, 
   }
 }
 
-template <typename T, typename O, bool PAIR>
+template <typename T, typename O, bool PARTS>
 __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
     const T* __restrict__ H, const T* __restrict__ W, const O* __restrict__ bias,
     const float* __restrict__ rowmask, O* __restrict__ reps, int32_t* __restrict__ argmax,
     float* __restrict__ reps_f32, int S, int D, int V, int n_vt, int ngrp,
     const int* __restrict__ meta, const int* __restrict__ list, float2* __restrict__ part,
-    const int* __restrict__ rexp, const int* __restrict__ cexp, int only_unheld) {
+    int only_unheld) {
   __shared__ Smem sm;
-  // fp32 operands: the launch on pairs or, after it, the one on the values, as the split found.
-  if constexpr (PAIR) {
+  // fp32 operands: the launch on parts or, after it, the one on the values, as the split found.
+  if constexpr (PARTS) {
     if (meta[1] != 0) return;
   } else if constexpr (sizeof(T) == 4) {
     if (only_unheld && meta[1] == 0) return;
@@ -1266,12 +1240,10 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: keep it scalar
 
-  Args<T, O, PAIR> a;
+  Args<T, O, PARTS> a;
   a.H = (const char*)H;
   a.W = (const char*)W;
   a.bias = bias;
-  a.rexp = rexp;
-  a.cexp = cexp;
   a.rowmask = rowmask;
   a.list = list;
   a.n_grp = __builtin_amdgcn_readfirstlane(meta[0]);
@@ -1279,10 +1251,10 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
   a.S = S;
   a.V = V;
   const int slab_elems = SLAB / (int)sizeof(T);
-  if constexpr (PAIR) {  // D: the padded part, whole slabs
+  if constexpr (PARTS) {  // D: the padded part, whole slabs
     a.part_bytes = D * (int)sizeof(T);
-    a.row_bytes = 2 * a.part_bytes;
-    a.nk_full = a.nk = 3 * (D / slab_elems);
+    a.row_bytes = N_PARTS * a.part_bytes;
+    a.nk_full = a.nk = PART_RUNS * (D / slab_elems);
   } else {
     a.part_bytes = 0;
     a.row_bytes = D * (int)sizeof(T);
@@ -1295,106 +1267,84 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
   const int n_mt = (a.n_grp + NGRP - 1) / NGRP;
   const int n_units = n_mt * n_vt;
   if (wave < COMPUTE_WAVES) {
-    compute_path<T, O, PAIR>(sm, a, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, wave, lane);
+    compute_path<T, O, PARTS>(sm, a, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, wave, lane);
   } else {
     Outputs<O> o{reps, argmax, reps_f32, part};
-    copy_path<T, O, PAIR>(sm, a, o, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, tid - 64 * COMPUTE_WAVES,
+    copy_path<T, O, PARTS>(sm, a, o, blockIdx.x, gridDim.x, n_units, n_mt, n_vt, tid - 64 * COMPUTE_WAVES,
                           wave - COMPUTE_WAVES, lane);
   }
 }
 
-// ---- fp32 operands as pairs of fp16 -------------------------------------------------
+// ---- fp32 operands as three bf16 parts -----------------------------------------------
 //
-// The fp32 MFMA runs at a sixteenth of the fp16 one's rate, so larger fp32 batches run on
-// fp16 MFMAs: each row of H and W is scaled by a power of two that brings its largest
-// magnitude to [2^14, 2^15) and written as hi = fp16(x), lo = fp16(x - hi). Both round to
-// nearest, so hi takes x's upper 12 bits and x - hi, at most 2^11 units of x's last place,
-// fits lo's 11: hi + lo = x exactly for every x within 2^-15 of its row's largest, and within
-// 2^-39 of that largest below (fp16's subnormals). A product is taken as lo hi + hi lo + hi hi,
-// each exact in fp32, accumulated in fp32; the dropped lo lo is at most 2^-24 of the product,
-// fp32's own rounding of it. The epilogue takes the scales out again before it adds the bias.
-// An element that is infinite or NaN has no such parts (an infinity would meet zeros among its
-// partners' that are none): the split then raises meta[1], the launch on pairs ends at once and
-// one on the fp32 MFMAs, which ends at once otherwise, follows.
-// Error of reps against 64 bits, fp32 MFMAs -> pairs (2-norm relative; the keys' 18 bits
-// included): 8 x 128 x 768 x 30522 normal 1.22e-6 -> 1.19e-6, rows scaled by e^N(0,16)
-// 2.6e-7 -> 2.4e-7, elements scaled by e^N(0,4) 2.61e-7 -> 2.56e-7; D = 4096 1.11e-6 -> 1.00e-6.
-// Bound by the fp16 MFMAs at three products per value, and by the two streams of W. Measured
-// at 8 x 128 x 768 x 30522, 757 live rows: main kernel 403 -> 116 us, this split 29 us
-// (188 MB, 6.5 TB/s).
-struct PairRows {
-  f16* hi_lo;      // [rows][2][Dp]: hi, lo
-  int* exp;        // [rows] the scale's exponent, negated
-};
+// The fp32 MFMA runs at a sixteenth of the bf16 one's rate, so larger fp32 batches run on
+// bf16 MFMAs, H and W as x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1
+// (each part rounds to nearest what the ones before left, 8 bits and a sign: together all 24).
+// A product is taken as x2 w0 + x0 w2 + x1 w1 + x1 w0 + x0 w1 + x0 w0, each exact in fp32,
+// accumulated in fp32 run by run; the dropped x1 w2, x2 w1 and x2 w2 are within 2^-22.9 of the
+// product (|x1| <= 2^-8 |x|, |x2| <= 2^-16 |x|). A logit takes 6 D / 16 accumulations, where the
+// fp32 MFMA's takes D / 2, so its bound is the smaller of the two. bf16 has fp32's exponents, so
+// no element loses bits to a larger one.
+// Error of reps against 64 bits, fp32 MFMAs -> parts (2-norm relative; the keys' 18 bits
+// included): 8 x 128 x 768 x 30522 normal 1.14e-6 -> 1.12e-6; logits 2^-12 of their products
+// 4.7e-4 -> 1.4e-4. Bound by the bf16 MFMAs at six products per value: 1.4 PFLOP/s at 8192 rows.
+// What that takes: |x| in [2^-50, 2^48) or 0. Then every part is a normal bf16, every product that
+// counts a normal fp32, and no sum of parts overflows where the values' would not. A value outside
+// (infinities, NaN) raises meta[1]: the launch on parts ends at once and one on the fp32 MFMAs,
+// which ends at once otherwise, follows.
+constexpr float PART_MIN = 0x1p-50f, PART_MAX = 0x1p48f;
 
 // One wave per row of W (rows 0 .. V - 1), then per row of H's tiles, in tile order (row t of
-// group list[t / 16]; rows past the last active group are left out).
+// group list[t / 16]; rows past the last active group are left out). Out: [row][part][Dp].
 __global__ __launch_bounds__(256) void fwd_split_rows_kernel(
-    const float* __restrict__ H, const float* __restrict__ W, PairRows hp, PairRows wp, int S, int D,
-    int Dp, int V, int ngrp, int* meta, const int* __restrict__ list) {
+    const float* __restrict__ H, const float* __restrict__ W, bf16* __restrict__ hp,
+    bf16* __restrict__ wp, int S, int D, int Dp, int V, int ngrp, int* meta,
+    const int* __restrict__ list) {
   const int lane = threadIdx.x & 63;
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const float* src;
-  f16* dst;
-  int* exp;
+  bf16* dst;
   if (r < V) {
     src = W + r * D;
-    dst = wp.hi_lo + r * 2 * Dp;
-    exp = wp.exp + r;
+    dst = wp + r * N_PARTS * Dp;
   } else {
     const int64_t t = r - V;
     if (t / GROUP >= meta[0]) return;
     const int code = list[t / GROUP], b = code / ngrp;
     const int s = min((code - b * ngrp) * GROUP + (int)(t % GROUP), S - 1);
     src = H + ((int64_t)b * S + s) * D;
-    dst = hp.hi_lo + t * 2 * Dp;
-    exp = hp.exp + t;
+    dst = hp + t * N_PARTS * Dp;
   }
-  constexpr int NR = 4;  // 256-column pieces kept in registers: D <= 1024 is read once
-  f32x4 x[NR];
-  float m = 0.0f;
   bool held = true;
-  auto piece = [&](int p) {
-    const int d = p * 256 + lane * 4;
-    return d < D ? *(const f32x4*)(src + d) : f32x4{0.f, 0.f, 0.f, 0.f};
-  };
-  auto top = [&](const f32x4& v) {
+  constexpr int NR = 4;  // 256-column pieces whose loads are in flight together
+  for (int p0 = 0; p0 * 256 < Dp; p0 += NR) {
+    f32x4 x[NR];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float y = fabsf(v[i]);
-      held &= y < INFINITY;
-      m = fmaxf(m, y);
+    for (int p = 0; p < NR; ++p) {
+      const int d = (p0 + p) * 256 + lane * 4;
+      x[p] = d < D ? *(const f32x4*)(src + d) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
-  };
 #pragma unroll
-  for (int p = 0; p < NR; ++p) x[p] = piece(p);
+    for (int p = 0; p < NR; ++p) {
+      const int d = (p0 + p) * 256 + lane * 4;
+      f32x4 v = x[p];
 #pragma unroll
-  for (int p = 0; p < NR; ++p) top(x[p]);
-  for (int p = NR; p * 256 < D; ++p) top(piece(p));
-  if (__ballot(!held) != 0) {  // uniform
-    if (lane == 0) meta[1] = 1;
-    return;
+      for (int i = 0; i < 4; ++i) {
+        const float y = fabsf(v[i]);
+        held &= y == 0.0f || (y >= PART_MIN && y < PART_MAX);
+      }
+      if (d < Dp) {
+#pragma unroll
+        for (int q = 0; q < N_PARTS; ++q) {
+          const bf16x4 b4 = __builtin_convertvector(v, bf16x4);
+          *(bf16x4*)(dst + q * Dp + d) = b4;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] -= (float)b4[i];
+        }
+      }
+    }
   }
-  m = wave_max(m);
-  int e = 15;  // m = f 2^e, 1/2 <= f < 1: the scale is 2^(15 - e)
-  if (m > 0.0f) (void)frexpf(m, &e);
-  if (lane == 0) *exp = e - 15;
-  auto put = [&](int p, const f32x4& v) {
-    const int d = p * 256 + lane * 4;
-    if (d >= Dp) return;
-    f16x4 hi, lo;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float y = __builtin_amdgcn_ldexpf(v[i], 15 - e);
-      hi[i] = (f16)y;
-      lo[i] = (f16)(y - (float)hi[i]);
-    }
-    *(f16x4*)(dst + d) = hi;
-    *(f16x4*)(dst + Dp + d) = lo;
-  };
-#pragma unroll
-  for (int p = 0; p < NR; ++p) put(p, x[p]);
-  for (int p = NR; p * 256 < Dp; ++p) put(p, piece(p));
+  if (__ballot(!held) != 0 && lane == 0) meta[1] = 1;
 }
 
 // ---- fixup ------------------------------------------------------------------------
@@ -1731,55 +1681,51 @@ static int64_t persistent_grid(int64_t n_units_max) {
   return std::min<int64_t>(g, n_units_max);
 }
 
-// The fp16 pairs of an fp32 launch, carved from the workspace after Work.
-struct Pairs {
-  PairRows h, w;
+// The bf16 parts of an fp32 launch, carved from the workspace after Work.
+struct Parts {
+  bf16 *h, *w;  // [rows][N_PARTS][Dp]
   int64_t Dp;
   size_t total;
 };
-// When fp32 batches take the pairs (whole forward, fp32 MFMAs -> pairs, one box): the split
-// passes over W cost what the fp32 MFMAs of about 100 rows do, so every batch past the
-// small-batch kernel gains (V = 30522, D = 768: 130 rows 139 -> 84 us, 1024 rows 414 -> 160 us,
-// 4096 rows 1162 -> 414 us), except where W is larger than the MALL holds beside its pairs
-// (140 rows, W of 983 MB: 727 -> 761 us; 512 rows, 614 MB: 1402 -> 682 us) or rows are narrow
-// (1024 rows, D = 64: 53 -> 56 us; D = 384: 112 -> 63 us).
-constexpr int64_t PAIR_MIN_D = 128;
-constexpr int64_t PAIR_W_BYTES = (int64_t)128 << 20, PAIR_BIG_W_ROWS = 256;
-static bool pairs_fit(int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
-  const int64_t Dp = round_up(D, SLAB / 2), n_mt_max = cdiv(B * cdiv(S, GROUP), NGRP);
-  return dtype == SPARTON_F32 && D >= PAIR_MIN_D && B * S > SMALL_MAX_ROWS &&
-         (V * D * 4 <= PAIR_W_BYTES || B * S >= PAIR_BIG_W_ROWS) &&
-         n_mt_max * BM * Dp * 4 < ((int64_t)1 << 31) && BN * Dp * 4 < ((int64_t)1 << 31);
+// When fp32 batches take the parts (whole forward, fp32 MFMAs -> parts, one box): splitting W costs
+// what the fp32 MFMAs of about 100 rows do (V = 30522, D = 768: 130 rows 141 -> 133 us, 200 rows
+// 184 -> 137, 512 rows 220 -> 164, 1024 rows 404 -> 262, 8192 rows 2890 -> 1648), more where the
+// parts of W do not stay in the MALL (V = 250002, D = 768: 256 rows 822 -> 871 us, 512 rows
+// 1608 -> 1237), and less is to be had from narrow rows (1024 rows, D = 128: 82 -> 67 us).
+constexpr int64_t PARTS_MIN_D = 128, PARTS_MIN_ROWS = 192;
+constexpr int64_t PARTS_W_BYTES = (int64_t)128 << 20, PARTS_BIG_W_ROWS = 257;
+static bool parts_fit(int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
+  const int64_t row = round_up(D, SLAB / 2) * N_PARTS * 2, n_mt_max = cdiv(B * cdiv(S, GROUP), NGRP);
+  return dtype == SPARTON_F32 && D >= PARTS_MIN_D && B * S >= PARTS_MIN_ROWS &&
+         (V * D * 4 <= PARTS_W_BYTES || B * S >= PARTS_BIG_W_ROWS) &&
+         n_mt_max * BM * row < ((int64_t)1 << 31) && BN * row < ((int64_t)1 << 31);
 }
-static Pairs carve_pairs(void* base, int64_t B, int64_t S, int64_t D, int64_t V) {
-  const int64_t n = cdiv(B * cdiv(S, GROUP), NGRP) * BM;
+static Parts carve_parts(void* base, int64_t B, int64_t S, int64_t D, int64_t V) {
   char* p = (char*)base;
-  Pairs x;
+  Parts x;
   x.Dp = round_up(D, SLAB / 2);
   size_t off = 0;
-  auto take = [&](int64_t bytes) {
+  auto take = [&](int64_t rows) {
     const size_t o = off;
-    off += (size_t)round_up(bytes, 256);
-    return p != nullptr ? p + o : nullptr;
+    off += (size_t)round_up(rows * N_PARTS * x.Dp * 2, 256);
+    return p != nullptr ? (bf16*)(p + o) : nullptr;
   };
-  x.h.hi_lo = (f16*)take(n * x.Dp * 4);
-  x.h.exp = (int*)take(n * 4);
-  x.w.hi_lo = (f16*)take(V * x.Dp * 4);
-  x.w.exp = (int*)take(V * 4);
+  x.h = take(cdiv(B * cdiv(S, GROUP), NGRP) * BM);
+  x.w = take(V);
   x.total = off;
   return x;
 }
 
 // ev_main: if non-null, two events recorded on `stream` just before and after the main
-// kernel (profiling).
+// kernel, and the split of fp32 operands before it (profiling).
 // split: fp32 products as bf16 hi/lo parts (SPARTON_F32_SPLIT) in the small-batch kernel;
-// the main kernel keeps fp32's precision either way. pairs: where its fp16 pairs lie, or null
+// the main kernel keeps fp32's precision either way. parts: where its bf16 parts lie, or null
 // for the fp32 MFMAs.
 template <typename T>
 static int launch(const void* H, const void* W, const void* bias, const void* mask,
                   int mask_dtype, void* reps, int32_t* argmax, float* reps_f32, int64_t B,
                   int64_t S, int64_t D, int64_t V, const Work& w, hipStream_t stream,
-                  hipEvent_t* ev_main, bool split, const Pairs* pairs) {
+                  hipEvent_t* ev_main, bool split, const Parts* parts) {
   const int64_t ngrp = cdiv(S, GROUP);
   const int64_t n_vt = cdiv(V, BN);
   const int64_t n_mt_max = cdiv(B * ngrp, NGRP);
@@ -1821,26 +1767,23 @@ static int launch(const void* H, const void* W, const void* bias, const void* ma
                        0, stream, mask, mask_dtype, (int)S, (int)ngrp, (const int*)w.meta,
                        (const int*)w.list, w.rowmask);
   }
-  if (pairs != nullptr)
-    hipLaunchKernelGGL(fwd_split_rows_kernel, dim3((unsigned)cdiv(V + n_mt_max * BM, 4)), dim3(256), 0,
-                       stream, (const float*)H, (const float*)W, pairs->h, pairs->w, (int)S, (int)D,
-                       (int)pairs->Dp, (int)V, (int)ngrp, w.meta, (const int*)w.list);
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[0], stream);
   if (grid > 0) {  // S == 0: no blocks, the fixup writes every row
     if constexpr (sizeof(T) == 4) {
-      if (pairs != nullptr)
-        hipLaunchKernelGGL((sparton_fwd_kernel<f16, float, true>), dim3((unsigned)grid), dim3(NTHREADS), 0,
-                           stream, (const f16*)pairs->h.hi_lo, (const f16*)pairs->w.hi_lo,
-                           (const float*)bias, (const float*)w.rowmask, (float*)reps, argmax, reps_f32,
-                           (int)S, (int)pairs->Dp, (int)V, (int)n_vt, (int)ngrp, (const int*)w.meta,
-                           (const int*)w.list, w.part, (const int*)pairs->h.exp,
-                           (const int*)pairs->w.exp, 0);
+      if (parts != nullptr) {
+        hipLaunchKernelGGL(fwd_split_rows_kernel, dim3((unsigned)cdiv(V + n_mt_max * BM, 4)), dim3(256), 0,
+                           stream, (const float*)H, (const float*)W, parts->h, parts->w, (int)S, (int)D,
+                           (int)parts->Dp, (int)V, (int)ngrp, w.meta, (const int*)w.list);
+        hipLaunchKernelGGL((sparton_fwd_kernel<bf16, float, true>), dim3((unsigned)grid), dim3(NTHREADS), 0,
+                           stream, (const bf16*)parts->h, (const bf16*)parts->w, (const float*)bias,
+                           (const float*)w.rowmask, (float*)reps, argmax, reps_f32, (int)S, (int)parts->Dp,
+                           (int)V, (int)n_vt, (int)ngrp, (const int*)w.meta, (const int*)w.list, w.part, 0);
+      }
     }
     hipLaunchKernelGGL((sparton_fwd_kernel<T, T, false>), dim3((unsigned)grid), dim3(NTHREADS), 0, stream,
                        (const T*)H, (const T*)W, (const T*)bias, (const float*)w.rowmask, (T*)reps,
                        argmax, reps_f32, (int)S, (int)D, (int)V, (int)n_vt, (int)ngrp,
-                       (const int*)w.meta, (const int*)w.list, w.part, nullptr, nullptr,
-                       pairs != nullptr ? 1 : 0);
+                       (const int*)w.meta, (const int*)w.list, w.part, parts != nullptr ? 1 : 0);
   }
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[1], stream);
   hipLaunchKernelGGL(fwd_fixup_kernel<T>, dim3((unsigned)cdiv(V, FIX_COLS), (unsigned)B), dim3(256), 0,
@@ -1875,7 +1818,7 @@ static int64_t mask_elem_bytes(int mask_dtype) {
 
 using namespace sparton;
 
-// Workspace without the fp16 pairs of fp32 operands: the plan and the partials.
+// Workspace without the parts of fp32 operands: the plan and the partials.
 static size_t plan_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
   if (B <= 0 || S < 0 || D < 0 || V <= 0) return 0;
   const int64_t esz = (dtype & ~SPARTON_F32_SPLIT) == SPARTON_F32 ? 4 : 2;
@@ -1885,8 +1828,8 @@ static size_t plan_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t V, i
 extern "C" __attribute__((visibility("default"))) size_t sparton_fwd_workspace_bytes(
     int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
   size_t n = plan_workspace_bytes(B, S, D, V, dtype);
-  if (n > 0 && fwd::pairs_fit(B, S, D, V, dtype & ~SPARTON_F32_SPLIT))
-    n += fwd::carve_pairs(nullptr, B, S, D, V).total;
+  if (n > 0 && fwd::parts_fit(B, S, D, V, dtype & ~SPARTON_F32_SPLIT))
+    n += fwd::carve_parts(nullptr, B, S, D, V).total;
   return n;
 }
 
@@ -1926,10 +1869,10 @@ static int fwd_run(const void* hidden, const void* weight, const void* bias, con
   hipStream_t st = (hipStream_t)stream;
   const int64_t Bc = fwd::rows_per_launch(B, S, D, esz);
   // A workspace that holds the plan only (sparton_fwd_noalloc's) keeps the fp32 MFMAs.
-  const bool use_pairs = fwd::pairs_fit(B, S, D, V, dtype) && Bc >= B &&
+  const bool use_parts = fwd::parts_fit(B, S, D, V, dtype) && Bc >= B &&
                          workspace_bytes >= sparton_fwd_workspace_bytes(B, S, D, V, dtype);
-  fwd::Pairs pairs{};
-  if (use_pairs) pairs = fwd::carve_pairs((char*)workspace + need, B, S, D, V);
+  fwd::Parts parts{};
+  if (use_parts) parts = fwd::carve_parts((char*)workspace + need, B, S, D, V);
   for (int64_t b0 = 0; b0 < B; b0 += Bc) {
     const int64_t nb = std::min(Bc, B - b0);
     const fwd::Work w = fwd::carve(workspace, nb, S, V);
@@ -1956,7 +1899,7 @@ static int fwd_run(const void* hidden, const void* weight, const void* bias, con
         break;
       default:
         rc = fwd::launch<float>(h, weight, bias, mk, mask_dtype, r, am, r32, nb, S, D, V, w, st, evp, split,
-                                use_pairs ? &pairs : nullptr);
+                                use_parts ? &parts : nullptr);
         break;
     }
     if (main_ms != nullptr) {

@@ -1006,8 +1006,8 @@ def test_fp32_split_precision(case, device):
         assert not torch.equal(r32, exact[2])
 
 
-def _fwd_capi_fp32(H, W, b, m, pairs):
-    """sparton_fwd on fp32 device tensors: with the whole workspace (fp16 pairs where the size
+def _fwd_capi_fp32(H, W, b, m, parts):
+    """sparton_fwd on fp32 device tensors: with the whole workspace (bf16 parts where the size
     takes them), or one byte less (the fp32 MFMAs)."""
     B, S, D = H.shape
     V = W.shape[0]
@@ -1018,24 +1018,25 @@ def _fwd_capi_fp32(H, W, b, m, pairs):
     idx = torch.empty((B, V), dtype=torch.int32, device=H.device)
     rc = L.sparton_fwd(H.data_ptr(), W.data_ptr(), _lib.ptr(b), m.data_ptr(), _lib.MASK_CODE[m.dtype],
                        reps.data_ptr(), idx.data_ptr(), None, B, S, D, V, 0, ws.data_ptr(),
-                       n if pairs else n - 1, torch.cuda.current_stream().cuda_stream)
+                       n if parts else n - 1, torch.cuda.current_stream().cuda_stream)
     assert rc == 0, L.sparton_strerror(rc)
     torch.cuda.synchronize()
     return reps, idx
 
 
 @pytest.mark.parametrize("case,spread", [
-    (("fp32", 1, 129, 128, 300, True, "int64"), 0),     # the fewest rows and columns that take pairs
+    (("fp32", 1, 192, 128, 300, True, "int64"), 0),     # the fewest rows and columns that take parts
     (("fp32", 3, 70, 132, 900, False, "frac"), 0),      # a padded last slab, fractional mask
     (("fp32", 8, 64, 772, 257, True, "holes"), 2),      # rows and elements of very different size
-    (("fp32", 2, 100, 1540, 515, True, "bool"), 2),     # rows longer than the split keeps in registers
+    (("fp32", 2, 100, 1540, 515, True, "bool"), 2),     # rows longer than the split loads at once
     (("fp32", 40, 30, 256, 1000, True, "gaps"), 0),     # rows with no active position
 ], ids=lambda c: "-".join(map(str, c)) if isinstance(c, tuple) else f"spread{c}")
-def test_fp32_pairs_precision(case, spread, device):
-    """fp32 batches past 128 positions run as pairs of fp16 (hi + lo, three products): against
+def test_fp32_parts_precision(case, spread, device):
+    """fp32 batches from 192 positions on run as bf16 parts (three, six products): against
     the oracle like any fp32 forward, and no further from 64 bits than the fp32 MFMAs. Both
-    errors are dominated by the keys' 2^-18, so theirs may differ by a tenth either way."""
-    say(f"fp32 pairs, case {case}, spread {spread}")
+    errors are dominated by the keys' 2^-18, so theirs may differ by a tenth either way (the next
+    test's are not)."""
+    say(f"fp32 parts, case {case}, spread {spread}")
     H, W, b, m, _ = make_case(*case)
     if spread:
         g = torch.Generator().manual_seed(3)
@@ -1044,23 +1045,54 @@ def test_fp32_pairs_precision(case, spread, device):
     Hd, Wd, md = H.to(device), W.to(device), m.to(device)
     bd = None if b is None else b.to(device)
     err = []
-    for pairs in (True, False):
-        reps, idx = _fwd_capi_fp32(Hd, Wd, bd, md, pairs)
+    for parts in (True, False):
+        reps, idx = _fwd_capi_fp32(Hd, Wd, bd, md, parts)
         check_fwd(H, W, b, m, reps, idx)
         x = torch.einsum("bsd,vd->bsv", H.double(), W.double())
         if b is not None:
             x = x + b.double()
         want = torch.log1p((x * m.double()[..., None]).amax(1).clamp_min(0.0))
         err.append(float((reps.cpu().double() - want).norm() / want.norm()))
-    say(f"  error against 64 bits: pairs {err[0]:.3g}, fp32 MFMAs {err[1]:.3g}")
+    say(f"  error against 64 bits: parts {err[0]:.3g}, fp32 MFMAs {err[1]:.3g}")
     assert err[0] <= 1.1 * err[1]
 
 
-def test_fp32_pairs_infinite_and_extreme_entries(device):
-    """Infinite entries, and rows at the ends of fp32's range, in a batch that runs as fp16
-    pairs: the fp32 MFMAs' reps, infinities and NaNs included, as long as no product has both
-    operands infinite."""
-    say("fp32 pairs with infinite and extreme entries")
+@pytest.mark.parametrize("what", ["outlier", "weight outlier", "cancel"])
+def test_fp32_parts_past_the_keys(what, device):
+    """Inputs where a lost bit shows past the keys' 2^-18: a hidden (or weight) column 2^28 times
+    the rest whose partners are 0, and logits 2^-12 of their products' magnitudes. Within the bound of
+    the fp32 MFMAs' order (D / 2 accumulations of 2^-24 of the sum of magnitudes), and no further
+    from 64 bits than they are, up to a tenth."""
+    say(f"fp32 parts, {what}")
+    g = torch.Generator().manual_seed(31)
+    B, S, D, V = 2, 96, 256, 700
+    H, W = torch.randn(B, S, D, generator=g), torch.randn(V, D, generator=g) * 0.02
+    if what == "outlier":
+        H[..., 7], W[:, 7] = 2.0 ** 28, 0.0
+    elif what == "weight outlier":
+        W[:, 9], H[..., 9] = 2.0 ** 28, 0.0
+    else:
+        H[..., D // 2:] = H[..., :D // 2]
+        W[:, D // 2:] = -W[:, :D // 2] * (1 + 2.0 ** -12 * torch.randn(V, D // 2, generator=g))
+    m = torch.ones(B, S, dtype=torch.int64)
+    x = torch.einsum("bsd,vd->bsv", H.double(), W.double())
+    top = x.amax(1).clamp_min(0.0)
+    mag = torch.einsum("bsd,vd->bsv", H.abs().double(), W.abs().double()).amax(1)
+    err = []
+    for parts in (True, False):
+        reps, _ = _fwd_capi_fp32(H.to(device), W.to(device), None, m.to(device), parts)
+        e = reps.cpu().double() - torch.log1p(top)
+        bound = 2.0 ** -18 * top + D / 2 * 2.0 ** -24 * mag + 2.0 ** -21 * torch.log1p(top)
+        assert bool((e.abs() <= bound).all()), float((e.abs() / bound).max())
+        err.append(float(e.norm() / torch.log1p(top).norm()))
+    say(f"  error against 64 bits: parts {err[0]:.3g}, fp32 MFMAs {err[1]:.3g}")
+    assert err[0] <= 1.1 * err[1]
+
+
+def test_fp32_parts_infinite_and_extreme_entries(device):
+    """Infinite entries, and rows at the ends of fp32's range, in a batch of a size that runs as
+    bf16 parts: the fp32 MFMAs' reps, infinities and NaNs included."""
+    say("fp32 parts, infinite and extreme entries")
     g = torch.Generator().manual_seed(22)
     B, S, D, V = 3, 64, 256, 700
     H = torch.randn(B, S, D, generator=g)
@@ -1092,12 +1124,13 @@ def test_fp32_pairs_infinite_and_extreme_entries(device):
     torch.testing.assert_close(r_p[same], r_e[same], rtol=2e-5, atol=1e-30)
 
 
-@pytest.mark.parametrize("where", ["tiny", "both", "nan", "weight", "padding"])
-def test_fp32_large_batch_nonfinite_entries(where, device):
-    """An infinite or NaN entry in an fp32 batch past the small-batch kernel: reps and argmax are the
-    fp32 MFMAs', bit for bit, whatever it meets: a finite partner far below its row's largest
-    (an infinity times it is infinite), another infinity, or a position the mask leaves out."""
-    say(f"fp32 large batch, entries that are not finite: {where}")
+@pytest.mark.parametrize("where", ["tiny", "both", "nan", "weight", "padding", "small", "large"])
+def test_fp32_large_batch_entries_without_parts(where, device):
+    """An entry that bf16 parts do not hold, in an fp32 batch past the small-batch kernel: reps and
+    argmax are the fp32 MFMAs', bit for bit. Infinities and NaN, whatever they meet: a finite
+    partner far below its row's largest (an infinity times it is infinite), another infinity, or
+    a position that the mask leaves out; a value under 2^-50, or of 2^48."""
+    say(f"fp32 large batch, entries without parts: {where}")
     g = torch.Generator().manual_seed(23)
     B, S, D, V = 3, 64, 256, 700
     H, W = torch.randn(B, S, D, generator=g), torch.randn(V, D, generator=g) * 0.02
@@ -1112,6 +1145,12 @@ def test_fp32_large_batch_nonfinite_entries(where, device):
         H[2, 63, 255] = float("nan")
     elif where == "weight":
         W[699, 255], H[..., 255] = inf, 1e-20
+    elif where == "small":
+        H[..., 4:] = 0.0
+        H[1, 2] *= 2.0 ** -118
+        W *= 2.0 ** 40
+    elif where == "large":
+        W[300, 255] = 2.0 ** 48
     else:
         H[1, 25, 3], W[:, 3] = inf, 1e-20
     Hd, Wd, md = H.to(device), W.to(device), m.to(device)
