@@ -78,13 +78,19 @@ enum sparton_status {
 /*
  * Bytes of device scratch sparton_fwd needs for these sizes (256-byte aligned
  * sections: the per-row block plan, the partial results of batch rows whose
- * positions span several row tiles, and for larger fp32 batches (B*S >= 192) H and W
- * as three bf16 parts, on whose MFMAs such a batch runs; given less than these bytes but
+ * positions span several row tiles, and for larger fp32 batches (from B*S = 192 on) H
+ * and W as three bf16 parts, a range of columns at a time, on whose MFMAs such a batch runs; given less than these bytes but
  * enough for the rest, it runs on the fp32 MFMAs instead, as do operands with a nonzero
  * magnitude outside [2^-50, 2^48), infinities and NaN among them). No counterpart in the reference: its forward
  * materializes a [B,S,C] logits tile per vocab tile instead (sparton_kernel.py:245-247).
  */
 size_t sparton_fwd_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t V, int dtype);
+
+/*
+ * The same without the bf16 parts, which take up to 512 MiB each for H's rows and for W: the least
+ * that sparton_fwd takes.
+ */
+size_t sparton_fwd_workspace_min_bytes(int64_t B, int64_t S, int64_t D, int64_t V, int dtype);
 
 /*
  * Forward: reps[B,V] (in `dtype`) and argmax I[B,V] (int32).

@@ -44,6 +44,7 @@ EXPORTED_SYMBOLS = (
     "sparton_fwd",
     "sparton_fwd_profile",
     "sparton_fwd_workspace_bytes",
+    "sparton_fwd_workspace_min_bytes",
     "sparton_fwd_noalloc",
     "sparton_fwd_noalloc_max_workspace",
     "sparton_bwd",
@@ -102,8 +103,9 @@ def load() -> ctypes.CDLL:
         L.sparton_fwd_noalloc.restype = ctypes.c_int
         L.sparton_fwd_noalloc_max_workspace.argtypes = []
         L.sparton_fwd_noalloc_max_workspace.restype = ctypes.c_size_t
-        L.sparton_fwd_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, ctypes.c_int]
-        L.sparton_fwd_workspace_bytes.restype = ctypes.c_size_t
+        for size in (L.sparton_fwd_workspace_bytes, L.sparton_fwd_workspace_min_bytes):
+            size.argtypes = [_i64, _i64, _i64, _i64, ctypes.c_int]
+            size.restype = ctypes.c_size_t
         L.sparton_bwd.argtypes = [_vp, _vp, ctypes.c_int, _vp, _vp, ctypes.c_int, _vp, _vp, _vp,
                                   _vp, _vp, ctypes.c_int, _vp, ctypes.c_size_t, _i64, _i64, _i64,
                                   _i64, ctypes.c_int, _vp]

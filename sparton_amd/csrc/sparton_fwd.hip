@@ -612,6 +612,8 @@ struct Args {
   int nk;             // slabs per unit
   int V;
   int part_bytes;     // PARTS: bytes of one part of a row
+  int v_beg;          // PARTS: the launch's first column
+  __device__ __forceinline__ int first() const { return PARTS ? v_beg : 0; }
   // Byte offsets of K slab k in a row of A and of W. A product of PARTS runs over K six times,
   // smallest first: A's parts 2 0 1 1 0 0 with W's 0 2 1 0 1 0.
   __device__ __forceinline__ void slab_at(int k, uint32_t* ka, uint32_t* kb) const {
@@ -797,7 +799,7 @@ struct Unit {
   int u, m, v0, n_valid;
 };
 __device__ __forceinline__ Unit unit_of(int w, int r, int G, int n_units, int n_mt, int n_vt,
-                                        int n_grp) {
+                                        int n_grp, int v_beg) {
   Unit x;
   x.u = unit_at(w, r, G, n_units);
   x.m = 0;
@@ -806,7 +808,7 @@ __device__ __forceinline__ Unit unit_of(int w, int r, int G, int n_units, int n_
   if (x.u >= 0) {
     int vt;
     unit_tile(x.u, n_mt, n_vt, &x.m, &vt);
-    x.v0 = vt * BN;
+    x.v0 = v_beg + vt * BN;
     x.n_valid = min(NGRP, n_grp - x.m * NGRP);
   }
   return x;
@@ -923,7 +925,7 @@ template <typename T, typename O, bool PARTS>
 __device__ void copy_path(Smem& sm, const Args<T, O, PARTS>& a, const Outputs<O>& o, int w, int G,
                           int n_units, int n_mt, int n_vt, int ct, int c, int lane) {
   const int nk = a.nk;
-  Unit cur = unit_of(w, 0, G, n_units, n_mt, n_vt, a.n_grp);
+  Unit cur = unit_of(w, 0, G, n_units, n_mt, n_vt, a.n_grp, a.first());
   if (cur.u < 0) return;
   Unit prev;
   prev.u = -1;
@@ -951,7 +953,7 @@ __device__ void copy_path(Smem& sm, const Args<T, O, PARTS>& a, const Outputs<O>
     }
     return mr;
   };
-  Unit next = unit_of(w, 1, G, n_units, n_mt, n_vt, a.n_grp);
+  Unit next = unit_of(w, 1, G, n_units, n_mt, n_vt, a.n_grp, a.first());
   MetaRegs meta = load_meta(next);
   for (int r = 1;; ++r) {
     const bool pre = next.u >= 0 && nk >= PREFETCH_MIN_NK;
@@ -1000,7 +1002,7 @@ __device__ void copy_path(Smem& sm, const Args<T, O, PARTS>& a, const Outputs<O>
     if (pre) issue_slab(sm, a, nx, 1, buf_next ^ 1, c, lane);
     // the unit after next, worked out while the compute waves run their epilogue, and its
     // metadata loads
-    const Unit next2 = next.u >= 0 ? unit_of(w, r + 1, G, n_units, n_mt, n_vt, a.n_grp) : next;
+    const Unit next2 = next.u >= 0 ? unit_of(w, r + 1, G, n_units, n_mt, n_vt, a.n_grp, a.first()) : next;
     if (pre) meta = load_meta(next2);
     lds_barrier();  // E: the compute waves' keys are written
     if (next.u < 0) {
@@ -1195,7 +1197,7 @@ __device__ void compute_path(Smem& sm, const Args<T, O, PARTS>& a, int w, int G,
                              int n_vt, int wave, int lane) {
   const int nk = a.nk;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  Unit cur = unit_of(w, 0, G, n_units, n_mt, n_vt, a.n_grp);
+  Unit cur = unit_of(w, 0, G, n_units, n_mt, n_vt, a.n_grp, a.first());
   if (cur.u < 0) return;
   lds_barrier();  // S1
   lds_barrier();  // S2
@@ -1211,7 +1213,7 @@ __device__ void compute_path(Smem& sm, const Args<T, O, PARTS>& a, int w, int G,
       case 3: compute_unit<T, 3>(sm, um, nk, buf, lane, wm, wn); break;
       default: compute_unit<T, 4>(sm, um, nk, buf, lane, wm, wn); break;
     }
-    const Unit next = unit_of(w, r, G, n_units, n_mt, n_vt, a.n_grp);
+    const Unit next = unit_of(w, r, G, n_units, n_mt, n_vt, a.n_grp, a.first());
     if (next.u < 0) return;
     if (nk < PREFETCH_MIN_NK) {
       lds_barrier();  // S1
@@ -1229,7 +1231,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
     const float* __restrict__ rowmask, O* __restrict__ reps, int32_t* __restrict__ argmax,
     float* __restrict__ reps_f32, int S, int D, int V, int n_vt, int ngrp,
     const int* __restrict__ meta, const int* __restrict__ list, float2* __restrict__ part,
-    int only_unheld) {
+    int v_beg, int only_unheld) {
   __shared__ Smem sm;
   // fp32 operands: the launch on parts or, after it, the one on the values, as the split found.
   if constexpr (PARTS) {
@@ -1255,6 +1257,8 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
     a.part_bytes = D * (int)sizeof(T);
     a.row_bytes = N_PARTS * a.part_bytes;
     a.nk_full = a.nk = PART_RUNS * (D / slab_elems);
+    a.v_beg = v_beg;
+    a.W -= (int64_t)v_beg * a.row_bytes;  // the parts' first row is column v_beg's
   } else {
     a.part_bytes = 0;
     a.row_bytes = D * (int)sizeof(T);
@@ -1286,30 +1290,31 @@ __global__ __launch_bounds__(NTHREADS, 1) void sparton_fwd_kernel(
 // fp32 MFMA's takes D / 2, so its bound is the smaller of the two. bf16 has fp32's exponents, so
 // no element loses bits to a larger one.
 // Error of reps against 64 bits, fp32 MFMAs -> parts (2-norm relative; the keys' 18 bits
-// included): 8 x 128 x 768 x 30522 normal 1.14e-6 -> 1.12e-6; logits 2^-12 of their products
-// 4.7e-4 -> 1.4e-4. Bound by the bf16 MFMAs at six products per value: 1.4 PFLOP/s at 8192 rows.
+// included), 192 rows, D = 384, V = 700: with a column 2^28 times the rest, its partners 0, 1.19e-6
+// -> 1.18e-6; with logits 2^-12 of their products 5.7e-4 -> 1.7e-4. Bound by the bf16 MFMAs at six
+// products per value: 1.4 PFLOP/s at 8192 rows (D = 768, V = 30522, the split included).
 // What that takes: |x| in [2^-50, 2^48) or 0. Then every part is a normal bf16, every product that
 // counts a normal fp32, and no sum of parts overflows where the values' would not. A value outside
 // (infinities, NaN) raises meta[1]: the launch on parts ends at once and one on the fp32 MFMAs,
 // which ends at once otherwise, follows.
 constexpr float PART_MIN = 0x1p-50f, PART_MAX = 0x1p48f;
 
-// One wave per row of W (rows 0 .. V - 1), then per row of H's tiles, in tile order (row t of
+// One wave per row of W (n_w of them), then per row of H's tiles (n_h), in tile order (row t of
 // group list[t / 16]; rows past the last active group are left out). Out: [row][part][Dp].
 __global__ __launch_bounds__(256) void fwd_split_rows_kernel(
     const float* __restrict__ H, const float* __restrict__ W, bf16* __restrict__ hp,
-    bf16* __restrict__ wp, int S, int D, int Dp, int V, int ngrp, int* meta,
+    bf16* __restrict__ wp, int S, int D, int Dp, int n_w, int n_h, int ngrp, int* meta,
     const int* __restrict__ list) {
   const int lane = threadIdx.x & 63;
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const float* src;
   bf16* dst;
-  if (r < V) {
+  if (r < n_w) {
     src = W + r * D;
     dst = wp + r * N_PARTS * Dp;
   } else {
-    const int64_t t = r - V;
-    if (t / GROUP >= meta[0]) return;
+    const int64_t t = r - n_w;
+    if (t >= n_h || t / GROUP >= meta[0]) return;
     const int code = list[t / GROUP], b = code / ngrp;
     const int s = min((code - b * ngrp) * GROUP + (int)(t % GROUP), S - 1);
     src = H + ((int64_t)b * S + s) * D;
@@ -1681,40 +1686,11 @@ static int64_t persistent_grid(int64_t n_units_max) {
   return std::min<int64_t>(g, n_units_max);
 }
 
-// The bf16 parts of an fp32 launch, carved from the workspace after Work.
+// The bf16 parts of an fp32 launch: H's rows, and W's vc rows at a time.
 struct Parts {
   bf16 *h, *w;  // [rows][N_PARTS][Dp]
-  int64_t Dp;
-  size_t total;
+  int64_t Dp, vc;
 };
-// When fp32 batches take the parts (whole forward, fp32 MFMAs -> parts, one box): splitting W costs
-// what the fp32 MFMAs of about 100 rows do (V = 30522, D = 768: 130 rows 141 -> 133 us, 200 rows
-// 184 -> 137, 512 rows 220 -> 164, 1024 rows 404 -> 262, 8192 rows 2890 -> 1648), more where the
-// parts of W do not stay in the MALL (V = 250002, D = 768: 256 rows 822 -> 871 us, 512 rows
-// 1608 -> 1237), and less is to be had from narrow rows (1024 rows, D = 128: 82 -> 67 us).
-constexpr int64_t PARTS_MIN_D = 128, PARTS_MIN_ROWS = 192;
-constexpr int64_t PARTS_W_BYTES = (int64_t)128 << 20, PARTS_BIG_W_ROWS = 257;
-static bool parts_fit(int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
-  const int64_t row = round_up(D, SLAB / 2) * N_PARTS * 2, n_mt_max = cdiv(B * cdiv(S, GROUP), NGRP);
-  return dtype == SPARTON_F32 && D >= PARTS_MIN_D && B * S >= PARTS_MIN_ROWS &&
-         (V * D * 4 <= PARTS_W_BYTES || B * S >= PARTS_BIG_W_ROWS) &&
-         n_mt_max * BM * row < ((int64_t)1 << 31) && BN * row < ((int64_t)1 << 31);
-}
-static Parts carve_parts(void* base, int64_t B, int64_t S, int64_t D, int64_t V) {
-  char* p = (char*)base;
-  Parts x;
-  x.Dp = round_up(D, SLAB / 2);
-  size_t off = 0;
-  auto take = [&](int64_t rows) {
-    const size_t o = off;
-    off += (size_t)round_up(rows * N_PARTS * x.Dp * 2, 256);
-    return p != nullptr ? (bf16*)(p + o) : nullptr;
-  };
-  x.h = take(cdiv(B * cdiv(S, GROUP), NGRP) * BM);
-  x.w = take(V);
-  x.total = off;
-  return x;
-}
 
 // ev_main: if non-null, two events recorded on `stream` just before and after the main
 // kernel, and the split of fp32 operands before it (profiling).
@@ -1770,20 +1746,22 @@ static int launch(const void* H, const void* W, const void* bias, const void* ma
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[0], stream);
   if (grid > 0) {  // S == 0: no blocks, the fixup writes every row
     if constexpr (sizeof(T) == 4) {
-      if (parts != nullptr) {
-        hipLaunchKernelGGL(fwd_split_rows_kernel, dim3((unsigned)cdiv(V + n_mt_max * BM, 4)), dim3(256), 0,
-                           stream, (const float*)H, (const float*)W, parts->h, parts->w, (int)S, (int)D,
-                           (int)parts->Dp, (int)V, (int)ngrp, w.meta, (const int*)w.list);
-        hipLaunchKernelGGL((sparton_fwd_kernel<bf16, float, true>), dim3((unsigned)grid), dim3(NTHREADS), 0,
+      for (int64_t v = 0; parts != nullptr && v < V; v += parts->vc) {
+        const int64_t n_w = std::min(V - v, parts->vc), n_h = v == 0 ? n_mt_max * BM : 0, vts = cdiv(n_w, BN);
+        hipLaunchKernelGGL(fwd_split_rows_kernel, dim3((unsigned)cdiv(n_w + n_h, 4)), dim3(256), 0, stream,
+                           (const float*)H, (const float*)W + v * D, parts->h, parts->w, (int)S, (int)D,
+                           (int)parts->Dp, (int)n_w, (int)n_h, (int)ngrp, w.meta, (const int*)w.list);
+        hipLaunchKernelGGL((sparton_fwd_kernel<bf16, float, true>),
+                           dim3((unsigned)persistent_grid(n_mt_max * vts)), dim3(NTHREADS), 0,
                            stream, (const bf16*)parts->h, (const bf16*)parts->w, (const float*)bias,
                            (const float*)w.rowmask, (float*)reps, argmax, reps_f32, (int)S, (int)parts->Dp,
-                           (int)V, (int)n_vt, (int)ngrp, (const int*)w.meta, (const int*)w.list, w.part, 0);
+                           (int)V, (int)vts, (int)ngrp, (const int*)w.meta, (const int*)w.list, w.part, (int)v, 0);
       }
     }
     hipLaunchKernelGGL((sparton_fwd_kernel<T, T, false>), dim3((unsigned)grid), dim3(NTHREADS), 0, stream,
                        (const T*)H, (const T*)W, (const T*)bias, (const float*)w.rowmask, (T*)reps,
                        argmax, reps_f32, (int)S, (int)D, (int)V, (int)n_vt, (int)ngrp,
-                       (const int*)w.meta, (const int*)w.list, w.part, parts != nullptr ? 1 : 0);
+                       (const int*)w.meta, (const int*)w.list, w.part, 0, parts != nullptr ? 1 : 0);
   }
   if (ev_main != nullptr) (void)hipEventRecord(ev_main[1], stream);
   hipLaunchKernelGGL(fwd_fixup_kernel<T>, dim3((unsigned)cdiv(V, FIX_COLS), (unsigned)B), dim3(256), 0,
@@ -1801,6 +1779,41 @@ static int64_t rows_per_launch(int64_t B, int64_t S, int64_t D, int64_t esz) {
   const int64_t per_row = std::max<int64_t>(1, S * D * esz);
   const int64_t cap = std::min<int64_t>(MAX_ROWS_PER_LAUNCH, ((int64_t)1 << 31) / per_row);
   return std::max<int64_t>(1, std::min<int64_t>(B, cap));
+}
+
+// How an fp32 launch takes the parts: Bc batch rows and vc columns at a time, which bounds H's parts
+// and W's to PARTS_BYTES each whatever the sizes.
+// When it does (whole forward, fp32 MFMAs -> parts, one box): splitting W costs what the fp32 MFMAs
+// of about 100 rows do (V = 30522, D = 768: 130 rows 141 -> 133 us, 200 rows 184 -> 136, 512 rows
+// 225 -> 166, 1024 rows 399 -> 270, 8192 rows 2884 -> 1698), more where the parts of W do not stay
+// in the MALL (V = 250002, D = 768: 256 rows 822 -> 871 us, 300 rows 1610 -> 1218), and little work
+// leaves little to gain (1024 rows, D = 128: 85 -> 68 us; 512 rows 48 -> 53; 256 rows, D = 384:
+// 111 -> 80). Ranges of columns that leave a quarter of the chip idle would lose it again
+// (256 rows, D = 4096, V = 128256: 2148 -> 2746 us, ranges or not).
+struct PartsPlan {
+  bool fits;
+  int64_t Dp, Bc, vc, h_bytes, w_bytes;
+};
+constexpr int64_t PARTS_BYTES = (int64_t)512 << 20;
+constexpr int64_t PARTS_MIN_D = 128, PARTS_MIN_ROWS = 192, PARTS_MIN_H = 72 << 10;
+constexpr int64_t PARTS_W_BYTES = (int64_t)128 << 20, PARTS_BIG_W_ROWS = 257;
+static PartsPlan parts_plan(int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
+  PartsPlan p{};
+  if (dtype != SPARTON_F32 || D < PARTS_MIN_D || B * S < PARTS_MIN_ROWS || B * S * D < PARTS_MIN_H ||
+      (V * D * 4 > PARTS_W_BYTES && B * S < PARTS_BIG_W_ROWS))
+    return p;
+  p.Dp = round_up(D, SLAB / 2);
+  const int64_t row = p.Dp * N_PARTS * 2, ngrp = cdiv(S, GROUP);
+  if (BN * row >= ((int64_t)1 << 31)) return p;
+  p.Bc = std::min(rows_per_launch(B, S, D, 4), PARTS_BYTES / (row * BM) * NGRP / ngrp);
+  if (p.Bc < 1) return p;
+  const int64_t n_mt = cdiv(p.Bc * ngrp, NGRP), nv = cdiv(V * row, PARTS_BYTES);
+  p.vc = round_up(cdiv(V, nv), BN * GROUP_V);
+  p.h_bytes = round_up(n_mt * BM * row, 256);
+  p.w_bytes = round_up(std::min(V, p.vc) * row, 256);
+  const int64_t units = n_mt * (p.vc / BN), rounds = cdiv(units, 256);
+  p.fits = nv == 1 || 4 * units >= 3 * 256 * rounds;
+  return p;
 }
 
 static int64_t mask_elem_bytes(int mask_dtype) {
@@ -1827,10 +1840,15 @@ static size_t plan_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t V, i
 
 extern "C" __attribute__((visibility("default"))) size_t sparton_fwd_workspace_bytes(
     int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
-  size_t n = plan_workspace_bytes(B, S, D, V, dtype);
-  if (n > 0 && fwd::parts_fit(B, S, D, V, dtype & ~SPARTON_F32_SPLIT))
-    n += fwd::carve_parts(nullptr, B, S, D, V).total;
-  return n;
+  const size_t n = plan_workspace_bytes(B, S, D, V, dtype);
+  if (n == 0) return 0;
+  const fwd::PartsPlan p = fwd::parts_plan(B, S, D, V, dtype & ~SPARTON_F32_SPLIT);
+  return n + (p.fits ? (size_t)(p.h_bytes + p.w_bytes) : 0);
+}
+
+extern "C" __attribute__((visibility("default"))) size_t sparton_fwd_workspace_min_bytes(
+    int64_t B, int64_t S, int64_t D, int64_t V, int dtype) {
+  return plan_workspace_bytes(B, S, D, V, dtype);
 }
 
 // dtype: an enum sparton_dtype, or SPARTON_F32 | SPARTON_F32_SPLIT.
@@ -1848,7 +1866,7 @@ static int fwd_run(const void* hidden, const void* weight, const void* bias, con
                    size_t workspace_bytes, void* stream, float* main_ms) {
   if (B < 0 || S < 0 || D < 0 || V < 0) return SPARTON_EINVAL;
   if (!fwd_dtype_ok(dtype)) return SPARTON_EINVAL;
-  const bool split = (dtype & SPARTON_F32_SPLIT) != 0;
+  const bool split = (dtype & SPARTON_F32_SPLIT) != 0 && B * S <= fwd::SMALL_MAX_ROWS;  // of the whole batch
   dtype &= ~SPARTON_F32_SPLIT;
   if (mask_dtype < SPARTON_MASK_I64 || mask_dtype > SPARTON_MASK_F16) return SPARTON_EINVAL;
   if (B == 0 || V == 0) return SPARTON_OK;
@@ -1867,12 +1885,12 @@ static int fwd_run(const void* hidden, const void* weight, const void* bias, con
   if (workspace == nullptr || workspace_bytes < need) return SPARTON_EWORKSPACE;
   if ((uintptr_t)workspace % 256 != 0) return SPARTON_EALIGN;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t Bc = fwd::rows_per_launch(B, S, D, esz);
   // A workspace that holds the plan only (sparton_fwd_noalloc's) keeps the fp32 MFMAs.
-  const bool use_parts = fwd::parts_fit(B, S, D, V, dtype) && Bc >= B &&
-                         workspace_bytes >= sparton_fwd_workspace_bytes(B, S, D, V, dtype);
-  fwd::Parts parts{};
-  if (use_parts) parts = fwd::carve_parts((char*)workspace + need, B, S, D, V);
+  const fwd::PartsPlan pp = fwd::parts_plan(B, S, D, V, dtype);
+  const bool use_parts = pp.fits && workspace_bytes >= sparton_fwd_workspace_bytes(B, S, D, V, dtype);
+  const int64_t Bc = use_parts ? pp.Bc : fwd::rows_per_launch(B, S, D, esz);
+  const fwd::Parts parts{(bf16*)((char*)workspace + need), (bf16*)((char*)workspace + need + pp.h_bytes),
+                         pp.Dp, pp.vc};
   for (int64_t b0 = 0; b0 < B; b0 += Bc) {
     const int64_t nb = std::min(Bc, B - b0);
     const fwd::Work w = fwd::carve(workspace, nb, S, V);

@@ -112,8 +112,17 @@ FwdOut head_fwd(const Tensor& h, const Tensor& w, const Tensor& b, const Tensor&
   o.reps = at::empty({B, V}, h.options());
   if (with_idx) o.idx = at::empty({B, V}, h.options().dtype(at::kInt));
   if (with_f32) o.reps32 = at::empty({B, V}, h.options().dtype(at::kFloat));
-  const size_t ws_bytes = sparton_fwd_workspace_bytes(B, S, D, V, dt);
-  Tensor ws = workspace(ws_bytes, h);
+  size_t ws_bytes = sparton_fwd_workspace_bytes(B, S, D, V, dt);
+  Tensor ws;
+  try {
+    ws = workspace(ws_bytes, h);
+  } catch (const c10::OutOfMemoryError&) {
+    // the plan alone: larger fp32 batches then run without the bf16 parts of H and W
+    const size_t least = sparton_fwd_workspace_min_bytes(B, S, D, V, dt);
+    if (least == ws_bytes) throw;
+    ws_bytes = least;
+    ws = workspace(ws_bytes, h);
+  }
   check(sparton_fwd(h.data_ptr(), w.data_ptr(), ptr(b), m.data_ptr(), mask_code(m.scalar_type()),
                     o.reps.data_ptr(), with_idx ? o.idx.data_ptr<int32_t>() : nullptr,
                     with_f32 ? o.reps32.data_ptr<float>() : nullptr, B, S, D, V, dt, ws.data_ptr(),

@@ -87,7 +87,15 @@ def _fwd_impl(hidden: Tensor, embed: Tensor, bias: Optional[Tensor], mask: Tenso
     L = _lib.load()
     dt = _lib.fwd_dtype_code(hidden.dtype)
     ws_bytes = int(L.sparton_fwd_workspace_bytes(B, S, D, V, dt))
-    ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
+    try:
+        ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        # the plan alone: larger fp32 batches then run without the bf16 parts of H and W
+        least = int(L.sparton_fwd_workspace_min_bytes(B, S, D, V, dt))
+        if least == ws_bytes:
+            raise
+        ws_bytes = least
+        ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
         rc = L.sparton_fwd(hidden.data_ptr(), embed.data_ptr(), _lib.ptr(bias), mask.data_ptr(),
                            _lib.MASK_CODE[mask.dtype], reps.data_ptr(), _lib.ptr(idx),

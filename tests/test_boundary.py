@@ -118,6 +118,21 @@ def test_bwd_argument_validation(kw, code):
     assert bwd(**kw) == code
 
 
+@pytest.mark.parametrize("B,S,D,V", [(8, 128, 768, 30522), (16, 512, 4096, 128256), (32, 256, 1024, 250002),
+                                     (100000, 16, 768, 30522), (1, 400000, 1024, 1000), (4, 64, 87040, 10000)])
+def test_fwd_workspace_of_fp32_parts_is_bounded(B, S, D, V):
+    """The bf16 parts of an fp32 batch take six bytes for each of H's and W's elements (16-position
+    groups, K in slabs of 64), or 512 MiB for each of the two and no more, whatever the sizes;
+    16-bit batches and a plan without them take none."""
+    L = _lib.load()
+    full, least = (f(B, S, D, V, 0) for f in (L.sparton_fwd_workspace_bytes, L.sparton_fwd_workspace_min_bytes))
+    row = 6 * -(-D // 64) * 64
+    h, w = (-(-B * -(-S // 16) // 16) * 256 + 256) * row, (V + 1024) * row
+    assert 0 <= full - least <= min(h, 2 ** 29) + min(w, 2 ** 29) + 1024 * row + 512
+    assert L.sparton_fwd_workspace_bytes(B, S, D, V, 1) == L.sparton_fwd_workspace_min_bytes(B, S, D, V, 1)
+    assert L.sparton_fwd_workspace_bytes(B, S, D, V, 0x100) == full
+
+
 @pytest.mark.parametrize("B,S,V", [(65536, 8, 30522), (65536, 16, 1000), (10 ** 6, 1, 128), (100000, 8, 1000),
                                    (9000, 3, 64), (40, 8192, 300), (3, 500000, 70000)])
 def test_bwd_workspace_is_bounded_in_batch_rows(B, S, V):

@@ -1013,6 +1013,7 @@ def _fwd_capi_fp32(H, W, b, m, parts):
     V = W.shape[0]
     L = _lib.load()
     n = int(L.sparton_fwd_workspace_bytes(B, S, D, V, 0))
+    assert n > L.sparton_fwd_workspace_min_bytes(B, S, D, V, 0)  # a size that takes parts
     ws = torch.empty(n, dtype=torch.uint8, device=H.device)
     reps = torch.empty((B, V), dtype=torch.float32, device=H.device)
     idx = torch.empty((B, V), dtype=torch.int32, device=H.device)
@@ -1025,8 +1026,8 @@ def _fwd_capi_fp32(H, W, b, m, parts):
 
 
 @pytest.mark.parametrize("case,spread", [
-    (("fp32", 1, 192, 128, 300, True, "int64"), 0),     # the fewest rows and columns that take parts
-    (("fp32", 3, 70, 132, 900, False, "frac"), 0),      # a padded last slab, fractional mask
+    (("fp32", 1, 192, 384, 300, True, "int64"), 0),     # the fewest rows and values that take parts
+    (("fp32", 9, 70, 132, 900, False, "frac"), 0),      # a padded last slab, fractional mask
     (("fp32", 8, 64, 772, 257, True, "holes"), 2),      # rows and elements of very different size
     (("fp32", 2, 100, 1540, 515, True, "bool"), 2),     # rows longer than the split loads at once
     (("fp32", 40, 30, 256, 1000, True, "gaps"), 0),     # rows with no active position
@@ -1065,7 +1066,7 @@ def test_fp32_parts_past_the_keys(what, device):
     from 64 bits than they are, up to a tenth."""
     say(f"fp32 parts, {what}")
     g = torch.Generator().manual_seed(31)
-    B, S, D, V = 2, 96, 256, 700
+    B, S, D, V = 2, 96, 384, 700
     H, W = torch.randn(B, S, D, generator=g), torch.randn(V, D, generator=g) * 0.02
     if what == "outlier":
         H[..., 7], W[:, 7] = 2.0 ** 28, 0.0
@@ -1089,12 +1090,63 @@ def test_fp32_parts_past_the_keys(what, device):
     assert err[0] <= 1.1 * err[1]
 
 
+@pytest.mark.parametrize("B,S,V", [(4, 160, 720000), (1400, 512, 300)])
+def test_fp32_parts_in_ranges(B, S, V, device):
+    """fp32 batches whose bf16 parts are made a range of columns (or of batch rows) at a time: the fp32
+    MFMAs' reps, in every range. Two values may differ by the keys' 2^-17 and by the two sums'
+    roundings, D / 2 of 2^-24 of the sum of magnitudes each."""
+    say(f"fp32 parts in ranges, B={B} S={S} V={V}")
+    D = 128
+    g = torch.Generator(device=device).manual_seed(33)
+    H = torch.randn(B, S, D, generator=g, device=device)
+    W = torch.randn(V, D, generator=g, device=device) * D ** -0.5
+    m = (torch.arange(S, device=device)[None] < torch.randint(1, S + 1, (B, 1), generator=g, device=device)).long()
+    L = _lib.load()
+    extra = L.sparton_fwd_workspace_bytes(B, S, D, V, 0) - L.sparton_fwd_workspace_min_bytes(B, S, D, V, 0)
+    assert 0 < extra < 6 * D * (B * S + V)  # not all of them at once
+    r_p, i_p = _fwd_capi_fp32(H, W, None, m, True)
+    r_e, i_e = _fwd_capi_fp32(H, W, None, m, False)
+    mag = H.abs().amax() * W.abs().sum(1).amax()
+    assert bool(((r_p - r_e).abs() <= 2.0 ** -17 * r_e.expm1() + D * 2.0 ** -24 * mag).all())
+    assert float((i_p != i_e).float().mean()) < 1e-3
+
+
+def test_fp32_forward_without_room_for_parts(device):
+    """Where the allocator has no room for the bf16 parts, a forward that fits without them runs on
+    the fp32 MFMAs: through the torch op and through the eager one."""
+    say("fp32 forward without room for its parts")
+    from sparton_amd import _eager
+    H, W, b, m, _ = make_case("fp32", 4, 128, 1024, 60000, True, "int64")
+    Hd, Wd, bd, md = H.to(device), W.to(device), b.to(device), m.to(device)
+    want, _ = _fwd_capi_fp32(Hd, Wd, bd, md, False)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(device).total_memory
+    L = _lib.load()
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (256 << 20)) / total)
+        fill = []
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                fill.append(torch.empty(96 << 20, dtype=torch.uint8, device=device))
+        fill.pop()  # room for reps and the plan
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(L.sparton_fwd_workspace_bytes(4, 128, 1024, 60000, 0), dtype=torch.uint8, device=device)
+        reps, _ = torch.ops.sparton.fused_sparton_fwd(Hd, Wd, bd, md)
+        eager = _eager.load().head_encode(Hd, Wd, bd, md)
+    finally:
+        fill = None
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    torch.cuda.synchronize()
+    assert torch.equal(reps, want) and torch.equal(eager, want)
+
+
 def test_fp32_parts_infinite_and_extreme_entries(device):
     """Infinite entries, and rows at the ends of fp32's range, in a batch of a size that runs as
     bf16 parts: the fp32 MFMAs' reps, infinities and NaNs included."""
     say("fp32 parts, infinite and extreme entries")
     g = torch.Generator().manual_seed(22)
-    B, S, D, V = 3, 64, 256, 700
+    B, S, D, V = 3, 64, 384, 700
     H = torch.randn(B, S, D, generator=g)
     W = torch.randn(V, D, generator=g) * 0.02
     b = torch.randn(V, generator=g) * 0.02
@@ -1132,7 +1184,7 @@ def test_fp32_large_batch_entries_without_parts(where, device):
     a position that the mask leaves out; a value under 2^-50, or of 2^48."""
     say(f"fp32 large batch, entries without parts: {where}")
     g = torch.Generator().manual_seed(23)
-    B, S, D, V = 3, 64, 256, 700
+    B, S, D, V = 3, 64, 384, 700
     H, W = torch.randn(B, S, D, generator=g), torch.randn(V, D, generator=g) * 0.02
     m = torch.ones(B, S, dtype=torch.long)
     m[1, 20:] = 0
