@@ -453,8 +453,8 @@ __device__ __forceinline__ void store_chunk(O* out, const float* a) {
 // would outlast the launch. A workgroup's lane groups therefore share such rows: each step
 // every group computes the batch partials of 16 consecutive entries into LDS, and the
 // slice's columns add them in batch order: the same sums. A workgroup takes DH_GROUPS rows,
-// of which those past max(HOT_MIN, HOT_REL times its mean) are shared, or one row, which is unless it is short
-// (HOT_FEW).
+// of which those past max(HOT_MIN, HOT_REL times its mean) are shared, or one row, which is
+// unless it is short (HOT_FEW).
 constexpr int HOT_MIN = 128;
 constexpr int HOT_REL = 4;
 constexpr int HOT_FEW = 32;
@@ -477,8 +477,8 @@ struct HotSmem {
 template <typename T, typename O, bool WIDE>
 __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
     const T* __restrict__ W, const int* __restrict__ off, const int2* __restrict__ run,
-    O* __restrict__ dH, int B, int S, int D, int V, int runs, int cap, int S_row, int n_slices, int rpw,
-    int hot_min) {
+    O* __restrict__ dH, int B, int S, int D, int V, int runs, int cap, int S_row, int n_slices, int n16,
+    int dense, int hot_min) {
   constexpr int E = Chunk<T>::E;
   static_assert(Chunk<T>::COLS <= 64 * DH_WAVES, "one thread per column");
   static_assert(FOLD % DH_LANES == 0 && DH_GROUPS * DH_LANES % FOLD == 0 &&
@@ -487,13 +487,26 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
   __shared__ HotSmem<T> sm;
   const int slice = (int)blockIdx.x % n_slices, blk = (int)blockIdx.x / n_slices;
   const int tid = threadIdx.x, grp = tid / DH_LANES, l = tid % DH_LANES;
+  // n16 workgroups of DH_GROUPS rows a slice, then, with dense >= 0, one for each row: a batch
+  // row's positions go to those where it holds more than `dense` entries (dh_dense).
+  const bool single = blk >= n16;
+  const int rpw = single ? 1 : DH_GROUPS;
+  auto many_entries = [&](int64_t b) {  // (lane l of each group adds run l's)
+    int n = l < runs ? off[(b * (S + 1) + S) * runs + l] : 0;
+    n += __builtin_amdgcn_update_dpp(0, n, 0x111, 0xF, 0xF, true);  // row_shr:1
+    n += __builtin_amdgcn_update_dpp(0, n, 0x112, 0xF, 0xF, true);
+    n += __builtin_amdgcn_update_dpp(0, n, 0x114, 0xF, 0xF, true);
+    n += __builtin_amdgcn_update_dpp(0, n, 0x118, 0xF, 0xF, true);
+    return (int)row_bcast<15>((uint32_t)n) > dense;
+  };
+  const int64_t n_rows = (int64_t)B * S, row0 = single ? blk - n16 : (int64_t)blk * DH_GROUPS;
+  if (single && !many_entries(row0 / S)) return;  // workgroup-uniform
   const uint64_t row16 = (uint64_t)D * sizeof(T) / 16;  // 16-byte units per row
   const int d0 = slice * Chunk<T>::COLS;
   // Lanes past the row's end work on its last chunk (the row broadcasts need them) and do not
   // store.
   const int d = d0 + l * E;
   const char* wp = (const char*)(W + min(d, D - E));
-  const int64_t n_rows = (int64_t)B * S, row0 = (int64_t)blk * rpw;
   auto entries_of = [&](int64_t row, RowEntries& re) {  // returns the batch row's runs
     const int64_t b = row / S;
     re.load(off + (b * (S + 1) + (row - b * S)) * runs, runs, cap, l);
@@ -503,7 +516,8 @@ __global__ __launch_bounds__(64 * DH_WAVES) void bwd_dh_kernel(
     const int64_t b = row / S;
     return dH + (b * S_row + (row - b * S)) * D;
   };
-  const bool live = grp < rpw && row0 + grp < n_rows;
+  bool live = grp < rpw && row0 + grp < n_rows;
+  if (live && !single && dense >= 0) live = !many_entries((row0 + grp) / S);  // uniform in a group
   RowEntries re;
   re.total = 0;
   const int2* rb = nullptr;
@@ -893,17 +907,16 @@ static int passes_for(int64_t D) {
   return (int)std::min<int64_t>(MAX_NP, std::max<int64_t>(1, cdiv(D, 256)));
 }
 
-// Rows a dH workgroup takes: all its lane groups' worth once there are enough rows to fill the
-// chip, one (shared by the groups) below. Measured as whole passes with bf16 rows of 768,
-// V = 30522, at 16 rows / 1 row a workgroup: dense gradients, 16 x 64 positions 295 / 214 us,
-// 16 x 128 256 / 233 us, 16 x 200 282 / 263 us; 5% dense, 16 x 64 93 / 89 us, 16 x 128 99 /
-// 116 us (8 x 512, dH alone: 11 / 48 us).
+// From this many rows on every dH workgroup takes 16: they fill the chip then. A launch of fewer
+// also holds a workgroup for each row, last, and a batch row's positions get one each where it
+// holds more than 48 entries a position, or less in proportion under 1024 rows; the workgroups of
+// the other kind end at once. Backward with bf16 rows of 768, V = 30522, at 16 rows / 1 row a
+// workgroup: 12 x 150 with 9 entries a position 42 / 54 us, 38 61 / 66, 190 180 / 140; 16 x 64 with
+// 22 45 / 50, 90 76 / 62, 440 248 / 164; 16 x 32 with 9 34 / 40, 45 43 / 44, 180 75 / 59; 4 x 64
+// with 24 36 / 33.
 constexpr int64_t DH_MANY_ROWS = 2048;
-// Rows too long for a workgroup each within a launch (65 of 2^24 fp32 columns) share them too.
+static int64_t dh_dense(int64_t S, int64_t rows) { return S * 48 * std::min<int64_t>(rows, 1024) / 1024; }
 static_assert(DH_MAX_WG == MAX_THREADS / (64 * DH_WAVES), "workgroups of a dH launch");
-static int dh_rows_per_group(int64_t rows, int64_t n_slices) {
-  return rows >= DH_MANY_ROWS || rows * n_slices > DH_MAX_WG ? DH_GROUPS : 1;
-}
 // SPARTON_BWD_HOT_MIN sets the number of entries past which a row is shared (tests compare
 // shared and unshared rows).
 static int dh_hot_min() {
@@ -1298,13 +1311,15 @@ static void launch_rows(const T* g, const RT* r, const int32_t* idx, const void*
                            H, dW, dbias, (int)B, (int)S, (int)D, (int)V, nbk, (int)c.runs, (int)c.cap,
                            (int)s0, (int)sw, off, run);
         dw_done |= with_dw;
-        const int rpw = dh_rows_per_group(nb * sw, n_slices);
+        const int64_t rows = nb * sw, n16 = cdiv(rows, DH_GROUPS);
+        // (rows so long that a launch cannot hold a workgroup for each share them all)
+        const bool singles = rows < DH_MANY_ROWS && (n16 + rows) * n_slices <= DH_MAX_WG;
         const bool wide = (uint64_t)V * ((uint64_t)D * sizeof(T) / 16) > DH_WIDE_16;
         hipLaunchKernelGGL((wide ? bwd_dh_kernel<T, O, true> : bwd_dh_kernel<T, O, false>),
-                           dim3((unsigned)(cdiv(nb * sw, rpw) * n_slices)),
+                           dim3((unsigned)((n16 + (singles ? rows : 0)) * n_slices)),
                            dim3(64 * DH_WAVES), 0, st, W, (const int*)off, (const int2*)run,
                            dH + (b0 * S + s0) * D, (int)nb, (int)sw, (int)D, (int)V, (int)c.runs, (int)c.cap,
-                           (int)S, (int)n_slices, rpw, dh_hot_min());
+                           (int)S, (int)n_slices, (int)n16, singles ? (int)dh_dense(sw, rows) : -1, dh_hot_min());
       }
     }
   }

@@ -339,13 +339,21 @@ def test_backward_hot_rows_five_kernel(case, device, monkeypatch):
     ("bf16", 2, 5000, 16, 300, True, "int64"),      # two windows of positions
     ("fp16", 1, 90, 40, 70000, True, "int64"),      # two turns per bucketing wave; 1 row a workgroup
     ("bf16", 3, 30, 2056, 130, True, "holes"),      # 17 slices, the last of one chunk
+    ("bf16", 9, 70, 72, 30522, True, "mixed"),      # dense, sparse and empty batch rows, none of 16
+    ("fp32", 3, 700, 40, 20000, False, "mixed"),    # 2100 rows: no row a workgroup
 ], ids=lambda c: "-".join(map(str, c)))
 def test_backward_row_sharing(case, device, monkeypatch):
     """dH at the edges of its bucketing and its workgroups: rows shared by a workgroup's lane
     groups, or never (SPARTON_BWD_HOT_MIN past every row), or always (0), are the same bits,
-    and the oracle's."""
+    and the oracle's. Under 2048 rows a batch row's positions get a workgroup each or share one
+    by its entries ("mixed": one batch row of three each way, and one of none)."""
     say(f"dH row sharing, case {case}")
-    H, W, b, m, G = make_case(*case)
+    mixed = case[-1] == "mixed"
+    H, W, b, m, G = make_case(*case[:-1], "int64" if mixed else case[-1])
+    if mixed:
+        g = torch.Generator().manual_seed(5)
+        keep = torch.tensor([1.0, 0.02, 0.0]).repeat(3)[:case[1], None]
+        G = torch.rand(G.shape, generator=g).to(G.dtype) * (torch.rand(G.shape, generator=g) < keep)
     Hd, Wd, md, Gd = H.to(device), W.to(device), m.to(device), G.to(device)
     bd = None if b is None else b.to(device)
     _, idx, reps32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
