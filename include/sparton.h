@@ -217,6 +217,11 @@ int sparton_transform_bwd(const void* dy, const void* z, const float* dense_bias
 int sparton_transform_fwd_typed(const void* z, const void* dense_bias, const void* ln_weight,
                                 const void* ln_bias, int vec_dtype, float eps, void* y, float* mean,
                                 float* rstd, int64_t M, int64_t D, int dtype, void* stream);
+/* The forward that also copies dense_bias and ln_weight into kept[2][D] (vec_dtype; may be NULL), for a
+ * backward on their values of now. */
+int sparton_transform_fwd_keep(const void* z, const void* dense_bias, const void* ln_weight,
+                               const void* ln_bias, int vec_dtype, float eps, void* y, float* mean,
+                               float* rstd, void* kept, int64_t M, int64_t D, int dtype, void* stream);
 int sparton_transform_bwd_typed(const void* dy, const void* z, const void* dense_bias,
                                 const void* ln_weight, int vec_dtype, const float* mean,
                                 const float* rstd, void* dz, void* d_ln_weight, void* d_ln_bias,

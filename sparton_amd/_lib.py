@@ -52,6 +52,7 @@ EXPORTED_SYMBOLS = (
     "sparton_transform_fwd",
     "sparton_transform_bwd",
     "sparton_transform_fwd_typed",
+    "sparton_transform_fwd_keep",
     "sparton_transform_bwd_typed",
     "sparton_transform_workspace_bytes",
     "sparton_transform_dz_chunks",

@@ -444,12 +444,16 @@ struct TransformFn : public torch::autograd::Function<TransformFn> {
     Tensor mean = at::empty({M}, x.options().dtype(at::kFloat));
     Tensor rstd = at::empty({M}, x.options().dtype(at::kFloat));
     Tensor vb = dense(dense_bias), vg = dense(ln_weight), vt = dense(ln_bias);
-    check(sparton_transform_fwd_typed(z.data_ptr(), vb.data_ptr(), vg.data_ptr(), vt.data_ptr(),
-                                      dtype_code(vb.scalar_type()), (float)eps, y.data_ptr(),
-                                      mean.data_ptr<float>(), rstd.data_ptr<float>(), M, D,
-                                      dtype_code(x.scalar_type()), stream_of(x)),
+    // 16-bit vectors are the module's parameters themselves: the backward takes the copies that the
+    // kernel leaves, so that the parameters may change before it, as float32 copies of them did.
+    Tensor kept = vb.scalar_type() == at::kFloat ? Tensor() : at::empty({2, D}, vb.options());
+    check(sparton_transform_fwd_keep(z.data_ptr(), vb.data_ptr(), vg.data_ptr(), vt.data_ptr(),
+                                     dtype_code(vb.scalar_type()), (float)eps, y.data_ptr(),
+                                     mean.data_ptr<float>(), rstd.data_ptr<float>(), mptr(kept), M, D,
+                                     dtype_code(x.scalar_type()), stream_of(x)),
           "sparton_transform_fwd");
-    ctx->save_for_backward({x, weight, z, vb, vg, mean, rstd});
+    if (kept.defined()) ctx->save_for_backward({x, weight, z, kept, Tensor(), mean, rstd});
+    else ctx->save_for_backward({x, weight, z, vb, vg, mean, rstd});
     return y.view(x.sizes());
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -462,11 +466,14 @@ struct TransformFn : public torch::autograd::Function<TransformFn> {
     const int64_t M = x2.size(0);
     Tensor dy2 = grads[0].reshape({-1, D}).to(x.scalar_type()).contiguous();
     Tensor dz = at::empty_like(z);
+    const void* bias = vb.data_ptr();
+    const void* gamma = vg.defined() ? vg.data_ptr()  // or [2][D]: both
+                                     : static_cast<const char*>(bias) + D * vb.element_size();
     Tensor dg = at::empty({D}, vb.options());
     Tensor dbt = at::empty_like(dg), dbd = at::empty_like(dg);
     const size_t ws_bytes = sparton_transform_workspace_bytes(M, D);
     Tensor ws = workspace(ws_bytes, x);
-    check(sparton_transform_bwd_typed(dy2.data_ptr(), z.data_ptr(), vb.data_ptr(), vg.data_ptr(),
+    check(sparton_transform_bwd_typed(dy2.data_ptr(), z.data_ptr(), bias, gamma,
                                       dtype_code(vb.scalar_type()), mean.data_ptr<float>(),
                                       rstd.data_ptr<float>(), dz.data_ptr(), dg.data_ptr(), dbt.data_ptr(),
                                       dbd.data_ptr(), ws.data_ptr(), ws_bytes, M, D,

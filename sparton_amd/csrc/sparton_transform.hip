@@ -111,12 +111,14 @@ __device__ __forceinline__ f32x4 load4p(const VT* p, int d, int D) {
 }
 
 // ---- forward epilogue: one wave per row ------------------------------------------------
-// u = gelu(Z + b_d), mean and 1/std of u over the row, Y = (u - mean) / std * gamma + beta.
+// u = gelu(Z + b_d), mean and 1/std of u over the row, Y = (u - mean) / std * gamma + beta. Row 0's
+// wave leaves copies of b_d and gamma in `kept` [2][D], if given, for a backward that must not see
+// them change meanwhile.
 template <typename T, typename VT, int NP, bool FULL>
 __global__ __launch_bounds__(64 * FWD_WAVES) void xf_fwd_kernel(
     const T* __restrict__ Z, const VT* __restrict__ bd, const VT* __restrict__ gamma,
     const VT* __restrict__ beta, float eps, T* __restrict__ Y, float* __restrict__ mean_out,
-    float* __restrict__ rstd_out, int M, int D) {
+    float* __restrict__ rstd_out, VT* __restrict__ kept, int M, int D) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * FWD_WAVES + (threadIdx.x >> 6);
   if (row >= M) return;
@@ -162,6 +164,11 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void xf_fwd_kernel(
     mean_out[row] = mu;
     rstd_out[row] = rs;
   }
+  if (row == 0 && kept != nullptr)
+    for (int d = lane; d < D; d += 64) {
+      kept[d] = bd[d];
+      kept[D + d] = gamma[d];
+    }
 }
 
 // ---- backward epilogue -----------------------------------------------------------------
@@ -409,17 +416,17 @@ static int64_t bwd_blocks(int64_t M, int64_t D) {
 
 template <typename T, typename VT>
 static int fwd(const void* z, const VT* bd, const VT* gamma, const VT* beta, float eps,
-               void* y, float* mean, float* rstd, int64_t M, int64_t D, hipStream_t st) {
+               void* y, float* mean, float* rstd, VT* kept, int64_t M, int64_t D, hipStream_t st) {
   const dim3 grid((unsigned)cdiv(M, FWD_WAVES)), block(64 * FWD_WAVES);
   const bool full = D % 256 == 0;
 #define XF_FWD(NP)                                                                            \
   do {                                                                                        \
     if (full && D == NP * 256)                                                                \
       hipLaunchKernelGGL((xf_fwd_kernel<T, VT, NP, true>), grid, block, 0, st, (const T*)z, bd,   \
-                         gamma, beta, eps, (T*)y, mean, rstd, (int)M, (int)D);                \
+                         gamma, beta, eps, (T*)y, mean, rstd, kept, (int)M, (int)D);          \
     else                                                                                      \
       hipLaunchKernelGGL((xf_fwd_kernel<T, VT, NP, false>), grid, block, 0, st, (const T*)z, bd,  \
-                         gamma, beta, eps, (T*)y, mean, rstd, (int)M, (int)D);                \
+                         gamma, beta, eps, (T*)y, mean, rstd, kept, (int)M, (int)D);          \
   } while (0)
   switch (passes(D)) {
     case 1: XF_FWD(1); break;
@@ -492,9 +499,10 @@ extern "C" __attribute__((visibility("default"))) size_t sparton_transform_works
 static bool xf_vec_ok(int vec_dtype, int dtype) { return vec_dtype == SPARTON_F32 || vec_dtype == dtype; }
 static uintptr_t xf_vec_align(int vec_dtype) { return vec_dtype == SPARTON_F32 ? 16 : 8; }
 
-extern "C" __attribute__((visibility("default"))) int sparton_transform_fwd_typed(
+extern "C" __attribute__((visibility("default"))) int sparton_transform_fwd_keep(
     const void* z, const void* dense_bias, const void* ln_weight, const void* ln_bias, int vec_dtype,
-    float eps, void* y, float* mean, float* rstd, int64_t M, int64_t D, int dtype, void* stream) {
+    float eps, void* y, float* mean, float* rstd, void* kept, int64_t M, int64_t D, int dtype,
+    void* stream) {
   const int rc = xf_check(M, D, dtype);
   if (rc != SPARTON_OK) return rc;
   if (!xf_vec_ok(vec_dtype, dtype)) return SPARTON_EINVAL;
@@ -506,13 +514,21 @@ extern "C" __attribute__((visibility("default"))) int sparton_transform_fwd_type
     return SPARTON_EALIGN;
   hipStream_t st = (hipStream_t)stream;
 #define XF(T, VT) \
-  xf::fwd<T, VT>(z, (const VT*)dense_bias, (const VT*)ln_weight, (const VT*)ln_bias, eps, y, mean, rstd, M, D, st)
+  xf::fwd<T, VT>(z, (const VT*)dense_bias, (const VT*)ln_weight, (const VT*)ln_bias, eps, y, mean, rstd, \
+                 (VT*)kept, M, D, st)
   switch (dtype) {
     case SPARTON_BF16: return vec_dtype == SPARTON_F32 ? XF(bf16, float) : XF(bf16, bf16);
     case SPARTON_F16: return vec_dtype == SPARTON_F32 ? XF(f16, float) : XF(f16, f16);
     default: return XF(float, float);
   }
 #undef XF
+}
+
+extern "C" __attribute__((visibility("default"))) int sparton_transform_fwd_typed(
+    const void* z, const void* dense_bias, const void* ln_weight, const void* ln_bias, int vec_dtype,
+    float eps, void* y, float* mean, float* rstd, int64_t M, int64_t D, int dtype, void* stream) {
+  return sparton_transform_fwd_keep(z, dense_bias, ln_weight, ln_bias, vec_dtype, eps, y, mean, rstd, nullptr,
+                                    M, D, dtype, stream);
 }
 
 extern "C" __attribute__((visibility("default"))) int sparton_transform_bwd_typed(

@@ -246,3 +246,26 @@ def test_module_in_16_bits_equals_float_vectors(dt, M, D, device):
         assert torch.equal(module(x), y)
     with pytest.raises(RuntimeError):
         _eager.load().mlm_transform(x2, w2, dense.bias, norm.weight, norm.bias, 1e-5)
+
+
+@pytest.mark.parametrize("dt,D", [("bf16", 768), ("fp16", 1000), ("bf16", 2052)])
+def test_module_in_16_bits_vectors_may_change_before_backward(dt, D, device):
+    """The bias and LayerNorm vectors of a 16-bit module updated in place between the forward and the
+    backward: the gradients are those at the forward's values, bit for bit."""
+    dtype = {"bf16": torch.bfloat16, "fp16": torch.float16}[dt]
+    torch.manual_seed(D)
+    module = sparton_amd.SpartonMLMTransform(torch.nn.Linear(D, D), torch.nn.LayerNorm(D)).to(device, dtype)
+    x, dy = torch.randn(2, 70, D, device=device, dtype=dtype)
+    grads = []
+    for change in (False, True):
+        module.zero_grad(set_to_none=True)
+        xs = x.clone().requires_grad_()
+        y = module(xs)
+        if change:
+            with torch.no_grad():
+                for v in (module.dense.bias, module.layer_norm.weight, module.layer_norm.bias):
+                    v.add_(1.0)
+        y.backward(dy)
+        grads.append([xs.grad] + [p.grad for p in module.parameters()])
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
