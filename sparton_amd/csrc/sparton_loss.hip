@@ -771,6 +771,9 @@ template <typename T> struct Parts {
   static constexpr int P = std::is_same<T, bf16>::value ? 2 : 3;
   static constexpr int X = sizeof(T) == 4 ? 3 : std::is_same<T, f16>::value ? 2 : 1;
   typedef typename std::conditional<sizeof(T) == 4, bf16, T>::type ST;  // the score MFMA's type
+  // Scale of P in the gradients, exact: the parts of a value under 2^-110 fall below bf16's smallest
+  // (probabilities of e^-83, and gradients of nothing else, came out with errors of 2e-4).
+  static constexpr float PS = X > 1 ? 0x1p48f : 1.0f;
 };
 
 // Two values as N parts, a pair of bf16 each.
@@ -1032,14 +1035,17 @@ __device__ __forceinline__ void load_p(const float* __restrict__ P, int Bq, int 
     }
   }
 }
-template <bool A_KC, int N>
+template <typename T, bool A_KC, int N>
 __device__ __forceinline__ void store_p(uint16_t* s, const float (&v)[2][8]) {
   const int t = threadIdx.x;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int m = A_KC ? (t >> 2) + 64 * u : t & 127, kg = A_KC ? t & 3 : (t >> 7) + 2 * u;
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = v[u][i] * Parts<T>::PS;
     u32x4 p[N];
-    parts8<N>(v[u], p);
+    parts8<N>(x, p);
 #pragma unroll
     for (int i = 0; i < N; ++i) *(u32x4*)(s + i * TM * LDH + m * LDH + 8 * kg) = p[i];
   }
@@ -1095,7 +1101,7 @@ __device__ __forceinline__ void store_x(uint16_t* s, const Two<T> (&v)[8]) {
 }
 
 // One GEMM tile: acc += A B^T over k in [0, K), A = P rows m0.. (A_KC) or P columns m0..,
-// B = X[k][c0 ..]. `meanwhile` (barriers in it are reached by every thread) runs under the first
+// B = X[k][c0 ..], times PS. `meanwhile` (barriers in it are reached by every thread) runs under the first
 // loads.
 template <typename T, bool A_KC, typename F>
 __device__ __forceinline__ void gemm16(uint16_t* sA, uint16_t* sB, const float* __restrict__ P, int Bq,
@@ -1116,7 +1122,7 @@ __device__ __forceinline__ void gemm16(uint16_t* sA, uint16_t* sB, const float* 
   auto stage = [&](int k0, float (&p)[2][8], Two<T> (&x)[8]) __attribute__((always_inline)) {
     if (k0 >= K) return;
     __syncthreads();  // the previous stage is read
-    store_p<A_KC, NP>(sA, p);
+    store_p<T, A_KC, NP>(sA, p);
     store_x<T, NX>(sB, x);
     __syncthreads();
     load(k0 + 2 * KS, p, x);
@@ -1132,7 +1138,7 @@ __device__ __forceinline__ void gemm16(uint16_t* sA, uint16_t* sB, const float* 
   if (NX > 1) add4(acc, low);
 }
 
-// G[i][c] = c_ce acc + c_s sign(X[i][c]) + c_f colsum[c] for the tile's rows below `rows`.
+// G[i][c] = c_ce acc / PS + c_s sign(X[i][c]) + c_f colsum[c] for the tile's rows below `rows`.
 template <typename T>
 __device__ __forceinline__ void grad16_epilogue(const f32x16 (&acc)[2][2], const T* __restrict__ X,
                                                 int rows, int m0, int c0, int V, float c_ce,
@@ -1162,7 +1168,7 @@ __device__ __forceinline__ void grad16_epilogue(const f32x16 (&acc)[2][2], const
         if (i < rows && c < V) {
           const float x = to_f32(xv[bi][bj][r]);
           const float sg = x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f);
-          G[(int64_t)i * V + c] = from_f32<T>(c_ce * acc[bi][bj][r] + c_s * sg + add);
+          G[(int64_t)i * V + c] = from_f32<T>(c_ce * (acc[bi][bj][r] * (1.0f / Parts<T>::PS)) + c_s * sg + add);
         }
       }
     }

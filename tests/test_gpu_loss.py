@@ -185,6 +185,27 @@ def test_loss_parts_against_fp64(dt, Bq, Bd, V, off, device, monkeypatch):
         assert a <= b + e, (err, eps)
 
 
+@pytest.mark.parametrize("margin", [20.0, 83.0])
+def test_loss_parts_of_small_probabilities(margin, device):
+    """Gradients that are sums of small probabilities, down to fp32's smallest normal values: documents
+    that no query owns, whose probabilities are about e^-margin. Relative to fp64 no further off
+    than the probabilities are: an absolute error of a score, at most 16 roundings of its size."""
+    say(f"loss parts, margin {margin}")
+    g = torch.Generator().manual_seed(1)
+    Bq, Bd, V = 66, 140, 513
+    q, d = torch.zeros(Bq, V + 130), torch.zeros(Bd, V + 130)
+    q[:, :V], d[:, :V] = torch.rand(Bq, V, generator=g) * 0.3, torch.rand(Bd, V, generator=g) * 0.3
+    for i in range(Bq):  # a column of its own for each query and its document
+        q[i, V + i] = d[i, V + i] = margin ** 0.5
+    q64, d64 = q.double().requires_grad_(), d.double().requires_grad_()
+    F.cross_entropy(q64 @ d64.T, torch.arange(Bq)).backward()
+    qs, ds = q.to(device).requires_grad_(), d.to(device).requires_grad_()
+    sl.splade_loss(qs, ds, 1.0, 0.0, 0.0).contrastive.backward()
+    score = float((q @ d.T).max())
+    got, want = ds.grad[Bq:, :V].cpu().double(), d64.grad[Bq:, :V]
+    assert float((got - want).norm() / want.norm()) <= 16 * 2.0 ** -24 * score
+
+
 @pytest.mark.parametrize("dt,big", [("fp32", float("inf")), ("fp32", 3.4e38), ("fp16", float("inf"))])
 def test_loss_parts_with_infinite_entries(dt, big, device, monkeypatch):
     """An entry with no finite parts (infinite, or one that bf16 rounds to infinity): every score,
