@@ -1,6 +1,7 @@
 """CPU checks of the drop-in boundary: the C-ABI library, the Python ops and the
 SpartonHead module surface. Nothing here launches a kernel."""
 import ctypes
+import glob
 import os
 import re
 import subprocess
@@ -461,3 +462,16 @@ def test_fwd_noalloc_rejections_before_any_hip_call():
     # config 2's fit
     assert L.sparton_fwd_workspace_bytes(32, 256, 768, 30522, 1) <= cap
     assert b"static scratch" in L.sparton_strerror(-5)
+
+
+def test_switches_that_tests_set_are_read():
+    """Every SPARTON_* variable that a test or the benchmark sets is read by the product: one that is not
+    would leave its test comparing a path with itself."""
+    read = lambda *paths: "\n".join(open(f).read() for p in paths for f in sorted(glob.glob(os.path.join(ROOT, p))))
+    used = set(re.findall(r"SPARTON_[A-Z0-9_]+", read("tests/*.py", "bench.py")))
+    c_names = set(re.findall(r"SPARTON_[A-Z0-9_]+", read("include/sparton.h")))  # enums and macros
+    src = read("sparton_amd/csrc/*", "sparton_amd/*.py")
+    read_names = set(re.findall(r"getenv\(\"(SPARTON_[A-Z0-9_]+)\"\)", src))
+    read_names |= set(re.findall(r"environ(?:\.get\(|\[)\"(SPARTON_[A-Z0-9_]+)\"", src))
+    assert {"SPARTON_BWD_HOT_MIN", "SPARTON_BWD_FEW", "SPARTON_FWD_PATH"} <= read_names
+    assert used - c_names - {"SPARTON_"} <= read_names, used - c_names - read_names

@@ -245,37 +245,43 @@ def test_deterministic_repeat(device):
     ("bf16", 37, 40, 256, 700, True, "int64"),      # many short rows
 ], ids=lambda c: "-".join(map(str, c)))
 def test_backward_paths_agree_bitwise(case, device, monkeypatch):
-    """The fused backward (entries compacted by the dW kernel) and the five-kernel one
-    (count, scan, scatter; with either dH load-group size) sum every gradient in the same
-    order: bitwise equal. (Shapes
-    where the fused path is taken: >= 64 row ranges, and >= 1024 rows, so that the
-    five-kernel path also gives each dH row one wave.)"""
+    """Gradients in the inputs' dtype, dH's rows shared among a workgroup's lane groups by their entries
+    (SPARTON_BWD_HOT_MIN unset), always (0) or never (2^30), and dW beside the bucketing or in a launch
+    of its own (SPARTON_BWD_DW_MERGE): every gradient is summed in the same order, bitwise equal, and
+    is the oracle's, rounded once."""
     say(f"backward paths, case {case}")
     H, W, b, m, G = make_case(*case)
     Hd, Wd, md, Gd = H.to(device), W.to(device), m.to(device), G.to(device)
     bd = None if b is None else b.to(device)
     _, idx, reps32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
-    fused = [t.clone() for t in torch.ops.sparton.fused_sparton_bwd_train(Gd, reps32, idx, Hd, Wd, bd, md)]
-    monkeypatch.setenv("SPARTON_BWD_PATH", "five")
-    five = [t.clone() for t in torch.ops.sparton.fused_sparton_bwd_train(Gd, reps32, idx, Hd, Wd, bd, md)]
-    monkeypatch.setenv("SPARTON_BWD_DH_LONG", "1")  # the large-vocabulary load groups
-    five_long = torch.ops.sparton.fused_sparton_bwd_train(Gd, reps32, idx, Hd, Wd, bd, md)
+    runs = []
+    for env in ({}, {"SPARTON_BWD_HOT_MIN": "0"}, {"SPARTON_BWD_HOT_MIN": str(2 ** 30)},
+                {"SPARTON_BWD_DW_MERGE": "0"}):
+        with monkeypatch.context() as mp:
+            for k, v in env.items():
+                mp.setenv(k, v)
+            runs.append([t.clone() for t in torch.ops.sparton.fused_sparton_bwd_train(
+                Gd, reps32, idx, Hd, Wd, bd, md)])
     torch.cuda.synchronize()
-    for a, c, d in zip(fused, five, five_long):
-        assert torch.equal(a, c) and torch.equal(a, d)
+    for out in runs[1:]:
+        for a, c in zip(runs[0], out):
+            assert torch.equal(a, c)
+    full = torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)
+    check_bwd_isolated(H, W, b, m, G, reps32, idx, *full)
+    for a, c in zip(runs[0], full):
+        assert a.dtype == H.dtype and torch.equal(a, c.to(a.dtype))
 
 
 @pytest.mark.parametrize("case", [
     ("bf16", 32, 256, 768, 30522, True, "int64"),   # the headline shape
     ("fp16", 8, 512, 768, 9000, False, "holes"),
     ("fp32", 16, 70, 132, 900, True, "frac"),
-    ("bf16", 20, 64, 1280, 3000, True, "int64"),    # two-group batches (bf16 rows past 768)
+    ("bf16", 20, 64, 1280, 3000, True, "int64"),    # ten slices a row
 ], ids=lambda c: "-".join(map(str, c)))
 def test_backward_hot_rows(case, device, monkeypatch):
-    """Rows that win most vocab ids (position 0 scaled up, like a [CLS] token): the fused
-    dH workgroup then shares the hot row's batches among its waves. Shared, per-row and
-    the automatic choice are bitwise equal, equal to the five-kernel path, and match
-    the oracle."""
+    """Rows that win most vocab ids (position 0 scaled up, like a [CLS] token): a workgroup shares the
+    hot row's batches among its lane groups. Shared always (SPARTON_BWD_HOT_MIN 0), never (2^30) and
+    by the automatic choice are bitwise equal, and match the oracle."""
     say(f"hot dH rows, case {case}")
     H, W, b, m, G = make_case(*case)
     H[:, 0, :] *= 3.0
@@ -283,18 +289,16 @@ def test_backward_hot_rows(case, device, monkeypatch):
     bd = None if b is None else b.to(device)
     _, idx, reps32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
     runs = {}
-    for mode in ("0", "1000", None):
+    for mode in ("0", str(2 ** 30), None):
         if mode is None:
-            monkeypatch.delenv("SPARTON_BWD_SHARE", raising=False)
+            monkeypatch.delenv("SPARTON_BWD_HOT_MIN", raising=False)
         else:
-            monkeypatch.setenv("SPARTON_BWD_SHARE", mode)
+            monkeypatch.setenv("SPARTON_BWD_HOT_MIN", mode)
         runs[mode] = [t.clone() for t in torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)]
-    monkeypatch.setenv("SPARTON_BWD_PATH", "five")
-    five = torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)
     torch.cuda.synchronize()
     hot = int(torch.bincount(idx[:1].flatten().long().cpu()).max())
     say(f"  row 0's most-won position holds {hot} vocab ids")
-    for out in list(runs.values())[1:] + [five]:
+    for out in list(runs.values())[1:]:
         for a, c in zip(runs["0"], out):
             assert (a is None and c is None) or torch.equal(a, c)
     dH, dW, db = runs[None]
@@ -302,22 +306,22 @@ def test_backward_hot_rows(case, device, monkeypatch):
 
 
 @pytest.mark.parametrize("case", [
-    ("bf16", 4, 64, 64, 70000, True, "int64"),      # V > 65536: the five-kernel path
-    ("fp32", 8, 100, 96, 8000, False, "int64"),     # five-kernel path forced
-    ("fp16", 4, 50, 1280, 12000, True, "int64"),    # five 256-column slices per row
+    ("bf16", 4, 64, 64, 70000, True, "int64"),      # V > 65536: two turns per bucketing wave
+    ("fp32", 8, 100, 96, 8000, False, "int64"),     # 800 rows, two slices
+    ("fp16", 4, 50, 1280, 12000, True, "int64"),    # ten slices a row
+    ("bf16", 40, 64, 72, 9000, True, "int64"),      # 2560 rows: sixteen a workgroup, the hot ones shared
 ], ids=lambda c: "-".join(map(str, c)))
-def test_backward_hot_rows_five_kernel(case, device, monkeypatch):
-    """Rows with more than 128 entries (position 0 scaled up) on the five-kernel path go to
-    bwd_dh_hot_kernel, whose workgroup shares a row's batches: bitwise the same dH as one
-    wave per row (SPARTON_BWD_HOT_MIN set past every row), and the oracle's."""
-    say(f"hot dH rows on the five-kernel path, case {case}")
+def test_backward_rows_past_hot_min(case, device, monkeypatch):
+    """Rows with more than 128 entries (position 0 scaled up), whose batches a workgroup shares:
+    bitwise the same dH as one lane group per row (SPARTON_BWD_HOT_MIN set past every row), and
+    the oracle's."""
+    say(f"dH rows past the shared rows' least, case {case}")
     H, W, b, m, G = make_case(*case)
     H[:, 0, :] *= 3.0
     Hd, Wd, md, Gd = H.to(device), W.to(device), m.to(device), G.to(device)
     bd = None if b is None else b.to(device)
-    monkeypatch.setenv("SPARTON_BWD_PATH", "five")
     _, idx, reps32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
-    hot = [t.clone() for t in torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)]
+    hot = [None if t is None else t.clone() for t in torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)]
     monkeypatch.setenv("SPARTON_BWD_HOT_MIN", str(2 ** 30))
     plain = torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)
     torch.cuda.synchronize()
@@ -704,27 +708,27 @@ def test_opcheck_and_compile(device):
 
 
 @pytest.mark.parametrize("case", [
-    ("fp32", 2, 32, 768, 3000, True, "int64"),     # 64 rows: 8 waves per dH row
-    ("bf16", 3, 100, 256, 2000, True, "holes"),    # 300 rows: 4 waves per row
-    ("fp16", 1, 700, 64, 500, False, "frac"),      # 700 rows: 2 waves per row
+    ("fp32", 2, 32, 768, 3000, True, "int64"),     # 64 rows
+    ("bf16", 3, 100, 256, 2000, True, "holes"),    # 300 rows
+    ("fp16", 1, 700, 64, 500, False, "frac"),      # 700 rows
 ], ids=lambda c: "-".join(map(str, c)))
 def test_backward_few_rows_split(case, device, monkeypatch):
-    """Few dH rows: the five-kernel path splits each row's entries over several waves and
-    adds their partial rows in wave order (SPARTON_BWD_FEW=0 keeps batches of at most 64 rows
-    on it too). Against the oracle, and bitwise repeatable."""
+    """Few dH rows: a workgroup's lane groups split each row's entries and add their partials in
+    order (SPARTON_BWD_FEW=0 keeps batches of at most 64 rows on that path too). Against the oracle,
+    and bitwise repeatable."""
     say(f"backward few rows, case {case}")
     monkeypatch.setenv("SPARTON_BWD_FEW", "0")
     H, W, b, m, G = make_case(*case)
     Hd, Wd, md, Gd = H.to(device), W.to(device), m.to(device), G.to(device)
     bd = None if b is None else b.to(device)
     _, idx, reps32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
-    outs = [[t.clone() for t in torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)]
+    outs = [[None if t is None else t.clone()
+             for t in torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)]
             for _ in range(2)]
     torch.cuda.synchronize()
     for a, c in zip(*outs):
-        assert torch.equal(a, c)
+        assert (a is None and c is None) or torch.equal(a, c)
     check_bwd_isolated(H, W, b, m, G, reps32, idx, *outs[0])
-
 
 
 FEW_ROW_CASES = [
@@ -741,7 +745,7 @@ FEW_ROW_CASES = [
 def test_backward_few_rows_single_w_read(case, device, monkeypatch):
     """At most 64 dH rows: each W row is read once and added into every dH row it serves
     (rows held in registers, per-range partials added in range order). Against the oracle,
-    bitwise repeatable, dW and dbias bitwise those of the five-kernel path, dH within fp32
+    bitwise repeatable, dW and dbias bitwise those of the bucketing path, dH within fp32
     rounding of it (the two sum in different orders)."""
     say(f"backward few rows, single W read, case {case}")
     H, W, b, m, G = make_case(*case)
@@ -812,24 +816,21 @@ def test_backward_few_rows_partial_outputs(case, device):
     assert torch.equal(no_db[0], full[0]) and torch.equal(no_db[1], full[1])
 
 
-@pytest.mark.parametrize("case,long_rows", [
-    (("fp32", 2, 32, 768, 3000, True, "int64"), False),    # few rows: split dH + dW, one launch
-    (("bf16", 3, 100, 256, 2000, False, "holes"), False),  # few rows, no bias
-    (("bf16", 8, 160, 1536, 1200, True, "int64"), False),  # 1280 rows, six register passes
-    (("fp16", 6, 200, 2048, 3000, True, "frac"), True),    # eight passes, long-row dH groups
-], ids=lambda c: "-".join(map(str, c)) if isinstance(c, tuple) else f"long{int(c)}")
-def test_backward_dw_in_dh_launch(case, long_rows, device, monkeypatch):
-    """On the five-kernel path, dW's workgroups run in the dH launch (few rows, or rows of
-    six or more register passes): bitwise the same dH, dW and dbias as a separate dW
-    launch (SPARTON_BWD_DW_MERGE=0), and the oracle's."""
-    say(f"dW in the dH launch, case {case}, long-row groups {long_rows}")
+@pytest.mark.parametrize("case", [
+    ("fp32", 2, 32, 768, 3000, True, "int64"),     # 64 rows
+    ("bf16", 3, 100, 256, 2000, False, "holes"),   # few rows, no bias
+    ("bf16", 8, 160, 1536, 1200, True, "int64"),   # 1280 rows, six register passes
+    ("fp16", 6, 200, 2048, 3000, True, "frac"),    # eight passes
+    ("bf16", 1, 1025, 72, 500, True, "int64"),     # S > 1024: dW in a launch of its own either way
+], ids=lambda c: "-".join(map(str, c)))
+def test_backward_dw_beside_bucketing(case, device, monkeypatch):
+    """dW's workgroups run in the bucketing's launch: bitwise the same dH, dW and dbias as a
+    separate dW launch (SPARTON_BWD_DW_MERGE=0), and the oracle's."""
+    say(f"dW beside the bucketing, case {case}")
     H, W, b, m, G = make_case(*case)
     Hd, Wd, md, Gd = H.to(device), W.to(device), m.to(device), G.to(device)
     bd = None if b is None else b.to(device)
-    monkeypatch.setenv("SPARTON_BWD_PATH", "five")
     monkeypatch.setenv("SPARTON_BWD_FEW", "0")
-    if long_rows:
-        monkeypatch.setenv("SPARTON_BWD_DH_LONG", "1")
     _, idx, reps32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
     merged = [None if t is None else t.clone()
               for t in torch.ops.sparton.fused_sparton_bwd(Gd, reps32, idx, Hd, Wd, bd, md)]
@@ -899,17 +900,18 @@ def test_backward_rows_past_the_launch_limit(device):
 
 
 @pytest.mark.parametrize("case", [
-    ("bf16", 2, 20000, 64, 320, True, "holes"),     # S > 16384: two dH windows
-    ("fp32", 1, 40000, 32, 200, False, "int64"),    # three windows, the last partial
+    ("bf16", 2, 20000, 64, 320, True, "holes"),     # five dH windows, the last partial
+    ("fp32", 1, 40960, 32, 200, False, "int64"),    # ten windows
     ("fp16", 20, 20000, 32, 64, True, "gaps"),      # 25000 groups: the three-kernel plan
     ("bf16", 9000, 3, 32, 64, True, "int64"),       # B > 8192: two dH batch chunks
+    ("fp16", 300, 4100, 8, 24, True, "int64"),      # 2^20 dH rows a chunk: two, of two windows each
     ("bf16", 33000, 1, 8, 16, True, "holes"),       # B > 32768: two forward launches
     ("bf16", 1, 70000, 16, 64, True, "int64"),      # S > 65536: dW without the 16-bit staging
 ], ids=lambda c: "-".join(map(str, c)))
 def test_long_sequences_and_many_rows(case, device):
     """Shapes past one pass of the kernels: the forward takes any S (and splits B over
-    launches of at most 32768 rows); the backward's dH passes run over windows of 16384
-    positions and chunks of 8192 batch rows. Against the oracle."""
+    launches of at most 32768 rows); the backward's dH passes run over windows of 4096
+    positions and chunks of 8192 batch rows and 2^20 dH rows. Against the oracle."""
     say(f"long / many rows, case {case}")
     H, W, b, m, G = make_case(*case)
     reps, idx, reps32, dH, dW, db = run_fwd_bwd(H, W, b, m, G, device)
