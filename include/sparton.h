@@ -255,7 +255,8 @@ int sparton_transform_chunk_sum(const float* part, void* out, int64_t C, int64_t
  * SPARTON_EUNSUPPORTED. Up to 64 rows per side run slice-staged kernels, larger batches
  * tiled GEMM kernels on the 16-bit matrix cores (products of 16-bit reps are exact in fp32;
  * fp32 values and, in the gradients, fp16 ones are sums of bf16 parts that hold all their
- * bits); the workspace size follows. Accumulated in fp32 whatever the reps dtype.
+ * bits, except that P against bf16 reps takes two parts, within 2^-17 of it); the workspace
+ * size follows. Accumulated in fp32 whatever the reps dtype.
  */
 size_t sparton_loss_workspace_bytes(int64_t Bq, int64_t Bd, int64_t V);
 

@@ -100,7 +100,7 @@ static int64_t mask_elem_bytes(int mdt) {
 
 // Entry (b, v): whether it carries gradient, its coefficient g' and index s.
 // Activity is decided by comparisons of loaded values only (never by the float
-// product), so the count and scatter kernels agree on every entry; an index outside
+// product), so the bucketing's count and its write agree on every entry; an index outside
 // [0, S) makes the entry inactive, so it can never turn into an out-of-bounds access.
 // g' = G * exp(-reps) (src/sparton/sparton_kernel.py:531) times mask[b, I], the torch
 // head's d x / d logits (training/model.py:60); 1 for a 0/1 mask.
@@ -118,7 +118,7 @@ __device__ __forceinline__ bool entry(T g_raw, RT r_raw, int s, const float* mas
   return true;
 }
 
-// ---- 1. bucketing --------------------------------------------------------------
+// ---- bucketing --------------------------------------------------------------
 //
 // The active entries of each batch row are sorted by position, ids ascending, a run of
 // consecutive ids at a time: workgroup (b, c) takes run c (at most BK_RUNS of them, so that
@@ -288,8 +288,9 @@ template <> struct Raw4<f16> {
 
 // The order every dH row is summed in (the few-row path aside): the row's entries, in v
 // order, are taken DH_BATCH at a time (the last batch may hold fewer); a batch's partial is
-// P = fma(g_u, W[v_u], P) over its entries from P = 0, and the row is ((0 + P_0) + P_1) + ...
-// So a row is the same bits whether one lane group sums it or a workgroup shares its batches.
+// P = fma(g_u, W[v_u], P) over its entries from P = 0. Partials are added in order in blocks of
+// FOLD entries, those in blocks of FOLD2 and these in order (below). So a row is the same bits
+// whether one lane group sums it or a workgroup shares its batches.
 constexpr int DH_BATCH = 4;
 
 // Rows gathered per batch: all their loads are in flight together (about 24 per lane).
@@ -309,7 +310,7 @@ template <typename T, int NP> struct DwPasses {
   static constexpr int value = NP < CAP ? NP : CAP;
 };
 
-// ---- 2. dH ---------------------------------------------------------------------
+// ---- dH ---------------------------------------------------------------------
 // A row of D elements is cut into slices of DH_LANES 16-byte chunks, and 16 lanes (one DPP
 // row) sum one slice of one row, a chunk each, over the row's entries. The lanes look up 16
 // entries together, one each, and hand them round with row broadcasts; then the 16 W chunks
@@ -641,7 +642,7 @@ __device__ __forceinline__ void entries_n(const T* grad, const RT* reps, const i
   }
 }
 
-// ---- 5. dW and dbias -------------------------------------------------------------
+// ---- dW and dbias -------------------------------------------------------------
 // One wave per vocab row v: lanes hold batch rows b (64 per pass), a ballot lists the
 // active ones, and their H rows are gathered in ascending b, two at a time. Lanes past the
 // row end load the row's last group (D >= 4 whenever D > 0), so the loads carry no per-lane
@@ -713,7 +714,7 @@ __global__ __launch_bounds__(256) void bwd_dw_kernel(
   }
 }
 
-// ---- 5b. dW and dbias, staged (B <= DW_STAGE_B) ---------------------------------
+// ---- dW and dbias, staged (B <= DW_STAGE_B) ---------------------------------
 constexpr int DW_STAGE_B = 128;
 // The staged dW: a workgroup of NW waves owns NIDS consecutive vocab ids (NIDS / NW per
 // wave). It loads G, reps and I of all batch rows for them (each load instruction reads
@@ -957,7 +958,7 @@ constexpr int FEW_ES_LD = 68;   // bytes per id of the index table: 17 words, od
                                 // 64 ids fall in 64 different banks
 constexpr uint8_t FEW_NONE = 0xff;  // index table: inactive entry (S <= FEW_ROWS < 255)
 
-// SPARTON_BWD_FEW=0 sends few-row batches down the count/scan/scatter path instead (tests
+// SPARTON_BWD_FEW=0 sends few-row batches to the bucketing and bwd_dh_kernel instead (tests
 // compare the two).
 static bool few_enabled() {
   const char* e = getenv("SPARTON_BWD_FEW");

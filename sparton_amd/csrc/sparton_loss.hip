@@ -733,7 +733,7 @@ __device__ __forceinline__ void grad_tile(float* sA, float* sB, const float* __r
 // fp32 value's 24 bits, two an fp16 value's 11, and bf16 has fp32's exponents, so no scales
 // are needed. A product takes the pairs of parts down to 2^-24 of it:
 //   scores     fp32 reps 3 x 3 parts, 6 MFMAs per step (against 8 fp32 ones of twice the time)
-//   gradients  P (fp32) against bf16 reps 2 x 1 parts (p within 2^-18), 2 MFMAs; fp16 reps
+//   gradients  P (fp32) against bf16 reps 2 x 1 parts (p within 2^-17), 2 MFMAs; fp16 reps
 //              3 x 2 parts, 5; fp32 reps 3 x 3, 6
 // The products of the lower parts have accumulators of their own, added at the end: the main
 // sums then round once per 16 k (the fp32 MFMA's: 8 times), and over batches of 65 to 500 rows

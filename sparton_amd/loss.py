@@ -19,7 +19,8 @@ runs in the reps dtype), deterministically. Device tensors only, like the head.
 
 Batches of up to 64 rows on each side take the slice-staged kernels above. Larger batches
 take GEMM-shaped HIP kernels on the matrix cores (the bf16/fp16 MFMA: products of 16-bit
-reps are exact in fp32, fp32 values are sums of bf16 parts that hold all their bits): a
+reps are exact in fp32, fp32 values are sums of bf16 parts that hold all their bits; P against bf16 reps, whose
+gradients are rounded to bf16, takes two parts, within 2^-17 of it): a
 split-vocabulary score GEMM with a fixed-order sum of its partials, per-slice row and column
 statistics, a row softmax, and a backward that recomputes each vocabulary slice's column sums
 and forms both gradients tile by tile (sparton_loss.hip). Limits: 1 <= Bq <= Bd when documents are given (the labels
