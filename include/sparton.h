@@ -79,10 +79,10 @@ enum sparton_status {
  * Bytes of device scratch sparton_fwd needs for these sizes (256-byte aligned
  * sections: the per-row block plan, the partial results of batch rows whose
  * positions span several row tiles, and for larger fp32 batches (from B*S = 192 on) H
- * and W as three bf16 parts, a range of columns at a time, on whose MFMAs such a batch runs; given less than these bytes but
- * enough for the rest, it runs on the fp32 MFMAs instead, as do operands with a nonzero
- * magnitude outside [2^-50, 2^48), infinities and NaN among them). No counterpart in the reference: its forward
- * materializes a [B,S,C] logits tile per vocab tile instead (sparton_kernel.py:245-247).
+ * and W as three bf16 parts, a range of columns at a time, on whose MFMAs such a batch
+ * runs; given less than these bytes but enough for the rest, it runs on the fp32 MFMAs
+ * instead, as do operands with a nonzero magnitude outside [2^-50, 2^48), infinities and
+ * NaN among them). No counterpart in the reference: its forward materializes a [B,S,C] logits tile per vocab tile instead (sparton_kernel.py:245-247).
  */
 size_t sparton_fwd_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t V, int dtype);
 
@@ -98,7 +98,7 @@ size_t sparton_fwd_workspace_min_bytes(int64_t B, int64_t S, int64_t D, int64_t 
  * `reps_f32` may be NULL; if given, it receives reps[B,V] unrounded in fp32, which a
  * training caller keeps for the backward instead of the rounded `reps`.
  * `bias` may be NULL (use_bias=False). `workspace` (256-byte aligned, at least
- * sparton_fwd_workspace_bytes) is overwritten; S <= 16384.
+ * sparton_fwd_workspace_min_bytes) is overwritten.
  *
  * Replaces the reference's forward path: fused_sparton_fwd_with_indices
  * (src/sparton/sparton_kernel.py:226-253), its V-tile GEMM (:204-210) and the

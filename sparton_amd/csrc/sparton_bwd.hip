@@ -18,8 +18,8 @@
 // two launches. At most 64 dH rows take the few-row path instead.
 // Measured against the kernels it replaced, which sorted by 64-id blocks and gave each dH row
 // one wave, 4 rows of W in flight (backward kernels, one box): dense gradients, 16 x 256 rows
-// bf16 into fp32 341 -> 187 us, 8 x 128 rows fp32 557 -> 161 us; 5% dense, 32 x 256 rows
-// 47 -> 48 us, 8 x 512 rows 23 -> 24 us, V = 250002 337 -> 298 us, D = 4096 515 -> 438 us.
+// bf16 into fp32 341 -> 186 us, 8 x 128 rows fp32 557 -> 153 us; 5% dense, 32 x 256 rows
+// 47 -> 48 us, 8 x 512 rows 23 -> 24 us, V = 250002 337 -> 290 us, D = 4096 515 -> 425 us.
 // The only atomics are integer counts in LDS, which are order-independent.
 //
 // Gradients are written as fp32 (what the reference returns) or in the input dtype
@@ -316,7 +316,7 @@ template <typename T, int NP> struct DwPasses {
 // entries together, one each, and hand them round with row broadcasts; then the 16 W chunks
 // are loaded, 256 bytes of a W row per lane group.
 // What bounds it: with dense gradients the W rows' way from the MALL into the L2s (every
-// entry's row is read once, 6 TB/s), with sparse ones the round trips of the longest row. So
+// entry's row is read once, 5.3 to 6.5 TB/s), with sparse ones the round trips of the longest row. So
 // many lane groups are in flight, each with 16 rows of W.
 constexpr int DH_LANES = 16;
 constexpr int DH_WAVES = 4;

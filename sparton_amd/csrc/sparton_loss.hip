@@ -980,7 +980,7 @@ __global__ __launch_bounds__(NT, 2) void loss_score16_kernel(const T* __restrict
 // its own side's columns (the FLOPS term) while the first stages of the GEMM load. No workspace:
 // everything stays in the workgroup.
 // Two workgroups fit a CU, so what bounds it is the latency that a stage does not hide, in turn
-// with the parts' vector arithmetic and the MFMAs (28% of the time for fp16): two stages are in
+// with the parts' vector arithmetic and the MFMAs (25% of the time for fp16): two stages are in
 // flight, from uniform addresses at constant distances, and the sums' and the epilogue's loads
 // are issued all at once. 256 x 512 x 30522 fp16, each with what comes before: parts in place of
 // fp32 MFMAs 273 -> 174 us, two stages 155, uniform addresses and one side a workgroup 128,

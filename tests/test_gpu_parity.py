@@ -1223,6 +1223,41 @@ def test_fp32_large_batch_entries_without_parts(where, device):
     assert torch.equal(r_p.view(torch.int32), r_e.view(torch.int32)) and torch.equal(i_p, i_e)
 
 
+def test_fp32_parts_in_a_graph(device):
+    """A captured fp32 training forward and backward whose input changes between replays, to one with an
+    entry that the bf16 parts do not hold and back: every replay is the eager result, bitwise, with
+    eager work between."""
+    say("fp32 parts in a graph")
+    H, W, b, m, G = make_case("fp32", 4, 64, 384, 3000, True, "int64")
+    good, bad = H.to(device), H.clone()
+    bad[1, 3, 7] = float("inf")
+    bad = bad.to(device)
+    Hd, Wd, bd, md, Gd = good.clone(), W.to(device), b.to(device), m.to(device), G.to(device)
+
+    def step():
+        reps, idx, r32 = torch.ops.sparton.fused_sparton_fwd_train(Hd, Wd, bd, md)
+        return reps, idx, *torch.ops.sparton.fused_sparton_bwd_train(Gd, r32, idx, Hd, Wd, bd, md)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step()
+    for x in (good, bad, good, bad, bad, good):
+        Hd.copy_(x)
+        want = [t.clone() for t in step()]
+        torch.cuda.synchronize()
+        for t in outs:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for t, w in zip(outs, want):
+            assert torch.equal(t.view(torch.int32), w.view(torch.int32))
+
+
 def test_fp32_split_infinite_entries(device):
     """Infinite entries in H and in W under 'high' (the bf16 hi/lo split kernel): reps and
     argmax equal the exact fp32 path's ('highest'), infinities and NaNs included, as long as
